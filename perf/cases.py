@@ -1,0 +1,188 @@
+"""The MoE layer's work as its users have it: which layers, on how many tokens, through which entry points.
+
+An inference layer is a handle and a set of weights that stay for the run, and one call per batch of tokens
+(`MoELayer.forward`, or the `MoE355` module over `torch.ops.moe355.forward`).  A training layer is a `MoE355Train` module:
+forward, then backward from a gradient of its output.  The shapes are those of `cuplayground_amd.workloads`, at the batch
+sizes that decoding, a chunk of a prompt, and a whole prompt bring, and a layer whose dimensions fit no large tile.
+"""
+import math
+
+import torch
+
+from cuplayground_amd import api, torch_op, training
+
+F32, TF32, BF16, FP16, FP8 = "f32", "tf32", "bf16", "fp16", "fp8"
+_DTYPE = {F32: api.DTYPE_F32, TF32: api.DTYPE_TF32, BF16: api.DTYPE_BF16, FP16: api.DTYPE_FP16, FP8: api.DTYPE_FP8}
+_ACT = {"relu": api.ACT_RELU, "gelu": api.ACT_GELU, "swiglu": api.ACT_SWIGLU}
+_GATE = {"softmax": api.GATE_SOFTMAX, "sigmoid": api.GATE_SIGMOID}
+
+
+def _case(S, H, I, E, k, act, dtype, **kw):
+    """capacity: the capacity factor of a layer that drops tokens (0: none is dropped).  zipf: a gate bias that loads the
+    experts like 1 / rank^1.1.  bias: the projections have biases.  entry: which entry point takes the batch."""
+    c = dict(S=S, H=H, I=I, E=E, k=k, act=act, dtype=dtype, gate="softmax", norm=True, capacity=0.0, zipf=False,
+             bias=False, entry="layer")
+    c.update(kw)
+    return c
+
+
+def listed():
+    def named(name, *a, **kw):
+        return dict(_case(*a, **kw), name=name)
+
+    return [
+        # a whole small layer in fp32, where a call is a handful of short launches
+        named("tiny_f32", 128, 256, 512, 8, 1, "gelu", F32, norm=False, capacity=1.0, entry="module"),
+        # one decoding step of 64 sequences, 256 experts with e4m3 weights: the weights of every expert hit, once
+        named("decode_fp8", 64, 7168, 2048, 256, 8, "swiglu", FP8, gate="sigmoid"),
+        # one decoding step of 16 sequences on the large bf16 layer: all its weights for two rows in each
+        named("decode_bf16", 16, 4096, 14336, 8, 2, "swiglu", BF16),
+        # a chunk of a prompt on many small experts: about 90 rows in each, in fp16
+        named("chunk_fp16", 1000, 2048, 1408, 64, 6, "swiglu", FP16, entry="module"),
+        # dimensions that fit no 128-wide tile, an odd number of tokens, biases on every projection
+        named("ragged_bf16", 1777, 1344, 2752, 12, 3, "gelu", BF16, bias=True, gate="sigmoid"),
+        # prompts on layers of increasing size; tokens past an expert's capacity are dropped in the first and the third
+        named("mid_bf16", 4096, 2048, 2048, 16, 2, "gelu", BF16, capacity=1.25),
+        named("mixtral_bf16", 8192, 4096, 14336, 8, 2, "swiglu", BF16),
+        named("finegrained_bf16", 16384, 2048, 1408, 64, 6, "swiglu", BF16, capacity=1.0, zipf=True),
+        # the same large layer with e4m3 weights
+        named("prefill_fp8", 8192, 4096, 14336, 8, 2, "swiglu", FP8),
+        # the reference's own knob file: one expert, fp32
+        named("reference_f32", 8192, 1024, 4096, 1, 1, "relu", F32, norm=False),
+        # a training step: forward, and the gradients of the tokens and of every weight
+        named("train_gelu_bf16", 4096, 2048, 2048, 16, 2, "gelu", BF16, capacity=1.25, entry="train"),
+        named("train_swiglu_bf16", 3000, 2048, 1408, 16, 4, "swiglu", BF16, entry="train"),
+    ]
+
+
+def draw(rng):
+    """One more layer and batch out of the ranges that the listed ones span."""
+
+    def tokens(lo, hi):
+        s = int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+        return s if rng.random() < 0.7 else max(lo, s // 64 * 64)     # most batches are not round numbers
+
+    def dims(lo, hi):
+        return 64 * rng.randint(lo // 64, hi // 64)
+
+    entry = rng.choice(("layer", "module"))
+    kind = rng.choice(("small_f32", "large_f32", "mid", "large", "finegrained", "ragged", "decode_fp8", "prefill_fp8", "train",
+                       "train_f32"))
+    if kind == "small_f32":
+        E = rng.choice((2, 4, 8, 16))
+        return _case(tokens(16, 1024), dims(128, 512), dims(256, 1024), E, rng.randint(1, 2), rng.choice(("relu", "gelu", "swiglu")),
+                     rng.choice((F32, TF32)), entry=entry)
+    if kind == "large_f32":
+        return _case(tokens(256, 8192), 1024, 4096, 1, 1, "relu", F32, norm=False, entry=entry)
+    if kind == "mid":
+        return _case(tokens(8, 8192), 2048, 2048, 16, 2, rng.choice(("gelu", "swiglu")), rng.choice((BF16, FP16)),
+                     capacity=rng.choice((0.0, 1.25)), entry=entry)
+    if kind == "large":
+        return _case(tokens(1, 8000), 4096, 14336, 8, 2, "swiglu", rng.choice((BF16, FP16)), entry=entry)
+    if kind == "finegrained":
+        zipf = rng.random() < 0.5
+        return _case(tokens(8, 16384), 2048, 1408, 64, 6, "swiglu", rng.choice((BF16, FP16)), capacity=1.0 if zipf else 0.0,
+                     zipf=zipf, entry=entry)
+    if kind == "ragged":
+        E = rng.randint(3, 24)
+        return _case(tokens(16, 4096), dims(512, 2048), dims(512, 3072), E, rng.randint(1, 3), rng.choice(("relu", "gelu", "swiglu")),
+                     rng.choice((BF16, FP16)), bias=rng.random() < 0.5, gate=rng.choice(("softmax", "sigmoid")), entry=entry)
+    if kind == "decode_fp8":
+        return _case(tokens(1, 256), 7168, 2048, 256, 8, "swiglu", FP8, gate="sigmoid", entry=entry)
+    if kind == "prefill_fp8":
+        return _case(tokens(1, 6000), 4096, 14336, 8, 2, "swiglu", FP8, entry=entry)
+    E = rng.choice((4, 8, 16))
+    k = rng.randint(1, 4)
+    if kind == "train":
+        return _case(tokens(256, 4096), 128 * rng.randint(8, 16), 128 * rng.randint(8, 20), E, k, rng.choice(("gelu", "swiglu")),
+                     rng.choice((BF16, FP16)), entry="train", capacity=rng.choice((0.0, 1.25)))
+    return _case(tokens(64, 1024), dims(256, 1024), dims(256, 1536), E, min(k, 2), rng.choice(("relu", "gelu", "swiglu")), F32, entry="train")
+
+
+def _config(c):
+    return api.MoEConfig(capacity_factor=c["capacity"] or 1.0, drop_tokens=int(c["capacity"] > 0), expert_top_k=c["k"],
+                         is_training=int(c["entry"] == "train"), hidden_act=_ACT[c["act"]], hidden_size=c["H"],
+                         intermediate_size=c["I"], micro_batch=1, num_experts=c["E"], sequence_len=c["S"],
+                         torch_dtype=_DTYPE[c["dtype"]], gate_fn=_GATE[c["gate"]], norm_topk_prob=int(c["norm"]))
+
+
+def _matrices(c):
+    """(name, rows, columns) of an expert's weight matrices."""
+    m = [("w_up", c["I"], c["H"]), ("w_down", c["H"], c["I"])]
+    return m + [("w_gate", c["I"], c["H"])] if c["act"] == "swiglu" else m
+
+
+def prepare(case, seed):
+    """Tokens N(0, 1), weights N(0, 0.02), rounded once to their storage types; the layer's handle and workspace."""
+    c, cfg = case, _config(case)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    act_dtype = {F32: torch.float32, TF32: torch.float32, FP16: torch.float16}.get(c["dtype"], torch.bfloat16)
+
+    def normal(*shape, std=1.0):
+        return torch.randn(*shape, generator=g, device="cuda").mul_(std)
+
+    x = normal(c["S"], c["H"]).to(act_dtype)
+    if c["entry"] == "train":
+        return {"train": training.MoE355Train(cfg, seed=seed), "x": x.requires_grad_(True),
+                "grad": normal(c["S"], c["H"]).to(act_dtype)}
+    w = {"gate_w": normal(c["E"], c["H"], std=0.02).to(act_dtype)}
+    for name, rows, cols in _matrices(c):
+        if c["dtype"] == FP8:
+            w[name], w["s" + name[1:]] = api.quantize_block128(normal(c["E"], rows, cols, std=0.02))
+        else:
+            w[name] = normal(c["E"], rows, cols, std=0.02).to(act_dtype)
+        if c["bias"]:
+            w["b" + name[1:]] = normal(c["E"], rows, std=0.02).to(act_dtype)
+    if c["zipf"]:
+        rank = torch.randperm(c["E"], generator=g, device="cuda").float() + 1.0
+        p = rank ** -1.1
+        w["gate_bias"] = torch.log(p / p.sum())
+    if c["entry"] == "module":
+        return {"module": torch_op.MoE355.from_packed(cfg, w), "x": x}
+    return {"layer": api.MoELayer(cfg), "weights": w, "x": x}
+
+
+def run(state):
+    if "train" in state:
+        m, x = state["train"], state["x"]
+        m.zero_grad(set_to_none=True)
+        x.grad = None
+        out = m(x)
+        out.backward(state["grad"])
+        return {"out": out.detach(), "x": x.grad, **{n: p.grad for n, p in m.named_parameters()}}
+    if "module" in state:
+        return state["module"](state["x"])
+    return state["layer"].forward(state["x"], state["weights"])
+
+
+def work(case):
+    """Every (token, expert) pair at 2 * rows * columns of each matrix; every matrix of an expert that is expected to be hit
+    read once, the tokens in and out.  A training step: three times the products; the weights and the tokens read, and a
+    gradient of the same size written for each of them, the output and its gradient."""
+    c = case
+    es = 4 if c["dtype"] in (F32, TF32) else 2
+    pairs, E = c["S"] * c["k"], c["E"]
+    if c["capacity"] and c["zipf"]:
+        p = [r ** -1.1 for r in range(1, E + 1)]
+        room, total = math.ceil(c["capacity"] * pairs / E), sum(p)
+        pairs = sum(min(room, min(1.0, c["k"] * v / total) * c["S"]) for v in p)
+    hit = E * (1.0 - (1.0 - c["k"] / E) ** c["S"])
+    elements = len(_matrices(c)) * c["H"] * c["I"]
+    weights = elements * (1.0 + 4.0 / 16384 if c["dtype"] == FP8 else es)
+    router = E * c["H"]
+    tokens = c["S"] * c["H"] * es
+    flops = 2.0 * pairs * elements + 2.0 * c["S"] * router
+    if c["entry"] == "train":
+        return {"bytes": 2.0 * (E * weights + router * es) + 4.0 * tokens, "flops": 3.0 * flops}
+    return {"bytes": hit * weights + router * es + 2.0 * tokens, "flops": flops}
+
+
+def tolerance(case):
+    """About four times the distance from the same layer computed with wider intermediate results (float64; the 16-bit
+    training steps: fp32): fp32 1e-6, fp16 3.6e-4, bf16 2.9e-3, e4m3 weights 4.1e-3; a training step in bf16 up to 5.1e-3
+    (the tokens' gradient, which adds up the most rounded terms), in fp16 an eighth of that."""
+    if case["dtype"] in (F32, TF32):
+        return {"rel": 5e-6}
+    if case["entry"] == "train":
+        return {"rel": 2e-2 if case["dtype"] == BF16 else 2.5e-3}
+    return {"rel": {FP16: 1.5e-3, BF16: 1.2e-2, FP8: 1.6e-2}[case["dtype"]]}

@@ -186,3 +186,61 @@ def tolerance(case):
     if case["entry"] == "train":
         return {"rel": 2e-2 if case["dtype"] == BF16 else 2.5e-3}
     return {"rel": {FP16: 1.5e-3, BF16: 1.2e-2, FP8: 1.6e-2}[case["dtype"]]}
+
+
+def _exact_layer(c, x, w):
+    """The layer in float64, an expert at a time; differentiable in x and every entry of w (w[name][e]: expert e's matrix)."""
+    S, E, k = c["S"], c["E"], c["k"]
+    logits = x @ w["gate_w"].t()
+    if w.get("gate_bias") is not None:
+        logits = logits + w["gate_bias"]
+    idx = logits.detach().topk(k, dim=1).indices
+    scores = torch.softmax(logits, dim=1) if c["gate"] == "softmax" else torch.sigmoid(logits)
+    tw = scores.gather(1, idx)
+    if c["norm"]:
+        tw = tw / tw.sum(1, keepdim=True)
+    room = math.ceil(c["capacity"] * S * k / E) if c["capacity"] else S * k
+    flat = idx.reshape(-1)
+    out = torch.zeros_like(x)
+    for e in range(E):
+        pairs = (flat == e).nonzero().flatten()[:room]      # pairs are numbered token by token; the first ones are kept
+        if pairs.numel() == 0:
+            continue
+
+        def project(rows, name):
+            y = rows @ w["w_" + name][e]().t()
+            return y + w["b_" + name][e] if "b_" + name in w else y
+
+        rows = x.index_select(0, pairs // k)
+        h = project(rows, "up")
+        if c["act"] == "swiglu":
+            h = torch.nn.functional.silu(project(rows, "gate")) * h
+        else:
+            h = torch.nn.functional.gelu(h) if c["act"] == "gelu" else torch.relu(h)
+        out = out.index_add(0, pairs // k, project(h, "down") * tw.reshape(-1)[pairs].unsqueeze(1))
+    return out
+
+
+def exact(case, seed):
+    """What `run` returns for these inputs, from plain torch operations in float64."""
+    c, state = case, prepare(case, seed)
+    if "train" in state:
+        params = {n: p.detach().double().requires_grad_(True) for n, p in state["train"].named_parameters()}
+        x = state["x"].detach().double().requires_grad_(True)
+        w = {n: p if n == "gate_w" else [(lambda m=m: m) for m in p.unbind(0)] for n, p in params.items()}
+        out = _exact_layer(c, x, w)
+        out.backward(state["grad"].double())
+        return {"out": out.detach(), "x": x.grad, **{n: p.grad for n, p in params.items()}}
+    held = state["weights"] if "weights" in state else {n: b for n, b in state["module"].named_buffers() if b is not None}
+    w = {n: v.double() for n, v in held.items() if n.startswith(("gate_", "b_"))}
+
+    def matrix(name, e):
+        m = held[name][e]
+        if c["dtype"] != FP8:
+            return m.double()
+        s = held["s" + name[1:]][e].double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+        return m.view(torch.float8_e4m3fn).double() * s
+
+    for name, _, _ in _matrices(c):
+        w[name] = [(lambda name=name, e=e: matrix(name, e)) for e in range(c["E"])]
+    return _exact_layer(c, state["x"].double(), w)

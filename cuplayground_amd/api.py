@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -162,6 +162,9 @@ def load_library():
     L.moe_act_backward.argtypes = [vp, vp, vp, vp, i64, vp, vp, vp]
     L.moe_bias_grad.argtypes = [vp, vp, vp, vp, i32, vp, vp]
     L.moe_combine_backward.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp]
+    L.moe_dispatch_rows.argtypes = [vp, vp, vp, vp, vp]
+    L.moe_act_forward.argtypes = [vp, vp, vp, vp, vp, vp, vp]
+    L.moe_dispatch_backward.argtypes = [vp, vp, vp, vp, vp, vp]
     L.moe_last_hip_error.argtypes = [vp]
     L.moe_status_string.argtypes = [C.c_int]; L.moe_status_string.restype = C.c_char_p
     L.moe_version.restype = C.c_int
@@ -581,10 +584,34 @@ class MoELayer:
                                     _ptr(db), _stream()), "moe_bias_grad")
         return db
 
-    def combine_backward(self, dout, y_rows, pair_row, topk_w):
-        """(dy_rows with the rows no pair maps to zero, dw [S, k] fp32)."""
+    def dispatch_rows(self, x, token_indices):
+        """x_rows[r] = x[token_indices[r]] for the kept packed rows; the rows behind them are not written."""
         import torch
-        dy = torch.zeros_like(y_rows)
+        rows = torch.empty(self.S * self.k, self.H, dtype=x.dtype, device=x.device)
+        _check(self.L.moe_dispatch_rows(self._h, _ptr(x), _ptr(token_indices), _ptr(rows), _stream()), "moe_dispatch_rows")
+        return rows
+
+    def act_forward(self, u_rows, g_rows, expert_count, expert_offset):
+        """act(u_rows), or silu(g_rows) * u_rows, over the kept packed rows; the rows behind them are not written."""
+        import torch
+        h = torch.empty_like(u_rows)
+        _check(self.L.moe_act_forward(self._h, _ptr(u_rows), _ptr(g_rows), _ptr(expert_count), _ptr(expert_offset), _ptr(h),
+                                      _stream()), "moe_act_forward")
+        return h
+
+    def dispatch_backward(self, da_rows, db_rows, pair_row):
+        """dx[t] = sum over ranks of da_rows[pair_row[t,r]] (+ db_rows[pair_row[t,r]] unless db_rows is None)."""
+        import torch
+        dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
+        _check(self.L.moe_dispatch_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(dx), _stream()),
+               "moe_dispatch_backward")
+        return dx
+
+    def combine_backward(self, dout, y_rows, pair_row, topk_w, dy=None):
+        """(dy_rows, dw [S, k] fp32).  Rows no pair maps to: zero in the buffer made here, untouched in the caller's."""
+        import torch
+        if dy is None:
+            dy = torch.zeros_like(y_rows)
         dw = torch.empty(self.S, self.k, dtype=torch.float32, device=dout.device)
         _check(self.L.moe_combine_backward(self._h, _ptr(dout), _ptr(y_rows), _ptr(pair_row), _ptr(topk_w), _ptr(dy),
                                            _ptr(dw), _stream()), "moe_combine_backward")

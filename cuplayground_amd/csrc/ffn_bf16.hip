@@ -98,27 +98,6 @@ struct TaskPtrs {
     uint16_t* c1_base;           // dg rows (SwiGLU), else null
 };
 
-// silu for a bf16 result: hardware exp2 and reciprocal (about 1 ulp each in fp32, far below the bf16 rounding of
-// the product that follows) instead of the library expf and an IEEE division.
-__device__ __forceinline__ float silu_fast(float g) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
-}
-
-// GELU (exact-erf form) for a bf16 result without the library erff, which costs some 40 instructions and two
-// divergent branches per element: u * Phi(u) with erfc(x) = t (a1 + t (a2 + t (a3 + t (a4 + t a5)))) exp(-x^2),
-// t = 1 / (1 + p x), x = |u| / sqrt 2 (Abramowitz & Stegun 7.1.26, |error| <= 1.5e-7 on erfc).  The error of the
-// result stays below 5e-7 in absolute terms and below one bf16 unit in the last place for |u| < 6.
-__device__ __forceinline__ float gelu_fast(float u) {
-    const float x = fabsf(u) * 0.70710678118654752440f;
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, x, 1.0f));
-    float q = fmaf(1.061405429f, t, -1.453152027f);
-    q = fmaf(q, t, 1.421413741f);
-    q = fmaf(q, t, -0.284496736f);
-    q = fmaf(q, t, 0.254829592f);
-    const float half_erfc = 0.5f * q * t * __builtin_amdgcn_exp2f(x * x * -1.4426950408889634f);
-    return u * (u >= 0.0f ? 1.0f - half_erfc : half_erfc);
-}
-
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // Two fp32 values rounded to the tile's 16-bit storage type (nearest even), and one stored value widened.
@@ -339,7 +318,7 @@ __device__ __forceinline__ void epilogue_impl(const TaskPtrs& p, f32x4 (&acc)[T:
                     float g = acc[i][j][r], u = acc[i][j + TN / 2][r];
                     if (p.bias1) g = g + widen1<T>(p.bias1[col + r]);
                     if (p.bias0) u = u + widen1<T>(p.bias0[col + r]);
-                    v[r] = silu_fast(g) * u;
+                    v[r] = silu16(g) * u;
                 }
                 store8(crow + col, pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), p.publish);
             }
@@ -353,7 +332,7 @@ __device__ __forceinline__ void epilogue_impl(const TaskPtrs& p, f32x4 (&acc)[T:
                 for (int r = 0; r < 4; ++r) {
                     float u = acc[i][j][r];
                     if (p.bias0) u = u + widen1<T>(p.bias0[col + r]);
-                    v[r] = MODE == 2 ? gelu_fast(u) : (u < relu_floor ? relu_floor : u);
+                    v[r] = MODE == 2 ? gelu16(u) : (u < relu_floor ? relu_floor : u);
                 }
                 store8(crow + col, pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), p.publish);
             }
@@ -510,12 +489,12 @@ __device__ __forceinline__ void epilogue_full_n_impl(const TaskPtrs& p, unsigned
             for (int r = 0; r < 4; ++r) {
                 if constexpr (MODE == 3) {
                     const float g = acc[i][j][r] + b1[j][r], u = acc[i][j + NJ][r] + b0[j][r];
-                    v[r] = silu_fast(g) * u;
+                    v[r] = silu16(g) * u;
                 } else {
                     float sum;
                     if constexpr (Parts::KP == 1) sum = acc[i][j][r]; else sum = whole[j][r];
                     const float u = sum + b0[j][r];
-                    v[r] = MODE == 2 ? gelu_fast(u) : (u < relu_floor ? relu_floor : u);
+                    v[r] = MODE == 2 ? gelu16(u) : (u < relu_floor ? relu_floor : u);
                 }
             }
             u32x2 o = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};

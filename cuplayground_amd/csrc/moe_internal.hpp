@@ -135,6 +135,7 @@ struct RouteArgs {
     int32_t* token_indices;     // [A]
     int32_t* expert_count;      // [E]
     int32_t* expert_offset;     // [E+1]
+    int32_t* offset_out;        // null, or a caller's [E] copy of the offsets
     MTile* mtiles;
     Segment* seg_phase0;
     Segment* seg_phase1;
@@ -218,6 +219,12 @@ hipError_t launch_act_backward(const void* dh, const void* u, const void* g, int
                                void* dg, hipStream_t st);
 hipError_t launch_bias_grad(const void* dy, const int32_t* count, const int32_t* offset, int E, int N, int dtype, void* db,
                             hipStream_t st);
+hipError_t launch_act_forward(const void* u, const void* g, const int32_t* count, const int32_t* offset, int E, int64_t A, int I,
+                              int act, int dtype, void* h, hipStream_t st);
+hipError_t launch_dispatch_rows(const void* x, const int32_t* token_indices, int64_t A, int S, int H, int dtype, void* rows,
+                                hipStream_t st);
+hipError_t launch_dispatch_backward(const void* a, const void* b, const int32_t* pair_row, int S, int k, int H, int dtype,
+                                    void* dx, hipStream_t st);
 hipError_t launch_combine_backward(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S,
                                    int k, int H, int dtype, void* dy, float* dw, hipStream_t st);
 

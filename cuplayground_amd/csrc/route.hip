@@ -191,6 +191,7 @@ __device__ __forceinline__ void route_scan_body(const RouteArgs& a, ScanShared& 
     if (e < a.E) {
         a.expert_count[e] = kept;
         a.expert_offset[e] = off;
+        if (a.offset_out) a.offset_out[e] = off;
         write_segment(a.seg_phase0 + e, mt0 * npg0, 0, e, mt0, nmt, a.nnt0, a.groups);
         write_segment(a.seg_phase1 + e, mt0 * npg1, 1, e, mt0, nmt, a.nnt1, a.groups);
     }

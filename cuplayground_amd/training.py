@@ -5,11 +5,11 @@ Here it has a consumer: `MoE355Train` runs the expert projections through `moe_e
 from `moe_expert_gemm` on the transposed weight (data gradient) and `moe_expert_wgrad` (weight gradient).  Routing
 decisions (top-k indices, slots, capacity drops) come from the library's router and are not differentiated; the gate
 weights that scale the expert outputs are recomputed in torch from the same logits formula, so the router's weight
-matrix and the tokens receive gradients through them.  The activation and the down projection are one autograd node
-(`_ActDown`): its backward is `moe_expert_gemm_act_backward` -- the data gradient of the down projection with the
-activation's derivative in the product's epilogue -- where the layer has it, else `moe_expert_gemm` followed by
-`moe_act_backward`.  Gather and the weighted combine are indexing work left to torch's autograd.  There is no CPU path:
-every tensor lives on the GPU.
+matrix and the tokens receive gradients through them.  Everything else -- dispatch, projections, activation, combine --
+is one autograd node (`_Experts`) whose backward runs the library's adjoints; the data gradient of the down projection
+carries the activation's derivative in its epilogue (`moe_expert_gemm_act_backward`) where the layer has that kernel,
+else `moe_expert_gemm` is followed by `moe_act_backward`.  `expert_linear` and `act_down` are the projections as nodes
+of their own, for layers composed in torch.  There is no CPU path: every tensor lives on the GPU.
 """
 from __future__ import annotations
 
@@ -82,6 +82,71 @@ def act_down(u_rows, g_rows, w_down, layer: api.MoELayer, expert_count, expert_o
                           expert_count, expert_offset)
 
 
+def _aligned(t):
+    """t, contiguous and at a 16-byte address (the row passes read 16 bytes at a time)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+class _Experts(torch.autograd.Function):
+    """(x [S,H], expert weights, topk_w [S,k]) -> the gate-weighted sum of the chosen experts' outputs.
+
+    The whole expert side of a training step as one node over packed rows: rows of no expert are never read, so no buffer
+    is cleared, and dispatch, activation, combine and their adjoints are one pass each."""
+
+    @staticmethod
+    def forward(ctx, x, w_up, w_gate, w_down, topk_w, layer, token_indices, pair_row, count, offset):
+        w_up, w_down, topk_w = w_up.contiguous(), w_down.contiguous(), topk_w.contiguous()
+        rows = layer.dispatch_rows(_aligned(x), token_indices)
+
+        def product(a, w):
+            out = torch.empty(a.shape[0], w.shape[1], dtype=a.dtype, device=a.device)
+            return layer.expert_gemm(a, w, None, count, offset, api.ACT_NONE, out=out)
+
+        u = product(rows, w_up)
+        g = None
+        if w_gate is not None:
+            w_gate = w_gate.contiguous()
+            g = product(rows, w_gate)
+        h = layer.act_forward(u, g, count, offset)
+        y = product(h, w_down)
+        ctx.save_for_backward(rows, u, g, h, y, w_up, w_gate, w_down, topk_w, pair_row, count, offset)
+        ctx.layer = layer
+        return api.combine(y, pair_row, topk_w)
+
+    @staticmethod
+    def backward(ctx, dout):
+        rows, u, g, h, y, w_up, w_gate, w_down, topk_w, pair_row, count, offset = ctx.saved_tensors
+        layer = ctx.layer
+        need_x, need_up, need_gate, need_down = ctx.needs_input_grad[:4]
+
+        def product(a, w_t):
+            out = torch.empty(a.shape[0], w_t.shape[1], dtype=a.dtype, device=a.device)
+            return layer.expert_gemm(a, w_t, None, count, offset, api.ACT_NONE, out=out)
+
+        dy, dtopk = layer.combine_backward(_aligned(dout), y, pair_row, topk_w, dy=torch.empty_like(y))
+        dx = dup = dgate = ddown = None
+        if need_down:
+            ddown = layer.expert_wgrad(dy, h, count, offset)
+        if need_x or need_up or need_gate:
+            w_t = api.transpose(w_down)                                                            # [E, I, H]
+            if layer.fused_act_backward:
+                du, dg = layer.expert_gemm_act_backward(dy, w_t, u, g, count, offset, du=torch.empty_like(u),
+                                                        dg=None if g is None else torch.empty_like(g))
+            else:
+                du, dg = layer.act_backward(product(dy, w_t), u, g)                                # dH = dY . W_down
+            del w_t
+            if need_x:
+                da = product(du, api.transpose(w_up))                                              # dA = dU . W_up
+                db = None if g is None else product(dg, api.transpose(w_gate))
+                dx = layer.dispatch_backward(da, db, pair_row)
+            if need_up:
+                dup = layer.expert_wgrad(du, rows, count, offset)                                  # dW[e] = dU_e^T . A_e
+            if need_gate:
+                dgate = layer.expert_wgrad(dg, rows, count, offset)
+        return dx, dup, dgate, ddown, dtopk, None, None, None, None, None
+
+
 class MoE355Train(torch.nn.Module):
     """forward(x [S,H]) -> [S,H] with gradients for x, gate_w, w_up, w_gate and w_down."""
 
@@ -119,14 +184,6 @@ class MoE355Train(torch.nn.Module):
         c = self.cfg
         idx, r = self.route(x)
         count, offset = r["expert_count"], r["expert_offset"]
-        tok = r["token_indices"].clamp(min=0).long()      # rows past the last kept one gather token 0 and are never used
-        x_rows = x.index_select(0, tok)
-        up = expert_linear(x_rows, self.w_up, self.layer, count, offset)
-        gate = expert_linear(x_rows, self.w_gate, self.layer, count, offset) if c.hidden_act == api.ACT_SWIGLU else None
-        y = act_down(up, gate, self.w_down, self.layer, count, offset)
         w = self.gate_weights(x, idx)
-        rows = r["pair_row"]
-        kept = (rows >= 0).unsqueeze(-1)
-        picked = y.index_select(0, rows.clamp(min=0).reshape(-1).long()).reshape(c.tokens, c.expert_top_k, -1)
-        out = (torch.where(kept, picked.float(), torch.zeros((), device=x.device)) * w.unsqueeze(-1)).sum(1)
-        return out.to(x.dtype)
+        return _Experts.apply(x, self.w_up, self.w_gate, self.w_down, w, self.layer, r["token_indices"], r["pair_row"],
+                              count, offset)

@@ -437,6 +437,18 @@ int moe_bias_grad(moe_handle* h, const void* dy_rows, const int32_t* expert_coun
                   void* db, void* stream);
 int moe_combine_backward(moe_handle* h, const void* dout, const void* y_rows, const int32_t* pair_row, const float* topk_w,
                          void* dy_rows, float* dw, void* stream);
+/* The passes of a training step that the fused forward keeps inside its tiles, and the adjoint of the dispatch.  All row
+ * buffers are 16-byte aligned (else MOE_ERR_BAD_ARGUMENT); rows that belong to no expert are neither read nor written.
+ * moe_dispatch_rows: x_rows[r, :H] = x[token_indices[r], :] for every kept packed row r (token_indices as moe_route wrote
+ *   it: negative behind the last kept row).
+ * moe_act_forward: h_rows = act(u_rows), or silu(g_rows) * u_rows (g_rows exactly when the layer is SwiGLU), width I.
+ * moe_dispatch_backward: dx[t, :] = sum over ranks r, ascending, of da_rows[pair_row[t,r], :] (+ db_rows[pair_row[t,r], :]
+ *   when db_rows is not null), dropped pairs skipped. */
+int moe_dispatch_rows(moe_handle* h, const void* x, const int32_t* token_indices, void* x_rows, void* stream);
+int moe_act_forward(moe_handle* h, const void* u_rows, const void* g_rows, const int32_t* expert_count,
+                    const int32_t* expert_offset, void* h_rows, void* stream);
+int moe_dispatch_backward(moe_handle* h, const void* da_rows, const void* db_rows, const int32_t* pair_row, void* dx,
+                          void* stream);
 
 int moe_last_hip_error(const moe_handle* h);
 const char* moe_status_string(int status);

@@ -63,3 +63,56 @@ def test_e4m3_layers_are_refused(moe):
     with pytest.raises(ValueError):
         training.MoE355Train(moe.MoEConfig(hidden_size=128, intermediate_size=128, micro_batch=1, sequence_len=128,
                                            torch_dtype=4))
+
+
+@pytest.mark.parametrize("dtype", [0, 2, 3])
+@pytest.mark.parametrize("S,H,I,E,k,act,cf", [(1, 64, 64, 2, 1, 0, 1.0), (37, 512, 128, 3, 2, 1, 0.6), (130, 576, 192, 5, 5, 2, 0.8),
+                                              (513, 1088, 64, 8, 6, 2, 1.0)])
+def test_row_passes_match_plain_torch(moe, S, H, I, E, k, act, cf, dtype):
+    """Dispatch, activation, the adjoint of the dispatch and of the combine, over kept and dropped pairs: one rounding to
+    the storage type behind fp32 arithmetic (2 ulp of it: the reference rounds the same fp64 value once)."""
+    import torch
+    cfg = moe.MoEConfig(capacity_factor=cf, drop_tokens=1, expert_top_k=k, hidden_act=act, hidden_size=H, intermediate_size=I,
+                        micro_batch=1, num_experts=E, sequence_len=S, torch_dtype=dtype, gate_fn=0, norm_topk_prob=1)
+    layer = moe.MoELayer(cfg)
+    dt = layer.act_dtype
+    g = torch.Generator(device="cuda").manual_seed(S + H)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(dt)
+
+    idx = torch.stack([torch.randperm(E, generator=g, device="cuda")[:k] for _ in range(S)]).int()
+    r = layer.route(idx)
+    kept, pr = int(r["expert_count"].sum()), r["pair_row"].long()
+    tok = r["token_indices"][:kept].long()
+    eps = {0: 2e-6, 2: 2.0 ** -7, 3: 2.0 ** -10}[dtype]
+
+    def close(a, b, scale=1.0):
+        a, b = a.double(), b.double()
+        return bool(((a - b).abs() <= eps * b.abs() + scale * (1e-6 if dtype else 2e-6)).all())
+
+    x = normal(S, H)
+    assert torch.equal(layer.dispatch_rows(x, r["token_indices"])[:kept], x[tok])
+    u, gt = normal(S * k, I), normal(S * k, I) if act == 2 else None
+    h = layer.act_forward(u, gt, r["expert_count"], r["expert_offset"])[:kept]
+    ud = u[:kept].double()
+    want = torch.nn.functional.silu(gt[:kept].double()) * ud if act == 2 else torch.nn.functional.gelu(ud) if act == 1 else torch.relu(ud)
+    assert close(h, want)
+    a, b = normal(S * k, H), normal(S * k, H)
+    on = (pr >= 0).unsqueeze(-1).double()
+    pick = lambda t: t.double()[pr.clamp(min=0)] * on
+    assert close(layer.dispatch_backward(a, None, r["pair_row"]), pick(a).sum(1), scale=k)
+    assert close(layer.dispatch_backward(a, b, r["pair_row"]), (pick(a) + pick(b)).sum(1), scale=2 * k)
+    w = torch.rand(S, k, generator=g, device="cuda")
+    dy, dw = layer.combine_backward(x, a, r["pair_row"], w)
+    want_dy = torch.zeros(S * k, H, dtype=torch.float64, device="cuda")
+    flat = pr.reshape(-1)
+    want_dy[flat[flat >= 0]] = (w.double().unsqueeze(-1) * x.double().unsqueeze(1)).reshape(S * k, H)[flat >= 0]
+    assert close(dy, want_dy)
+    want_dw = (pick(a) * x.double().unsqueeze(1)).sum(-1)
+    assert float((dw.double() - want_dw).abs().max()) <= 1e-6 * H       # fp32 sums of H products of order 1
+    # operands that are not 16-byte aligned take the element-wise kernel, with the same dy
+    pad = torch.zeros(S * H + 1, dtype=dt, device="cuda")
+    pad[1:] = x.reshape(-1)
+    dy2, dw2 = layer.combine_backward(pad[1:].view(S, H), a, r["pair_row"], w)
+    assert torch.equal(dy2, dy) and float((dw2.double() - want_dw).abs().max()) <= 1e-6 * H

@@ -138,7 +138,7 @@ WsLayout layout(const Derived& d) {
     w.done1 = take((size_t)d.max_mtiles * 4);
     w.pair_mt = take((size_t)d.A * 4);
     w.wg_clock = take((size_t)kMaxQueueWorkgroups * 2 * sizeof(int64_t));
-    w.arrive = take((size_t)d.S * d.plan.nnt1 * 4);
+    w.arrive = take((size_t)d.S * std::max(d.plan.nnt1, ceil_div(d.H, 128)) * 4);   // no smaller for a plan with wider column tiles
     w.stats_prob = take((size_t)kStatsBlocks * d.E * 8);
     w.stats_cnt = take((size_t)kStatsBlocks * d.E * 4);
     w.h = take((size_t)d.A * d.I * d.act_bytes);
@@ -360,6 +360,10 @@ int resolved_ffn_mode(const moe_handle* h) {
     // against 1.03-1.10 ms as two launches; the same file in bf16 0.183 against 0.170 ms; the Mixtral dimensions with one
     // expert: no difference).
     const bool tile16 = d.plan.kernel_dtype == MOE_DTYPE_BF16 || d.plan.kernel_dtype == MOE_DTYPE_FP16;
+    // The 128 x 128 tile of the general loop stores its rows in 8-byte pieces straight from the accumulators: written
+    // through, as the queue needs them, they cost it more than the overlap gives at every size measured (12 experts of
+    // 1344 x 2752, 444 rows each: 233 against 199 us; 8 of 4096 x 14336, 4 rows 775 / 631, 375 rows 2087 / 1424).
+    if (tile16 && d.plan.tile == 0) return MOE_FFN_TILED;
     if ((f32_tile || tile16) && d.E == 1) return MOE_FFN_TILED;
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }

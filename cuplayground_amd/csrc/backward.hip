@@ -17,7 +17,8 @@
 
 namespace moe355 {
 
-bool grouped_gemm_takes_large_tile(int64_t A, int E, int N, int K);
+bool grouped_hand_ok(int64_t A, int N, int K);
+int grouped_gemm_tile_16(int64_t A, int E, int N, int K);
 hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const MTile* mtiles,
                                   const int32_t* num_mtiles, const int32_t* count, int max_mtiles, int tile, int64_t A,
                                   int N, int K, int act, bool f16, hipStream_t st);
@@ -548,11 +549,10 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
         return (mfma ? launch_grouped_gemm_f32_tile : launch_grouped_gemm_f32)(a_rows, w, bias, out_rows, t.mtiles,
                                                                                t.num_mtiles, max_mtiles, N, K, act, st);
     }
-    int tile = grouped_gemm_takes_large_tile(A, E, N, K) ? 1 : 0;     // 1: 256 x 256, 0: 128 x 128
-    if (opt.grouped_tile != MOE_OPT_AUTO) {                            // option; 2: 128 x 256 (hand-ordered)
+    int tile = grouped_gemm_tile_16(A, E, N, K);                       // 1: 256 x 256, 2: 128 x 256, 0: 128 x 128
+    if (opt.grouped_tile != MOE_OPT_AUTO) {
         const int v = opt.grouped_tile;
-        const int64_t lim = (int64_t)1 << 32;
-        if ((v == 1 || v == 2) && N % 256 == 0 && K % 128 == 0 && A * K * 2 < lim && (int64_t)N * K * 2 < lim) tile = v;
+        if ((v == 1 || v == 2) && grouped_hand_ok(A, N, K)) tile = v;
         if (v == 0) tile = 0;
     }
     const int block_m = tile == 1 ? 256 : 128;
@@ -568,15 +568,12 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
 // when the shape or the options leave only the 128 x 128 tile, which has no such epilogue.
 int expert_gemm_dact_tile(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
     if (dtype != MOE_DTYPE_BF16 && dtype != MOE_DTYPE_FP16) return 0;
-    int tile = grouped_gemm_takes_large_tile(A, E, N, K) ? 1 : 0;
-    const int64_t lim = (int64_t)1 << 32;
-    const bool hand_ok = N % 256 == 0 && K % 128 == 0 && A * K * 2 < lim && (int64_t)N * K * 2 < lim;
+    const bool hand_ok = N % 256 == 0 && K % 128 == 0 && grouped_hand_ok(A, N, K);
+    int tile = hand_ok ? grouped_gemm_tile_16(A, E, N, K) : 0;
     if (opt.grouped_tile != MOE_OPT_AUTO) {
         const int v = opt.grouped_tile;
         if ((v == 1 || v == 2) && hand_ok) tile = v;
         if (v == 0) tile = 0;
-    } else if (tile == 0 && hand_ok) {
-        tile = 2;      // few rows per expert: the 128-row hand-ordered tile rather than no fusion at all
     }
     return tile;
 }

@@ -13,10 +13,10 @@
 //   * dispatch is fused into the A-tile load: phase 0 gathers token rows through token_indices[];
 //   * SwiGLU pairs gate and up columns inside one wavefront (first half of its tile rows from w_gate, second
 //     half from w_up), so silu(g)*u happens in registers.
-// Two plans.  "Large": 256-row blocks, 256 x 256 tiles for both projections, four wavefronts of 128 x 128 with the
-// slab loop ordered by hand (gemm_tile_ring) and an epilogue staged through LDS; chosen when experts see many rows
-// and every tile of the layer meets that loop's conditions (large_tile_ok).  "Small": 128 x 128 tiles, four
-// wavefronts of 64 x 64, compiler-scheduled loop (mainloop_generic), general epilogue; takes everything else.
+// Plans: "large", 256-row blocks and 256 x 256 tiles, four wavefronts of 128 x 128; "medium", 128-row blocks and 128 x 256
+// tiles, four wavefronts of 128 x 64; both with the slab loop ordered by hand (gemm_tile_ring) and an epilogue staged
+// through LDS, for operands below 4 GiB, chosen by bf16_tile.  "Small": 128 x 128 tiles, four wavefronts of 64 x 64,
+// compiler-scheduled loop (mainloop_generic), general epilogue; takes everything else.
 #include <type_traits>
 
 #include "ffn_common.hpp"
@@ -347,7 +347,7 @@ __device__ __forceinline__ void epilogue(const TaskPtrs& p, f32x4 (&acc)[T::TM][
     else epilogue_impl<T, 0>(p, acc);
 }
 
-// The epilogue of a tile that is not ragged in N (rows may be), staged through LDS.
+// The epilogue of the hand-ordered tiles, staged through LDS.
 //
 // In the accumulator layout the 16 lanes that are neighbours in the wavefront hold 16 different rows, so a store
 // straight from the registers writes 64 separate 8-byte pieces per instruction.  Each wavefront therefore writes its
@@ -416,13 +416,13 @@ __device__ __forceinline__ void epilogue_full_n_impl(const TaskPtrs& p, unsigned
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) b0[j][r] = widen1<T>(p.bias0[col0 + 16 * j + 4 * fk + r]);
+            for (int r = 0; r < 4; ++r) b0[j][r] = widen1<T>(p.bias0[min(col0 + 16 * j + 4 * fk, p.N - 4) + r]);
     }
     if (MODE == 3 && p.bias1) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) b1[j][r] = widen1<T>(p.bias1[col0 + 16 * j + 4 * fk + r]);
+            for (int r = 0; r < 4; ++r) b1[j][r] = widen1<T>(p.bias1[min(col0 + 16 * j + 4 * fk, p.N - 4) + r]);
     }
     // MODE 0: u below the floor becomes the floor.  Written as a compare and select, not as fmaxf: a max returns its
     // other operand for a NaN, and a NaN must stay a NaN (the reference's __hfma_relu propagates it too, processor/tiling.cuh:45,54)
@@ -431,7 +431,9 @@ __device__ __forceinline__ void epilogue_full_n_impl(const TaskPtrs& p, unsigned
     unsigned char* wr = stage + frow * PITCH + fk * 8;
     const int rd_row = lane / LANES_PER_ROW, rd_chunk = lane % LANES_PER_ROW;
     const unsigned char* rd = stage + rd_row * PITCH + rd_chunk * 16;
-    const int rows_left = p.rows - wm * 128 - rd_row;                 // this lane stores row r0 + rd_row when r0 < rows_left
+    // this lane stores row r0 + rd_row when r0 < rows_left; none if its eight columns lie behind the last one (N is a
+    // multiple of 64, so they do together or not at all)
+    const int rows_left = col0 + rd_chunk * 8 < p.N ? p.rows - wm * 128 - rd_row : 0;
     const uint32_t lane_off = (uint32_t)(rd_row * p.N + col0 + rd_chunk * 8);   // elements from the uniform row pointer
     const bool publish = p.publish;
     constexpr int NQ = 16 / ROWS_PER_PASS;
@@ -557,19 +559,6 @@ __device__ __forceinline__ void epilogue_full_n(const TaskPtrs& p, unsigned char
     else epilogue_full_n_impl<T, 0>(p, smem, acc, between);
 }
 
-// The slab loop of a full 256 x 256 tile on four wavefronts of 128 x 128, with the instruction order fixed by hand.
-//
-// Why not the compiler's order: with one wavefront per SIMD nothing else hides a stall, and the global->LDS loads of
-// a slab (64 KB per compute unit) need more than one slab of flight time to stream in at the rate the L2 delivers.
-// So (a) both k halves of a slab's fragments are double buffered in registers, which frees the slab's LDS stage at
-// mid-slab, (b) the loads of slab kt+2 are issued into that stage right away, two per MFMA row, and stay in flight
-// across the barriers (bare s_barrier: a __syncthreads() would wait for them), (c) MFMAs, LDS reads and their
-// s_waitcnt are inline asm in the order written by gen_slab_schedule.py (ffn_bf16_slab_steady.inc); the compiler places
-// nothing between them but the scalar address updates of the loads.  The accumulators are tied asm operands in
-// AGPRs, so they stay put for the whole loop.  Loads use buffer addressing: a 32-bit byte offset per row, computed
-// once per task, plus a scalar k offset -- no vector ALU instruction is left in the loop.
-// Takes partial row blocks too (the whole tile is computed, rows past the end are not stored).
-// Needs: K a multiple of 128, a tile that is not ragged in N, operand extents below 4 GiB.
 // What the loads of one task of the hand-ordered tile need; computed once per task (ring_prepare).
 struct RingLoads {
     unsigned voff_a[8], voff_b[8];   // byte offsets of this thread's eight token rows / weight rows (row + 16-byte chunk)
@@ -577,7 +566,7 @@ struct RingLoads {
     const void* base_b0;
     const void* base_b1;
     uint32_t a_extent, b_extent;
-    int KT;                          // slabs of 64: even, >= 2
+    int KT;                          // slabs of 64, >= 1
     int wrow;                        // first of the eight consecutive stage rows this wavefront's loads fill per pass
 };
 
@@ -599,6 +588,7 @@ __device__ __forceinline__ RingLoads ring_prepare_weights(const TaskPtrs& p) {
         // SwiGLU: a wavefront's weight rows are the gate rows of its output columns followed by their up rows
         const int j = prow + n * T::ROWS_PER_PASS;
         const int col = p.swiglu ? p.n0 + (j / T::WB) * (T::WB / 2) + (j % (T::WB / 2)) : p.n0 + j;
+        // (columns behind the last one of a ragged tile lie behind the end of the matrix, hence of the buffer)
         L.voff_b[n] = (unsigned)(((int64_t)col * p.b_ld + chunk * 8) * 2);
     }
     auto uniform = [](const void* q) {          // the bases are the same in every lane; say so, or each load loops over lanes
@@ -700,7 +690,9 @@ __device__ __forceinline__ void ring_first_loads(const RingLoads& L, unsigned ch
 // AGPRs, so they stay put for the whole loop.  Loads use buffer addressing: a 32-bit byte offset per row, computed
 // once per task, plus a scalar k offset -- no vector ALU instruction is left in the loop.
 // Takes partial row blocks too (the whole tile is computed, rows past the end are not stored).
-// Needs: K a multiple of 128, a tile that is not ragged in N, operand extents below 4 GiB.
+// Needs: K a multiple of 64 (an odd number of slabs runs one slab of zeros: the loads of slab KT go through descriptors of
+// zero length), N a multiple of 64 (columns behind the last one are loaded as zeros and not stored), operand extents
+// below 4 GiB.
 // On entry the loads of slabs 0 and 1 (ring_first_loads, in that order) are the 32 youngest vector loads of this
 // wavefront (stores issued behind them only make the first wait more conservative).  Returns false for a wavefront whose 128 rows are all
 // padding: it has taken part in the loads and barriers only and holds no results.
@@ -722,7 +714,7 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
         U.a_extent = uni(L.a_extent); U.b_extent = uni(L.b_extent);
         U.KT = (int)uni((unsigned)L.KT); U.wrow = (int)uni((unsigned)L.wrow);
     }
-    const int KT = U.KT;
+    const int KT = U.KT;                        // an odd one runs one slab more, on the zeros that its loads fetch
     auto load_one = [&](int slab, int n) { ring_load_one<T>(U, smem, slab, n); };
 
 #pragma unroll
@@ -1525,39 +1517,51 @@ int occupancy() {
 
 }  // namespace
 
-// Row-block height chosen for a layer: 256 when the average expert sees at least 256 rows and the up
-// projection still gives every compute unit a task at that size.
-//
-// The 256-row tile runs the hand-ordered slab loop only, which needs: K a multiple of 128 in both projections, no
-// ragged column tile (the SwiGLU tile covers 128 intermediate columns, the others 256), and operands below 4 GiB
-// (32-bit buffer offsets; `pairs` bounds the token count).
-static bool large_tile_ok(int64_t pairs, int H, int I, bool swiglu) {
-    const int64_t lim = (int64_t)1 << 32;
-    return H % 256 == 0 && I % (swiglu ? 128 : 256) == 0 && pairs * H * 2 < lim && pairs * I * 2 < lim &&
-           (int64_t)H * I * 2 < lim;
+// The hand-ordered slab loop needs 32-bit buffer offsets: operands below 4 GiB (`pairs` bounds the token count), and for
+// the weights also the columns behind the last one that a ragged tile reaches.  Dimensions are multiples of 64
+// (moe_config_validate).
+constexpr int64_t kBufferLimit = (int64_t)1 << 32;
+static bool hand_weights_ok(int64_t N, int64_t K) { return (N + 256) * K * 2 < kBufferLimit; }
+static bool large_tile_ok(int64_t pairs, int H, int I) {
+    return pairs * H * 2 < kBufferLimit && pairs * I * 2 < kBufferLimit && hand_weights_ok(H, I) && hand_weights_ok(I, H);
 }
 
-// Tile of a layer: 0 = 128 x 128, 1 = 256 x 256, 2 = 128 x 256, 3 = 256 x 256 with the 128 x 256 tile for the row
-// blocks of at most 128 rows.  1 where its conditions hold and the layer has enough rows, else 0; 2 and 3 are tuning
-// knobs (option tile16).
+// Which hand-ordered tile a grouped product runs on: the 256 x 256 one or the 128 x 256 one.
 //
-// Measured (FFN stage, one box, alternating runs): the 128 x 256 tile reaches 93 % of the 256 x 256 tile's rate on a
-// plain 4096 x 8192 x 4096 GEMM, but as the tile of a whole layer it loses everywhere (Mixtral shape 5.48 against
-// 4.26 ms, 16 experts of 512 rows 0.209 against 0.187 ms, 64 small experts 0.72 against 0.59 ms): twice the tasks,
-// each with the same 12 us between two slab loops.  As the tile of short last blocks only it is no better either
-// (Mixtral shape 4.38 against 4.26 ms, 16 experts 0.198 against 0.190 ms, 64 small experts 0.590 against 0.592 ms):
-// such a task runs through K faster than the full blocks that share its weight tile, drops out of their lockstep
-// and fetches its weights past the L2 on its own, with half the time per slab to hide that latency in (with a
-// routing that leaves no partial blocks both kernels take the same time).
+// The larger tile reads its operands half as often; the smaller one pads less behind an expert's last row and spreads few
+// rows over more compute units.  The estimate behind the choice, per projection: row blocks an expert is expected to have
+// (rows / height and a half, one if the expert's rows hardly ever reach the height) x column tiles, in rounds over the
+// compute units (at least one, and half a round of tail), x the time of a task: 1.3 us a slab + 10 us for 256 x 256,
+// 1.1 us + 3 us for 128 x 256 (cold weights; fill of the first slabs, epilogue and queue overhead in the constant).
+// Measured, whole layer, 256 x 256 / 128 x 256 / the 128 x 128 tile of the general loop (better of queue and launches):
+//   12 experts of 1344 x 2752, GELU: 150 rows each 127 / 112 / 115 us, 444 176 / 168 / 199, 1000 269 / 293 / 350
+//   12 experts of 704 x 1152, SwiGLU, 296 rows 107 / 81 / 87;  5 of 1856 x 2112, 200 rows 108 / 78 / 87
+//   64 experts of 2048 x 1408, SwiGLU: 93 rows 301 / 279 / 303, 281 492 / 552 / 611
+//   8 experts of 4096 x 14336, SwiGLU: 128 rows 775 / 728 / 804, 250 843 / 944 / 1118, 375 1035 / 1252 / 1424
+//   16 experts of 2048 x 2048, GELU: 125 rows 133 / 115 / 129, 250 158 / 175 / 195
+// The general loop is the fastest of the three at none of them.
+static double projection_cost(bool large, int64_t pairs, int experts, int column_tiles, int K) {
+    const double rows = (double)pairs / experts, height = large ? 256 : 128;
+    const double blocks = experts * (rows <= 0.75 * height ? 1.0 : rows / height + 0.5);
+    const double rounds = blocks * column_tiles / 256;
+    const double slabs = (K + kBK - 1) / kBK;
+    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * (large ? 1.3 * slabs + 10.0 : 1.1 * slabs + 3.0);
+}
+static int columns256(int N) { return (N + 255) / 256; }
+
+// Tile of a layer: 0 = 128 x 128 on the general loop (operands of 4 GiB and more), 1 = 256 x 256, 2 = 128 x 256,
+// 3 = 256 x 256 with the 128 x 256 tile for the row blocks of at most 128 rows (option tile16 only).
 int bf16_tile(int64_t pairs, int experts, int H, int I, int swiglu, int opt_block_rows, int opt_tile) {
-    if (!large_tile_ok(pairs, H, I, swiglu != 0)) return 0;
-    const int up_columns = swiglu ? 2 * I : I;
-    if (opt_block_rows == 128 || opt_block_rows == 256) return opt_block_rows == 256 ? 1 : 0;   // option block_rows ...
-    if (opt_tile >= 0 && opt_tile <= 3) return opt_tile;                                        // ... or tile16
-    const int64_t per_expert = pairs / (experts > 0 ? experts : 1);
-    if (per_expert < 256) return 0;
-    const int64_t tasks = (pairs / 256) * ((up_columns + Tile256::BN - 1) / Tile256::BN);
-    return tasks >= 256 ? 1 : 0;
+    if (!large_tile_ok(pairs, H, I)) return 0;
+    // option block_rows: 256 means the 256 x 256 tile where it is not ragged in either projection ...
+    if (opt_block_rows == 128 || opt_block_rows == 256)
+        return opt_block_rows == 256 && H % 256 == 0 && I % (swiglu ? 128 : 256) == 0 ? 1 : 0;
+    if (opt_tile >= 0 && opt_tile <= 3) return opt_tile;      // ... or tile16
+    const int E = experts > 0 ? experts : 1;
+    auto cost = [&](bool large) {
+        return projection_cost(large, pairs, E, columns256(swiglu ? 2 * I : I), H) + projection_cost(large, pairs, E, columns256(H), I);
+    };
+    return cost(true) <= cost(false) ? 1 : 2;
 }
 int bf16_block_m(int tile) { return tile == 1 || tile == 3 ? 256 : 128; }
 int bf16_block_n0(int tile) { return tile == 0 ? SmallPlan::T0::BN : 256; }
@@ -1629,9 +1633,12 @@ hipError_t launch_gemm_dense_bf16(const void* A, const void* B, const void* bias
 }
 
 // ---- building blocks of the backward pass (callers: csrc/backward.hip) ----
-bool grouped_gemm_takes_large_tile(int64_t A, int E, int N, int K) {
-    const int64_t lim = (int64_t)1 << 32;
-    return N % 256 == 0 && K % 128 == 0 && A * K * 2 < lim && (int64_t)N * K * 2 < lim && A / (E > 0 ? E : 1) >= 256;
+bool grouped_hand_ok(int64_t A, int N, int K) { return A * K * 2 < kBufferLimit && hand_weights_ok(N, K); }
+// Tile of one grouped product, as for a layer: 1, 2, or 0 when an operand has 4 GiB or more.
+int grouped_gemm_tile_16(int64_t A, int E, int N, int K) {
+    if (!grouped_hand_ok(A, N, K)) return 0;
+    const int e = E > 0 ? E : 1;
+    return projection_cost(true, A, e, columns256(N), K) <= projection_cost(false, A, e, columns256(N), K) ? 1 : 2;
 }
 
 template <class T>
@@ -1703,8 +1710,7 @@ static hipError_t launch_wgrad(const void* dyT, const void* aT, void* dw, const 
 
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
                            int64_t ld, bool f16, hipStream_t st) {
-    const int64_t lim = (int64_t)1 << 32;
-    const bool large = N >= 1024 && K >= 1024 && K % 256 == 0 && N * ld * 2 < lim && K * ld * 2 < lim;
+    const bool large = N >= 1024 && K >= 1024 && hand_weights_ok(N, ld) && hand_weights_ok(K, ld);
     if (large) return f16 ? launch_wgrad<LargePlanH::T0>(dyT, aT, dw, poff, E, N, K, ld, st)
                           : launch_wgrad<LargePlan::T0>(dyT, aT, dw, poff, E, N, K, ld, st);
     return f16 ? launch_wgrad<SmallPlanH::T0>(dyT, aT, dw, poff, E, N, K, ld, st)

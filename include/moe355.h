@@ -105,8 +105,8 @@ typedef struct moe_handle moe_handle;
  * (CMakeLists.txt:204-216), and chooses tiles and schedulers at compile time (processor/tiling.cuh:97-159,
  * scheduling.cuh:170-200 against warpScheduler.cuh:167-265); these are the same choices as run-time values of a handle.
  * Every field is MOE_OPT_AUTO (the library chooses) or one of the values named beside it; a value outside its domain
- * makes moe_create_with_options return MOE_ERR_BAD_ARGUMENT, a value the layer's shape cannot take (the 256-row tile on
- * a layer with H % 256 != 0, say) falls back to the library's choice.  Results never depend on these options beyond
+ * makes moe_create_with_options return MOE_ERR_BAD_ARGUMENT, a value the layer's shape cannot take (block_rows = 256
+ * on a layer with H % 256 != 0, say) falls back to the library's choice.  Results never depend on these options beyond
  * what is said here: schedules and tiles of one dtype agree bit for bit except where a field says otherwise.
  * Options are fixed when the handle is created; two handles of one process may differ in every one of them.
  */
@@ -114,7 +114,8 @@ typedef struct moe_handle moe_handle;
 typedef struct moe_options {
     int32_t tile16;          /* bf16 / fp16 layers: 0 = 128x128 tile, 1 = 256x256 (hand-ordered), 2 = 128x256 (hand-ordered),
                                 3 = 256x256 with the 128x256 tile for row blocks of at most 128 rows */
-    int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1) */
+    int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1; 256 needs
+                                H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0) */
     int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile; also read by the
                                 backward entry points of an fp32 handle (there 1 means "where the shape allows") */
     int32_t fp8_tile;        /* e4m3 layers: 0 = weight streamer (decode), 1 = 128x128 tile GEMM */

@@ -51,6 +51,7 @@ CASES = [  # S, H, I, E, k, capacity factor, router skew
     (512, 128, 320, 4, 1, 2.0, 0.7),        # skewed: one expert takes most rows, one may stay empty
     (2048, 512, 1024, 4, 2, 1.25, 0.0),     # 256-row blocks in the grouped product
     (1024, 1024, 1024, 2, 2, 2.0, 0.0),     # 256 x 256 tiles in the weight gradient as well
+    (700, 1088, 1216, 2, 1, 2.0, 0.2),      # the same, ragged in both dimensions
 ]
 
 

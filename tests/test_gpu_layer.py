@@ -212,6 +212,36 @@ def test_large_tile_and_queue_groups(moe, name):
         assert np.array_equal(got["out"], first), ("early", groups)
 
 
+RAGGED_HAND = {
+    # column tiles cut at 64, 128 and 192 of 256 columns (64 of 128 with SwiGLU), an odd number of 64-wide slabs in one or
+    # both projections, one slab only, partial row blocks
+    "gelu_bias_odd_slabs": ob.Cfg(S=700, H=448, I=832, E=3, k=2, act=ob.ACT_GELU, dtype=ob.BF16, drop=0),
+    "swiglu_bias_odd_slabs": ob.Cfg(S=500, H=320, I=448, E=2, k=1, act=ob.ACT_SWIGLU, dtype=ob.BF16, norm_topk=0, drop=0),
+    "relu_one_slab": ob.Cfg(S=300, H=64, I=64, E=2, k=1, act=ob.ACT_RELU, dtype=ob.F16, norm_topk=0, drop=0),
+    "fp16_swiglu_bias_drop": ob.Cfg(S=900, H=576, I=192, E=3, k=2, act=ob.ACT_SWIGLU, dtype=ob.F16, drop=1, capacity_factor=0.8),
+}
+
+
+@pytest.mark.parametrize("name", sorted(RAGGED_HAND))
+def test_hand_ordered_tiles_on_ragged_dimensions(moe, name):
+    """The hand-ordered tiles where the dimensions fit neither their columns nor their pairs of slabs: the same bits from
+    each of them in both FFN modes, also behind a layer that left other data in LDS, and the oracle's values."""
+    cfg = RAGGED_HAND[name]
+    inp = ob.make_inputs(cfg, seed=11, with_bias="bias" in name)
+    want = ob.forward(cfg, inp)
+    other = ob.Cfg(S=600, H=512, I=512, E=2, k=1, act=ob.ACT_GELU, dtype=cfg.dtype, norm_topk=0, drop=0)
+    first = None
+    for tile in (1, 2, 3):
+        for mode in (FFN_TILED, FFN_PERSISTENT):
+            run_layer(moe, other, ob.make_inputs(other, seed=1), mode, {"tile16": tile})
+            got = run_layer(moe, cfg, inp, mode, {"tile16": tile})
+            check_routing(got, want)
+            assert got["plan"]["block_rows"] == (128 if tile == 2 else 256)
+            assert max_rel_err(ob.to_f32(got["out"], cfg.act_dtype), ob.to_f32(want["out"], cfg.act_dtype)) <= OUT_TOL[cfg.dtype]
+            first = got["out"] if first is None else first
+            assert np.array_equal(got["out"], first), (tile, mode)
+
+
 @pytest.mark.parametrize("name", ["bf16_gelu_ragged", "bf16_swiglu_skew", "f32_swiglu_ragged", "fp8_many_rows_bias",
                                   "fp16_swiglu_skew_bias", "tf32_gelu_ragged", "capacity_one", "many_experts_bias",
                                   "all_experts_selected", "one_token"])

@@ -17,7 +17,7 @@ namespace moe355 {
 // per-dtype pieces defined next to their kernels
 int bf16_tile(int64_t pairs, int experts, int H, int I, int swiglu, int opt_block_rows, int opt_tile);
 int bf16_block_m(int tile);
-int bf16_block_n0(int tile);
+int bf16_block_n0(int tile, int swiglu);
 int bf16_block_n1(int tile);
 int f32_block_m();
 int f32_block_n();
@@ -206,7 +206,7 @@ FfnPlan ffn_plan(int dtype, int act, int H, int I, int64_t A, int E, const moe_o
     } else {
         p.tile = bf16_tile(A, E, H, I, sw, o.block_rows, o.tile16);
         p.block_m = bf16_block_m(p.tile);
-        p.nnt0 = sw ? ceil_div(I, bf16_block_n0(p.tile) / 2) : ceil_div(I, bf16_block_n0(p.tile));
+        p.nnt0 = ceil_div(I, bf16_block_n0(p.tile, sw) / (sw ? 2 : 1));
         p.nnt1 = ceil_div(H, bf16_block_n1(p.tile));
         // Partial sums for the down-projection tiles of the last row blocks: F tasks of a 1/F of the contraction
         // dimension each (the hand-ordered slab loop takes multiples of 128).  How many row blocks: the workgroups reach
@@ -214,7 +214,7 @@ FfnPlan ffn_plan(int dtype, int act, int H, int I, int64_t A, int E, const moe_o
         // spread on average, one more round is the tail proper.  Sized for kSplitWorkgroups resident workgroups whatever
         // the device has (the workspace size must not depend on the device).
         const int F = o.tail_split == 2 || o.tail_split == 4 ? o.tail_split : 1;
-        if (F > 1 && p.tile != 0 && I % (128 * F) == 0 && o.combine <= 0 && o.queue_early != 1) {
+        if (F > 1 && p.tile != 0 && p.tile < kStream16Tile && I % (128 * F) == 0 && o.combine <= 0 && o.queue_early != 1) {
             p.ksplit = F;
             p.tail_blocks = ceil_div((int64_t)(F / 2 + 1) * kSplitWorkgroups, (int64_t)p.nnt1 * F);
         }
@@ -363,7 +363,8 @@ int resolved_ffn_mode(const moe_handle* h) {
     // The 128 x 128 tile of the general loop stores its rows in 8-byte pieces straight from the accumulators: written
     // through, as the queue needs them, they cost it more than the overlap gives at every size measured (12 experts of
     // 1344 x 2752, 444 rows each: 233 against 199 us; 8 of 4096 x 14336, 4 rows 775 / 631, 375 rows 2087 / 1424).
-    if (tile16 && d.plan.tile == 0) return MOE_FFN_TILED;
+    // So do the weight streamer's rows, and its tasks are shorter still (ffn_stream16.hip).
+    if (tile16 && (d.plan.tile == 0 || d.plan.tile >= kStream16Tile)) return MOE_FFN_TILED;
     if ((f32_tile || tile16) && d.E == 1) return MOE_FFN_TILED;
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }
@@ -518,8 +519,8 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
     h->arch.persistent_blocks = prop.multiProcessorCount * per_cu;
     // One task queue per XCD for the MFMA-bound bf16 tiles, whose operand tiles are then shared in that XCD's L2;
     // so does the e4m3 tile GEMM; the fp32 kernels (the matrix-core tile measured 5 % faster on one queue than on eight)
-    // and the e4m3 weight streamer keep a single queue.
-    h->queue_groups = (tile16 || (kdt == MOE_DTYPE_FP8_E4M3_B128 && d.plan.tile)) ? h->arch.xcds : 1;
+    // and the weight streamers (no operand is shared between their workgroups) keep a single queue.
+    h->queue_groups = ((tile16 && d.plan.tile < kStream16Tile) || (kdt == MOE_DTYPE_FP8_E4M3_B128 && d.plan.tile)) ? h->arch.xcds : 1;
     if (opt->queue_groups != MOE_OPT_AUTO && opt->queue_groups <= h->arch.xcds) h->queue_groups = opt->queue_groups;   // never more queues than XCDs
     if (h->queue_groups > h->arch.persistent_blocks) h->queue_groups = 1;   // every queue needs a home workgroup
     // The e4m3 tile GEMM holds 64 workgroups per XCD on 128 x 128 tiles whose token rows (bf16) take twice the L2 space
@@ -555,8 +556,11 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
         *h->stall_host = 0;
     }
     // what moe_get_options reports: the values in force
-    h->opt.tile16 = tile16 ? d.plan.tile : MOE_OPT_AUTO;
-    h->opt.block_rows = tile16 ? d.plan.block_m : MOE_OPT_AUTO;
+    const bool stream16 = tile16 && d.plan.tile >= kStream16Tile;      // has no value of its own among the options
+    h->opt.tile16 = tile16 && !stream16 ? d.plan.tile : MOE_OPT_AUTO;
+    // (the coarser of the two, which wins where both are given: reported where it names this very tile)
+    const bool named = tile16 && !stream16 && bf16_tile(d.A, d.E, d.H, d.I, cfg->hidden_act == MOE_ACT_SWIGLU, d.plan.block_m, MOE_OPT_AUTO) == d.plan.tile;
+    h->opt.block_rows = named ? d.plan.block_m : MOE_OPT_AUTO;
     h->opt.f32_tile = (kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) ? d.plan.tile : MOE_OPT_AUTO;
     h->opt.fp8_tile = kdt == MOE_DTYPE_FP8_E4M3_B128 ? d.plan.tile : MOE_OPT_AUTO;
     h->opt.fp8_widen = cfg->torch_dtype == MOE_DTYPE_FP8_E4M3_B128 ? (int)d.plan.widen : MOE_OPT_AUTO;

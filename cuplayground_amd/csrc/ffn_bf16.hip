@@ -1549,8 +1549,17 @@ static double projection_cost(bool large, int64_t pairs, int experts, int column
 }
 static int columns256(int N) { return (N + 255) / 256; }
 
+// The weight streamer's form for this many rows per expert, or -1: the tiles are faster.  The first line lies where too many
+// experts begin to have a second block of 16 rows, the second where the tiles' cost, which rows do not change below a row
+// block, is that of the streamer's token rows: both sides measured at 2 to 32 rows, figures in ffn_stream16.hip.
+static int stream16_form(int64_t pairs, int experts) {
+    const double rows = (double)pairs / experts;
+    return rows <= 9 ? 0 : rows <= 17 ? 1 : -1;
+}
+
 // Tile of a layer: 0 = 128 x 128 on the general loop (operands of 4 GiB and more), 1 = 256 x 256, 2 = 128 x 256,
-// 3 = 256 x 256 with the 128 x 256 tile for the row blocks of at most 128 rows (option tile16 only).
+// 3 = 256 x 256 with the 128 x 256 tile for the row blocks of at most 128 rows (option tile16 only), kStream16Tile + form =
+// the weight streamer (ffn_stream16.hip; no option names it).
 int bf16_tile(int64_t pairs, int experts, int H, int I, int swiglu, int opt_block_rows, int opt_tile) {
     if (!large_tile_ok(pairs, H, I)) return 0;
     // option block_rows: 256 means the 256 x 256 tile where it is not ragged in either projection ...
@@ -1558,14 +1567,26 @@ int bf16_tile(int64_t pairs, int experts, int H, int I, int swiglu, int opt_bloc
         return opt_block_rows == 256 && H % 256 == 0 && I % (swiglu ? 128 : 256) == 0 ? 1 : 0;
     if (opt_tile >= 0 && opt_tile <= 3) return opt_tile;      // ... or tile16
     const int E = experts > 0 ? experts : 1;
+    const int form = stream16_form(pairs, E);
+    if (form >= 0) return kStream16Tile + form;
     auto cost = [&](bool large) {
         return projection_cost(large, pairs, E, columns256(swiglu ? 2 * I : I), H) + projection_cost(large, pairs, E, columns256(H), I);
     };
     return cost(true) <= cost(false) ? 1 : 2;
 }
-int bf16_block_m(int tile) { return tile == 1 || tile == 3 ? 256 : 128; }
-int bf16_block_n0(int tile) { return tile == 0 ? SmallPlan::T0::BN : 256; }
-int bf16_block_n1(int tile) { return tile == 0 ? SmallPlan::T1::BN : 256; }
+int bf16_block_m(int tile) {
+    if (tile >= kStream16Tile) return stream16_block_m(tile - kStream16Tile);
+    return tile == 1 || tile == 3 ? 256 : 128;
+}
+// Weight rows of a task: with SwiGLU half of them are gate rows (the streamer's tasks have as many columns either way).
+int bf16_block_n0(int tile, int swiglu) {
+    if (tile >= kStream16Tile) return stream16_block_n(tile - kStream16Tile) * (swiglu ? 2 : 1);
+    return tile == 0 ? SmallPlan::T0::BN : 256;
+}
+int bf16_block_n1(int tile) {
+    if (tile >= kStream16Tile) return stream16_block_n(tile - kStream16Tile);
+    return tile == 0 ? SmallPlan::T1::BN : 256;
+}
 
 template <template <class> class F, class... Args>
 static auto for_plan(int tile, bool f16, Args&&... args) {
@@ -1592,14 +1613,19 @@ template <class P> struct RunOccupancy {
 
 hipError_t launch_ffn_tiled_bf16(const FfnArgs& a, int tile, int max_mtiles, int nnt0, int nnt1, hipStream_t st,
                                  bool f16) {
+    if (tile >= kStream16Tile) return launch_ffn_stream16(a, tile - kStream16Tile, f16, max_mtiles, nnt0, nnt1, 0, st);
     return for_plan<RunTiled>(tile, f16, a, max_mtiles, nnt0, nnt1, st);
 }
 
 hipError_t launch_ffn_persistent_bf16(const FfnArgs& a, int tile, int blocks, bool early, hipStream_t st, bool f16) {
+    if (tile >= kStream16Tile) return launch_ffn_stream16(a, tile - kStream16Tile, f16, 0, 0, 0, blocks, st);
     return for_plan<RunPersistent>(tile, f16, a, blocks, early, st);
 }
 
-int ffn_persistent_occupancy_bf16(int tile) { return for_plan<RunOccupancy>(tile, false); }
+int ffn_persistent_occupancy_bf16(int tile) {
+    if (tile >= kStream16Tile) return ffn_persistent_occupancy_stream16(tile - kStream16Tile);
+    return for_plan<RunOccupancy>(tile, false);
+}
 
 template <class T>
 static hipError_t launch_dense(const void* A, const void* B, const void* bias, void* C, int64_t M, int64_t N, int64_t K,

@@ -1,0 +1,312 @@
+// Expert FFN of bf16 / fp16 layers with a handful of token rows per expert (decoding): a weight streamer.
+//
+// Every weight of an expert that is hit is needed once, for a few rows: the time is the time the weights take from memory
+// (8 experts of 4096 x 14336, SwiGLU, 16 tokens: 2.8 GB).  The 256-column tiles cannot reach that: a tile streams 256 weight
+// rows through one compute unit's LDS behind one barrier per slab, and a down projection onto 4096 columns has 16 such tiles
+// an expert, half the chip.  Here a wavefront is on its own:
+//   * it owns 16 * CG output columns -- as many weight rows, or gate and up rows with SwiGLU -- over the whole contraction
+//     dimension, as the "A" operand of v_mfma_f32_16x16x32; the "B" operand is up to NT groups of 16 token rows, read through
+//     the caches that the neighbouring wavefronts read them through.  No LDS, no barrier;
+//   * weights go from memory into the fragment registers in which the matrix instruction wants them (16 bytes a lane, 64
+//     contiguous bytes of 16 rows an instruction, 8 KB in flight while the 8 KB before are multiplied);
+//   * one accumulator per output element, added to in the order of k as in the tiles: the same bits as theirs, and no sums
+//     to bring together.
+// A workgroup is four wavefronts on neighbouring columns of one row block.
+//
+// What bounds it: memory, and beside it the token rows, of which every wavefront reads NT * 16 for its 16 * CG weight rows.
+// Measured, whole layer, cold weights, two launches, us -- 128 x 256 tile / NT 1, CG 1 / NT 2, CG 1 / NT 2, CG 2:
+//   8 experts of 4096 x 14336, SwiGLU (2.8 GB): 2 rows each 507 / 438 / 468 / 445, 4 612 / 527 / 552 / 562,
+//     8 613 / 556 / 579 / 566, 12 614 / 590 / 613 / 583, 16 618 / 823 / 657 / 609, 24 621 / 1237 / 740 / 648
+//   16 of 2048 x 2048, GELU: 0.5 rows 96 / 50 / 54 / 67, 8 109 / 86 / 92 / 86, 12 108 / 103 / 97 / 88, 16 111 / 126 / 103 / 91,
+//     24 111 / 149 / 128 / 117
+//   64 of 2048 x 1408, SwiGLU: 2 rows 267 / 221 / 236 / 241, 8 284 / 264 / 276 / 261, 16 290 / 358 / 310 / 284, 24 294 / 468 / 349 / 309
+//   12 of 1344 x 2752, GELU: 2 rows 105 / 63 / 69 / 76, 8 107 / 74 / 82 / 92, 16 106 / 102 / 92 / 99, 24 107 / 117 / 104 / 107
+// (4 rows of the first: 5.7 TB/s of weights behind about 30 us of routing, launches and combine.)  An expert with more rows
+// than a block has its weights read again, which is where the steps upwards come from.  NT 4 is behind the tile from 24 rows
+// on the first and the third of these.  Non-temporal weight loads lose 1 to 15 % (an instruction takes half of a 128-byte
+// line; its other half must still be in the cache for the next one).  The task queue with its written-through rows and pops
+// of this much shorter tasks costs more than the overlap of the projections gives: 645 us against 520 (4 rows of the first),
+// 158 against 81 (4 of the second).
+#include "act_deriv.hpp"
+#include "ffn_common.hpp"
+
+namespace moe355 {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int STHREADS = 256;
+
+template <class ET, int NT, int CG>
+struct Stream {
+    using Elem = ET;
+    static constexpr bool F16 = std::is_same<ET, f16_s>::value;
+    static constexpr int T = NT;             // groups of 16 token rows
+    static constexpr int BM = 16 * NT;
+    static constexpr int C = CG;             // groups of 16 columns a wavefront owns
+    static constexpr int BN = 64 * CG;       // columns of a task
+};
+
+template <class P>
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (P::F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <class P>
+__device__ __forceinline__ uint32_t pack2s(float lo, float hi) {
+    if constexpr (P::F16) {
+        typedef float f32x2_t __attribute__((ext_vector_type(2)));
+        typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+        const f32x2_t v = {lo, hi};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+    } else {
+        return pack2_bf16(lo, hi);
+    }
+}
+template <class P>
+__device__ __forceinline__ float widen1s(uint16_t v) {
+    if constexpr (P::F16) return (float)__builtin_bit_cast(_Float16, v);
+    else return bf16_bits_to_f32(v);
+}
+
+struct StreamTask {
+    const uint16_t* w[2];      // weight matrices of the expert: {w_up or w_down, w_gate or null}
+    const uint16_t* bias[2];
+    const uint16_t* a_base;    // x or h
+    const int32_t* gather;     // token_indices + row0, or null
+    int64_t a_row0;
+    uint16_t* c_base;          // h or y at the first row of the block
+    int K, N, rows, n0, act;
+    bool publish;              // rows are read by other workgroups of the same launch
+};
+
+// MATS: weight matrices (2: SwiGLU's up and gate).  K and N are multiples of 64 (moe_config_validate), so a wavefront's
+// columns exist together or not at all.
+template <class P, int MATS>
+__device__ __forceinline__ void stream_tile(const StreamTask& t) {
+    constexpr int NT = P::T, CG = P::C, G = MATS * CG;
+    constexpr int U = 8 / G;      // 32-wide slabs in flight
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int idx = lane & 15, kg = lane >> 4;
+    const int c0 = t.n0 + 16 * CG * wave;
+    if (c0 >= t.N) return;
+
+    const uint16_t* wp[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) wp[g] = t.w[g / CG] + (int64_t)(c0 + 16 * (g % CG) + idx) * t.K + 8 * kg;
+    // rows behind the block's last one read row 0 again and are never stored
+    const uint16_t* xp[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int r = 16 * i + idx < t.rows ? 16 * i + idx : 0;
+        xp[i] = t.a_base + (t.gather ? (int64_t)t.gather[r] : t.a_row0 + r) * t.K + 8 * kg;
+    }
+
+    f32x4 acc[G][NT];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[g][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int slabs = t.K >> 5, full = slabs / U, left = slabs - full * U;
+    u32x4 w[G][U], wn[G][U], x[NT][U];
+    // slabs behind the last one read it again (and are not multiplied)
+    auto load_w = [&](u32x4 (&d)[G][U], int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s0 + u, slabs - 1) << 5;
+#pragma unroll
+            for (int g = 0; g < G; ++g) d[g][u] = *reinterpret_cast<const u32x4*>(wp[g] + k);
+        }
+    };
+    auto load_x = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s0 + u, slabs - 1) << 5;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) x[i][u] = *reinterpret_cast<const u32x4*>(xp[i] + k);
+        }
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) acc[g][i] = mfma32<P>(w[g][u], x[i][u], acc[g][i]);
+    };
+    load_w(w, 0);
+    for (int c = 0; c < full; ++c) {
+        // The token rows first: loads return in order, so waiting for them does not wait for the weights behind.
+        load_x(c * U);
+        if ((c + 1) * U < slabs) load_w(wn, (c + 1) * U);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(u);
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[g][u] = wn[g][u];
+    }
+    if (left) {
+        load_x(full * U);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < left) multiply(u);
+    }
+
+    // this lane holds token rows 16 i + idx, columns c0 + 16 c + 4 kg ..+3
+    const float relu_floor = t.act == MOE_ACT_RELU ? 0.0f : -INFINITY;      // compare and select: a NaN stays a NaN
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+        const int col = c0 + 16 * c + 4 * kg;
+        float b[MATS][4];
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) b[m][r] = t.bias[m] ? widen1s<P>(t.bias[m][col + r]) : -0.0f;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int row = 16 * i + idx;
+            if (row >= t.rows) continue;
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float u = acc[c][i][r] + b[0][r];
+                if constexpr (MATS == 2) {
+                    const float g = acc[CG + c][i][r] + b[1][r];
+                    v[r] = silu16(g) * u;
+                } else {
+                    v[r] = t.act == MOE_ACT_GELU ? gelu16(u) : (u < relu_floor ? relu_floor : u);
+                }
+            }
+            uint16_t* p = t.c_base + (int64_t)row * t.N + col;
+            const uint32_t lo = pack2s<P>(v[0], v[1]), hi = pack2s<P>(v[2], v[3]);
+            if (t.publish) publish8(p, lo, hi);
+            else *reinterpret_cast<uint2*>(p) = uint2{lo, hi};
+        }
+    }
+}
+
+template <class P>
+__device__ __forceinline__ StreamTask resolve_stream(const FfnArgs& a, const Task& t, bool publish) {
+    StreamTask p;
+    const int64_t HI = (int64_t)a.H * a.I;
+    p.publish = publish;
+    p.rows = t.rows;
+    p.n0 = t.ntile * P::BN;
+    if (t.phase == 0) {
+        const bool sw = a.act == MOE_ACT_SWIGLU;
+        p.K = a.H;
+        p.N = a.I;
+        p.w[0] = (const uint16_t*)a.w_up + t.expert * HI;
+        p.w[1] = sw ? (const uint16_t*)a.w_gate + t.expert * HI : nullptr;
+        p.bias[0] = a.b_up ? (const uint16_t*)a.b_up + (int64_t)t.expert * a.I : nullptr;
+        p.bias[1] = sw && a.b_gate ? (const uint16_t*)a.b_gate + (int64_t)t.expert * a.I : nullptr;
+        p.a_base = (const uint16_t*)a.x;
+        p.gather = a.token_indices + t.row0;
+        p.a_row0 = 0;
+        p.c_base = (uint16_t*)a.h + (int64_t)t.row0 * a.I;
+        p.act = a.act;
+    } else {
+        p.K = a.I;
+        p.N = a.H;
+        p.w[0] = (const uint16_t*)a.w_down + t.expert * HI;
+        p.w[1] = nullptr;
+        p.bias[0] = a.b_down ? (const uint16_t*)a.b_down + (int64_t)t.expert * a.H : nullptr;
+        p.bias[1] = nullptr;
+        p.a_base = (const uint16_t*)a.h;
+        p.gather = nullptr;
+        p.a_row0 = t.row0;
+        p.c_base = (uint16_t*)a.y + (int64_t)t.row0 * a.H;
+        p.act = MOE_ACT_NONE;
+    }
+    return p;
+}
+
+template <class P>
+__device__ __forceinline__ void stream_task(const FfnArgs& a, const Task& t, bool publish) {
+    const StreamTask p = resolve_stream<P>(a, t, publish);
+    if (t.phase == 0 && a.act == MOE_ACT_SWIGLU) stream_tile<P, 2>(p);
+    else stream_tile<P, 1>(p);
+}
+
+template <class P>
+__global__ __launch_bounds__(STHREADS) void ffn_tiled_stream16_kernel(FfnArgs a, int phase) {
+    __shared__ int s_list[1 + P::BM];
+    if (phase == 0) zero_unrouted_rows(a, 2);
+    Task t;
+    if (!tiled_task(a, phase, blockIdx.x, t)) return;
+    stream_task<P>(a, t, phase == 1 && a.arrive);
+    if (phase == 1 && a.arrive) combine_arrivals<typename P::Elem>(combine_args(a), t.row0, t.rows, t.ntile, t.ntile * P::BN, P::BN, s_list);
+}
+
+template <class P>
+__global__ __launch_bounds__(STHREADS) void ffn_persistent_stream16_kernel(FfnArgs a) {
+    __shared__ int s_task, s_ok;
+    __shared__ int s_cmb[kCombineLds];
+    __shared__ int s_list[1 + P::BM];
+    queue_kernel_entry();
+    queue_clock_stamp(a.wg_clock, 0);
+    zero_unrouted_rows(a, 2);
+    const int ids = a.q->ids_queue;
+    const int nseg = a.q->nseg;
+    const int nnt0 = a.seg_phase0[0].nnt;
+    QueueCursor cur = queue_cursor(a.groups);
+    Task t;
+    while (next_task(a, cur, &s_task, ids, nseg, nnt0, t)) {
+        int ok = 1;
+        if (t.phase == 1) ok = wait_phase0_done(a.done0, t.mtile, nnt0, a.spin_limit, a.q, a.host_stall, &s_ok);
+        const long long started = trace_clock(a.task_trace);
+        const bool publish = t.phase == 0 || publish_y(a);
+        if (ok) {
+            stream_task<P>(a, t, publish);
+        } else {
+            const StreamTask p = resolve_stream<P>(a, t, publish);
+            poison_tile(p.c_base, p.rows, p.N, p.n0, P::BN, 2);
+        }
+        if (a.task_trace) trace_task(a.task_trace, a.task_trace_cap, t.phase, t.expert, t.mtile, t.ntile, t.rows, started);
+        if (t.phase == 0) signal_phase0_done(a.done0, t.mtile);
+        else after_down_tile<typename P::Elem>(a, t.row0, t.rows, t.mtile, t.ntile, t.ntile * P::BN, P::BN, s_list);
+    }
+    if (a.combined) combine_while_idle_narrow<typename P::Elem>(sweep_args(a), &s_task, s_cmb);
+    queue_clock_stamp(a.wg_clock, 1);
+}
+
+template <class P>
+hipError_t launch(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
+    if (blocks > 0) {
+        ffn_persistent_stream16_kernel<P><<<blocks, STHREADS, 0, st>>>(a);
+    } else {
+        ffn_tiled_stream16_kernel<P><<<tiled_grid(max_mtiles, nnt0, a.groups), STHREADS, 0, st>>>(a, 0);
+        ffn_tiled_stream16_kernel<P><<<tiled_grid(max_mtiles, nnt1, a.groups), STHREADS, 0, st>>>(a, 1);
+    }
+    return hipGetLastError();
+}
+
+template <class P>
+int occupancy() {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&ffn_persistent_stream16_kernel<P>), STHREADS, 0) != hipSuccess || n < 1)
+        n = 1;
+    return n;
+}
+
+}  // namespace
+
+// The two forms: 0 = blocks of 16 rows, tasks of 64 columns; 1 = 32 rows, 128 columns.
+template <class ET> using Narrow = Stream<ET, 1, 1>;
+template <class ET> using Wide = Stream<ET, 2, 2>;
+
+int stream16_block_m(int form) { return form ? Wide<bf16_s>::BM : Narrow<bf16_s>::BM; }
+int stream16_block_n(int form) { return form ? Wide<bf16_s>::BN : Narrow<bf16_s>::BN; }
+int ffn_persistent_occupancy_stream16(int form) { return form ? occupancy<Wide<bf16_s>>() : occupancy<Narrow<bf16_s>>(); }
+
+// blocks > 0: workgroups of the task queue; 0: a launch per projection.
+hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
+    if (f16) return form ? launch<Wide<f16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch<Narrow<f16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st);
+    return form ? launch<Wide<bf16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch<Narrow<bf16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st);
+}
+
+}  // namespace moe355

@@ -178,6 +178,13 @@ hipError_t launch_combine(const void* y_rows, const int32_t* pair_row, const flo
                           int act_dtype, void* out, const int32_t* taken, hipStream_t st);
 
 // FFN stage.  block_m / block_n are the tile sizes the routing stage must be told about.
+// FfnPlan::tile of a 16-bit layer from this value on: the weight streamer (ffn_stream16.hip) in its form tile - kStream16Tile.
+constexpr int kStream16Tile = 4;
+struct FfnArgs;
+int stream16_block_m(int form);
+int stream16_block_n(int form);
+int ffn_persistent_occupancy_stream16(int form);
+hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st);
 struct FfnPlan {
     int kernel_dtype;   // the dtype whose kernels run: the layer's, or bf16 for an e4m3 layer whose weights are widened
     bool widen;         // e4m3 layer run as a bf16 layer on weights widened into the workspace by every call

@@ -113,7 +113,8 @@ typedef struct moe_handle moe_handle;
 #define MOE_OPT_AUTO (-1)
 typedef struct moe_options {
     int32_t tile16;          /* bf16 / fp16 layers: 0 = 128x128 tile, 1 = 256x256 (hand-ordered), 2 = 128x256 (hand-ordered),
-                                3 = 256x256 with the 128x256 tile for row blocks of at most 128 rows */
+                                3 = 256x256 with the 128x256 tile for row blocks of at most 128 rows; AUTO also has the weight
+                                streamer for a few rows per expert, which moe_get_options reports as AUTO here and below */
     int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1; 256 needs
                                 H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0) */
     int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile; also read by the

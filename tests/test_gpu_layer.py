@@ -242,6 +242,42 @@ def test_hand_ordered_tiles_on_ragged_dimensions(moe, name):
             assert np.array_equal(got["out"], first), (tile, mode)
 
 
+FEW_ROWS = {
+    # rows per expert on average, over every one of them: one; up to and past a block of 16 or 32 rows; dimensions of one
+    # column task and of a cut one, of 2 slabs (one partial chunk), of a whole number of chunks and of one slab more
+    "one_row": (ob.Cfg(S=1, H=64, I=64, E=2, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=0), 16),
+    "gelu_bias_empty_experts": (ob.Cfg(S=9, H=192, I=320, E=12, k=1, act=ob.ACT_GELU, dtype=ob.BF16, norm_topk=0, drop=0), 16),
+    "fp16_swiglu_bias_skew": (ob.Cfg(S=70, H=256, I=448, E=16, k=2, act=ob.ACT_SWIGLU, dtype=ob.F16, drop=0, zipf_bias=True), 16),
+    "relu_last_narrow": (ob.Cfg(S=36, H=320, I=576, E=4, k=1, act=ob.ACT_RELU, dtype=ob.BF16, norm_topk=0, drop=0, zipf_bias=True), 16),
+    "swiglu_first_wide": (ob.Cfg(S=37, H=320, I=192, E=4, k=1, act=ob.ACT_SWIGLU, dtype=ob.BF16, norm_topk=0, drop=0), 32),
+    "fp16_gelu_wide_skew_drop": (ob.Cfg(S=66, H=576, I=256, E=8, k=2, act=ob.ACT_GELU, dtype=ob.F16, drop=1, capacity_factor=2.5,
+                                        zipf_bias=True), 32),
+    "swiglu_bias_last_wide": (ob.Cfg(S=51, H=512, I=832, E=3, k=1, act=ob.ACT_SWIGLU, dtype=ob.BF16, norm_topk=0, drop=0), 32),
+    "tile_behind_the_last": (ob.Cfg(S=52, H=256, I=256, E=3, k=1, act=ob.ACT_SWIGLU, dtype=ob.BF16, norm_topk=0, drop=0), 128),
+}
+
+
+@pytest.mark.parametrize("name", sorted(FEW_ROWS))
+def test_weight_streamer_gives_the_bits_of_the_tiles(moe, name):
+    """A few rows per expert: the streamer (csrc/ffn_stream16.hip) in both FFN modes, with the combine behind it, by arrival
+    counters and as queue tasks, against the oracle and, bit for bit, against the 128 x 256 tile: each of its output elements
+    is accumulated by the same matrix instructions in the same order."""
+    cfg, rows = FEW_ROWS[name]
+    inp = ob.make_inputs(cfg, seed=23, with_bias="bias" in name)
+    want = ob.forward(cfg, inp)
+    tile = run_layer(moe, cfg, inp, FFN_TILED, {"tile16": 2})
+    for mode in (FFN_TILED, FFN_PERSISTENT):
+        for combine in (0, 1, 2):
+            got = run_layer(moe, cfg, inp, mode, {"combine": combine})
+            check_routing(got, want)
+            assert got["plan"]["block_rows"] == rows
+            assert max_rel_err(ob.to_f32(got["out"], cfg.act_dtype), ob.to_f32(want["out"], cfg.act_dtype)) <= OUT_TOL[cfg.dtype]
+            assert np.array_equal(got["out"], tile["out"]), (mode, combine)
+    layer = moe.MoELayer(product_config(cfg))
+    again = moe.MoELayer(product_config(cfg), options=layer.options)        # the options in force make the same handle
+    assert again.plan == layer.plan and layer.plan["block_rows"] == rows
+
+
 @pytest.mark.parametrize("name", ["bf16_gelu_ragged", "bf16_swiglu_skew", "f32_swiglu_ragged", "fp8_many_rows_bias",
                                   "fp16_swiglu_skew_bias", "tf32_gelu_ragged", "capacity_one", "many_experts_bias",
                                   "all_experts_selected", "one_token"])

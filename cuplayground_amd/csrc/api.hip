@@ -26,8 +26,8 @@ hipError_t launch_ffn_persistent_bf16(const FfnArgs&, int tile, int blocks, bool
 int ffn_persistent_occupancy_bf16(int tile);
 hipError_t launch_gemm_dense_bf16(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int,
                                   int opt_tile, hipStream_t, bool f16);
-hipError_t launch_ffn_tiled_f32(const FfnArgs&, int max_mtiles, int nnt0, int nnt1, hipStream_t);
-hipError_t launch_ffn_persistent_f32(const FfnArgs&, int blocks, hipStream_t);
+hipError_t launch_ffn_tiled_f32(const FfnArgs&, bool stream, int max_mtiles, int nnt0, int nnt1, hipStream_t);
+hipError_t launch_ffn_persistent_f32(const FfnArgs&, bool stream, int blocks, hipStream_t);
 hipError_t launch_gemm_dense_f32(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int,
                                  hipStream_t);
 hipError_t launch_ffn_fp8(const FfnArgs&, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t);
@@ -179,19 +179,22 @@ FfnPlan ffn_plan(int dtype, int act, int H, int I, int64_t A, int E, const moe_o
         if (p.widen) p.kernel_dtype = dtype = MOE_DTYPE_BF16;
     }
     if (dtype == MOE_DTYPE_F32 || dtype == MOE_DTYPE_TF32) {
-        // 0: 64 x 64 tiles on the vector ALUs (small and ragged layers); 1: 128 x 128 tiles on the matrix cores
+        // 0: 64 x 64 tiles on the vector ALUs (ragged layers), or kF32StreamTile, the weight streamer on blocks of the same height
+        // (small ones); 1: 128 x 128 tiles on the matrix cores
         // (from a full row block per expert on average, and enough 128 x 128 tiles to occupy the compute units twice over:
-        // below that the smaller tiles of the vector kernel spread the same work over more of the chip)
+        // below that the smaller tiles spread the same work over more of the chip)
         const int64_t tiles = (A / f32_tile_block_m()) * (ceil_div(I, f32_tile_block_n0(sw)) + ceil_div(H, f32_tile_block_n1()));
         p.tile = H % 128 == 0 && I % 128 == 0 && A / (E > 0 ? E : 1) >= kF32TileRowsPerExpert && tiles >= kF32TileMinTiles ? 1 : 0;
+        const int64_t stream_tasks = (A / f32_block_m() + E) * (ceil_div(I, f32_block_n()) + ceil_div(H, f32_block_n()));
+        if (p.tile == 0 && (A <= (int64_t)E * kF32StreamRowsPerExpert || stream_tasks <= kF32StreamMaxTasks)) p.tile = kF32StreamTile;
         if (o.f32_tile == 0 || (o.f32_tile == 1 && H % 128 == 0 && I % 128 == 0)) p.tile = o.f32_tile;
-        if (p.tile) {
+        if (p.tile == 1) {
             p.block_m = f32_tile_block_m();
             p.nnt0 = ceil_div(I, f32_tile_block_n0(sw));
             p.nnt1 = ceil_div(H, f32_tile_block_n1());
         } else {
             p.block_m = f32_block_m();
-            p.nnt0 = sw ? ceil_div(I, f32_block_n() / 2) : ceil_div(I, f32_block_n());
+            p.nnt0 = sw && p.tile == 0 ? ceil_div(I, f32_block_n() / 2) : ceil_div(I, f32_block_n());
             p.nnt1 = ceil_div(H, f32_block_n());
         }
     } else if (dtype == MOE_DTYPE_FP8_E4M3_B128) {
@@ -354,7 +357,7 @@ int resolved_ffn_mode(const moe_handle* h) {
     // The queue pays off from a couple of tasks per resident workgroup on.  The fp32 matrix-core tile has long tasks
     // (a down-projection tile of the reference's knob file takes half a millisecond) and needs twice that to balance:
     // 4096 tokens of that file, 2.6 tasks per workgroup, take 0.79 ms on the queue and 0.60 ms as two launches.
-    const bool f32_tile = (d.plan.kernel_dtype == MOE_DTYPE_F32 || d.plan.kernel_dtype == MOE_DTYPE_TF32) && d.plan.tile;
+    const bool f32_tile = (d.plan.kernel_dtype == MOE_DTYPE_F32 || d.plan.kernel_dtype == MOE_DTYPE_TF32) && d.plan.tile == 1;
     // With a single expert the queue has no second expert's up projection to run beside the down projection: it is the
     // two launches plus dependency waits and written-through intermediate rows (the reference's knob file: 1.13 ms
     // against 1.03-1.10 ms as two launches; the same file in bf16 0.183 against 0.170 ms; the Mixtral dimensions with one
@@ -365,6 +368,8 @@ int resolved_ffn_mode(const moe_handle* h) {
     // 1344 x 2752, 444 rows each: 233 against 199 us; 8 of 4096 x 14336, 4 rows 775 / 631, 375 rows 2087 / 1424).
     // So do the weight streamer's rows, and its tasks are shorter still (ffn_stream16.hip).
     if (tile16 && (d.plan.tile == 0 || d.plan.tile >= kStream16Tile)) return MOE_FFN_TILED;
+    // (the fp32 one: 1.26 against 1.02 ms, 16 tokens on 8 experts of 4096 x 14336; 2.89 against 2.21 for 128 tokens)
+    if ((d.plan.kernel_dtype == MOE_DTYPE_F32 || d.plan.kernel_dtype == MOE_DTYPE_TF32) && d.plan.tile == kF32StreamTile) return MOE_FFN_TILED;
     if ((f32_tile || tile16) && d.E == 1) return MOE_FFN_TILED;
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }
@@ -561,7 +566,8 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
     // (the coarser of the two, which wins where both are given: reported where it names this very tile)
     const bool named = tile16 && !stream16 && bf16_tile(d.A, d.E, d.H, d.I, cfg->hidden_act == MOE_ACT_SWIGLU, d.plan.block_m, MOE_OPT_AUTO) == d.plan.tile;
     h->opt.block_rows = named ? d.plan.block_m : MOE_OPT_AUTO;
-    h->opt.f32_tile = (kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) ? d.plan.tile : MOE_OPT_AUTO;
+    // (the streamer's layers keep the products outside the layer on the 64 x 64 tile: moe_get_options says AUTO for both)
+    h->opt.f32_tile = (kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) ? (d.plan.tile == kF32StreamTile ? 0 : d.plan.tile) : MOE_OPT_AUTO;
     h->opt.fp8_tile = kdt == MOE_DTYPE_FP8_E4M3_B128 ? d.plan.tile : MOE_OPT_AUTO;
     h->opt.fp8_widen = cfg->torch_dtype == MOE_DTYPE_FP8_E4M3_B128 ? (int)d.plan.widen : MOE_OPT_AUTO;
     h->opt.queue_groups = h->queue_groups;
@@ -581,6 +587,8 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
 int moe_get_options(const moe_handle* h, moe_options* opt) {
     if (!h || !opt) return MOE_ERR_BAD_ARGUMENT;
     *opt = h->opt;
+    const int kdt = h->d.plan.kernel_dtype;
+    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && h->d.plan.tile == kF32StreamTile) opt->f32_tile = MOE_OPT_AUTO;
     return MOE_OK;
 }
 
@@ -1244,20 +1252,21 @@ namespace moe355 {
 
 hipError_t launch_ffn_tiled(const FfnArgs& a, int dtype, const FfnPlan& p, int max_mtiles, hipStream_t st) {
     if (dtype == MOE_DTYPE_F32 || dtype == MOE_DTYPE_TF32)
-        return p.tile ? launch_ffn_f32_tile(a, max_mtiles, p.nnt0, p.nnt1, 0, st)
-                      : launch_ffn_tiled_f32(a, max_mtiles, p.nnt0, p.nnt1, st);
+        return p.tile == 1 ? launch_ffn_f32_tile(a, max_mtiles, p.nnt0, p.nnt1, 0, st)
+                           : launch_ffn_tiled_f32(a, p.tile == kF32StreamTile, max_mtiles, p.nnt0, p.nnt1, st);
     return launch_ffn_tiled_bf16(a, p.tile, max_mtiles, p.nnt0, p.nnt1, st, dtype == MOE_DTYPE_FP16);
 }
 
 hipError_t launch_ffn_persistent(const FfnArgs& a, int dtype, const FfnPlan& p, int blocks, bool early, hipStream_t st) {
     if (dtype == MOE_DTYPE_F32 || dtype == MOE_DTYPE_TF32)
-        return p.tile ? launch_ffn_f32_tile(a, 0, p.nnt0, p.nnt1, blocks, st) : launch_ffn_persistent_f32(a, blocks, st);
+        return p.tile == 1 ? launch_ffn_f32_tile(a, 0, p.nnt0, p.nnt1, blocks, st)
+                           : launch_ffn_persistent_f32(a, p.tile == kF32StreamTile, blocks, st);
     return launch_ffn_persistent_bf16(a, p.tile, blocks, early, st, dtype == MOE_DTYPE_FP16);
 }
 
 int ffn_persistent_blocks(int dtype, int tile, int compute_units) {
     if (dtype == MOE_DTYPE_F32 || dtype == MOE_DTYPE_TF32)
-        return compute_units * (tile ? ffn_persistent_occupancy_f32_tile() : 4);
+        return compute_units * (tile == 1 ? ffn_persistent_occupancy_f32_tile() : tile == kF32StreamTile ? 3 : 4);      // 3: the streamer's __launch_bounds__
     if (dtype == MOE_DTYPE_FP8_E4M3_B128)
         return compute_units * (tile ? ffn_persistent_occupancy_fp8_tile() : ffn_persistent_occupancy_fp8());
     return compute_units * ffn_persistent_occupancy_bf16(tile);

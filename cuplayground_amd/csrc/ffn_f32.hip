@@ -1,12 +1,15 @@
 // Expert FFN in fp32 (torch_dtype 0): the reference's tile GEMM contract, C = act(A.B^T + bias)
-// (mma.cuh:46-179; its only instantiated case is fp32 + ReLU, mma.cuh:378-384), on the vector ALUs.
-// This is the kernel of small and ragged fp32 layers (large ones take ffn_f32_tile.hip): a plain LDS-tiled FMA kernel, 64x64 output tile,
-// 16-wide K slabs, 256 threads with a 4x4 register block each.  Task decoding, dispatch-by-gather and the
+// (mma.cuh:46-179; its only instantiated case is fp32 + ReLU, mma.cuh:378-384).
+// The kernels of small and ragged fp32 layers (large ones take ffn_f32_tile.hip): a plain LDS-tiled FMA kernel, 64x64 output
+// tile, 16-wide K slabs, 256 threads with a 4x4 register block each, and for layers of few rows or few tasks wavefronts that
+// stream weights into the fp32 matrix instructions.  Task decoding, dispatch-by-gather and the
 // phase dependency protocol are shared with the bf16 path.
 #include "ffn_common.hpp"
 
 namespace moe355 {
 namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int FBM = 64, FBN = 64, FBK = 16, FPAD = 4;
 
@@ -103,6 +106,139 @@ __device__ __forceinline__ void gemm_tile_f32(const TaskPtrsF& p, float (*As)[FB
     }
 }
 
+// ---- the weight streamer ----
+// 64 rows x 64 columns of one projection (SwiGLU: of both, 64 gate and 64 up rows) on v_mfma_f32_16x16x4_f32 without LDS or
+// barriers.  A wavefront owns 16 columns over the whole contraction dimension: weight rows as the "A" operand, up to NT
+// groups of 16 token rows as "B", each fetched as 16 bytes a lane and 16 values of k an instruction, the next chunk of
+// weights in flight while this one is multiplied.  Lane group g holds k = 4 g .. 4 g + 3 of a slab, and matrix instruction j
+// multiplies element j of every lane group: a permutation of the slab's k that both operands share.  Two accumulators per
+// output element (even and odd slabs), added at the end.
+//
+// What bounds a small layer is latency: 128 rows on 8 experts of 256 x 512 are 1 us of arithmetic for 64 and 32 tasks.  The
+// LDS-tiled FMA kernel above waits for memory and two barriers every 16 values of k and always computes 64 rows;
+// here eight slabs (16 KB a wavefront) are in flight, nothing is waited for but the operands, and groups of 16 rows that a
+// block does not have cost nothing.  Whole layer, that kernel -> this one, us: 128 tokens, 8 experts of 256 x 512, GELU 67.6 ->
+// 33.2; 40 tokens top-2 of 16, 128 x 768 76 -> 34; 192 tokens, 4 of 448 x 640 90 -> 72; 537 tokens, 8 of 384 x 256 64 -> 52; 332
+// tokens, one of 1024 x 4096 331 -> 255; 16 tokens, 8 of 4096 x 14336, SwiGLU 2990 -> 1020.  Error against float64: 5.2e-7 -> 3.7e-7
+// (first), 1.0e-6 -> 7.0e-7 (fifth).  Where full blocks keep the chip busy it loses to the LDS kernel, which reads a token row
+// once for 64 columns and not for 16 (api.hip: ffn_plan has the line).
+template <int MATS, int NT>
+__device__ __forceinline__ void stream_tile_f32(const TaskPtrsF& p) {
+    constexpr int U = (NT >= 4 ? 4 : 8) / MATS;      // slabs of 16 in flight
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int idx = lane & 15, kg = lane >> 4;
+    const int c0 = p.n0 + 16 * wave;                 // N is a multiple of 64: a wavefront's columns exist together or not at all
+    if (c0 >= p.N) return;
+
+    const float* wp[MATS];
+#pragma unroll
+    for (int m = 0; m < MATS; ++m) wp[m] = (m ? p.b1 : p.b0) + (int64_t)(c0 + idx) * p.b_ld + 4 * kg;
+    // rows behind the block's last one read row 0 again and are never stored
+    const float* xp[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int r = 16 * i + idx < p.rows ? 16 * i + idx : 0;
+        xp[i] = p.a_base + (p.gather ? (int64_t)p.gather[r] : p.a_row0 + r) * p.a_ld + 4 * kg;
+    }
+
+    f32x4 acc[2][MATS][NT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) acc[h][m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int slabs = p.K >> 4, full = slabs / U, left = slabs - full * U;
+    f32x4 w[MATS][U], wn[MATS][U], x[NT][U];
+    // slabs behind the last one read it again (and are not multiplied)
+    auto load_w = [&](f32x4 (&d)[MATS][U], int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s0 + u, slabs - 1) << 4;
+#pragma unroll
+            for (int m = 0; m < MATS; ++m) d[m][u] = *reinterpret_cast<const f32x4*>(wp[m] + k);
+        }
+    };
+    auto load_x = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s0 + u, slabs - 1) << 4;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) x[i][u] = *reinterpret_cast<const f32x4*>(xp[i] + k);
+        }
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int m = 0; m < MATS; ++m)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+                    acc[u & 1][m][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[m][u][j], x[i][u][j], acc[u & 1][m][i], 0, 0, 0);
+    };
+    load_w(w, 0);
+    for (int c = 0; c < full; ++c) {
+        load_x(c * U);                               // first: loads return in order, and these are needed first
+        if ((c + 1) * U < slabs) load_w(wn, (c + 1) * U);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(u);
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[m][u] = wn[m][u];
+    }
+    if (left) {
+        load_x(full * U);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < left) multiply(u);
+    }
+
+    // this lane holds token rows 16 i + idx, columns c0 + 4 kg ..+3
+    const int col = c0 + 4 * kg;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int row = 16 * i + idx;
+        if (row >= p.rows) continue;
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float u = acc[0][0][i][q] + acc[1][0][i][q];
+            if (p.bias0) u = u + p.bias0[col + q];
+            if constexpr (MATS == 2) {
+                float g = acc[0][1][i][q] + acc[1][1][i][q];
+                if (p.bias1) g = g + p.bias1[col + q];
+                v[q] = silu(g) * u;
+            } else {
+                v[q] = act_apply(u, p.act);
+            }
+        }
+        float* out = p.c_base + (int64_t)row * p.N + col;
+        if (p.publish) {
+            publish8(out, __float_as_uint(v[0]), __float_as_uint(v[1]));
+            publish8(out + 2, __float_as_uint(v[2]), __float_as_uint(v[3]));
+        } else {
+            *reinterpret_cast<f32x4*>(out) = f32x4{v[0], v[1], v[2], v[3]};
+        }
+    }
+}
+
+// Groups of 16 rows that the block does not have are neither read nor multiplied.
+__device__ __forceinline__ void stream_rows_f32(const TaskPtrsF& p) {
+    if (p.swiglu) {
+        if (p.rows <= 16) stream_tile_f32<2, 1>(p);
+        else if (p.rows <= 32) stream_tile_f32<2, 2>(p);
+        else stream_tile_f32<2, 4>(p);
+    } else {
+        if (p.rows <= 16) stream_tile_f32<1, 1>(p);
+        else if (p.rows <= 32) stream_tile_f32<1, 2>(p);
+        else stream_tile_f32<1, 4>(p);
+    }
+}
+
+template <bool STREAM>
 __device__ __forceinline__ TaskPtrsF resolve_f32(const FfnArgs& a, const Task& t, bool publish) {
     TaskPtrsF p;
     const int64_t HI = (int64_t)a.H * a.I;
@@ -120,7 +256,7 @@ __device__ __forceinline__ TaskPtrsF resolve_f32(const FfnArgs& a, const Task& t
         p.c_base = (float*)a.h + (int64_t)t.row0 * a.I;
         p.N = a.I;
         p.K = a.H;
-        p.n0 = t.ntile * (sw ? FBN / 2 : FBN);
+        p.n0 = t.ntile * (sw && !STREAM ? FBN / 2 : FBN);
         p.act = a.act;
         p.swiglu = sw;
         p.publish = publish;
@@ -146,21 +282,24 @@ __device__ __forceinline__ TaskPtrsF resolve_f32(const FfnArgs& a, const Task& t
     return p;
 }
 
-__global__ __launch_bounds__(256) void ffn_tiled_f32_kernel(FfnArgs a, int phase) {
-    __shared__ __align__(16) float As[FBK][FBM + FPAD];
-    __shared__ __align__(16) float Bs[FBK][FBN + FPAD];
+template <bool STREAM>
+__global__ __launch_bounds__(256, STREAM ? 3 : 1) void ffn_tiled_f32_kernel(FfnArgs a, int phase) {
+    __shared__ __align__(16) float As[STREAM ? 1 : FBK][FBM + FPAD];
+    __shared__ __align__(16) float Bs[STREAM ? 1 : FBK][FBN + FPAD];
     Task t;
     __shared__ int s_list[1 + FBM];
     if (phase == 0) zero_unrouted_rows(a, 4);
     if (!tiled_task(a, phase, blockIdx.x, t)) return;
-    const TaskPtrsF p = resolve_f32(a, t, phase == 1 && a.arrive);
-    gemm_tile_f32(p, As, Bs);
+    const TaskPtrsF p = resolve_f32<STREAM>(a, t, phase == 1 && a.arrive);
+    if constexpr (STREAM) stream_rows_f32(p);
+    else gemm_tile_f32(p, As, Bs);
     if (phase == 1 && a.arrive) combine_arrivals<float>(combine_args(a), t.row0, t.rows, t.ntile, p.n0, FBN, s_list);
 }
 
-__global__ __launch_bounds__(256) void ffn_persistent_f32_kernel(FfnArgs a) {
-    __shared__ __align__(16) float As[FBK][FBM + FPAD];
-    __shared__ __align__(16) float Bs[FBK][FBN + FPAD];
+template <bool STREAM>
+__global__ __launch_bounds__(256, STREAM ? 3 : 1) void ffn_persistent_f32_kernel(FfnArgs a) {
+    __shared__ __align__(16) float As[STREAM ? 1 : FBK][FBM + FPAD];
+    __shared__ __align__(16) float Bs[STREAM ? 1 : FBK][FBN + FPAD];
     __shared__ int s_task, s_ok;
     __shared__ int s_cmb[kCombineLds];
     __shared__ int s_list[1 + FBM];
@@ -175,10 +314,12 @@ __global__ __launch_bounds__(256) void ffn_persistent_f32_kernel(FfnArgs a) {
     while (next_task(a, cur, &s_task, ids, nseg, nnt0, t)) {
         int ok = 1;
         if (t.phase == 1) ok = wait_phase0_done(a.done0, t.mtile, nnt0, a.spin_limit, a.q, a.host_stall, &s_ok);
-        const TaskPtrsF p = resolve_f32(a, t, t.phase == 0 || publish_y(a));
+        const TaskPtrsF p = resolve_f32<STREAM>(a, t, t.phase == 0 || publish_y(a));
         const long long started = trace_clock(a.task_trace);
-        if (ok) gemm_tile_f32(p, As, Bs);
-        else poison_tile(p.c_base, p.rows, p.N, p.n0, FBN, 4);
+        if (ok) {
+            if constexpr (STREAM) stream_rows_f32(p);
+            else gemm_tile_f32(p, As, Bs);
+        } else poison_tile(p.c_base, p.rows, p.N, p.n0, FBN, 4);
         if (a.task_trace) trace_task(a.task_trace, a.task_trace_cap, t.phase, t.expert, t.mtile, t.ntile, t.rows, started);
         if (t.phase == 0) signal_phase0_done(a.done0, t.mtile);
         else after_down_tile<float>(a, t.row0, t.rows, t.mtile, t.ntile, p.n0, FBN, s_list);
@@ -241,14 +382,20 @@ __global__ __launch_bounds__(256) void wgrad_f32_kernel(const float* dyT, const 
 int f32_block_m() { return FBM; }
 int f32_block_n() { return FBN; }
 
-hipError_t launch_ffn_tiled_f32(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, hipStream_t st) {
-    ffn_tiled_f32_kernel<<<tiled_grid(max_mtiles, nnt0, a.groups), 256, 0, st>>>(a, 0);
-    ffn_tiled_f32_kernel<<<tiled_grid(max_mtiles, nnt1, a.groups), 256, 0, st>>>(a, 1);
+template <bool STREAM>
+static void launch_tiled(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, hipStream_t st) {
+    ffn_tiled_f32_kernel<STREAM><<<tiled_grid(max_mtiles, nnt0, a.groups), 256, 0, st>>>(a, 0);
+    ffn_tiled_f32_kernel<STREAM><<<tiled_grid(max_mtiles, nnt1, a.groups), 256, 0, st>>>(a, 1);
+}
+hipError_t launch_ffn_tiled_f32(const FfnArgs& a, bool stream, int max_mtiles, int nnt0, int nnt1, hipStream_t st) {
+    if (stream) launch_tiled<true>(a, max_mtiles, nnt0, nnt1, st);
+    else launch_tiled<false>(a, max_mtiles, nnt0, nnt1, st);
     return hipGetLastError();
 }
 
-hipError_t launch_ffn_persistent_f32(const FfnArgs& a, int blocks, hipStream_t st) {
-    ffn_persistent_f32_kernel<<<blocks, 256, 0, st>>>(a);
+hipError_t launch_ffn_persistent_f32(const FfnArgs& a, bool stream, int blocks, hipStream_t st) {
+    if (stream) ffn_persistent_f32_kernel<true><<<blocks, 256, 0, st>>>(a);
+    else ffn_persistent_f32_kernel<false><<<blocks, 256, 0, st>>>(a);
     return hipGetLastError();
 }
 

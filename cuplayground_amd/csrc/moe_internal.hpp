@@ -45,6 +45,12 @@ constexpr int kF32TileRowsPerExpert = 128;
 // (H 1024, I 4096: one expert x 1024 rows, 320 tiles, 0.391 / 0.348 ms; one expert x 2048 rows 0.644 / 0.398; four experts,
 // top-2, SwiGLU, 2048 tokens 1.705 / 1.119 ms.)
 constexpr int kF32TileMinTiles = 320;
+// FfnPlan::tile of an fp32 layer below that: the weight streamer of ffn_f32.hip (no option names it) up to this many rows per
+// expert, or up to this many 64 x 64 tasks in both projections; else the 64 x 64 vector-ALU kernel.  Measured, vector / streamer:
+// 16 rows, 8 experts of 4096 x 14336, SwiGLU, 4 rows each 2.99 / 1.02 ms, 32 rows 3.11 / 2.21; 24 rows, 64 of 2048 x 1408 1.05 / 0.79;
+// more rows: 288 tasks 74 / 58 us (128 rows, 8 of 256 x 512), 480 126 / 108 (256, 4 of 512 x 1024) and 331 / 255 (332, one of
+// 1024 x 4096), 748 129 / 110 (1024, 2 of 448 x 960), 832 301 / 353 (150, 4 of 2048 x 2048), 3300 804 / 984 (512, 8 of 960 x 1984).
+constexpr int kF32StreamTile = 2, kF32StreamRowsPerExpert = 32, kF32StreamMaxTasks = 600;
 struct QueueState {
     int32_t groups;        // queue groups (1 or the number of XCDs)
     int32_t total_tasks;   // tasks of both phases (holes not counted)

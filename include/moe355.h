@@ -117,7 +117,7 @@ typedef struct moe_options {
                                 streamer for a few rows per expert, which moe_get_options reports as AUTO here and below */
     int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1; 256 needs
                                 H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0) */
-    int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile; also read by the
+    int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile (AUTO: also the weight streamer, other bits); also read by the
                                 backward entry points of an fp32 handle (there 1 means "where the shape allows") */
     int32_t fp8_tile;        /* e4m3 layers: 0 = weight streamer (decode), 1 = 128x128 tile GEMM */
     int32_t fp8_widen;       /* e4m3 layers: 1 = run the bf16 tiles on bf16 copies of the weights (widened into the workspace

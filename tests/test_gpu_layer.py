@@ -278,6 +278,25 @@ def test_weight_streamer_gives_the_bits_of_the_tiles(moe, name):
     assert again.plan == layer.plan and layer.plan["block_rows"] == rows
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("act", [ob.ACT_RELU, ob.ACT_SWIGLU], ids=["relu", "swiglu"])
+def test_f32_layer_at_the_edges_of_its_row_groups(moe, rows, act):
+    """Small fp32 layers (csrc/ffn_f32.hip) with 1, 2 and 4 groups of 16 rows in a block, a partial last group, several blocks,
+    and contraction dimensions of half a chunk, whole chunks and a remainder; both FFN modes and every combine agree."""
+    cfg = ob.Cfg(S=rows, H=64 if rows % 2 else 320, I=192, E=2, k=2, act=act, dtype=ob.F32, drop=0)
+    inp = ob.make_inputs(cfg, seed=29, with_bias=rows % 2 == 1)
+    want = ob.forward(cfg, inp)
+    first = None
+    for mode in (FFN_TILED, FFN_PERSISTENT):
+        for combine in (0, 1, 2):
+            got = run_layer(moe, cfg, inp, mode, {"combine": combine})
+            check_routing(got, want)
+            assert got["plan"]["block_rows"] == 64
+            assert max_rel_err(got["out"], want["out"]) <= OUT_TOL[cfg.dtype]
+            first = got["out"] if first is None else first
+            assert np.array_equal(got["out"], first), (mode, combine)
+
+
 @pytest.mark.parametrize("name", ["bf16_gelu_ragged", "bf16_swiglu_skew", "f32_swiglu_ragged", "fp8_many_rows_bias",
                                   "fp16_swiglu_skew_bias", "tf32_gelu_ragged", "capacity_one", "many_experts_bias",
                                   "all_experts_selected", "one_token"])

@@ -244,6 +244,14 @@ def _ptr(t):
     return None if t is None else C.c_void_p(t.data_ptr())
 
 
+def _operand(name, t, dtype, elements=0):
+    """The kernels read raw addresses: an operand of another type, or with fewer elements than they read, is refused here."""
+    if t.dtype != dtype:
+        raise TypeError("%s is %s: expected %s" % (name, t.dtype, dtype))
+    if t.numel() < elements:
+        raise ValueError("%s holds %d elements: at least %d are read" % (name, t.numel(), elements))
+
+
 def _stream():
     import torch
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -587,6 +595,8 @@ class MoELayer:
     def dispatch_rows(self, x, token_indices):
         """x_rows[r] = x[token_indices[r]] for the kept packed rows; the rows behind them are not written."""
         import torch
+        _operand("x", x, self.act_dtype, self.S * self.H)
+        _operand("token_indices", token_indices, torch.int32, self.S * self.k)
         rows = torch.empty(self.S * self.k, self.H, dtype=x.dtype, device=x.device)
         _check(self.L.moe_dispatch_rows(self._h, _ptr(x), _ptr(token_indices), _ptr(rows), _stream()), "moe_dispatch_rows")
         return rows
@@ -594,6 +604,9 @@ class MoELayer:
     def act_forward(self, u_rows, g_rows, expert_count, expert_offset):
         """act(u_rows), or silu(g_rows) * u_rows, over the kept packed rows; the rows behind them are not written."""
         import torch
+        for name, t in (("u_rows", u_rows), ("g_rows", g_rows)):
+            if t is not None:
+                _operand(name, t, self.act_dtype)
         h = torch.empty_like(u_rows)
         _check(self.L.moe_act_forward(self._h, _ptr(u_rows), _ptr(g_rows), _ptr(expert_count), _ptr(expert_offset), _ptr(h),
                                       _stream()), "moe_act_forward")
@@ -602,6 +615,10 @@ class MoELayer:
     def dispatch_backward(self, da_rows, db_rows, pair_row):
         """dx[t] = sum over ranks of da_rows[pair_row[t,r]] (+ db_rows[pair_row[t,r]] unless db_rows is None)."""
         import torch
+        for name, t in (("da_rows", da_rows), ("db_rows", db_rows)):
+            if t is not None:
+                _operand(name, t, self.act_dtype)
+        _operand("pair_row", pair_row, torch.int32, self.S * self.k)
         dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
         _check(self.L.moe_dispatch_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(dx), _stream()),
                "moe_dispatch_backward")
@@ -610,6 +627,10 @@ class MoELayer:
     def combine_backward(self, dout, y_rows, pair_row, topk_w, dy=None):
         """(dy_rows, dw [S, k] fp32).  Rows no pair maps to: zero in the buffer made here, untouched in the caller's."""
         import torch
+        _operand("dout", dout, self.act_dtype, self.S * self.H)
+        _operand("y_rows", y_rows, self.act_dtype)
+        _operand("pair_row", pair_row, torch.int32, self.S * self.k)
+        _operand("topk_w", topk_w, torch.float32, self.S * self.k)
         if dy is None:
             dy = torch.zeros_like(y_rows)
         dw = torch.empty(self.S, self.k, dtype=torch.float32, device=dout.device)
@@ -708,6 +729,8 @@ def combine(y_rows, pair_row, topk_w, out=None):
     S, k = pair_row.shape
     H = y_rows.shape[1]
     dtype = {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_FP16}[y_rows.dtype]
+    _operand("pair_row", pair_row, torch.int32, S * k)
+    _operand("topk_w", topk_w, torch.float32, S * k)
     if out is None:
         out = torch.empty(S, H, dtype=y_rows.dtype, device=y_rows.device)
     _check(load_library().moe_combine(_ptr(y_rows), _ptr(pair_row), _ptr(topk_w), S, k, H, dtype, _ptr(out),

@@ -184,6 +184,8 @@ class MoE355Train(torch.nn.Module):
         c = self.cfg
         idx, r = self.route(x)
         count, offset = r["expert_count"], r["expert_offset"]
-        w = self.gate_weights(x, idx)
+        # fp32 whatever gate_weights computed in: the combine reads fp32 (under autocast the logits, and with them a sigmoid's
+        # weights, are 16 bits wide); the cast is undone by autograd
+        w = self.gate_weights(x, idx).float()
         return _Experts.apply(x, self.w_up, self.w_gate, self.w_down, w, self.layer, r["token_indices"], r["pair_row"],
                               count, offset)

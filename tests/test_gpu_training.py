@@ -116,3 +116,27 @@ def test_row_passes_match_plain_torch(moe, S, H, I, E, k, act, cf, dtype):
     pad[1:] = x.reshape(-1)
     dy2, dw2 = layer.combine_backward(pad[1:].view(S, H), a, r["pair_row"], w)
     assert torch.equal(dy2, dy) and float((dw2.double() - want_dw).abs().max()) <= 1e-6 * H
+
+
+@pytest.mark.parametrize("norm", [0, 1])
+def test_a_step_under_autocast_uses_its_gate_weights(moe, norm):
+    """torch.autocast computes the router's logits, and with them a sigmoid's weights, in 16 bits: the step must be the one
+    with exactly those weights, widened."""
+    import torch
+    from cuplayground_amd import training, torch_op
+    cfg = moe.MoEConfig(capacity_factor=1.0, drop_tokens=0, expert_top_k=2, hidden_act=1, hidden_size=256, intermediate_size=128,
+                        micro_batch=1, num_experts=5, sequence_len=301, torch_dtype=2, gate_fn=1, norm_topk_prob=norm, is_training=1)
+    m = training.MoE355Train(cfg, init_std=0.05, seed=3)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").bfloat16()
+    dout = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = m(x)
+        idx, _ = m.route(x)
+        w = m.gate_weights(x, idx)
+    out.backward(dout)
+    ps = {n: p.detach().float() for n, p in m.named_parameters()}
+    ref = torch_op.torch_reference(x.float(), cfg, ps["gate_w"], ps["w_up"], None, ps["w_down"], topk=(idx, w.detach().float()))
+    assert rel(out.float(), ref) <= 1e-2
+    for n, p in m.named_parameters():
+        assert torch.isfinite(p.grad.float()).all() and float(p.grad.float().abs().max()) > 0, n

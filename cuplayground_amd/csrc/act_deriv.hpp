@@ -46,14 +46,14 @@ __device__ __forceinline__ float dgelu16(float d, float u) {
     return settled(d * __builtin_fmaf(u, pdf, cdf));
 }
 
-// The activations themselves for a 16-bit result, shared by the forward tiles' epilogues and moe_act_forward.
+// The activations themselves for a 16-bit result, shared by the epilogues of the forward tiles and the weight streamer.
 // silu: hardware exp2 and reciprocal (about 1 ulp each in fp32, far below the 16-bit rounding of the product that follows)
 // instead of the library expf and an IEEE division.
 __device__ __forceinline__ float silu16(float g) {
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
 }
 // GELU (exact-erf form) without the library erff, which costs some 40 instructions and two divergent branches per element:
-// u * Phi(u) with the erfc of dgelu16 above (|error| <= 1.5e-7 on erfc).  The error of the result stays below 5e-7 in
+// u * Phi(u) with the erfc of dgelu16 above (Abramowitz & Stegun 7.1.26, |error| <= 1.5e-7).  The error of the result stays below 5e-7 in
 // absolute terms and below one bf16 unit in the last place for |u| < 6.
 __device__ __forceinline__ float gelu16(float u) {
     const float x = fabsf(u) * 0.70710678118654752440f;

@@ -110,7 +110,15 @@ class _Experts(torch.autograd.Function):
             g = product(rows, w_gate)
         h = layer.act_forward(u, g, count, offset)
         y = product(h, w_down)
-        ctx.save_for_backward(rows, u, g, h, y, w_up, w_gate, w_down, topk_w, pair_row, count, offset)
+        # kept: what the gradients that are asked for read (a step that trains the router alone reads y)
+        need_x, need_up, need_gate, need_down = ctx.needs_input_grad[:4]
+        need_u = need_x or need_up or need_gate
+
+        def kept(needed, t):
+            return t if needed else None
+
+        ctx.save_for_backward(kept(need_up or need_gate, rows), kept(need_u, u), kept(need_u, g), kept(need_down, h), y,
+                              kept(need_x, w_up), kept(need_x, w_gate), kept(need_u, w_down), topk_w, pair_row, count, offset)
         ctx.layer = layer
         return api.combine(y, pair_row, topk_w)
 

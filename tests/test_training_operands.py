@@ -69,3 +69,69 @@ def test_row_passes_refuse_operands_of_another_type():
     for call in (lambda: layer.dispatch_rows(x[:7], tok), lambda: layer.combine_backward(x[:7], rows, pairs, w)):
         with pytest.raises(ValueError):
             call()
+
+
+class _RowsLayer:
+    """The passes of the expert node as plain torch expressions (one expert, one rank): enough to run the node on the CPU."""
+    fused_act_backward = False
+
+    def dispatch_rows(self, x, tok):
+        return x.clone()
+
+    def expert_gemm(self, a, w, bias, count, offset, act, out=None):
+        return out.copy_(a @ w[0].t())
+
+    def act_forward(self, u, g, count, offset):
+        return torch.relu(u) if g is None else torch.nn.functional.silu(g) * u
+
+    def combine_backward(self, dout, y, pair_row, w, dy=None):
+        return dy.copy_(dout * w), (dout * y).sum(1, keepdim=True)
+
+    def act_backward(self, dh, u, g):
+        with torch.enable_grad():
+            args = [t.detach().requires_grad_(True) for t in (u, g) if t is not None]
+            grads = torch.autograd.grad(self.act_forward(args[0], args[1] if g is not None else None, None, None), args, dh)
+        return grads if g is not None else (grads[0], None)
+
+    def dispatch_backward(self, da, db, pair_row):
+        return da if db is None else da + db
+
+    def expert_wgrad(self, dy, a, count, offset):
+        return (dy.t() @ a).unsqueeze(0)
+
+
+@pytest.mark.parametrize("swiglu", [False, True], ids=["relu", "swiglu"])
+@pytest.mark.parametrize("needs", ["w", "x", "w_up", "w_gate", "w_down", "x w_up w_gate w_down w"])
+def test_the_node_keeps_only_what_its_gradients_read(monkeypatch, swiglu, needs):
+    """Rows, pre-activations, activations and weights stay alive until the backward only where a gradient that is asked for
+    reads them; the gradients are torch's in every combination."""
+    monkeypatch.setattr(api, "combine", lambda y, rows, w: y * w)
+    monkeypatch.setattr(api, "transpose", lambda t: t.transpose(1, 2))
+    S, H, I = 5, 4, 6
+    g = torch.Generator().manual_seed(0)
+    t = {n: torch.randn(*s, generator=g, dtype=torch.float64) for n, s in
+         dict(x=(S, H), w_up=(1, I, H), w_gate=(1, I, H), w_down=(1, H, I), w=(S, 1)).items()}
+    if not swiglu:
+        t["w_gate"] = None
+    want = [n for n in needs.split() if t[n] is not None]
+    if not want:
+        pytest.skip("the layer has no such matrix")
+    for n in want:
+        t[n].requires_grad_(True)
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda v: saved.append(tuple(v.shape)) or v, lambda v: v):
+        out = training._Experts.apply(t["x"], t["w_up"], t["w_gate"], t["w_down"], t["w"], _RowsLayer(), None, None, None, None)
+    wide = 0                                          # [S, I] buffers: u, g and h
+    if {"x", "w_up", "w_gate"} & set(want):
+        wide += 2 if swiglu else 1
+    wide += "w_down" in want
+    assert saved.count((S, I)) == wide
+    assert saved.count((S, H)) == 1 + bool({"w_up", "w_gate"} & set(want))      # y, and the dispatched rows
+    assert saved.count((1, I, H)) == (2 if swiglu else 1) * ("x" in want)
+    dout = torch.randn(S, H, generator=g, dtype=torch.float64)
+    got = torch.autograd.grad(out, [t[n] for n in want], dout)
+    u = t["x"] @ t["w_up"][0].t()
+    h = torch.relu(u) if not swiglu else torch.nn.functional.silu(t["x"] @ t["w_gate"][0].t()) * u
+    ref = torch.autograd.grad(h @ t["w_down"][0].t() * t["w"], [t[n] for n in want], dout)
+    for n, a, b in zip(want, got, ref):
+        assert torch.allclose(a, b, rtol=1e-12, atol=1e-12), n

@@ -195,5 +195,6 @@ class MoE355Train(torch.nn.Module):
         # fp32 whatever gate_weights computed in: the combine reads fp32 (under autocast the logits, and with them a sigmoid's
         # weights, are 16 bits wide); the cast is undone by autograd
         w = self.gate_weights(x, idx).float()
-        return _Experts.apply(x, self.w_up, self.w_gate, self.w_down, w, self.layer, r["token_indices"], r["pair_row"],
+        rows = x if x.shape[0] == c.tokens else x[:c.tokens]      # rows behind the layer's tokens: zero gradients
+        return _Experts.apply(rows, self.w_up, self.w_gate, self.w_down, w, self.layer, r["token_indices"], r["pair_row"],
                               count, offset)

@@ -135,3 +135,15 @@ def test_the_node_keeps_only_what_its_gradients_read(monkeypatch, swiglu, needs)
     ref = torch.autograd.grad(h @ t["w_down"][0].t() * t["w"], [t[n] for n in want], dout)
     for n, a, b in zip(want, got, ref):
         assert torch.allclose(a, b, rtol=1e-12, atol=1e-12), n
+
+
+@pytest.mark.parametrize("extra", [0, 3])
+def test_rows_behind_the_layers_tokens_get_zero_gradients(monkeypatch, extra):
+    """A longer x is a longer buffer with the layer's tokens in front: the node takes those, the gradient has x's shape."""
+    seen = []
+    m = _module(_cfg(), monkeypatch, seen)
+    monkeypatch.setattr(training._Experts, "apply", staticmethod(lambda *a: seen.append(a) or a[0].sum() + a[4].sum()))
+    x = torch.randn(m.cfg.tokens + extra, m.cfg.hidden_size, requires_grad=True)
+    m(x).backward()
+    assert seen[0][0].shape == (m.cfg.tokens, m.cfg.hidden_size) and seen[0][0].data_ptr() == x.data_ptr()
+    assert x.grad.shape == x.shape and (x.grad[:m.cfg.tokens] != 0).all() and not x.grad[m.cfg.tokens:].any()

@@ -1551,7 +1551,7 @@ static int columns256(int N) { return (N + 255) / 256; }
 
 // The weight streamer's form for this many rows per expert, or -1: the tiles are faster.  The first line lies where too many
 // experts begin to have a second block of 16 rows, the second where the tiles' cost, which rows do not change below a row
-// block, is that of the streamer's token rows: both sides measured at 2 to 32 rows, figures in ffn_stream16.hip.
+// block, is that of the streamer's token rows: both sides measured at 2 to 32 rows, figures in ffn_stream16.hip, for uneven routing as well.
 static int stream16_form(int64_t pairs, int experts) {
     const double rows = (double)pairs / experts;
     return rows <= 9 ? 0 : rows <= 17 ? 1 : -1;

@@ -22,11 +22,21 @@
 //   64 of 2048 x 1408, SwiGLU: 2 rows 267 / 221 / 236 / 241, 8 284 / 264 / 276 / 261, 16 290 / 358 / 310 / 284, 24 294 / 468 / 349 / 309
 //   12 of 1344 x 2752, GELU: 2 rows 105 / 63 / 69 / 76, 8 107 / 74 / 82 / 92, 16 106 / 102 / 92 / 99, 24 107 / 117 / 104 / 107
 // (4 rows of the first: 5.7 TB/s of weights behind about 30 us of routing, launches and combine.)  An expert with more rows
-// than a block has its weights read again, which is where the steps upwards come from.  NT 4 is behind the tile from 24 rows
-// on the first and the third of these.  Non-temporal weight loads lose 1 to 15 % (an instruction takes half of a 128-byte
+// than a block had its weights read again for every block in these, which is where the steps upwards come from.  NT 4 was behind
+// the tile from 24 rows on the first and the third of these.  Non-temporal weight loads lose 1 to 15 % (an instruction takes half of a 128-byte
 // line; its other half must still be in the cache for the next one).  The task queue with its written-through rows and pops
 // of this much shorter tasks costs more than the overlap of the projections gives: 645 us against 520 (4 rows of the first),
 // 158 against 81 (4 of the second).
+//
+// The form goes by the average; a skewed router gives some experts many times that.  Their blocks are taken up to 64 rows at a
+// time, the token rows shared through LDS (take_group, stream_group).  Two launches, us -- 128 x 128 tile / every block by itself /
+// groups, for router biases of 1 / rank^s:
+//   64 experts of 2048 x 1408, top-6, 64 tokens: s = 0 338 / 254 / 253, 1.1 222 / 207 / 192, 2 137 / 157 / 136, one set of six 92 / 146 / 73;
+//     96 tokens: 343 / 268 / 265, 233 / 245 / 201, 142 / 185 / 159, 96 / 170 / 112;  170: 348 / 283 / 283, 259 / 258 / 243, 169 / 192 / 173, 119 / 176 / 137
+//   8 of 4096 x 14336, top-2, 32 tokens: 744 / 551 / 538, 745 / 686 / 619, 682 / 679 / 583, one set of two 362 / 352 / 292;
+//     64 tokens: 748 / 610 / 610, 749 / 776 / 708, 687 / 755 / 674, 367 / 418 / 354
+//   16 of 2048 x 2048, top-2, 64 tokens: 122 / 87 / 87, 117 / 92 / 91, 103 / 83 / 78;  128: 125 / 93 / 93, 123 / 127 / 115, 106 / 87 / 85
+// What is left behind the tile are routers that send nearly every one of 96 tokens and more to the same few of many experts.
 #include "act_deriv.hpp"
 #include "ffn_common.hpp"
 
@@ -39,6 +49,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int STHREADS = 256;
+constexpr int kGroupRows = 64, kGroupStage = kGroupRows * 128;      // rows of a group, bytes of 64 values of k of theirs
 
 template <class ET, int NT, int CG>
 struct Stream {
@@ -48,6 +59,7 @@ struct Stream {
     static constexpr int BM = 16 * NT;
     static constexpr int C = CG;             // groups of 16 columns a wavefront owns
     static constexpr int BN = 64 * CG;       // columns of a task
+    static constexpr int WAVES = NT * CG > 1 ? 3 : 4;      // wavefronts per SIMD whose registers its own blocks leave room for
 };
 
 template <class P>
@@ -82,6 +94,45 @@ struct StreamTask {
     int K, N, rows, n0, act;
     bool publish;              // rows are read by other workgroups of the same launch
 };
+
+// Bias, activation and the rows' store.  acc[m * CG + c][i]: matrix m, 16 columns c, 16 token rows i.
+template <class P, int MATS, int NT>
+__device__ __forceinline__ void stream_store(const StreamTask& t, int c0, f32x4 (&acc)[MATS * P::C][NT]) {
+    constexpr int CG = P::C;
+    const int lane = threadIdx.x & 63;
+    const int idx = lane & 15, kg = lane >> 4;
+    // this lane holds token rows 16 i + idx, columns c0 + 16 c + 4 kg ..+3
+    const float relu_floor = t.act == MOE_ACT_RELU ? 0.0f : -INFINITY;      // compare and select: a NaN stays a NaN
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+        const int col = c0 + 16 * c + 4 * kg;
+        float b[MATS][4];
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) b[m][r] = t.bias[m] ? widen1s<P>(t.bias[m][col + r]) : -0.0f;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int row = 16 * i + idx;
+            if (row >= t.rows) continue;
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float u = acc[c][i][r] + b[0][r];
+                if constexpr (MATS == 2) {
+                    const float g = acc[CG + c][i][r] + b[1][r];
+                    v[r] = silu16(g) * u;
+                } else {
+                    v[r] = t.act == MOE_ACT_GELU ? gelu16(u) : (u < relu_floor ? relu_floor : u);
+                }
+            }
+            uint16_t* p = t.c_base + (int64_t)row * t.N + col;
+            const uint32_t lo = pack2s<P>(v[0], v[1]), hi = pack2s<P>(v[2], v[3]);
+            if (t.publish) publish8(p, lo, hi);
+            else *reinterpret_cast<uint2*>(p) = uint2{lo, hi};
+        }
+    }
+}
 
 // MATS: weight matrices (2: SwiGLU's up and gate).  K and N are multiples of 64 (moe_config_validate), so a wavefront's
 // columns exist together or not at all.
@@ -156,37 +207,7 @@ __device__ __forceinline__ void stream_tile(const StreamTask& t) {
             if (u < left) multiply(u);
     }
 
-    // this lane holds token rows 16 i + idx, columns c0 + 16 c + 4 kg ..+3
-    const float relu_floor = t.act == MOE_ACT_RELU ? 0.0f : -INFINITY;      // compare and select: a NaN stays a NaN
-#pragma unroll
-    for (int c = 0; c < CG; ++c) {
-        const int col = c0 + 16 * c + 4 * kg;
-        float b[MATS][4];
-#pragma unroll
-        for (int m = 0; m < MATS; ++m)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) b[m][r] = t.bias[m] ? widen1s<P>(t.bias[m][col + r]) : -0.0f;
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            const int row = 16 * i + idx;
-            if (row >= t.rows) continue;
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float u = acc[c][i][r] + b[0][r];
-                if constexpr (MATS == 2) {
-                    const float g = acc[CG + c][i][r] + b[1][r];
-                    v[r] = silu16(g) * u;
-                } else {
-                    v[r] = t.act == MOE_ACT_GELU ? gelu16(u) : (u < relu_floor ? relu_floor : u);
-                }
-            }
-            uint16_t* p = t.c_base + (int64_t)row * t.N + col;
-            const uint32_t lo = pack2s<P>(v[0], v[1]), hi = pack2s<P>(v[2], v[3]);
-            if (t.publish) publish8(p, lo, hi);
-            else *reinterpret_cast<uint2*>(p) = uint2{lo, hi};
-        }
-    }
+    stream_store<P, MATS, NT>(t, c0, acc);
 }
 
 template <class P>
@@ -225,20 +246,129 @@ __device__ __forceinline__ StreamTask resolve_stream(const FfnArgs& a, const Tas
     return p;
 }
 
-template <class P>
-__device__ __forceinline__ void stream_task(const FfnArgs& a, const Task& t, bool publish) {
-    const StreamTask p = resolve_stream<P>(a, t, publish);
-    if (t.phase == 0 && a.act == MOE_ACT_SWIGLU) stream_tile<P, 2>(p);
-    else stream_tile<P, 1>(p);
+// The same for up to 16 NT rows, more than a block has (take_group): the token rows go through LDS, 64 values of k at a time,
+// once for the four wavefronts.  Weights as above, in the same order of k, hence the same bits.  Few workgroups have such a
+// task, so nothing but a wavefront's own requests hides the memory's latency: two slabs of weights are always on their way,
+// each requested as soon as the registers of the slab before the last are free.
+template <class P, int MATS, int NT>
+__device__ __forceinline__ void stream_group(const StreamTask& t, unsigned char* smem) {
+    constexpr int CG = P::C, G = MATS * CG, PASSES = NT / 2;      // a pass brings 32 rows of 128 bytes
+    constexpr int XD = G > 2 ? 1 : 2;            // slabs of rows in registers on their way to LDS (one: four weight fragments leave no room)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int idx = lane & 15, kg = lane >> 4;
+    const int c0 = t.n0 + 16 * CG * wave;
+    const bool live = c0 < t.N;                  // a wavefront without columns helps to bring the rows
+    // 32-bit offsets from bases that are the same in every lane: operands are below 4 GiB (large_tile_ok)
+    const uint32_t w_off = (uint32_t)(idx * t.K + 8 * kg) * 2;
+    uint32_t x_off[PASSES];
+#pragma unroll
+    for (int n = 0; n < PASSES; ++n) {
+        const int row = (tid >> 3) + 32 * n, r = row < t.rows ? row : 0;      // rows behind the last one are never stored
+        x_off[n] = (uint32_t)(((t.gather ? (int64_t)t.gather[r] : t.a_row0 + r) * t.K + 8 * (tid & 7)) * 2);
+    }
+    // 16-byte piece p of row r lies at p ^ (r >> 1 & 7): the 16 rows of a fragment read then meet all banks
+    unsigned char* put = smem + (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 4) & 7)) << 4);
+    const unsigned char* get = smem + idx * 128;
+    const int sw = (idx >> 1) & 7;
+
+    f32x4 acc[G][NT];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[g][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int slabs = t.K >> 6;
+    u32x4 w[2][G][2], x[XD][PASSES];
+    // slabs behind the last one read it again (and are not multiplied)
+    auto load_x = [&](u32x4 (&d)[PASSES], int slab) {
+        const char* base = reinterpret_cast<const char*>(t.a_base + (min(slab, slabs - 1) << 6));
+#pragma unroll
+        for (int n = 0; n < PASSES; ++n) d[n] = *reinterpret_cast<const u32x4*>(base + x_off[n]);
+    };
+    auto load_w = [&](u32x4 (&d)[G][2], int slab) {
+        const int k = min(slab, slabs - 1) << 6;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const char* base = reinterpret_cast<const char*>(t.w[g / CG] + (int64_t)((live ? c0 : 0) + 16 * (g % CG)) * t.K + k);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) d[g][u] = *reinterpret_cast<const u32x4*>(base + 64 * u + w_off);
+        }
+    };
+    auto put_x = [&](const u32x4 (&d)[PASSES], int stage) {
+#pragma unroll
+        for (int n = 0; n < PASSES; ++n) *reinterpret_cast<u32x4*>(put + stage * kGroupStage + n * 32 * 128) = d[n];
+    };
+    // slab's rows lie in stage S; its successor's go into the other one, which was last read in front of the last barrier
+    auto step = [&](auto S, int slab) {
+        constexpr int st = decltype(S)::value;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                const u32x4 b = *reinterpret_cast<const u32x4*>(get + st * kGroupStage + i * 16 * 128 + (((4 * u + kg) ^ sw) << 4));
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[g][i] = mfma32<P>(w[st][g][u], b, acc[g][i]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        put_x(x[(st ^ 1) % XD], st ^ 1);
+        load_x(x[(st ^ 1) % XD], slab + 1 + XD);
+        load_w(w[st], slab + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    load_x(x[0], 0);
+    load_w(w[0], 0);
+    if constexpr (XD == 2) load_x(x[1], 1);
+    load_w(w[1], 1);
+    put_x(x[0], 0);
+    load_x(x[0], XD);
+    __syncthreads();
+    for (int slab = 0; slab < slabs; slab += 2) {
+        step(std::integral_constant<int, 0>{}, slab);
+        if (slab + 1 < slabs) step(std::integral_constant<int, 1>{}, slab + 1);
+    }
+    if (live) stream_store<P, MATS, NT>(t, c0, acc);
+}
+
+// smem: null where a task never has more rows than a block.
+template <class P, int MATS>
+__device__ __forceinline__ void stream_rows(const StreamTask& p, unsigned char* smem) {
+    if (!smem || p.rows <= P::BM) stream_tile<P, MATS>(p);
+    else if (P::BM < 32 && p.rows <= 32) stream_group<P, MATS, 2>(p, smem);
+    else stream_group<P, MATS, kGroupRows / 16>(p, smem);
 }
 
 template <class P>
-__global__ __launch_bounds__(STHREADS) void ffn_tiled_stream16_kernel(FfnArgs a, int phase) {
-    __shared__ int s_list[1 + P::BM];
+__device__ __forceinline__ void stream_task(const FfnArgs& a, const Task& t, bool publish, unsigned char* smem) {
+    const StreamTask p = resolve_stream<P>(a, t, publish);
+    if (t.phase == 0 && a.act == MOE_ACT_SWIGLU) stream_rows<P, 2>(p, smem);
+    else stream_rows<P, 1>(p, smem);
+}
+
+// The row blocks of an expert that was given more rows than a block holds, kGroupRows rows at a time: one block's task takes
+// the group, the others have nothing to do (false).  The average that chooses the streamer says nothing about the fullest
+// expert, and without this its weights are read again for every block.  Which block's varies with the column, because the
+// blocks of a column are neighbours in the launch and go to the XCDs in turn: with the first one's, four blocks to an expert
+// would leave the work to two of the eight XCDs.
+template <class P>
+__device__ __forceinline__ bool take_group(const FfnArgs& a, Task& t) {
+    const Segment& s = a.seg_phase0[t.expert];
+    constexpr int N = kGroupRows / P::BM;
+    const int pos = t.mtile - s.mt0, first = pos / N * N, blocks = min(N, s.nmt - first);
+    if (blocks == 1) return true;
+    if (pos - first != (t.ntile * s.nmt >> 3) % blocks) return false;
+    t.row0 -= (pos - first) * P::BM;
+    t.rows = (blocks - 1) * P::BM + a.mtiles[s.mt0 + first + blocks - 1].rows;
+    return true;
+}
+
+template <class P>
+__global__ __launch_bounds__(STHREADS, P::WAVES) void ffn_tiled_stream16_kernel(FfnArgs a, int phase) {
+    __shared__ int s_list[1 + kGroupRows];
+    __shared__ __align__(16) unsigned char smem[2 * kGroupStage];
     if (phase == 0) zero_unrouted_rows(a, 2);
     Task t;
-    if (!tiled_task(a, phase, blockIdx.x, t)) return;
-    stream_task<P>(a, t, phase == 1 && a.arrive);
+    if (!tiled_task(a, phase, blockIdx.x, t) || !take_group<P>(a, t)) return;
+    stream_task<P>(a, t, phase == 1 && a.arrive, smem);
     if (phase == 1 && a.arrive) combine_arrivals<typename P::Elem>(combine_args(a), t.row0, t.rows, t.ntile, t.ntile * P::BN, P::BN, s_list);
 }
 
@@ -261,7 +391,7 @@ __global__ __launch_bounds__(STHREADS) void ffn_persistent_stream16_kernel(FfnAr
         const long long started = trace_clock(a.task_trace);
         const bool publish = t.phase == 0 || publish_y(a);
         if (ok) {
-            stream_task<P>(a, t, publish);
+            stream_task<P>(a, t, publish, nullptr);
         } else {
             const StreamTask p = resolve_stream<P>(a, t, publish);
             poison_tile(p.c_base, p.rows, p.N, p.n0, P::BN, 2);

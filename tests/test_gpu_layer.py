@@ -278,6 +278,40 @@ def test_weight_streamer_gives_the_bits_of_the_tiles(moe, name):
     assert again.plan == layer.plan and layer.plan["block_rows"] == rows
 
 
+HOT_EXPERT = {
+    # rows of one expert beside a few of the others: up to and past 16, 32, 64 and 128 rows.  Dimensions of one slab of 64, an odd and an even
+    # number of them, column tasks that the last wavefronts have no columns of (form of 32 rows: 128 columns a task)
+    **{"narrow_%d_rows" % n: (ob.Cfg(S=n, H=320, I=192, E=2 + n * 2 // 9, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=0), 16)
+       for n in (17, 32, 33, 48, 49, 64, 65, 81, 130)},
+    **{"wide_%d_rows" % n: (ob.Cfg(S=n, H=192, I=320, E=1 + n * 2 // 17, k=2, act=ob.ACT_SWIGLU, dtype=ob.F16, drop=0), 32)
+       for n in (33, 63, 64, 65, 97, 130)},
+    "narrow_one_slab_gelu_bias": (ob.Cfg(S=60, H=64, I=64, E=16, k=2, act=ob.ACT_GELU, dtype=ob.F16, drop=0), 16),
+    "wide_one_slab_relu_bias": (ob.Cfg(S=75, H=64, I=64, E=10, k=2, act=ob.ACT_RELU, dtype=ob.BF16, drop=0), 32),
+    "narrow_drop": (ob.Cfg(S=90, H=256, I=448, E=24, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=1, capacity_factor=5.0), 16),
+    "wide_drop_bias": (ob.Cfg(S=99, H=448, I=256, E=14, k=2, act=ob.ACT_GELU, dtype=ob.BF16, drop=1, capacity_factor=5.0), 32),
+}
+
+
+@pytest.mark.parametrize("name", sorted(HOT_EXPERT))
+def test_weight_streamer_takes_the_rows_of_a_full_expert_together(moe, name):
+    """A router that sends every token to one expert: its row blocks go through the streamer in groups of up to 64 rows in
+    the two launches, whatever order the tasks have, and singly from the queue, with the bits of the 128 x 256 tile."""
+    cfg, rows = HOT_EXPERT[name]
+    inp = ob.make_inputs(cfg, seed=31, with_bias="bias" in name)
+    inp["gate_bias"] = np.zeros(cfg.E, np.float32)
+    inp["gate_bias"][cfg.E // 2] = 20.0
+    want = ob.forward(cfg, inp)
+    assert want["expert_count"][cfg.E // 2] == (min(cfg.S, cfg.capacity) if cfg.drop else cfg.S) > rows
+    tile = run_layer(moe, cfg, inp, FFN_TILED, {"tile16": 2})
+    for mode, options in [(FFN_TILED, {"combine": 0}), (FFN_TILED, {"combine": 1}), (FFN_TILED, {"queue_groups": 8}),
+                          (FFN_TILED, {"row_chunk": 3}), (FFN_PERSISTENT, {"combine": 0})]:
+        got = run_layer(moe, cfg, inp, mode, options)
+        check_routing(got, want)
+        assert got["plan"]["block_rows"] == rows
+        assert max_rel_err(ob.to_f32(got["out"], cfg.act_dtype), ob.to_f32(want["out"], cfg.act_dtype)) <= OUT_TOL[cfg.dtype]
+        assert np.array_equal(got["out"], tile["out"]), (mode, options)
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 130])
 @pytest.mark.parametrize("act", [ob.ACT_RELU, ob.ACT_SWIGLU], ids=["relu", "swiglu"])
 def test_f32_layer_at_the_edges_of_its_row_groups(moe, rows, act):

@@ -102,7 +102,7 @@ def test_no_accumulator_access_behind_asm_mfma():
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-@pytest.mark.parametrize("source", ["ffn_bf16.hip", "ffn_f32.hip", "ffn_f32_tile.hip", "ffn_fp8.hip", "ffn_fp8_tile.hip"])
+@pytest.mark.parametrize("source", ["ffn_bf16.hip", "ffn_stream16.hip", "ffn_f32.hip", "ffn_f32_tile.hip", "ffn_fp8.hip", "ffn_fp8_tile.hip"])
 def test_phase0_results_are_complete_before_they_are_signalled(source):
     """The hand-off of the intermediate rows between workgroups: in signal_phase0_done every wavefront must wait for
     its own stores (s_waitcnt vmcnt(0)) before the workgroup barrier and the counter increment that publishes the

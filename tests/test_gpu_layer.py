@@ -35,6 +35,7 @@ def run_layer(moe, cfg, inp, mode, options=None):
     res = {k: from_device(v) for k, v in routing.items()}
     res["out"] = from_device(out)
     res["plan"] = layer.plan
+    res["options"] = layer.options
     layer.close()
     return res
 
@@ -325,7 +326,7 @@ def test_f32_layer_at_the_edges_of_its_row_groups(moe, rows, act):
         for combine in (0, 1, 2):
             got = run_layer(moe, cfg, inp, mode, {"combine": combine})
             check_routing(got, want)
-            assert got["plan"]["block_rows"] == 64
+            assert got["plan"]["block_rows"] == 64 and got["options"]["f32_tile"] == -1      # the streamer: the vector kernel reports 0
             assert max_rel_err(got["out"], want["out"]) <= OUT_TOL[cfg.dtype]
             first = got["out"] if first is None else first
             assert np.array_equal(got["out"], first), (mode, combine)

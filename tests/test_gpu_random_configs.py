@@ -23,7 +23,7 @@ def _cases(n=36, seed=2024):
             act = ob.ACT_SWIGLU                  # e4m3 layers: SwiGLU at least every other time
         E = int(rng.choice([1, 2, 3, 4, 6, 8, 16, 40]))
         k = int(rng.integers(1, min(E, 4) + 1))
-        mult = 128 if dtype == ob.FP8 else (256 if i % 2 == 0 else 64)        # multiples of 256 reach the hand-ordered tiles
+        mult = 128 if dtype == ob.FP8 else (256 if i % 2 == 0 else 64)        # multiples of 256: whole column tiles and pairs of slabs of the hand-ordered tiles
         H = mult * int(rng.integers(1, 3))
         I = mult * int(rng.integers(1, 4))
         S = int(rng.integers(1, 2600 if i % 2 == 0 else 900))     # the larger ones give experts several row blocks
@@ -53,7 +53,28 @@ def _cases(n=36, seed=2024):
     return out
 
 
-@pytest.mark.parametrize("cfg,knobs,mode,with_bias", _cases())
+def _few_row_cases(n=20, seed=77):
+    """Layers of a few rows per expert with the tile left to the library: the weight streamers (_cases names a tile in each)."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for i in range(n):
+        dtype = [ob.BF16, ob.F16, ob.F32][i % 3]
+        E = int(rng.choice([2, 3, 5, 8, 16, 40]))
+        k = int(rng.integers(1, min(E, 4) + 1))
+        rows = float(rng.uniform(1, 32 if dtype == ob.F32 else 17))           # per expert on average
+        S = max(1, int(rows * E / k))
+        drop = int(rng.integers(0, 2))
+        cfg = ob.Cfg(S=S, H=64 * int(rng.integers(1, 9)), I=64 * int(rng.integers(1, 9)), E=E, k=k,
+                     act=int(rng.choice([ob.ACT_RELU, ob.ACT_GELU, ob.ACT_SWIGLU])), dtype=dtype, drop=drop,
+                     capacity_factor=float(rng.choice([0.5, 1.0, 3.0])), norm_topk=int(k > 1), gate_fn=int(rng.integers(0, 2)),
+                     zipf_bias=bool(i % 2))
+        knobs = dict(queue_groups=int(rng.choice([1, 2, 8])), combine=int(rng.integers(0, 3)), row_chunk=i % 4, tail_round=i % 2,
+                     tail_split=(1, 2, 4)[i % 3])
+        out.append(pytest.param(cfg, knobs, int(rng.integers(1, 3)), bool(rng.integers(0, 2)), id="few_rows%02d" % i))
+    return out
+
+
+@pytest.mark.parametrize("cfg,knobs,mode,with_bias", _cases() + _few_row_cases())
 def test_random_shape_and_knobs_vs_oracle(cfg, knobs, mode, with_bias):
     import torch
     import cuplayground_amd as moe
@@ -61,6 +82,8 @@ def test_random_shape_and_knobs_vs_oracle(cfg, knobs, mode, with_bias):
     inp = ob.make_inputs(cfg, seed=17, with_bias=with_bias)
     want = ob.forward(cfg, inp)
     layer = moe.MoELayer(product_config(cfg), ffn_mode=mode, options=knobs)
+    if "tile16" not in knobs:
+        assert layer.options["f32_tile"] == -1 if cfg.dtype == ob.F32 else layer.plan["block_rows"] in (16, 32)
     dev = upload_inputs(cfg, inp)
     routing = layer.new_routing()
     out = torch.full((cfg.S, cfg.H), float("nan"), dtype=layer.act_dtype, device="cuda")

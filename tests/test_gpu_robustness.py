@@ -9,6 +9,7 @@ from helpers import OUT_TOL, from_device, max_rel_err, product_config, to_device
 pytestmark = pytest.mark.gpu
 FFN_TILED, FFN_PERSISTENT = 1, 2
 STALL = 7   # MOE_ERR_QUEUE_STALL
+AUTO = -1   # MOE_OPT_AUTO
 
 
 @pytest.fixture(scope="module")
@@ -85,6 +86,10 @@ def test_route_drops_out_of_range_expert_ids(moe):
     ("fp8_tile", ob.Cfg(S=600, H=256, I=256, E=4, k=2, act=ob.ACT_SWIGLU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, drop=0)),
     # the fp32 matrix-core tile (forced: the layer is too small for the plan to pick it)
     ("f32_tile", ob.Cfg(S=600, H=256, I=128, E=2, k=1, act=ob.ACT_SWIGLU, dtype=ob.F32, norm_topk=0, drop=0)),
+    # the 16-bit weight streamer in both forms, and the fp32 one
+    ("stream_narrow", ob.Cfg(S=33, H=192, I=320, E=8, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=0)),
+    ("stream_wide", ob.Cfg(S=65, H=320, I=192, E=8, k=2, act=ob.ACT_GELU, dtype=ob.F16, drop=0)),
+    ("stream_f32", ob.Cfg(S=100, H=192, I=320, E=4, k=2, act=ob.ACT_SWIGLU, dtype=ob.F32, drop=0)),
 ])
 @pytest.mark.parametrize("combine", [0, 1, 2], ids=["combine_launch", "combine_arrivals", "combine_queue"])
 def test_expired_dependency_wait_poisons_the_output_and_is_reported(moe, name, cfg, combine):
@@ -97,8 +102,10 @@ def test_expired_dependency_wait_poisons_the_output_and_is_reported(moe, name, c
     want = ob.forward(cfg, inp)
     # the combine inside the FFN kernels must carry the NaNs too
     layer = moe.MoELayer(product_config(cfg), ffn_mode=FFN_PERSISTENT,
-                         options={"combine": combine, "f32_tile": 1 if name == "f32_tile" else 0})
+                         options={"combine": combine, "f32_tile": {"f32_tile": 1, "stream_f32": AUTO}.get(name, 0)})
     assert name != "f32_tile" or layer.plan["block_rows"] == 128
+    assert name not in ("stream_narrow", "stream_wide") or layer.plan["block_rows"] == (16 if name == "stream_narrow" else 32)
+    assert name != "stream_f32" or layer.options["f32_tile"] == AUTO      # reported for the streamer alone
     dev = upload_inputs(cfg, inp)
     layer.set_spin_limit(-1)
     out = layer.forward(dev["x"], dev)          # enqueues; the stall is not known yet

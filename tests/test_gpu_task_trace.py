@@ -8,6 +8,7 @@ from helpers import product_config, upload_inputs
 from test_gpu_layer import FFN_PERSISTENT, FFN_TILED
 
 pytestmark = pytest.mark.gpu
+AUTO = -1   # MOE_OPT_AUTO
 
 CASES = {
     "bf16_large_tile": ob.Cfg(S=2500, H=256, I=512, E=4, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=0),
@@ -15,6 +16,10 @@ CASES = {
     "f32": ob.Cfg(S=333, H=192, I=320, E=7, k=3, act=ob.ACT_SWIGLU, dtype=ob.F32, drop=1, capacity_factor=0.75),
     "f32_tile": ob.Cfg(S=900, H=256, I=384, E=3, k=2, act=ob.ACT_GELU, dtype=ob.F32, drop=0),
     "fp8_streamer": ob.Cfg(S=64, H=512, I=256, E=32, k=8, act=ob.ACT_SWIGLU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, drop=0),
+    # the weight streamers, with experts of several row blocks
+    "stream_narrow": ob.Cfg(S=60, H=192, I=320, E=16, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, drop=0, zipf_bias=True),
+    "stream_wide": ob.Cfg(S=120, H=320, I=192, E=16, k=2, act=ob.ACT_GELU, dtype=ob.F16, drop=0, zipf_bias=True),
+    "stream_f32": ob.Cfg(S=120, H=192, I=320, E=5, k=2, act=ob.ACT_SWIGLU, dtype=ob.F32, drop=0, zipf_bias=True),
     "fp8_tile": ob.Cfg(S=1500, H=384, I=256, E=6, k=2, act=ob.ACT_SWIGLU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, drop=0),
 }
 
@@ -29,12 +34,15 @@ def test_every_task_is_recorded_once_and_in_dependency_order(name):
         options["queue_early"] = 1
         name = name[:-len("_early_start")]
     cfg = CASES[name]
-    options["f32_tile"] = 1 if name == "f32_tile" else 0
+    options["f32_tile"] = {"f32_tile": 1, "stream_f32": AUTO}.get(name, 0)
     inp = ob.make_inputs(cfg, seed=13)
     want = ob.route(cfg, inp)
     layer = moe.MoELayer(product_config(cfg), ffn_mode=FFN_PERSISTENT, options=options)
     dev = upload_inputs(cfg, inp)
     plan = layer.plan
+    if name.startswith("stream"):
+        assert plan["block_rows"] == {"stream_narrow": 16, "stream_wide": 32, "stream_f32": 64}[name]
+        assert name != "stream_f32" or layer.options["f32_tile"] == AUTO      # reported for the streamer alone
     layer.enable_task_trace(1 << 14)
     ref = layer.forward(dev["x"], dev).clone()
     for _ in range(2):                       # the trace holds the last call only

@@ -165,3 +165,36 @@ def test_training_activation_is_the_fp32_function(moe, act, dtype):
     tail = ok & (f < 0) & (f >= -4)                       # where 1 + erf cancels
     assert float((got != want)[tail].float().mean()) <= 1e-3
     assert float((got != want)[ok].float().mean()) <= 1e-3
+
+
+@pytest.mark.parametrize("act,dtype,inter", [(2, 2, 384), (1, 3, 512), (0, 0, 384), (2, 0, 128)])
+def test_a_layer_composed_of_the_projection_nodes_is_the_layer(moe, act, dtype, inter):
+    """expert_linear and act_down with gather and combine as torch indexing against MoE355Train on the same weights: each is
+    within the tolerance of test_trainable_layer_matches_torch_autograd of the same fp32 layer, so they are within twice that."""
+    import torch
+    from cuplayground_amd import training
+    cfg = moe.MoEConfig(capacity_factor=0.9, drop_tokens=1, expert_top_k=2, hidden_act=act, hidden_size=256,
+                        intermediate_size=inter, micro_batch=1, num_experts=5, sequence_len=333,
+                        torch_dtype=dtype, gate_fn=0, norm_topk_prob=1, is_training=1)
+    m = training.MoE355Train(cfg, init_std=0.05, seed=3)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype).requires_grad_(True)
+    dout = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype)
+    leaves = dict(m.named_parameters(), x=x)
+
+    def step(out):
+        return out, dict(zip(leaves, torch.autograd.grad(out, leaves.values(), dout)))
+
+    idx, r = m.route(x)
+    count, offset, pairs = r["expert_count"], r["expert_offset"], r["pair_row"]
+    x_rows = x.index_select(0, r["token_indices"].clamp(min=0).long())      # rows of no expert gather token 0 and are not used
+    up = training.expert_linear(x_rows, m.w_up, m.layer, count, offset)
+    gate = training.expert_linear(x_rows, m.w_gate, m.layer, count, offset) if act == 2 else None
+    y = training.act_down(up, gate, m.w_down, m.layer, count, offset)
+    picked = y[pairs.clamp(min=0).long()].float() * (pairs >= 0).unsqueeze(-1)
+    composed, grads = step((picked * m.gate_weights(x, idx).unsqueeze(-1)).sum(1).to(x.dtype))
+    out, want = step(m(x))
+    assert int((pairs < 0).sum()) > 0
+    assert rel(composed, out) <= 2 * {2: 1e-2, 3: 2e-3}.get(dtype, 2e-5)
+    for n in leaves:
+        assert rel(grads[n], want[n]) <= 2 * {2: 2e-2, 3: 4e-3}.get(dtype, 1e-4), n

@@ -604,9 +604,9 @@ class MoELayer:
     def act_forward(self, u_rows, g_rows, expert_count, expert_offset):
         """act(u_rows), or silu(g_rows) * u_rows, over the kept packed rows; the rows behind them are not written."""
         import torch
-        for name, t in (("u_rows", u_rows), ("g_rows", g_rows)):
-            if t is not None:
-                _operand(name, t, self.act_dtype)
+        _operand("u_rows", u_rows, self.act_dtype)
+        if g_rows is not None:
+            _operand("g_rows", g_rows, self.act_dtype, u_rows.numel())
         h = torch.empty_like(u_rows)
         _check(self.L.moe_act_forward(self._h, _ptr(u_rows), _ptr(g_rows), _ptr(expert_count), _ptr(expert_offset), _ptr(h),
                                       _stream()), "moe_act_forward")
@@ -615,9 +615,9 @@ class MoELayer:
     def dispatch_backward(self, da_rows, db_rows, pair_row):
         """dx[t] = sum over ranks of da_rows[pair_row[t,r]] (+ db_rows[pair_row[t,r]] unless db_rows is None)."""
         import torch
-        for name, t in (("da_rows", da_rows), ("db_rows", db_rows)):
-            if t is not None:
-                _operand(name, t, self.act_dtype)
+        _operand("da_rows", da_rows, self.act_dtype)
+        if db_rows is not None:
+            _operand("db_rows", db_rows, self.act_dtype, da_rows.numel())
         _operand("pair_row", pair_row, torch.int32, self.S * self.k)
         dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
         _check(self.L.moe_dispatch_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(dx), _stream()),

@@ -66,7 +66,8 @@ def test_row_passes_refuse_operands_of_another_type():
     for call in bad:
         with pytest.raises(TypeError):
             call()
-    for call in (lambda: layer.dispatch_rows(x[:7], tok), lambda: layer.combine_backward(x[:7], rows, pairs, w)):
+    for call in (lambda: layer.dispatch_rows(x[:7], tok), lambda: layer.combine_backward(x[:7], rows, pairs, w),
+                 lambda: layer.act_forward(rows, rows[:15], None, None), lambda: layer.dispatch_backward(rows, rows[:15], pairs)):
         with pytest.raises(ValueError):
             call()
 

@@ -557,8 +557,10 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
                                   dtype == MOE_DTYPE_FP16, st);
 }
 
-// The tile the fused data gradient (product + activation derivative) would run on: 1 or 2 (the hand-ordered tiles), or 0
-// when the shape or the options leave only the 128 x 128 tile, which has no such epilogue.
+// The tile the fused data gradient (product + activation derivative) runs on: 1 or 2 (the hand-ordered tiles), or 0 where
+// there is none: option grouped_tile = 0 (the 128 x 128 tile has no such epilogue), operands of 4 GiB and more, and ragged
+// dimensions.  The tiles themselves take those; what moe_expert_gemm_act_backward_supported answers for them, and the
+// two-call chain behind it, is from before they did.
 int expert_gemm_dact_tile(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
     if (dtype != MOE_DTYPE_BF16 && dtype != MOE_DTYPE_FP16) return 0;
     const bool hand_ok = N % 256 == 0 && K % 128 == 0 && grouped_hand_ok(A, N, K);

@@ -116,8 +116,8 @@ __device__ __forceinline__ void gemm_tile_f32(const TaskPtrsF& p, float (*As)[FB
 //
 // What bounds a small layer is latency: 128 rows on 8 experts of 256 x 512 are 1 us of arithmetic for 64 and 32 tasks.  The
 // LDS-tiled FMA kernel above waits for memory and two barriers every 16 values of k and always computes 64 rows;
-// here eight slabs (16 KB a wavefront) are in flight, nothing is waited for but the operands, and groups of 16 rows that a
-// block does not have cost nothing.  Whole layer, that kernel -> this one, us: 128 tokens, 8 experts of 256 x 512, GELU 67.6 ->
+// here 8 KB of weights a wavefront are in flight (eight slabs of one matrix, four of SwiGLU's two; half of that for blocks of more than
+// 32 rows, whose token rows take the registers), nothing is waited for but the operands, and groups of 16 rows that a block does not have cost nothing.  Whole layer, that kernel -> this one, us: 128 tokens, 8 experts of 256 x 512, GELU 67.6 ->
 // 33.2; 40 tokens top-2 of 16, 128 x 768 76 -> 34; 192 tokens, 4 of 448 x 640 90 -> 72; 537 tokens, 8 of 384 x 256 64 -> 52; 332
 // tokens, one of 1024 x 4096 331 -> 255; 16 tokens, 8 of 4096 x 14336, SwiGLU 2990 -> 1020.  Error against float64: 5.2e-7 -> 3.7e-7
 // (first), 1.0e-6 -> 7.0e-7 (fifth).  Where full blocks keep the chip busy it loses to the LDS kernel, which reads a token row

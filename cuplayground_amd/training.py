@@ -91,8 +91,9 @@ def _aligned(t):
 class _Experts(torch.autograd.Function):
     """(x [S,H], expert weights, topk_w [S,k]) -> the gate-weighted sum of the chosen experts' outputs.
 
-    The whole expert side of a training step as one node over packed rows: rows of no expert are never read, so no buffer
-    is cleared, and dispatch, activation, combine and their adjoints are one pass each."""
+    The whole expert side of a training step as one node over packed rows.  No result depends on the rows of no expert, so no
+    buffer is cleared (the activation's derivative as a pass of its own computes on what lies there; nobody reads that), and
+    dispatch, activation, combine and their adjoints are one pass each."""
 
     @staticmethod
     def forward(ctx, x, w_up, w_gate, w_down, topk_w, layer, token_indices, pair_row, count, offset):

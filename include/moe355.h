@@ -105,8 +105,8 @@ typedef struct moe_handle moe_handle;
  * (CMakeLists.txt:204-216), and chooses tiles and schedulers at compile time (processor/tiling.cuh:97-159,
  * scheduling.cuh:170-200 against warpScheduler.cuh:167-265); these are the same choices as run-time values of a handle.
  * Every field is MOE_OPT_AUTO (the library chooses) or one of the values named beside it; a value outside its domain
- * makes moe_create_with_options return MOE_ERR_BAD_ARGUMENT, a value the layer's shape cannot take (block_rows = 256
- * on a layer with H % 256 != 0, say) falls back to the library's choice.  Results never depend on these options beyond
+ * makes moe_create_with_options return MOE_ERR_BAD_ARGUMENT, a value the layer's shape cannot take (f32_tile = 1 on a
+ * layer with H % 128 != 0, say) falls back to the library's choice, except where its field names another.  Results never depend on these options beyond
  * what is said here: schedules and tiles of one dtype agree bit for bit except where a field says otherwise.
  * Options are fixed when the handle is created; two handles of one process may differ in every one of them.
  */
@@ -116,9 +116,11 @@ typedef struct moe_options {
                                 3 = 256x256 with the 128x256 tile for row blocks of at most 128 rows; AUTO also has the weight
                                 streamer for a few rows per expert, which moe_get_options reports as AUTO here and below */
     int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1; 256 needs
-                                H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0) */
-    int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile (AUTO: also the weight streamer, other bits); also read by the
-                                backward entry points of an fp32 handle (there 1 means "where the shape allows") */
+                                H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0; elsewhere 256 gives the 128x128 tile) */
+    int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile (AUTO: also the weight
+                                streamer, other bits).  The backward entry points of an fp32 handle use the matrix-core tile,
+                                where their shape allows, on a handle whose layer runs on it, and the 64x64 tile on any other
+                                one, the streamer's included (which moe_get_options reports as AUTO) */
     int32_t fp8_tile;        /* e4m3 layers: 0 = weight streamer (decode), 1 = 128x128 tile GEMM */
     int32_t fp8_widen;       /* e4m3 layers: 1 = run the bf16 tiles on bf16 copies of the weights (widened into the workspace
                                 by every call, or taken from moe_prepare_weights), 0 = never */
@@ -305,7 +307,8 @@ int moe_get_stage_ms(moe_handle* h, int stage, float* ms, int32_t* calls);
 int moe_get_stage_samples(moe_handle* h, int stage, float* ms, int32_t capacity, int32_t* count);
 
 /* How evenly the task queue of the last moe_forward kept its workgroups busy (task-queue FFN only; MOE_ERR_UNSUPPORTED
- * in the two-launch mode).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
+ * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers and for single experts:
+ * moe_get_ffn_mode tells).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
  * the queue kernel: span_us = first entry to last exit, mean_active_us = mean of (exit - entry), mean_tail_idle_us =
  * mean of (last exit - own exit), i.e. the time a workgroup had nothing left to pop while others still worked.
  * Synchronises `stream`.  No counterpart in the reference, whose scheduler keeps no statistics. */
@@ -416,7 +419,7 @@ int moe_expert_wgrad(moe_handle* h, const void* dy_rows, const void* a_rows, con
  * without dh ever reaching memory.  N = intermediate_size, K = hidden_size; the activation is the layer's hidden_act;
  * u_rows / g_rows / du_rows / dg_rows are [rows, N] (g_rows and dg_rows exactly when the layer is SwiGLU).  The product
  * is rounded to the storage type before the derivative, as the two calls do when they store dh, so both give the same
- * bits.  Exists for bf16 and fp16 layers whose shape meets the hand-ordered tiles' conditions (N % 256 == 0,
+ * bits.  Exists for bf16 and fp16 layers of whole column tiles and pairs of slabs of the hand-ordered tiles (N % 256 == 0,
  * K % 128 == 0, operands below 4 GiB; option grouped_tile = 0 switches it off): moe_expert_gemm_act_backward_supported
  * tells, and the call returns MOE_ERR_UNSUPPORTED otherwise -- the two calls remain the general path. */
 int moe_expert_gemm_act_backward_supported(const moe_handle* h, int32_t* supported);

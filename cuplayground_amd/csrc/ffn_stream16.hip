@@ -36,6 +36,8 @@
 //   8 of 4096 x 14336, top-2, 32 tokens: 744 / 551 / 538, 745 / 686 / 619, 682 / 679 / 583, one set of two 362 / 352 / 292;
 //     64 tokens: 748 / 610 / 610, 749 / 776 / 708, 687 / 755 / 674, 367 / 418 / 354
 //   16 of 2048 x 2048, top-2, 64 tokens: 122 / 87 / 87, 117 / 92 / 91, 103 / 83 / 78;  128: 125 / 93 / 93, 123 / 127 / 115, 106 / 87 / 85
+// (Groups of 64 rows in a wavefront's own fragments, without LDS, lose to single blocks: 890 us against 418 for 64 tokens on one set of two of the
+// second; with one slab of weights on its way instead of two the groups take 469 there.)
 // What is left behind the tile are routers that send nearly every one of 96 tokens and more to the same few of many experts.
 #include "act_deriv.hpp"
 #include "ffn_common.hpp"

@@ -33,7 +33,7 @@ PEAK_HBM_GBS = 8000.0         # MI355X HBM3E
 # script (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch), each scaled by what the same counter showed for a 1 GiB
 # device copy in the same run (--calibrate-copy).  Each entry names the summary under profiles/ it comes from and the
 # digest of the kernel sources it was collected with: when the sources have changed since, the figure is withheld.
-BF16_SOURCES = ("ffn_bf16.hip", "ffn_bf16_slab_steady.inc", "ffn_common.hpp", "route.hip")
+BF16_SOURCES = ("ffn_bf16.hip", "ffn_bf16_tile.hpp", "ffn_bf16_slab_steady.inc", "ffn_common.hpp", "route.hip")
 FP8_SOURCES = ("ffn_fp8.hip", "ffn_common.hpp", "route.hip")
 FP8_TILE_SOURCES = ("ffn_fp8_tile.hip", "ffn_common.hpp", "route.hip")
 WIDEN_SOURCES = BF16_SOURCES + ("quant.hip",)

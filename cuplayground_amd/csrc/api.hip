@@ -1159,6 +1159,31 @@ int moe_expert_gemm_act_backward_supported(const moe_handle* h, int32_t* support
     return MOE_OK;
 }
 
+int moe_expert_gemm_kn_supported(const moe_handle* h, int32_t N, int32_t K, int32_t* supported) {
+    if (!h || !supported) return MOE_ERR_BAD_ARGUMENT;
+    const bool dims_ok = (N == h->d.H && K == h->d.I) || (N == h->d.I && K == h->d.H);
+    if (!dims_ok) return MOE_ERR_BAD_ARGUMENT;
+    *supported = h->cfg.torch_dtype == MOE_DTYPE_FP8_E4M3_B128 ? 0 : expert_gemm_kn_supported(h->d.A, h->d.E, N, K, h->d.act_dtype, h->opt);
+    return MOE_OK;
+}
+
+int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const void* u_rows, const void* g_rows,
+                       const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K, void* out_rows,
+                       void* out1_rows, void* stream) {
+    if (!h || !a_rows || !w || !expert_count || !expert_offset || !out_rows) return MOE_ERR_BAD_ARGUMENT;
+    const bool gated = u_rows && h->cfg.hidden_act == MOE_ACT_SWIGLU;
+    if (gated != (g_rows != nullptr) || gated != (out1_rows != nullptr)) return MOE_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)a_rows | (uintptr_t)w | (uintptr_t)u_rows | (uintptr_t)g_rows | (uintptr_t)out_rows | (uintptr_t)out1_rows) % 16) return MOE_ERR_BAD_ARGUMENT;
+    int32_t supported = 0;
+    const int rc = moe_expert_gemm_kn_supported(h, N, K, &supported);
+    if (rc) return rc;
+    if (u_rows && (N != h->d.I || K != h->d.H)) return MOE_ERR_BAD_ARGUMENT;
+    if (!supported) return MOE_ERR_UNSUPPORTED;
+    const hipError_t e = launch_expert_gemm_kn(a_rows, w, u_rows, g_rows, expert_count, expert_offset, h->d.A, h->d.E, N, K, h->cfg.hidden_act,
+                                               h->d.act_dtype, out_rows, out1_rows, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
 int moe_expert_wgrad(moe_handle* h, const void* dy_rows, const void* a_rows, const int32_t* expert_count,
                      const int32_t* expert_offset, int32_t N, int32_t K, void* dw, void* scratch, size_t scratch_bytes,
                      void* stream) {

@@ -19,15 +19,14 @@ namespace moe355 {
 
 bool grouped_hand_ok(int64_t A, int N, int K);
 int grouped_gemm_tile_16(int64_t A, int E, int N, int K);
-hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const MTile* mtiles,
-                                  const int32_t* num_mtiles, const int32_t* count, int max_mtiles, int tile, int64_t A,
-                                  int N, int K, int act, bool f16, hipStream_t st);
+hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const int32_t* count,
+                                  const int32_t* offset, int tile, int64_t A, int E, int N, int K, int act, bool f16, hipStream_t st);
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
                            int64_t ld, bool f16, hipStream_t st);
 
-hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const void* u, const void* g, void* du, void* dg,
-                                        const MTile* mtiles, const int32_t* num_mtiles, const int32_t* count, int max_mtiles,
-                                        int tile, int64_t A, int N, int K, int hidden_act, bool f16, hipStream_t st);
+hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* du, void* dg,
+                                        const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
+                                        int hidden_act, bool f16, hipStream_t st);
 hipError_t launch_grouped_gemm_f32(const void* a_rows, const void* w, const void* bias, void* out, const MTile* mtiles,
                                    const int32_t* num_mtiles, int max_mtiles, int N, int K, int act, hipStream_t st);
 hipError_t launch_wgrad_f32(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K, int64_t ld,
@@ -530,8 +529,8 @@ ScratchTables scratch_tables(void* scratch, int64_t A, int E) {
 hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bias, const int32_t* count,
                               const int32_t* offset, int64_t A, int E, int N, int K, int act, int dtype,
                               const moe_options& opt, void* out_rows, void* scratch, hipStream_t st) {
-    const ScratchTables t = scratch_tables(scratch, A, E);
     if (dtype == MOE_DTYPE_F32) {
+        const ScratchTables t = scratch_tables(scratch, A, E);
         bool mfma = grouped_gemm_f32_takes_tile(A, N, K);
         if (opt.f32_tile == 0) mfma = false;   // option: keep the vector-ALU kernel
         const int block_m = mfma ? 128 : 64;
@@ -548,13 +547,7 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
         if ((v == 1 || v == 2) && grouped_hand_ok(A, N, K)) tile = v;
         if (v == 0) tile = 0;
     }
-    const int block_m = tile == 1 ? 256 : 128;
-    const int max_mtiles = (int)(A / block_m + E);
-    backward_tables_kernel<<<1, kMaxExperts, 0, st>>>(count, offset, E, block_m, t.mtiles, t.num_mtiles, nullptr);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_grouped_gemm_16(a_rows, w, bias, out_rows, t.mtiles, t.num_mtiles, count, max_mtiles, tile, A, N, K, act,
-                                  dtype == MOE_DTYPE_FP16, st);
+    return launch_grouped_gemm_16(a_rows, w, bias, out_rows, count, offset, tile, A, E, N, K, act, dtype == MOE_DTYPE_FP16, st);
 }
 
 // The tile the fused data gradient (product + activation derivative) runs on: 1 or 2 (the hand-ordered tiles), or 0 where
@@ -582,14 +575,8 @@ hipError_t launch_expert_gemm_dact(const void* dy_rows, const void* w, const voi
                                    hipStream_t st) {
     const int tile = expert_gemm_dact_tile(A, E, N, K, dtype, opt);
     if (tile == 0) return hipErrorNotSupported;
-    const ScratchTables t = scratch_tables(scratch, A, E);
-    const int block_m = tile == 1 ? 256 : 128;
-    const int max_mtiles = (int)(A / block_m + E);
-    backward_tables_kernel<<<1, kMaxExperts, 0, st>>>(count, offset, E, block_m, t.mtiles, t.num_mtiles, nullptr);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_grouped_gemm_deriv_16(dy_rows, w, u_rows, g_rows, du_rows, dg_rows, t.mtiles, t.num_mtiles, count, max_mtiles,
-                                        tile, A, N, K, hidden_act, dtype == MOE_DTYPE_FP16, st);
+    return launch_grouped_gemm_deriv_16(dy_rows, w, u_rows, g_rows, du_rows, dg_rows, count, offset, tile, A, E, N, K, hidden_act,
+                                        dtype == MOE_DTYPE_FP16, st);
 }
 
 // dw[e] [N,K] = dy_e^T . a_e; scratch holds the window offsets and the two transposed operands.

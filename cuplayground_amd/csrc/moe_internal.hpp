@@ -224,6 +224,10 @@ hipError_t launch_expert_gemm_dact(const void* dy_rows, const void* w, const voi
 hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bias, const int32_t* count,
                               const int32_t* offset, int64_t A, int E, int N, int K, int act, int dtype,
                               const moe_options& opt, void* out_rows, void* scratch, hipStream_t st);
+int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const moe_options& opt);
+hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
+                                 const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows,
+                                 void* out1_rows, hipStream_t st);
 hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const int32_t* count, const int32_t* offset,
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st);

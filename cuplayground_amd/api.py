@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -159,6 +159,8 @@ def load_library():
     L.moe_expert_wgrad.argtypes = [vp, vp, vp, vp, vp, i32, i32, vp, vp, C.c_size_t, vp]
     L.moe_expert_gemm_act_backward.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp, C.c_size_t, vp]
     L.moe_expert_gemm_act_backward_supported.argtypes = [vp, C.POINTER(C.c_int32)]
+    L.moe_expert_gemm_kn.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp]
+    L.moe_expert_gemm_kn_supported.argtypes = [vp, i32, i32, C.POINTER(C.c_int32)]
     L.moe_act_backward.argtypes = [vp, vp, vp, vp, i64, vp, vp, vp]
     L.moe_bias_grad.argtypes = [vp, vp, vp, vp, i32, vp, vp]
     L.moe_combine_backward.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp]
@@ -562,6 +564,28 @@ class MoELayer:
                                                    _ptr(expert_count), _ptr(expert_offset), N, K, _ptr(du), _ptr(dg),
                                                    _ptr(sc), sc.numel(), _stream()), "moe_expert_gemm_act_backward")
         return du, dg
+
+    def gemm_kn_supported(self, N: int, K: int) -> int:
+        """0: no expert_gemm_kn for these dimensions; 1: there is; 2: and it is expected to beat transpose + expert_gemm."""
+        v = C.c_int32(0)
+        _check(self.L.moe_expert_gemm_kn_supported(self._h, N, K, C.byref(v)), "moe_expert_gemm_kn_supported")
+        return v.value
+
+    def expert_gemm_kn(self, a_rows, w, expert_count, expert_offset, u_rows=None, g_rows=None):
+        """a_rows[r] . w[e(r)] with w [E, K, N]; with u_rows (and g_rows): (du_rows, dg_rows), that times act'(u_rows, g_rows).
+        Rows of no expert are not written."""
+        import torch
+        K, N = w.shape[1], w.shape[2]
+        for name, t in (("a_rows", a_rows), ("w", w)):
+            _operand(name, t, self.act_dtype)
+        for name, t in (("u_rows", u_rows), ("g_rows", g_rows)):
+            if t is not None:
+                _operand(name, t, self.act_dtype, a_rows.shape[0] * N)
+        out = torch.empty(a_rows.shape[0], N, dtype=a_rows.dtype, device=a_rows.device)
+        out1 = None if g_rows is None else torch.empty_like(out)
+        _check(self.L.moe_expert_gemm_kn(self._h, _ptr(a_rows), _ptr(w), _ptr(u_rows), _ptr(g_rows), _ptr(expert_count),
+                                         _ptr(expert_offset), N, K, _ptr(out), _ptr(out1), _stream()), "moe_expert_gemm_kn")
+        return out if u_rows is None else (out, out1)
 
     def expert_wgrad(self, dy_rows, a_rows, expert_count, expert_offset, out=None):
         """dw[e] [N,K] = sum over expert e's rows of dy_rows[r,:N]^T a_rows[r,:K]."""

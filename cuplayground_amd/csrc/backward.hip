@@ -24,6 +24,14 @@ hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void*
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
                            int64_t ld, bool f16, hipStream_t st);
 
+bool wgrad_rows_16_better(int64_t A, int E, int N, int K);
+bool grouped_kn_16_ok(int64_t A, int N, int K);
+bool grouped_kn_16_better(int64_t A, int E, int N, int K);
+hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
+                                     const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
+                                     hipStream_t st);
+hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K,
+                                bool f16, hipStream_t st);
 hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* du, void* dg,
                                         const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
                                         int hidden_act, bool f16, hipStream_t st);
@@ -579,10 +587,26 @@ hipError_t launch_expert_gemm_dact(const void* dy_rows, const void* w, const voi
                                         dtype == MOE_DTYPE_FP16, st);
 }
 
-// dw[e] [N,K] = dy_e^T . a_e; scratch holds the window offsets and the two transposed operands.
+// out_rows[r,:] = a_rows[r,:] . w[e(r)] with w [E, K, N] as the other direction stores it, and with u_rows the derivative behind it
+// (launch_expert_gemm_dact): no transposed copy of the weight.  16-bit layers.
+int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
+    if (dtype == MOE_DTYPE_F32 || !grouped_kn_16_ok(A, N, K)) return 0;
+    return opt.grouped_tile == MOE_OPT_AUTO && grouped_kn_16_better(A, E, N, K) ? 2 : 1;
+}
+hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
+                                 const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows, void* out1_rows,
+                                 hipStream_t st) {
+    if (dtype == MOE_DTYPE_F32 || !grouped_kn_16_ok(A, N, K)) return hipErrorNotSupported;
+    return launch_grouped_gemm_kn_16(a_rows, w, u_rows, g_rows, out_rows, out1_rows, count, offset, A, E, N, K, hidden_act, dtype == MOE_DTYPE_FP16, st);
+}
+
+// dw[e] [N,K] = dy_e^T . a_e, from the rows as they are or from transposed copies: scratch holds the window offsets and those.
 hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const int32_t* count, const int32_t* offset,
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st) {
+    const bool aligned = ((uintptr_t)dy_rows | (uintptr_t)a_rows | (uintptr_t)dw) % 16 == 0;
+    if (dtype != MOE_DTYPE_F32 && aligned && wgrad_rows_16_better(A, E, N, K))
+        return launch_wgrad_rows_16(dy_rows, a_rows, dw, count, offset, E, N, K, dtype == MOE_DTYPE_FP16, st);
     const ScratchTables t = scratch_tables(scratch, A, E);
     const int64_t ld = wgrad_ld(A, E);
     const size_t eb = dtype == MOE_DTYPE_F32 ? 4 : 2;

@@ -195,6 +195,274 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
     grouped_tile<P, EPI>(p, smem);
 }
 
+// ---- products whose operands may lie the other way round ----
+//
+// C[i, j] = sum over k of A(i, k) B(j, k) on 128 x 128 tiles, where either operand may be stored with k as its slow index: the
+// weight as it is in a data gradient (dX = dY . W), both operands in a weight gradient (dW[e] = dY_e^T . X_e).  A transposed
+// operand is turned round on its way through the registers: a thread fetches 16 bytes of four consecutive k and writes, for each
+// of the eight i, the four values of k side by side (one byte permute a dword), so that LDS holds what it holds for the other
+// tiles and nothing else is ever written to memory.
+template <bool F16_>
+struct ProdTile {
+    static constexpr int BM = 128, BN = 128, WM = 2, WN = 2, NS = 2, THREADS = 256, TM = 4, TN = 4, WB = 64;
+    static constexpr bool F16 = F16_, RING = false, HALF = false, HAND = true;
+    static constexpr int STAGE_BYTES = (BM + BN) * kRowBytes;
+    static constexpr int STAGING_BYTES = 4 * 16 * (TN * 32 + 16);
+    static constexpr int LDS_BYTES = NS * STAGE_BYTES + STAGING_BYTES;
+    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per compute unit");
+};
+// An operand of one tile: 128 rows i (or columns j) from `base` on.
+struct ProdOperand {
+    const uint16_t* base;
+    int ld;                // elements between consecutive i (as it is) or consecutive k (transposed)
+    uint32_t extent;       // bytes from base that exist; loads behind read zeros
+};
+// LDS: 128-byte rows of 64 k, 16-byte piece c of row i at c ^ prod_swizzle(i).  The 16 rows of a fragment read meet all banks, and
+// so do eight rows that lie eight apart, which is what a transposed operand writes at a time.
+__device__ __forceinline__ int prod_swizzle(int i) { return ((i >> 1) ^ (i >> 4)) & 7; }
+template <bool TR>
+struct ProdLoads {
+    uint32_t off[4];       // rows behind the operand's last one lie behind its extent, whatever the tile
+    int put;
+    __device__ __forceinline__ ProdLoads(int ld, int tid) {
+        if constexpr (TR) {
+            // Eight lanes in a row fetch 128 bytes in a row: the address unit takes four neighbouring lanes a cycle only where
+            // their addresses follow each other, else one (with the lanes of a row eight apart: 64 cycles a request, the unit busy
+            // 94 % of the time, 1.6 times the kernel's time).
+            const int lane = tid & 63, wave = tid >> 6;
+            const int kq = (lane >> 3) + 8 * (wave & 1), ig = (lane & 7) + 8 * (wave >> 1);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) off[q] = (uint32_t)((4 * kq + q) * ld + 8 * ig) * 2;
+            put = ig * 8 * kRowBytes + (((kq >> 1) ^ prod_swizzle(8 * ig)) << 4) + (kq & 1) * 8;
+        } else {
+            const int row = tid >> 3;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) off[q] = (uint32_t)((row + 32 * q) * ld + 8 * (tid & 7)) * 2;
+            put = row * kRowBytes + (((tid & 7) ^ prod_swizzle(row)) << 4);
+        }
+    }
+    // slab s of 64 k.  Transposed: k behind the extent are zeros.
+    __device__ __forceinline__ void load(const ProdOperand& o, int slab, u32x4 (&d)[4]) const {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(o.base), 0, (int)o.extent, 0x00020000);
+        if constexpr (TR) {
+            const uint32_t k = (uint32_t)(slab * kBK) * o.ld * 2;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) d[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off[q] + k), 0, 0));
+        } else {
+            const int k = slab * kRowBytes;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) d[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[q], k, 0));
+        }
+    }
+    __device__ __forceinline__ void store(const u32x4 (&d)[4], unsigned char* st) const {
+        if constexpr (TR) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {      // row i = 8 ig + j: its swizzle differs from that of 8 ig by j >> 1
+                const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+                const u32x2 v = {__builtin_amdgcn_perm(d[1][j >> 1], d[0][j >> 1], sel), __builtin_amdgcn_perm(d[3][j >> 1], d[2][j >> 1], sel)};
+                *reinterpret_cast<u32x2*>(st + ((put ^ ((j >> 1) << 4)) + j * kRowBytes)) = v;
+            }
+        } else {                               // row + 32 q: by 2 q
+#pragma unroll
+            for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(st + ((put ^ (q << 5)) + q * 32 * kRowBytes)) = d[q];
+        }
+    }
+};
+
+// The same in every lane, and said so: else each load loops over the lanes.
+__device__ __forceinline__ ProdOperand prod_uniform(const ProdOperand& o) {
+    const uint64_t v = (uint64_t)o.base;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return ProdOperand{(const uint16_t*)(((uint64_t)hi << 32) | lo), __builtin_amdgcn_readfirstlane(o.ld), (uint32_t)__builtin_amdgcn_readfirstlane((int)o.extent)};
+}
+
+// One tile of a launch: its operands and how many slabs of 64 k it has (at least one).
+struct ProdJob {
+    ProdOperand a, b;
+    int slabs;
+};
+
+// The slab loop of one tile.  What bounds it: LDS (a 64 x 64 wavefront tile reads 16 KB of fragments a slab at 256 bytes a cycle,
+// the slab's 32 KB are written at 128), the address unit (64 bytes a cycle) and the matrix instructions, each about half of the
+// time; two workgroups share a compute unit and fill each other's waits.  0.9 PFLOP/s in 2048 rows an expert.  (Workgroups that stay and
+// request the next tile's first slabs under this one's last: no faster, what they save at the ends of tiles they lose in the
+// last round of an uneven number of tiles.)
+template <class T, bool TA, bool TB>
+__device__ __forceinline__ void prod_slabs(const ProdJob& job, unsigned char* smem, f32x4 (&acc)[T::TM][T::TN]) {
+    constexpr int D = 2;                       // slabs on their way in registers
+    typedef typename std::conditional<T::F16, f16x8, bf16x8>::type frag_t;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / T::WN, wn = wave % T::WN;
+    const ProdLoads<TA> la(job.a.ld, tid);
+    const ProdLoads<TB> lb(job.b.ld, tid);
+    const int slabs = job.slabs;
+    const int frow = lane & 15, fk = lane >> 4, sw = (frow >> 1) & 7;
+    int get_a[T::TM], get_b[T::TN];            // this lane's pieces of k half 0; those of half 1 lie 64 bytes up or down
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) get_a[i] = (16 * (wm * T::TM + i) + frow) * kRowBytes + ((fk ^ sw ^ ((wm * T::TM + i) & 7)) << 4);
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) get_b[j] = (T::BM + 16 * (wn * T::TN + j) + frow) * kRowBytes + ((fk ^ sw ^ ((wn * T::TN + j) & 7)) << 4);
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 ra[D][4], rb[D][4];
+    frag_t fa[2][T::TM], fb[2][T::TN];
+    auto read = [&](int st, int s) {
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j) fb[s][j] = *reinterpret_cast<const frag_t*>(smem + st * T::STAGE_BYTES + (get_b[j] ^ (s << 6)));
+#pragma unroll
+        for (int i = 0; i < T::TM; ++i) fa[s][i] = *reinterpret_cast<const frag_t*>(smem + st * T::STAGE_BYTES + (get_a[i] ^ (s << 6)));
+    };
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < T::TN; ++j) {
+                if constexpr (T::F16) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);
+                else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);
+            }
+    };
+    auto put = [&](int u) {
+        la.store(ra[u], smem + u * T::STAGE_BYTES);
+        lb.store(rb[u], smem + u * T::STAGE_BYTES + T::BM * kRowBytes);
+    };
+    auto fetch = [&](int u, int slab) {        // slabs behind the last one: operands of no extent, zeros without a memory access
+        ProdOperand a = job.a, b = job.b;
+        if (slab >= slabs) a.extent = b.extent = 0;
+        la.load(a, slab, ra[u]);
+        lb.load(b, slab, rb[u]);
+    };
+    // The slab lies in stage u, the fragments of its first half in registers.  The second half's are read and the next slab is
+    // written under the first half's MFMAs; behind the barrier the next slab's first half is read under the second half's.
+    // (One body for every slab: with bodies of their own for the last ones, which need not write and request, the compiler spills.)
+    auto step = [&](auto U, int slab) {
+        constexpr int u = decltype(U)::value;
+        read(u, 1);
+        multiply(0);
+        put(u ^ 1);
+        fetch(u ^ 1, slab + 1 + D);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        read(u ^ 1, 0);
+        multiply(1);
+    };
+    fetch(0, 0);
+    fetch(1, 1);
+    put(0);
+    fetch(0, D);
+    __syncthreads();
+    read(0, 0);
+    int slab = 0;
+    for (; slab + 2 <= slabs; slab += 2) {
+        step(std::integral_constant<int, 0>{}, slab);
+        step(std::integral_constant<int, 1>{}, slab + 1);
+    }
+    if (slab < slabs) step(std::integral_constant<int, 0>{}, slab);
+}
+// Tiles: job(id, j) the operands of tile `id` (false: no such tile), finish(id, acc, smem) its epilogue.
+template <class T, bool TA, bool TB, class Tiles>
+__device__ __forceinline__ void prod_tile(const Tiles& tiles, unsigned char* smem) {
+    ProdJob job;
+    if (!tiles.job(blockIdx.x, job)) return;
+    job = ProdJob{prod_uniform(job.a), prod_uniform(job.b), __builtin_amdgcn_readfirstlane(job.slabs)};
+    f32x4 acc[T::TM][T::TN];
+    prod_slabs<T, TA, TB>(job, smem, acc);
+    tiles.finish(blockIdx.x, acc, smem);
+}
+
+// What the epilogue of a tile without bias needs: rows of C from `c` on, N columns a row, this tile's from n0 on.
+__device__ __forceinline__ TaskPtrs prod_epilogue(uint16_t* c, int N, int n0, int rows) {
+    TaskPtrs p{};
+    p.c_base = c;
+    p.N = N;
+    p.rows = rows;
+    p.n0 = n0;
+    p.act = MOE_ACT_NONE;
+    return p;
+}
+
+// Weight gradient of one projection from the packed rows as they are: dw[e] [N, K] = sum over expert e's rows of
+// dy[r, :]^T a[r, :].  Tiles expert by expert.  The workgroups of an XCD (launched eight apart) take neighbouring tiles, four
+// columns wide, whose operands meet in its L2: 16 experts of 2048 x 1408, 750 rows each, 104 us against 124 with columns fastest.
+template <class T>
+struct WgradTiles {
+    const uint16_t* dy;
+    const uint16_t* a;
+    uint16_t* dw;
+    const int32_t* count;
+    const int32_t* offset;
+    int E, N, K;
+    __device__ __forceinline__ bool place(int id, int& e, int& n0, int& k0) const {
+        const int cols = (K + T::BN - 1) / T::BN, rows = (N + T::BM - 1) / T::BM, share = (cols * rows + 7) / 8;
+        e = id / (8 * share);
+        const int r = id - e * 8 * share, t = (r & 7) * share + (r >> 3);
+        const int band = t / (4 * rows), in = t - band * 4 * rows, width = min(4, cols - 4 * band);
+        if (t >= cols * rows) return false;
+        n0 = in / width * T::BM;
+        k0 = (4 * band + in % width) * T::BN;
+        return e < E;
+    }
+    __device__ __forceinline__ bool job(int id, ProdJob& j) const {
+        int e, n0, k0;
+        if (!place(id, e, n0, k0)) return false;
+        const int n = max(count[e], 0);
+        const int64_t off = offset[e];
+        j.a = ProdOperand{dy + off * N + n0, N, n > 0 ? (uint32_t)(((int64_t)n * N - n0) * 2) : 0u};
+        j.b = ProdOperand{a + off * K + k0, K, n > 0 ? (uint32_t)(((int64_t)n * K - k0) * 2) : 0u};
+        j.slabs = max((n + kBK - 1) / kBK, 1);
+        return true;
+    }
+    __device__ __forceinline__ void finish(int id, f32x4 (&acc)[T::TM][T::TN], unsigned char* smem) const {
+        int e, n0, k0;
+        place(id, e, n0, k0);
+        grouped_epilogue<T, kSums>(prod_epilogue(dw + ((int64_t)e * N + n0) * K, K, k0, min(T::BM, N - n0)), smem, acc);
+    }
+};
+template <class T>
+__global__ __launch_bounds__(T::THREADS, 2) void wgrad_rows_kernel(WgradTiles<T> tiles) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    prod_tile<T, true, true>(tiles, smem);
+}
+
+// A grouped product with the weight as it is stored for the other direction: out[r, :] = a[r, :] . w[e(r)], w [E, K, N].
+template <class T, int EPI>
+struct GroupedTiles {
+    GroupedArgs g;
+    __device__ __forceinline__ bool place(int id, GroupedTask& t) const {
+        return grouped_task<T::BM>(g.count, g.offset, g.E, (g.N + T::BN - 1) / T::BN, id, t);
+    }
+    __device__ __forceinline__ bool job(int id, ProdJob& j) const {
+        GroupedTask t;
+        if (!place(id, t)) return false;
+        const int n0 = t.ctile * T::BN;
+        const uint16_t* w = g.w + (int64_t)t.expert * g.N * g.K;
+        j.a = ProdOperand{g.a_rows + (int64_t)t.row0 * g.K, g.K, (uint32_t)((int64_t)t.rows * g.K * 2)};
+        j.b = ProdOperand{w + n0, g.N, (uint32_t)(((int64_t)g.K * g.N - n0) * 2)};
+        j.slabs = g.K / kBK;
+        return true;
+    }
+    __device__ __forceinline__ void finish(int id, f32x4 (&acc)[T::TM][T::TN], unsigned char* smem) const {
+        GroupedTask t;
+        place(id, t);
+        const int64_t at = (int64_t)t.row0 * g.N;
+        TaskPtrs p = prod_epilogue(g.out + at, g.N, t.ctile * T::BN, t.rows);
+        if constexpr (EPI == kDeriv) {
+            p.deriv = 1 + g.act;
+            p.aux0 = g.u_rows + at;
+            p.aux1 = g.g_rows ? g.g_rows + at : nullptr;
+            p.c1_base = g.out1 ? g.out1 + at : nullptr;
+        }
+        grouped_epilogue<T, EPI>(p, smem, acc);
+    }
+};
+template <class T, int EPI>
+__global__ __launch_bounds__(T::THREADS, 2) void grouped_kn_kernel(GroupedArgs g) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    prod_tile<T, false, true>(GroupedTiles<T, EPI>{g}, smem);
+}
+
 // Weight gradient of one projection: dw[e] [N, K] = dy_e^T . a_e, the sum running over the rows of expert e.  Both
 // operands arrive transposed and padded: dyT [N, ld] and aT [K, ld] hold expert e's rows in columns
 // [poff[e], poff[e+1]) (zeros behind the last real row; every window is a multiple of 128 wide), so each expert is one
@@ -338,6 +606,71 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
                           : launch_wgrad<Tile256>(dyT, aT, dw, poff, E, N, K, ld, st);
     return f16 ? launch_wgrad<Tile128H>(dyT, aT, dw, poff, E, N, K, ld, st)
                : launch_wgrad<Tile128>(dyT, aT, dw, poff, E, N, K, ld, st);
+}
+
+// The 128 x 128 tiles that turn operands round, against the larger hand-ordered tile behind transposes.  An estimate of either, us;
+// constants and checks are measurements of whole calls (transposes and launches included, bf16, one card):
+//   hand-ordered: 1.3 us a slab of 64 and 8 us a task, rounds of 256 tasks and half a one; transposes at 4.5 TB/s read and written;
+//   these: 1.25 us a slab and round of 512 tasks (two on a compute unit share its time), 5 us a round.
+static double prod_us(double tiles, double slabs) {
+    const double rounds = tiles / 512;
+    return (rounds < 1.0 ? 1.0 : rounds) * (1.25 * slabs + 5.0);
+}
+static double hand_us(double tiles, double slabs, double transposed_bytes) {
+    const double rounds = tiles / 256;
+    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * (1.3 * slabs + 8.0) + 2.0 * transposed_bytes / 4.5e6 + 8.0;
+}
+static bool prod_operands_ok(int64_t rows, int N, int K) { return (rows + 128) * std::max(N, K) * 2 < kBufferLimit && (int64_t)(N + 128) * K * 2 < kBufferLimit && (int64_t)(K + 128) * N * 2 < kBufferLimit; }
+//   weight gradient, hand-ordered / these: 16 experts of 2048 x 2048, 512 rows each 120 / 111; 750 rows of 1408 x 2048 125 / 108; 136 of
+//   1280 x 1408 47 / 26; 19 of 1024 x 2560 49 / 21; 4 of 2048 x 2560, 4096 rows 225 / 212; 64 of 1408 x 2048, 1536 rows 903 / 761;
+//   16 of 2048 x 2560, 1024 rows 238 / 240; 8 of 4096 x 2048, 2048 rows 304 / 339; 8 of 4096 x 14336, 512 rows 664 / 790, 2048 rows 1680 / 2410
+bool wgrad_rows_16_better(int64_t A, int E, int N, int K) {
+    if (!prod_operands_ok(A, N, K)) return false;
+    const double rows = (double)A / std::max(E, 1);
+    return prod_us((double)E * ((N + 127) / 128) * ((K + 127) / 128), rows / 64 + 0.5) <
+           hand_us((double)E * columns256(N) * columns256(K), rows / 64 + 1.0, 2.0 * A * (N + K));
+}
+bool grouped_kn_16_ok(int64_t A, int N, int K) { return prod_operands_ok(A, N, K); }
+bool grouped_kn_16_better(int64_t A, int E, int N, int K) {
+    if (!prod_operands_ok(A, N, K)) return false;
+    const double rows = (double)A / std::max(E, 1);
+    const double blocks = E * (rows <= 96 ? 1.0 : rows / 128 + 0.5), big = E * (rows <= 192 ? 1.0 : rows / 256 + 0.25);
+    return prod_us(blocks * ((N + 127) / 128), K / 64.0) < hand_us(big * columns256(N), K / 64.0, 2.0 * E * N * K);
+}
+
+template <class T>
+static hipError_t launch_wgrad_rows(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K, hipStream_t st) {
+    hipError_t e = allow_lds(&wgrad_rows_kernel<T>, T::LDS_BYTES);
+    if (e != hipSuccess) return e;
+    const int64_t tiles = ((int64_t)((K + T::BN - 1) / T::BN) * ((N + T::BM - 1) / T::BM) + 7) / 8 * 8 * E;
+    if (tiles > INT32_MAX) return hipErrorInvalidValue;
+    wgrad_rows_kernel<T><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(WgradTiles<T>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K});
+    return hipGetLastError();
+}
+hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K,
+                                bool f16, hipStream_t st) {
+    return f16 ? launch_wgrad_rows<ProdTile<true>>(dy, a, dw, count, offset, E, N, K, st)
+               : launch_wgrad_rows<ProdTile<false>>(dy, a, dw, count, offset, E, N, K, st);
+}
+
+template <bool F16, int EPI>
+static hipError_t launch_grouped_kn(const GroupedArgs& g, int64_t A, hipStream_t st) {
+    using T = ProdTile<F16>;
+    hipError_t e = allow_lds(&grouped_kn_kernel<T, EPI>, T::LDS_BYTES);
+    if (e != hipSuccess) return e;
+    const int64_t tiles = (A / T::BM + g.E) * ((g.N + T::BN - 1) / T::BN);
+    if (tiles > INT32_MAX) return hipErrorInvalidValue;
+    grouped_kn_kernel<T, EPI><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(g);
+    return hipGetLastError();
+}
+// out = a . w[e], or, with u, du (and dg) = (a . w[e]) * act'(u, g).
+hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
+                                     const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
+                                     hipStream_t st) {
+    const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)out,
+                        (uint16_t*)out1, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2)};
+    if (u) return f16 ? launch_grouped_kn<true, kDeriv>(g, A, st) : launch_grouped_kn<false, kDeriv>(g, A, st);
+    return f16 ? launch_grouped_kn<true, kSums>(g, A, st) : launch_grouped_kn<false, kSums>(g, A, st);
 }
 
 }  // namespace moe355

@@ -88,6 +88,11 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _as_stored(layer, w):
+    """Whether a data gradient [rows, K] . w[e] takes the weight w [E, K, N] as it is (else: a transposed copy)."""
+    return isinstance(layer, api.MoELayer) and w.data_ptr() % 16 == 0 and layer.gemm_kn_supported(w.shape[2], w.shape[1]) == 2
+
+
 class _Experts(torch.autograd.Function):
     """(x [S,H], expert weights, topk_w [S,k]) -> the gate-weighted sum of the chosen experts' outputs.
 
@@ -138,16 +143,19 @@ class _Experts(torch.autograd.Function):
         if need_down:
             ddown = layer.expert_wgrad(dy, h, count, offset)
         if need_x or need_up or need_gate:
-            w_t = api.transpose(w_down)                                                            # [E, I, H]
-            if layer.fused_act_backward:
-                du, dg = layer.expert_gemm_act_backward(dy, w_t, u, g, count, offset, du=torch.empty_like(u),
+            if _as_stored(layer, w_down):
+                du, dg = layer.expert_gemm_kn(dy, w_down, count, offset, u, g)                     # dH = dY . W_down, times act'
+            elif layer.fused_act_backward:
+                du, dg = layer.expert_gemm_act_backward(dy, api.transpose(w_down), u, g, count, offset, du=torch.empty_like(u),
                                                         dg=None if g is None else torch.empty_like(g))
             else:
-                du, dg = layer.act_backward(product(dy, w_t), u, g)                                # dH = dY . W_down
-            del w_t
+                du, dg = layer.act_backward(product(dy, api.transpose(w_down)), u, g)
             if need_x:
-                da = product(du, api.transpose(w_up))                                              # dA = dU . W_up
-                db = None if g is None else product(dg, api.transpose(w_gate))
+                def data_gradient(d, w):                                                           # dA = dU . W_up
+                    return layer.expert_gemm_kn(d, w, count, offset) if _as_stored(layer, w) else product(d, api.transpose(w))
+
+                da = data_gradient(du, w_up)
+                db = None if g is None else data_gradient(dg, w_gate)
                 dx = layer.dispatch_backward(da, db, pair_row)
             if need_up:
                 dup = layer.expert_wgrad(du, rows, count, offset)                                  # dW[e] = dU_e^T . A_e

@@ -426,6 +426,16 @@ int moe_expert_gemm_act_backward_supported(const moe_handle* h, int32_t* support
 int moe_expert_gemm_act_backward(moe_handle* h, const void* dy_rows, const void* w, const void* u_rows, const void* g_rows,
                                  const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K,
                                  void* du_rows, void* dg_rows, void* scratch, size_t scratch_bytes, void* stream);
+/* The same products with the weight as the other direction stores it, w [E, K, N] (k-major): out_rows[r, :] = a_rows[r, :] . w[e(r)],
+ * a projection's data gradient without a transposed copy of its weight; with u_rows (and, for a SwiGLU layer, g_rows and
+ * out1_rows) what moe_expert_gemm_act_backward gives, N = intermediate_size and K = hidden_size.  The sums run in the same order of
+ * k as in moe_expert_gemm: the same bits as behind moe_transpose.  *supported: 0 = no such kernel for this layer (fp32, operands of
+ * 4 GiB and more), 1 = it exists, 2 = and is expected to be faster than a transpose and the k-contiguous product (few rows per
+ * expert, small matrices; option grouped_tile asks for the latter).  Every pointer 16-byte aligned.  No scratch. */
+int moe_expert_gemm_kn_supported(const moe_handle* h, int32_t N, int32_t K, int32_t* supported);
+int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const void* u_rows, const void* g_rows,
+                       const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K, void* out_rows,
+                       void* out1_rows, void* stream);
 /* The elementwise and reduction steps between those products (same layers; fp32 arithmetic, one rounding on store):
  * moe_act_backward: for the first `rows` packed rows of width I, du = dh * act'(u) for hidden_act ReLU (1 where u > 0)
  *   and GELU (Phi(u) + u phi(u)); for SwiGLU, where h = silu(g) * u, du = dh * silu(g) and dg = dh * u * s * (1 + g (1 - s))

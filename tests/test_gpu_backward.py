@@ -1,5 +1,7 @@
 """GPU parity of the backward building blocks (batched transpose, grouped product over packed expert rows, per-expert
 weight gradient), called through the C ABI, against the CPU oracle."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -374,3 +376,45 @@ def test_fused_activation_backward_says_where_it_does_not_exist(moe):
         layer.expert_gemm_act_backward(z(256, 256), z(4, 128, 256), z(256, 128), z(256, 128), cnt, cnt)
     assert e.value.status == 4
     layer.close()
+
+
+@pytest.mark.parametrize("dtype", [ob.BF16, ob.F16])
+@pytest.mark.parametrize("shape", [(97, 64, 192, 3, 1), (700, 320, 192, 5, 2), (300, 256, 448, 70, 2), (1030, 192, 128, 2, 1)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_products_on_operands_as_stored(moe, dtype, shape, gated):
+    """The 128 x 128 tiles that turn operands round on their way (k-major weight, packed rows of a weight gradient), at remainders
+    of rows, columns and slabs, more experts than a wavefront has lanes, experts without rows.  The product keeps the order of
+    its sums: the bits of transpose + moe_expert_gemm (+ moe_act_backward).  The weight gradient against float64: fp32 sums
+    (2^-24 sqrt(rows) of the terms' size, far below) and one rounding, 2^-9 (bf16) or 2^-12 (fp16) of the value, with a factor of two."""
+    import torch
+    S, H, I, E, k = shape
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=S, drop=0, skew=0.3)
+    if gated:
+        cfg = dataclasses.replace(cfg, act=ob.ACT_SWIGLU)
+    R = int(count.sum())
+    layer = moe.MoELayer(product_config(cfg))
+    assert layer.gemm_kn_supported(H, I) and layer.gemm_kn_supported(I, H)
+    dev = lambda a: to_device(a, KIND[dtype])
+    dcount, doff = to_device(count, "i32"), to_device(offset, "i32")
+    rows = {n: dev(ob.from_f32(rng.standard_normal((S * k, n)).astype(np.float32), dtype)) for n in (H, I)}
+    u, g = (dev(ob.from_f32(rng.standard_normal((S * k, I)).astype(np.float32), dtype)) for _ in range(2))
+    rows[I][R:] = float("nan")                   # rows of no expert must not reach a result
+    rows[H][R:] = float("nan")
+    w_down = dev(ob.from_f32((rng.standard_normal((E, H, I)) * 0.1).astype(np.float32), dtype))
+    w_up = dev(ob.from_f32((rng.standard_normal((E, I, H)) * 0.1).astype(np.float32), dtype))
+    import cuplayground_amd.api as api
+    none = api.ACT_NONE
+    da = layer.expert_gemm_kn(rows[I], w_up, dcount, doff)
+    want = layer.expert_gemm(rows[I], api.transpose(w_up), None, dcount, doff, none)
+    assert torch.equal(da[:R], want[:R])
+    du, dg = layer.expert_gemm_kn(rows[H], w_down, dcount, doff, u, g if gated else None)
+    dh = layer.expert_gemm(rows[H], api.transpose(w_down), None, dcount, doff, none)
+    wu, wg = layer.act_backward(dh, u, g if gated else None)
+    assert torch.equal(du[:R], wu[:R]) and (not gated or torch.equal(dg[:R], wg[:R]))
+    dw = layer.expert_wgrad(rows[H], rows[I], dcount, doff)
+    tol = 2 * (2.0 ** -9 if dtype == ob.BF16 else 2.0 ** -12)
+    for e in range(E):
+        r = slice(int(offset[e]), int(offset[e] + count[e]))
+        ref = rows[H][r].double().t() @ rows[I][r].double()
+        scale = rows[H][r].double().abs().t() @ rows[I][r].double().abs()
+        assert ((dw[e].double() - ref).abs() <= tol * ref.abs() + 1e-6 * scale + 1e-7).all(), e

@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -167,6 +167,10 @@ def load_library():
     L.moe_dispatch_rows.argtypes = [vp, vp, vp, vp, vp]
     L.moe_act_forward.argtypes = [vp, vp, vp, vp, vp, vp, vp]
     L.moe_dispatch_backward.argtypes = [vp, vp, vp, vp, vp, vp]
+    L.moe_router_grad_bytes.argtypes = [vp, C.POINTER(C.c_size_t)]
+    L.moe_combine_router_backward.argtypes = [vp] * 10
+    L.moe_dispatch_router_backward.argtypes = [vp] * 9
+    L.moe_gate_wgrad.argtypes = [vp, vp, vp, vp, vp, C.c_size_t, vp]
     L.moe_last_hip_error.argtypes = [vp]
     L.moe_status_string.argtypes = [C.c_int]; L.moe_status_string.restype = C.c_char_p
     L.moe_version.restype = C.c_int
@@ -661,6 +665,53 @@ class MoELayer:
         _check(self.L.moe_combine_backward(self._h, _ptr(dout), _ptr(y_rows), _ptr(pair_row), _ptr(topk_w), _ptr(dy),
                                            _ptr(dw), _stream()), "moe_combine_backward")
         return dy, dw
+
+
+    # the router's share of a training step
+    @property
+    def router_grad_bytes(self) -> int:
+        """Bytes of the router's gradient buffer; 0 where the gate has no such kernels (softmax not normalised over the chosen)."""
+        n = C.c_size_t(0)
+        return n.value if self.L.moe_router_grad_bytes(self._h, C.byref(n)) == 0 else 0
+
+    def combine_router_backward(self, dout, y_rows, pair_row, topk_w, topk_idx, logits, dy, router_grad):
+        _operand("dout", dout, self.act_dtype, self.S * self.H)
+        _operand("y_rows", y_rows, self.act_dtype)
+        for name, t, dt in (("pair_row", pair_row, _i32()), ("topk_idx", topk_idx, _i32()), ("topk_w", topk_w, _f32())):
+            _operand(name, t, dt, self.S * self.k)
+        if logits is not None:
+            _operand("logits", logits, _f32(), self.S * self.E)
+        _check(self.L.moe_combine_router_backward(self._h, _ptr(dout), _ptr(y_rows), _ptr(pair_row), _ptr(topk_w), _ptr(topk_idx),
+                                                  _ptr(logits), _ptr(dy), _ptr(router_grad), _stream()), "moe_combine_router_backward")
+
+    def dispatch_router_backward(self, da_rows, db_rows, pair_row, topk_idx, router_grad, gate_w):
+        import torch
+        _operand("da_rows", da_rows, self.act_dtype)
+        if db_rows is not None:
+            _operand("db_rows", db_rows, self.act_dtype, da_rows.numel())
+        _operand("gate_w", gate_w, self.act_dtype, self.E * self.H)
+        dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
+        _check(self.L.moe_dispatch_router_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(topk_idx),
+                                                   _ptr(router_grad), _ptr(gate_w), _ptr(dx), _stream()), "moe_dispatch_router_backward")
+        return dx
+
+    def gate_wgrad(self, x, router_grad):
+        import torch
+        _operand("x", x, self.act_dtype, self.S * self.H)
+        sc = self.backward_scratch()
+        dw = torch.empty(self.E, self.H, dtype=self.act_dtype, device=x.device)
+        _check(self.L.moe_gate_wgrad(self._h, _ptr(x), _ptr(router_grad), _ptr(dw), _ptr(sc), sc.numel(), _stream()), "moe_gate_wgrad")
+        return dw
+
+
+def _i32():
+    import torch
+    return torch.int32
+
+
+def _f32():
+    import torch
+    return torch.float32
 
 
 def transpose(src, out=None):

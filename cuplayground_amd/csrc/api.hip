@@ -1258,7 +1258,49 @@ int moe_dispatch_backward(moe_handle* h, const void* da_rows, const void* db_row
     if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
     if (((uintptr_t)da_rows | (uintptr_t)db_rows | (uintptr_t)dx) % 16) return MOE_ERR_BAD_ARGUMENT;
     const hipError_t e = launch_dispatch_backward(da_rows, db_rows, pair_row, h->d.S, h->d.k, h->d.H, h->d.act_dtype, dx,
-                                                  (hipStream_t)stream);
+                                                  nullptr, nullptr, nullptr, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_router_grad_bytes(const moe_handle* h, size_t* bytes) {
+    if (!h || !bytes) return MOE_ERR_BAD_ARGUMENT;
+    // the weights of a softmax that are not normalised over the chosen experts depend on every logit: no such kernel
+    if (!backward_dtype(h) || (h->cfg.gate_fn == MOE_GATE_SOFTMAX && !h->cfg.norm_topk_prob)) return MOE_ERR_UNSUPPORTED;
+    *bytes = router_grad_bytes(h->d.S, h->d.E, h->d.k);
+    return MOE_OK;
+}
+
+int moe_combine_router_backward(moe_handle* h, const void* dout, const void* y_rows, const int32_t* pair_row, const float* topk_w,
+                                const int32_t* topk_idx, const float* logits, void* dy_rows, void* router_grad, void* stream) {
+    if (!h || !dout || !y_rows || !pair_row || !topk_w || !topk_idx || !dy_rows || !router_grad) return MOE_ERR_BAD_ARGUMENT;
+    size_t bytes = 0;
+    const int rc = moe_router_grad_bytes(h, &bytes);
+    if (rc) return rc;
+    if (!logits && h->cfg.gate_fn != MOE_GATE_SOFTMAX && h->cfg.norm_topk_prob) return MOE_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)dout | (uintptr_t)y_rows | (uintptr_t)dy_rows) % 16 || (uintptr_t)router_grad % kAlign) return MOE_ERR_BAD_ARGUMENT;
+    const hipError_t e = launch_combine_backward_router(dout, y_rows, pair_row, topk_w, topk_idx, logits, h->d.S, h->d.E, h->d.k, h->d.H,
+                                                        h->cfg.gate_fn, h->cfg.norm_topk_prob, h->d.act_dtype, dy_rows, router_grad,
+                                                        (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_dispatch_router_backward(moe_handle* h, const void* da_rows, const void* db_rows, const int32_t* pair_row, const int32_t* topk_idx,
+                                 const void* router_grad, const void* gate_w, void* dx, void* stream) {
+    if (!h || !da_rows || !pair_row || !topk_idx || !router_grad || !gate_w || !dx) return MOE_ERR_BAD_ARGUMENT;
+    if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
+    if (((uintptr_t)da_rows | (uintptr_t)db_rows | (uintptr_t)gate_w | (uintptr_t)dx) % 16 || (uintptr_t)router_grad % kAlign) return MOE_ERR_BAD_ARGUMENT;
+    const hipError_t e = launch_dispatch_backward(da_rows, db_rows, pair_row, h->d.S, h->d.k, h->d.H, h->d.act_dtype, dx, topk_idx,
+                                                  router_grad, gate_w, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_gate_wgrad(moe_handle* h, const void* x, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream) {
+    if (!h || !x || !router_grad || !dgate_w) return MOE_ERR_BAD_ARGUMENT;
+    if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
+    if ((uintptr_t)x % 16 || (uintptr_t)router_grad % kAlign) return MOE_ERR_BAD_ARGUMENT;
+    if (!scratch || (uintptr_t)scratch % kAlign || scratch_bytes < backward_scratch_bytes(h->d.A, h->d.E, h->d.H, h->d.I, (int)h->d.act_bytes))
+        return MOE_ERR_WORKSPACE;
+    const hipError_t e = launch_gate_wgrad(x, router_grad, h->d.S, h->d.E, h->d.k, h->d.H, h->d.act_dtype, dgate_w, scratch, (hipStream_t)stream);
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 

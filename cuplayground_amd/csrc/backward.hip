@@ -324,6 +324,104 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(const RAW* __restrict__ 
     db[(size_t)e * N + n] = st16<T16>(acc);
 }
 
+// Where the combine's adjoint leaves the gradient of the router's logits (null dl: not asked for).
+struct RouterGrad {
+    const int32_t* topk_idx;     // [S, k]
+    const float* logits;         // [S, E], read where the gate is a normalised sigmoid only
+    float* dl;                   // [S, k]: of the chosen experts' logits (those of the others are zero)
+    float* dl_dense;             // [S, ld]: the same as rows over the experts, zeros elsewhere
+    int E, ld, gate_fn, norm;
+};
+// The adjoint of the gate weights of one token (one wavefront; lane j < k holds dw of rank j), in fp32:
+//   softmax, normalised over the chosen: w = softmax of the chosen logits,  dl_j = w_j (dw_j - sum_m w_m dw_m);
+//   sigmoid: dl_j = s_j (1 - s_j) dw_j, s = w;  normalised: ds_j = (dw_j - sum_m w_m dw_m) / sum_m s_m, dl_j = s_j (1 - s_j) ds_j.
+__device__ __forceinline__ void router_grad_token(const RouterGrad& r, const float* __restrict__ topk_w, float dw, int t, int k) {
+    const int lane = threadIdx.x & 63;
+    const bool have = lane < k;
+    const int e = have ? r.topk_idx[(size_t)t * k + lane] : -1;
+    const float w = have ? topk_w[(size_t)t * k + lane] : 0.0f;
+    auto sum = [](float v) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        return v;
+    };
+    float g = dw;
+    if (r.norm) g -= sum(w * dw);
+    float dl;
+    if (r.gate_fn == MOE_GATE_SOFTMAX) {
+        dl = w * g;
+    } else {
+        float s = w;
+        if (r.norm) {
+            s = have ? 1.0f / (1.0f + expf(-r.logits[(size_t)t * r.E + e])) : 0.0f;
+            g /= sum(s);
+        }
+        dl = s * (1.0f - s) * g;
+    }
+    if (have) r.dl[(size_t)t * k + lane] = dl;
+    for (int c = lane; c - lane < r.ld; c += 64) {       // every lane takes every turn: the shuffles read all of them
+        float v = 0.0f;
+        for (int j = 0; j < k; ++j) {
+            const float d = __shfl(dl, j, 64);
+            if (__shfl(e, j, 64) == c) v = d;
+        }
+        if (c < r.ld) r.dl_dense[(size_t)t * r.ld + c] = v;
+    }
+}
+
+// The router's weight gradient, dgate_w[e, :] = sum over tokens of dl[t, e] x[t, :], in fp32: a share of the tokens a wavefront,
+// 256 columns x 16 experts of sums in its registers, the coefficients as scalars; the four wavefronts' sums meet in LDS and the
+// workgroups' in gate_wgrad_sum_kernel, both in a fixed order.  grid = (columns / 256, shares, experts / 16).
+constexpr int kGateShareMax = 64;      // partial sums of E * H * 4 bytes each: never more than the transposed operands the scratch is sized for
+template <class T16, class RAW = typename RawOf<T16>::type>
+__global__ __launch_bounds__(256) void gate_wgrad_kernel(const RAW* __restrict__ x, const float* __restrict__ dl, int S, int H, int E, int ld, float* __restrict__ part) {
+    __shared__ float red[4][64][64];   // [wavefront][expert * 4 + column of the lane][lane]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = blockIdx.x * 256 + 4 * lane, e0 = blockIdx.z * 16;
+    const int shares = gridDim.y * 4, per = (S + shares - 1) / shares;
+    const int t0 = (blockIdx.y * 4 + wave) * per, t1 = min(S, t0 + per);
+    float acc[16][4];
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[e][v] = 0.0f;
+    const int c = col < H ? col : 0;
+    struct alignas(4 * sizeof(RAW)) Four { RAW e[4]; };
+#pragma unroll 4
+    for (int t = t0; t < t1; ++t) {
+        const Four q = *reinterpret_cast<const Four*>(x + (size_t)t * H + c);
+        const float* d = dl + (size_t)t * ld + e0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float w = d[e];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[e][v] = fmaf(w, ld16<T16>(q.e, v), acc[e][v]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) red[wave][e * 4 + v][lane] = acc[e][v];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {              // this wavefront: experts 4 wave .. + 3
+        const int e = 4 * wave + i;
+        float o[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (red[0][e * 4 + v][lane] + red[1][e * 4 + v][lane]) + (red[2][e * 4 + v][lane] + red[3][e * 4 + v][lane]);
+        if (col < H && e0 + e < E) *reinterpret_cast<float4*>(part + ((size_t)blockIdx.y * E + e0 + e) * H + col) = float4{o[0], o[1], o[2], o[3]};
+    }
+}
+template <class T16, class RAW = typename RawOf<T16>::type>
+__global__ __launch_bounds__(256) void gate_wgrad_sum_kernel(const float* __restrict__ part, int shares, int n, RAW* __restrict__ dw) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float sum = 0.0f;
+#pragma unroll 8
+    for (int s = 0; s < shares; ++s) sum = sum + part[(size_t)s * n + i];
+    dw[i] = st16<T16>(sum);
+}
+
 // dy[row(t,r), :] = w[t,r] * dout[t, :]; dw[t,r] = <dout[t, :], y[row(t,r), :]>, one wavefront per token, four tokens per
 // workgroup.  Bound by memory (dout and y in, dy out): 16 bytes per lane and operand, the rows of four ranks in flight
 // beside one load of dout, and the dot products fold across the wavefront without LDS or a barrier.  8192 tokens x 2
@@ -332,11 +430,12 @@ template <class T16, class RAW = typename RawOf<T16>::type>
 __global__ __launch_bounds__(256) void combine_backward_kernel(const RAW* __restrict__ dout, const RAW* __restrict__ y,
                                                                const int32_t* __restrict__ pair_row,
                                                                const float* __restrict__ topk_w, int S, int k, int H,
-                                                               RAW* __restrict__ dy, float* __restrict__ dw) {
+                                                               RAW* __restrict__ dy, float* __restrict__ dw, RouterGrad router) {
     constexpr int VEC = 16 / (int)sizeof(RAW);
     union Pack { uint4 q; RAW e[VEC]; };
     const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= S) return;
+    float mine = 0.0f;                 // lane j: dw[t, j]
     for (int r0 = 0; r0 < k; r0 += 4) {
         int row[4];
         float w[4], acc[4];
@@ -368,9 +467,12 @@ __global__ __launch_bounds__(256) void combine_backward_kernel(const RAW* __rest
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) acc[j] += __shfl_xor(acc[j], off, 64);
-            if (lane == 0 && r0 + j < k) dw[(size_t)t * k + r0 + j] = row[j] >= 0 ? acc[j] : 0.0f;
+            if (row[j] < 0) acc[j] = 0.0f;
+            if (lane == r0 + j) mine = acc[j];
+            if (dw && lane == 0 && r0 + j < k) dw[(size_t)t * k + r0 + j] = acc[j];
         }
     }
+    if (router.dl) router_grad_token(router, topk_w, mine, t, k);
 }
 
 // The same one element at a time, for operands that are not 16-byte aligned: one workgroup per token.
@@ -445,14 +547,15 @@ __global__ __launch_bounds__(256) void dispatch_rows_kernel(const uint4* __restr
     for (int c = lane; c < row_vec; c += 64) rows[r * row_vec + c] = x[(int64_t)t * row_vec + c];
 }
 
-// dx[t, :] = sum over ranks r, ascending, of a[pair_row[t,r], :] + b[pair_row[t,r], :] (b may be null), in fp32 and rounded
-// once: the adjoint of the dispatch for one or two row gradients.  One wavefront per token and 64 16-byte pieces of its row,
+// dx[t, :] = sum over ranks r, ascending, of a[pair_row[t,r], :] + b[pair_row[t,r], :] (b may be null), and, with dl, behind
+// them of dl[t,r] gate_w[topk_idx[t,r], :], in fp32 and rounded once: the adjoint of the dispatch for one or two row gradients.  One wavefront per token and 64 16-byte pieces of its row,
 // the rows of four ranks in flight.  (torch's index_add backward of the same gather, 8192 rows x 2048 columns in bf16:
 // 55 us, behind two zero fills and, for two projections, two more sums over the rows.)
 template <class T16, class RAW = typename RawOf<T16>::type>
 __global__ __launch_bounds__(256) void dispatch_backward_kernel(const RAW* __restrict__ a, const RAW* __restrict__ b,
                                                                 const int32_t* __restrict__ pair_row, int S, int k, int H,
-                                                                RAW* __restrict__ dx) {
+                                                                RAW* __restrict__ dx, const int32_t* __restrict__ topk_idx,
+                                                                const float* __restrict__ dl, const RAW* __restrict__ gate_w) {
     constexpr int VEC = 16 / (int)sizeof(RAW);
     union Pack { uint4 q; RAW e[VEC]; };
     const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -479,6 +582,16 @@ __global__ __launch_bounds__(256) void dispatch_backward_kernel(const RAW* __res
                     acc[i] = acc[i] + ld16<T16>(va[j].e, i);
                     if (b) acc[i] = acc[i] + ld16<T16>(vb[j].e, i);
                 }
+            }
+        }
+        if (dl) {                          // the router's share: its weight rows of the chosen experts times their logits' gradients
+            for (int j = 0; j < k; ++j) {
+                const int e = __builtin_amdgcn_readfirstlane(topk_idx[(size_t)t * k + j]);
+                const float d = dl[(size_t)t * k + j];
+                Pack w;
+                w.q = *reinterpret_cast<const uint4*>(gate_w + (size_t)e * H + c);
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) acc[i] = fmaf(d, ld16<T16>(w.e, i), acc[i]);
             }
         }
         Pack o;
@@ -664,20 +777,55 @@ hipError_t launch_bias_grad(const void* dy, const int32_t* count, const int32_t*
 
 template <class T16, class RAW>
 static void launch_combine_backward_t(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S,
-                                      int k, int H, void* dy, float* dw, hipStream_t st) {
+                                      int k, int H, void* dy, float* dw, const RouterGrad& router, hipStream_t st) {
     const uintptr_t bits = (uintptr_t)dout | (uintptr_t)y | (uintptr_t)dy;
-    if (bits % 16 == 0)
-        combine_backward_kernel<T16><<<(S + 3) / 4, 256, 0, st>>>((const RAW*)dout, (const RAW*)y, pair_row, topk_w, S, k, H, (RAW*)dy, dw);
+    if (bits % 16 == 0)        // (the entry point of the router's share refuses others)
+        combine_backward_kernel<T16><<<(S + 3) / 4, 256, 0, st>>>((const RAW*)dout, (const RAW*)y, pair_row, topk_w, S, k, H, (RAW*)dy, dw, router);
     else
         combine_backward_unaligned_kernel<T16><<<S, 256, 0, st>>>((const RAW*)dout, (const RAW*)y, pair_row, topk_w, k, H, (RAW*)dy, dw);
 }
-
+static hipError_t combine_backward(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S, int k, int H,
+                                   int dtype, void* dy, float* dw, const RouterGrad& router, hipStream_t st) {
+    if (S <= 0) return hipSuccess;
+    if (dtype == MOE_DTYPE_F32) launch_combine_backward_t<f32_s, float>(dout, y, pair_row, topk_w, S, k, H, dy, dw, router, st);
+    else if (dtype == MOE_DTYPE_FP16) launch_combine_backward_t<f16_s, uint16_t>(dout, y, pair_row, topk_w, S, k, H, dy, dw, router, st);
+    else launch_combine_backward_t<bf16_s, uint16_t>(dout, y, pair_row, topk_w, S, k, H, dy, dw, router, st);
+    return hipGetLastError();
+}
 hipError_t launch_combine_backward(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S,
                                    int k, int H, int dtype, void* dy, float* dw, hipStream_t st) {
-    if (S <= 0) return hipSuccess;
-    if (dtype == MOE_DTYPE_F32) launch_combine_backward_t<f32_s, float>(dout, y, pair_row, topk_w, S, k, H, dy, dw, st);
-    else if (dtype == MOE_DTYPE_FP16) launch_combine_backward_t<f16_s, uint16_t>(dout, y, pair_row, topk_w, S, k, H, dy, dw, st);
-    else launch_combine_backward_t<bf16_s, uint16_t>(dout, y, pair_row, topk_w, S, k, H, dy, dw, st);
+    return combine_backward(dout, y, pair_row, topk_w, S, k, H, dtype, dy, dw, RouterGrad{}, st);
+}
+
+// ---- the router's share of a backward pass ----
+static int router_ld(int E) { return (E + 15) / 16 * 16; }
+size_t router_grad_bytes(int S, int E, int k) { return align256((size_t)S * k * 4) + align256((size_t)S * router_ld(E) * 4); }
+static float* router_dense(void* grad, int S, int k) { return reinterpret_cast<float*>(static_cast<char*>(grad) + align256((size_t)S * k * 4)); }
+
+hipError_t launch_combine_backward_router(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w,
+                                          const int32_t* topk_idx, const float* logits, int S, int E, int k, int H, int gate_fn, int norm,
+                                          int dtype, void* dy, void* grad, hipStream_t st) {
+    const RouterGrad r{topk_idx, logits, static_cast<float*>(grad), router_dense(grad, S, k), E, router_ld(E), gate_fn, norm};
+    return combine_backward(dout, y, pair_row, topk_w, S, k, H, dtype, dy, nullptr, r, st);
+}
+
+hipError_t launch_gate_wgrad(const void* x, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st) {
+    const float* dense = router_dense(const_cast<void*>(grad), S, k);
+    // shares: 32 tokens a wavefront, at least enough workgroups for the compute units where there are tokens for them
+    const int shares = std::min(std::max((S + 127) / 128, 1), kGateShareMax), n = E * H;
+    const dim3 grid((unsigned)((H + 255) / 256), (unsigned)shares, (unsigned)(router_ld(E) / 16));
+    float* part = static_cast<float*>(scratch);
+    const unsigned sums = (unsigned)((n + 255) / 256);
+    if (dtype == MOE_DTYPE_F32) {
+        gate_wgrad_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_sum_kernel<f32_s><<<sums, 256, 0, st>>>(part, shares, n, (float*)dgate_w);
+    } else if (dtype == MOE_DTYPE_FP16) {
+        gate_wgrad_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_sum_kernel<f16_s><<<sums, 256, 0, st>>>(part, shares, n, (uint16_t*)dgate_w);
+    } else {
+        gate_wgrad_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_sum_kernel<bf16_s><<<sums, 256, 0, st>>>(part, shares, n, (uint16_t*)dgate_w);
+    }
     return hipGetLastError();
 }
 
@@ -701,13 +849,15 @@ hipError_t launch_dispatch_rows(const void* x, const int32_t* token_indices, int
     return hipGetLastError();
 }
 
+// topk_idx, grad, gate_w: null, or what adds the router's share to the tokens' gradient.
 hipError_t launch_dispatch_backward(const void* a, const void* b, const int32_t* pair_row, int S, int k, int H, int dtype,
-                                    void* dx, hipStream_t st) {
+                                    void* dx, const int32_t* topk_idx, const void* grad, const void* gate_w, hipStream_t st) {
     if (S <= 0) return hipSuccess;
     const int grid = (S + 3) / 4;
-    if (dtype == MOE_DTYPE_F32) dispatch_backward_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)a, (const float*)b, pair_row, S, k, H, (float*)dx);
-    else if (dtype == MOE_DTYPE_FP16) dispatch_backward_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx);
-    else dispatch_backward_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx);
+    const float* dl = static_cast<const float*>(grad);
+    if (dtype == MOE_DTYPE_F32) dispatch_backward_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)a, (const float*)b, pair_row, S, k, H, (float*)dx, topk_idx, dl, (const float*)gate_w);
+    else if (dtype == MOE_DTYPE_FP16) dispatch_backward_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
+    else dispatch_backward_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
     return hipGetLastError();
 }
 

@@ -241,7 +241,12 @@ hipError_t launch_act_forward(const void* u, const void* g, const int32_t* count
 hipError_t launch_dispatch_rows(const void* x, const int32_t* token_indices, int64_t A, int S, int H, int dtype, void* rows,
                                 hipStream_t st);
 hipError_t launch_dispatch_backward(const void* a, const void* b, const int32_t* pair_row, int S, int k, int H, int dtype,
-                                    void* dx, hipStream_t st);
+                                    void* dx, const int32_t* topk_idx, const void* grad, const void* gate_w, hipStream_t st);
+size_t router_grad_bytes(int S, int E, int k);
+hipError_t launch_combine_backward_router(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w,
+                                          const int32_t* topk_idx, const float* logits, int S, int E, int k, int H, int gate_fn, int norm,
+                                          int dtype, void* dy, void* grad, hipStream_t st);
+hipError_t launch_gate_wgrad(const void* x, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st);
 hipError_t launch_combine_backward(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S,
                                    int k, int H, int dtype, void* dy, float* dw, hipStream_t st);
 

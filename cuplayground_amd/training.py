@@ -4,9 +4,10 @@ The reference declares a training knob (`is_training`, aristos_config.schema.jso
 Here it has a consumer: `MoE355Train` runs the expert projections through `moe_expert_gemm` and gets their gradients
 from `moe_expert_gemm` on the transposed weight (data gradient) and `moe_expert_wgrad` (weight gradient).  Routing
 decisions (top-k indices, slots, capacity drops) come from the library's router and are not differentiated; the gate
-weights that scale the expert outputs are recomputed in torch from the same logits formula, so the router's weight
-matrix and the tokens receive gradients through them.  Everything else -- dispatch, projections, activation, combine --
-is one autograd node (`_Experts`) whose backward runs the library's adjoints; the data gradient of the down projection
+weights that scale the expert outputs are, by the router's own kernels (`_RoutedExperts`) or, where those do not exist, as
+torch ops on the same logits formula, so the router's weight matrix and the tokens receive gradients through them.
+Everything else -- dispatch, projections, activation, combine -- is one autograd node (`_Experts`, or that node with the
+router) whose backward runs the library's adjoints; the data gradient of the down projection
 carries the activation's derivative in its epilogue (`moe_expert_gemm_act_backward`) where the layer has that kernel,
 else `moe_expert_gemm` is followed by `moe_act_backward`.  `expert_linear` and `act_down` are the projections as nodes
 of their own, for layers composed in torch.  There is no CPU path: every tensor lives on the GPU.
@@ -93,6 +94,65 @@ def _as_stored(layer, w):
     return isinstance(layer, api.MoELayer) and w.data_ptr() % 16 == 0 and layer.gemm_kn_supported(w.shape[2], w.shape[1]) == 2
 
 
+def _expert_rows(x, w_up, w_gate, w_down, layer, token_indices, count, offset):
+    """The packed rows of the expert side's forward pass: tokens, projections u and g, activation h, outputs y."""
+    rows = layer.dispatch_rows(_aligned(x), token_indices)
+
+    def product(a, w):
+        out = torch.empty(a.shape[0], w.shape[1], dtype=a.dtype, device=a.device)
+        return layer.expert_gemm(a, w, None, count, offset, api.ACT_NONE, out=out)
+
+    u = product(rows, w_up)
+    g = None if w_gate is None else product(rows, w_gate)
+    h = layer.act_forward(u, g, count, offset)
+    return rows, u, g, h, product(h, w_down)
+
+
+def _kept(needs, rows, u, g, h, w_up, w_gate, w_down):
+    """What of the forward pass the gradients that are asked for read (a step that trains the router alone reads y)."""
+    need_x, need_up, need_gate, need_down = needs
+    need_u = need_x or need_up or need_gate
+
+    def kept(needed, t):
+        return t if needed else None
+
+    return (kept(need_up or need_gate, rows), kept(need_u, u), kept(need_u, g), kept(need_down, h),
+            kept(need_x, w_up), kept(need_x, w_gate), kept(need_u, w_down))
+
+
+def _expert_gradients(layer, needs, dy, kept, count, offset):
+    """(da rows, db rows or None, dw_up, dw_gate, dw_down), each None where it is not asked for."""
+    rows, u, g, h, w_up, w_gate, w_down = kept
+    need_x, need_up, need_gate, need_down = needs
+
+    def product(a, w_t):
+        out = torch.empty(a.shape[0], w_t.shape[1], dtype=a.dtype, device=a.device)
+        return layer.expert_gemm(a, w_t, None, count, offset, api.ACT_NONE, out=out)
+
+    da = db = dup = dgate = ddown = None
+    if need_down:
+        ddown = layer.expert_wgrad(dy, h, count, offset)
+    if need_x or need_up or need_gate:
+        if _as_stored(layer, w_down):
+            du, dg = layer.expert_gemm_kn(dy, w_down, count, offset, u, g)                         # dH = dY . W_down, times act'
+        elif layer.fused_act_backward:
+            du, dg = layer.expert_gemm_act_backward(dy, api.transpose(w_down), u, g, count, offset, du=torch.empty_like(u),
+                                                    dg=None if g is None else torch.empty_like(g))
+        else:
+            du, dg = layer.act_backward(product(dy, api.transpose(w_down)), u, g)
+        if need_x:
+            def data_gradient(d, w):                                                               # dA = dU . W_up
+                return layer.expert_gemm_kn(d, w, count, offset) if _as_stored(layer, w) else product(d, api.transpose(w))
+
+            da = data_gradient(du, w_up)
+            db = None if g is None else data_gradient(dg, w_gate)
+        if need_up:
+            dup = layer.expert_wgrad(du, rows, count, offset)                                      # dW[e] = dU_e^T . A_e
+        if need_gate:
+            dgate = layer.expert_wgrad(dg, rows, count, offset)
+    return da, db, dup, dgate, ddown
+
+
 class _Experts(torch.autograd.Function):
     """(x [S,H], expert weights, topk_w [S,k]) -> the gate-weighted sum of the chosen experts' outputs.
 
@@ -103,65 +163,61 @@ class _Experts(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_up, w_gate, w_down, topk_w, layer, token_indices, pair_row, count, offset):
         w_up, w_down, topk_w = w_up.contiguous(), w_down.contiguous(), topk_w.contiguous()
-        rows = layer.dispatch_rows(_aligned(x), token_indices)
-
-        def product(a, w):
-            out = torch.empty(a.shape[0], w.shape[1], dtype=a.dtype, device=a.device)
-            return layer.expert_gemm(a, w, None, count, offset, api.ACT_NONE, out=out)
-
-        u = product(rows, w_up)
-        g = None
-        if w_gate is not None:
-            w_gate = w_gate.contiguous()
-            g = product(rows, w_gate)
-        h = layer.act_forward(u, g, count, offset)
-        y = product(h, w_down)
-        # kept: what the gradients that are asked for read (a step that trains the router alone reads y)
-        need_x, need_up, need_gate, need_down = ctx.needs_input_grad[:4]
-        need_u = need_x or need_up or need_gate
-
-        def kept(needed, t):
-            return t if needed else None
-
-        ctx.save_for_backward(kept(need_up or need_gate, rows), kept(need_u, u), kept(need_u, g), kept(need_down, h), y,
-                              kept(need_x, w_up), kept(need_x, w_gate), kept(need_u, w_down), topk_w, pair_row, count, offset)
+        w_gate = None if w_gate is None else w_gate.contiguous()
+        rows, u, g, h, y = _expert_rows(x, w_up, w_gate, w_down, layer, token_indices, count, offset)
+        ctx.save_for_backward(*_kept(ctx.needs_input_grad[:4], rows, u, g, h, w_up, w_gate, w_down), y, topk_w, pair_row, count, offset)
         ctx.layer = layer
         return api.combine(y, pair_row, topk_w)
 
     @staticmethod
     def backward(ctx, dout):
-        rows, u, g, h, y, w_up, w_gate, w_down, topk_w, pair_row, count, offset = ctx.saved_tensors
-        layer = ctx.layer
-        need_x, need_up, need_gate, need_down = ctx.needs_input_grad[:4]
-
-        def product(a, w_t):
-            out = torch.empty(a.shape[0], w_t.shape[1], dtype=a.dtype, device=a.device)
-            return layer.expert_gemm(a, w_t, None, count, offset, api.ACT_NONE, out=out)
-
+        *kept, y, topk_w, pair_row, count, offset = ctx.saved_tensors
+        layer, needs = ctx.layer, ctx.needs_input_grad[:4]
         dy, dtopk = layer.combine_backward(_aligned(dout), y, pair_row, topk_w, dy=torch.empty_like(y))
-        dx = dup = dgate = ddown = None
-        if need_down:
-            ddown = layer.expert_wgrad(dy, h, count, offset)
-        if need_x or need_up or need_gate:
-            if _as_stored(layer, w_down):
-                du, dg = layer.expert_gemm_kn(dy, w_down, count, offset, u, g)                     # dH = dY . W_down, times act'
-            elif layer.fused_act_backward:
-                du, dg = layer.expert_gemm_act_backward(dy, api.transpose(w_down), u, g, count, offset, du=torch.empty_like(u),
-                                                        dg=None if g is None else torch.empty_like(g))
-            else:
-                du, dg = layer.act_backward(product(dy, api.transpose(w_down)), u, g)
-            if need_x:
-                def data_gradient(d, w):                                                           # dA = dU . W_up
-                    return layer.expert_gemm_kn(d, w, count, offset) if _as_stored(layer, w) else product(d, api.transpose(w))
-
-                da = data_gradient(du, w_up)
-                db = None if g is None else data_gradient(dg, w_gate)
-                dx = layer.dispatch_backward(da, db, pair_row)
-            if need_up:
-                dup = layer.expert_wgrad(du, rows, count, offset)                                  # dW[e] = dU_e^T . A_e
-            if need_gate:
-                dgate = layer.expert_wgrad(dg, rows, count, offset)
+        da, db, dup, dgate, ddown = _expert_gradients(layer, needs, dy, kept, count, offset)
+        dx = layer.dispatch_backward(da, db, pair_row) if needs[0] else None
         return dx, dup, dgate, ddown, dtopk, None, None, None, None, None
+
+
+class _RoutedExperts(torch.autograd.Function):
+    """(x [S,H], expert weights, gate_w [E,H]) -> the layer's output: `_Experts` with the router inside the node.
+
+    The gate weights are the routing kernel's own and their adjoint rides in passes that run anyway: the combine's adjoint, one
+    wavefront a token, goes on to the logits' gradients; the dispatch's adds their product with the router's weight rows to the
+    tokens' gradient in fp32; what is left is one pass over x for the router's weight gradient.  As torch ops the router took
+    about 25 launches and fp32 copies of x.  A bf16 step, before and after: 922 -> 786 us (GELU, the larger layer of the
+    benchmark table), 1302 -> 1172 us (SwiGLU), 720 -> 330 us for a few hundred tokens, where launches are the time."""
+
+    @staticmethod
+    def forward(ctx, x, w_up, w_gate, w_down, gate_w, layer):
+        x, gate_w, w_up, w_down = _aligned(x), _aligned(gate_w), w_up.contiguous(), w_down.contiguous()
+        w_gate = None if w_gate is None else w_gate.contiguous()
+        c = layer.cfg
+        need_router = ctx.needs_input_grad[0] or ctx.needs_input_grad[4]
+        gate = layer.gate(x, gate_w, want_logits=need_router and c.gate_fn != api.GATE_SOFTMAX and bool(c.norm_topk_prob))
+        idx, topk_w, logits = gate if len(gate) == 3 else (*gate, None)
+        r = layer.route(idx)
+        pair_row, count, offset = r["pair_row"], r["expert_count"], r["expert_offset"]
+        rows, u, g, h, y = _expert_rows(x, w_up, w_gate, w_down, layer, r["token_indices"], count, offset)
+        ctx.save_for_backward(*_kept(ctx.needs_input_grad[:4], rows, u, g, h, w_up, w_gate, w_down), y, topk_w, pair_row, count, offset,
+                              x if ctx.needs_input_grad[4] else None, gate_w if ctx.needs_input_grad[0] else None, idx, logits)
+        ctx.layer = layer
+        return api.combine(y, pair_row, topk_w)
+
+    @staticmethod
+    def backward(ctx, dout):
+        *kept, y, topk_w, pair_row, count, offset, x, gate_w, idx, logits = ctx.saved_tensors
+        layer, needs = ctx.layer, ctx.needs_input_grad[:4]
+        dout, dy, router = _aligned(dout), torch.empty_like(y), None
+        if needs[0] or ctx.needs_input_grad[4]:
+            router = torch.empty(layer.router_grad_bytes, dtype=torch.uint8, device=y.device)
+            layer.combine_router_backward(dout, y, pair_row, topk_w, idx, logits, dy, router)
+        else:
+            layer.combine_backward(dout, y, pair_row, topk_w, dy=dy)
+        da, db, dup, dgate, ddown = _expert_gradients(layer, needs, dy, kept, count, offset)
+        dx = layer.dispatch_router_backward(da, db, pair_row, idx, router, gate_w) if needs[0] else None
+        dgate_w = layer.gate_wgrad(x, router) if ctx.needs_input_grad[4] else None
+        return dx, dup, dgate, ddown, dgate_w, None
 
 
 class MoE355Train(torch.nn.Module):
@@ -197,8 +253,20 @@ class MoE355Train(torch.nn.Module):
         w = scores.gather(1, idx.long())
         return w / w.sum(1, keepdim=True) if c.norm_topk_prob else w
 
+    def _routed(self, x):
+        """Whether the router's gradients have kernels for this call; else the gate weights are torch ops.  Not under autocast,
+        which computes the logits in 16 bits, not with a route or gate weights of a subclass's own, and not for a softmax that is
+        not normalised over the chosen experts (every logit has a gradient there)."""
+        return (isinstance(self.layer, api.MoELayer) and x.is_cuda and x.dim() == 2 and x.shape[0] >= self.cfg.tokens
+                and x.shape[1] == self.cfg.hidden_size and x.dtype == self.gate_w.dtype == self.layer.act_dtype
+                and getattr(self.route, "__func__", None) is _ROUTE and getattr(self.gate_weights, "__func__", None) is _GATE_WEIGHTS
+                and not torch.is_autocast_enabled("cuda") and self.layer.router_grad_bytes > 0)
+
     def forward(self, x):
         c = self.cfg
+        if self._routed(x):
+            rows = x if x.shape[0] == c.tokens else x[:c.tokens]
+            return _RoutedExperts.apply(rows, self.w_up, self.w_gate, self.w_down, self.gate_w, self.layer)
         idx, r = self.route(x)
         count, offset = r["expert_count"], r["expert_offset"]
         # fp32 whatever gate_weights computed in: the combine reads fp32 (under autocast the logits, and with them a sigmoid's
@@ -207,3 +275,6 @@ class MoE355Train(torch.nn.Module):
         rows = x if x.shape[0] == c.tokens else x[:c.tokens]      # rows behind the layer's tokens: zero gradients
         return _Experts.apply(rows, self.w_up, self.w_gate, self.w_down, w, self.layer, r["token_indices"], r["pair_row"],
                               count, offset)
+
+
+_ROUTE, _GATE_WEIGHTS = MoE355Train.route, MoE355Train.gate_weights

@@ -436,6 +436,20 @@ int moe_expert_gemm_kn_supported(const moe_handle* h, int32_t N, int32_t K, int3
 int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const void* u_rows, const void* g_rows,
                        const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K, void* out_rows,
                        void* out1_rows, void* stream);
+/* The router's share of a training step, without the logits' gradients of all experts ever being multiplied:
+ * moe_combine_router_backward: moe_combine_backward whose gate-weight gradients go on through the gate -- softmax normalised over the
+ *   chosen experts, or sigmoid, normalised or not (logits [S, E] from moe_gate: the normalised sigmoid only) -- into router_grad
+ *   (moe_router_grad_bytes, 256-byte aligned; MOE_ERR_UNSUPPORTED for a softmax that is not normalised, whose weights depend on
+ *   every logit).  Everything in fp32.
+ * moe_dispatch_router_backward: moe_dispatch_backward plus sum over ranks of that gradient times gate_w's row of the chosen expert,
+ *   added up in fp32 and rounded once.
+ * moe_gate_wgrad: dgate_w [E, H] in the layer's storage type; scratch as for the expert products. */
+int moe_router_grad_bytes(const moe_handle* h, size_t* bytes);
+int moe_combine_router_backward(moe_handle* h, const void* dout, const void* y_rows, const int32_t* pair_row, const float* topk_w,
+                                const int32_t* topk_idx, const float* logits, void* dy_rows, void* router_grad, void* stream);
+int moe_dispatch_router_backward(moe_handle* h, const void* da_rows, const void* db_rows, const int32_t* pair_row, const int32_t* topk_idx,
+                                 const void* router_grad, const void* gate_w, void* dx, void* stream);
+int moe_gate_wgrad(moe_handle* h, const void* x, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream);
 /* The elementwise and reduction steps between those products (same layers; fp32 arithmetic, one rounding on store):
  * moe_act_backward: for the first `rows` packed rows of width I, du = dh * act'(u) for hidden_act ReLU (1 where u > 0)
  *   and GELU (Phi(u) + u phi(u)); for SwiGLU, where h = silu(g) * u, du = dh * silu(g) and dg = dh * u * s * (1 + g (1 - s))

@@ -198,3 +198,63 @@ def test_a_layer_composed_of_the_projection_nodes_is_the_layer(moe, act, dtype, 
     assert rel(composed, out) <= 2 * {2: 1e-2, 3: 2e-3}.get(dtype, 2e-5)
     for n in leaves:
         assert rel(grads[n], want[n]) <= 2 * {2: 2e-2, 3: 4e-3}.get(dtype, 1e-4), n
+
+
+@pytest.mark.parametrize("S,H,E,k,gate_fn,norm,dtype,drop", [
+    (257, 320, 5, 3, 0, 1, 2, 1), (1, 64, 2, 1, 1, 0, 0, 0), (1, 64, 70, 8, 0, 1, 3, 0), (4100, 256, 16, 2, 0, 1, 2, 1),
+    (300, 1024, 130, 6, 1, 1, 0, 1), (700, 448, 33, 4, 1, 1, 2, 0), (129, 576, 64, 16, 1, 0, 3, 1), (9000, 64, 8, 1, 0, 1, 0, 0)])
+def test_router_gradients(moe, S, H, E, k, gate_fn, norm, dtype, drop):
+    """The adjoint of the gate inside the combine's and the dispatch's, and the router's weight gradient, against float64."""
+    import torch
+    cfg = moe.MoEConfig(capacity_factor=0.8, drop_tokens=drop, expert_top_k=k, hidden_act=1, hidden_size=H, intermediate_size=64,
+                        micro_batch=1, num_experts=E, sequence_len=S, torch_dtype=dtype, gate_fn=gate_fn, norm_topk_prob=norm)
+    layer = moe.MoELayer(cfg)
+    gen = torch.Generator(device="cuda").manual_seed(S + E)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=gen, device="cuda").to(layer.act_dtype)
+
+    x, gate_w, y, dout = rand(S, H), rand(E, H) * H ** -0.5, rand(S * k, H), rand(S, H)
+    idx, w, logits = layer.gate(x, gate_w, want_logits=True)
+    rows = layer.route(idx)["pair_row"]
+    dy, router = torch.empty_like(y), torch.empty(layer.router_grad_bytes, dtype=torch.uint8, device="cuda")
+    layer.combine_router_backward(dout, y, rows, w, idx, logits if gate_fn and norm else None, dy, router)
+    want_dy, dw = layer.combine_backward(dout, y, rows, w)
+    assert torch.equal(dy[rows[rows >= 0].long()], want_dy[rows[rows >= 0].long()])
+
+    # the gate in float64 from the kernel's own logits, its adjoint from the combine's fp32 gradients
+    l64 = logits.double().requires_grad_(True)
+    s = torch.softmax(l64, 1) if gate_fn == 0 else torch.sigmoid(l64)
+    w64 = s.gather(1, idx.long())
+    w64 = w64 / w64.sum(1, keepdim=True) if norm else w64
+    w64.backward(dw.double())
+    want = l64.grad.gather(1, idx.long())
+    dl = router[:4 * S * k].view(torch.float32).view(S, k)
+    # k products and sums of fp32 and the weights' own fp32 error: some tens of units of 2^-24 of the largest gradient of the token
+    scale = dw.double().abs().amax(1, keepdim=True).clamp(min=1e-30) * (1.0 if not (gate_fn and norm) else k)
+    assert float(((dl.double() - want).abs() / scale).max()) <= 64 * 2.0 ** -24
+
+    # the sums: terms in fp32 (2^-24 of the sum of magnitudes for each of the terms one accumulator takes), then one rounding
+    unit = {0: 2.0 ** -24, 1: 2.0 ** -24, 2: 2.0 ** -8, 3: 2.0 ** -11}[dtype]         # half a step of the stored type
+    dense = torch.zeros(S, E, dtype=torch.float64, device="cuda").scatter_(1, idx.long(), dl.double())
+    got, ref, mag = layer.gate_wgrad(x, router).double(), dense.t() @ x.double(), dense.t().abs() @ x.double().abs()
+    tiny = 2.0 ** -24 if dtype == 3 else 0.0           # fp16 below its normal range
+    assert bool(((got - ref).abs() <= unit * ref.abs() + (S / 4 + 68) * 2.0 ** -24 * mag + tiny).all())
+    a, b = rand(S * k, H), rand(S * k, H)
+    got = layer.dispatch_router_backward(a, b, rows, idx, router, gate_w).double()
+    part = torch.where((rows >= 0)[..., None], a[rows.clamp(min=0).long()].double() + b[rows.clamp(min=0).long()].double(), 0.0).sum(1)
+    mag = torch.where((rows >= 0)[..., None], a[rows.clamp(min=0).long()].double().abs() + b[rows.clamp(min=0).long()].double().abs(), 0.0).sum(1)
+    ref, mag = part + dense @ gate_w.double(), mag + dense.abs() @ gate_w.double().abs()
+    assert bool(((got - ref).abs() <= unit * ref.abs() + (3 * k + 1) * 2.0 ** -24 * mag + tiny).all())
+
+
+def test_a_softmax_over_all_experts_keeps_its_torch_gate(moe):
+    """Not normalised over the chosen, each logit has a gradient: such a layer has no router kernels and says so."""
+    import torch
+    from cuplayground_amd import training
+    cfg = moe.MoEConfig(expert_top_k=2, hidden_act=1, hidden_size=64, intermediate_size=64, micro_batch=1, num_experts=4,
+                        sequence_len=32, torch_dtype=2, gate_fn=0, norm_topk_prob=0, is_training=1)
+    m = training.MoE355Train(cfg, init_std=0.2)
+    assert m.layer.router_grad_bytes == 0
+    m(torch.randn(32, 64, device="cuda", dtype=torch.bfloat16)).float().sum().backward()
+    assert bool((m.gate_w.grad.float().abs().sum(1) > 0).all())

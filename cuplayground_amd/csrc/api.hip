@@ -345,6 +345,7 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
+constexpr int kSplitComputeUnits = 256, kSplitRowsPerExpert = 192, kSplitRounds = 11;
 int resolved_ffn_mode(const moe_handle* h) {
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
     if (h->d.plan.mfma8) return MOE_FFN_TILED;
@@ -371,6 +372,18 @@ int resolved_ffn_mode(const moe_handle* h) {
     // (the fp32 one: 1.26 against 1.02 ms, 16 tokens on 8 experts of 4096 x 14336; 2.89 against 2.21 for 128 tokens)
     if ((d.plan.kernel_dtype == MOE_DTYPE_F32 || d.plan.kernel_dtype == MOE_DTYPE_TF32) && d.plan.tile == kF32StreamTile) return MOE_FFN_TILED;
     if ((f32_tile || tile16) && d.E == 1) return MOE_FFN_TILED;
+    // Two launches on row blocks and remainders (launch_ffn_split_16) against the queue.  128-row blocks: always faster where that tile is
+    // chosen (figures beside the launch).  256-row blocks, queue / two launches, us: few rows an expert, where remainders are most of the
+    // work: 64 experts of 2048 x 1408, 141 rows each 323 / 311, 188 rows 346 / 328; and many rounds of short tasks, where the queue's
+    // pops and written-through rows add up: 1536 rows 1707 / 1665, uneven and capped 728 / 720.  Between these the queue, which
+    // starts the down projection under the up projection's last round: 750 rows 913 / 907, 375 rows 541 / 559; 16 of 2048 x 2048, 512
+    // rows 214 / 223; 12 of 1344 x 2752, 1000 rows 259 / 289; 8 of 4096 x 14336, 256 rows 894 / 989, 2048 rows 4447 / 4463 (4 rounds down).
+    // (Options of the queue and its trace keep it.)
+    if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && h->opt.queue_early != 1 && !h->task_trace) {
+        if (d.plan.tile == 2) return MOE_FFN_TILED;
+        const int64_t rounds = (d.A / d.plan.block_m) * std::min(d.plan.nnt0, d.plan.nnt1) / kSplitComputeUnits;
+        if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || rounds >= kSplitRounds)) return MOE_FFN_TILED;
+    }
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }
 
@@ -804,6 +817,7 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
     FfnArgs fa{};        // every field starts null / zero: a member nobody sets must not reach a kernel as stack garbage
     fa.x = x;
     fa.token_indices = ra.token_indices;
+    fa.expert_count = ra.expert_count; fa.expert_offset = ra.expert_offset;
     fa.w_up = w->w_up; fa.w_gate = w->w_gate; fa.w_down = w->w_down;
     fa.b_up = w->b_up; fa.b_gate = w->b_gate; fa.b_down = w->b_down;
     fa.s_up = w->s_up; fa.s_gate = w->s_gate; fa.s_down = w->s_down;

@@ -1,4 +1,4 @@
-// Products on the 16-bit tiles (ffn_bf16_tile.hpp) outside the layer: dense operands, packed rows by expert, weight gradients.
+// Products on the 16-bit tiles (ffn_bf16_tile.hpp): dense operands, packed rows by expert (a layer's two launches too), weight gradients.
 #include <algorithm>
 
 #include "ffn_bf16_tile.hpp"
@@ -57,23 +57,48 @@ struct PlainSplit {
     static constexpr int BIG = 128, BN = 128, THREADS = 256, LDS_BYTES = TB::LDS_BYTES;
 };
 
+constexpr int kShareSlack = 14;      // workgroups without a tile, at most: the two lists are rounded up to eight equal shares
 struct GroupedTask {
     int expert, row0, rows, ctile;
 };
 // Which tile workgroup `id` of a grouped product takes, from the experts' row counts alone; false: none.  Order: the row blocks of
-// full height, expert by expert, column tile by column tile, an expert's row blocks fastest (neighbouring workgroups share a
-// weight tile, an expert's few row blocks stay in the caches while its column tiles pass by); with 256-row blocks, behind them the
-// remainders of at most 128 rows: the long tasks start first, and the short ones fill the compute units that the last round of
-// long ones leaves idle.  Every wavefront works it out for itself, an expert a lane, which takes less time than a launch
-// in front that writes tables.
+// full height, expert by expert, column tile by column tile, an expert's row blocks fastest (an expert's few row blocks stay in the
+// caches while its column tiles pass by); with 256-row blocks, behind them the remainders of at most 128 rows: the long tasks start
+// first, and the short ones fill the compute units that the last round of long ones leaves idle.  Workgroups go to the eight XCDs in
+// turn: each XCD takes an eighth of either list in a row, so that the tiles that share a weight tile or token rows share an L2.
+// Every wavefront works it out for itself, an expert a lane, which takes less time than a launch in front that writes tables.
 // 16 experts of 2048 x 2048, 512 rows each, bf16: 112 -> 93 us (320 tasks on 256 compute units, 64 of them remainders); 8 of
 // 4096 x 2048, 2048 rows 297 -> 258; 64 of 2048 x 1408, 94 rows 113 -> 106; 16 of 2048 x 1408, 750 rows, no remainders, 109 -> 110.
+// The share of an XCD in a row, against the list dealt out to them: whole layers, 8 experts of 4096 x 14336, 2048 rows 4825 -> 4463 us,
+// 1024 rows 2888 -> 2448; 64 of 2048 x 1408, 1536 rows 1862 -> 1665, 750 rows 1112 -> 907; 12 of 1344 x 2752, 444 rows 180 -> 166.
 template <int BIG>
 __device__ __forceinline__ bool grouped_task(const int32_t* __restrict__ count, const int32_t* __restrict__ offset, int E, int ncol, int id, GroupedTask& t) {
     constexpr int LEFT = BIG == 256 ? 128 : 0;          // rows up to which what is left of an expert is a block of its own kind
     const int lane = threadIdx.x & 63;
     auto rows_of = [&](int c) { return c + lane < E ? max(count[c + lane], 0) : 0; };
     auto big_of = [&](int n) { return (n + BIG - 1 - LEFT) / BIG; };
+    int big_sum = 0, left_sum = 0;         // full row blocks and remainders of all experts
+    for (int c = 0; c < E; c += kWave) {
+        const int n = rows_of(c), big = big_of(n);
+        big_sum += big;
+        left_sum += n > big * BIG ? 1 : 0;
+    }
+#pragma unroll
+    for (int off = kWave / 2; off; off >>= 1) {
+        big_sum += __shfl_xor(big_sum, off, kWave);
+        left_sum += __shfl_xor(left_sum, off, kWave);
+    }
+    const int bigs = __builtin_amdgcn_readfirstlane(big_sum) * ncol, lefts = __builtin_amdgcn_readfirstlane(left_sum) * ncol;
+    const int big_share = (bigs + 7) / 8, left_share = (lefts + 7) / 8;
+    if (id < 8 * big_share) {
+        id = (id & 7) * big_share + (id >> 3);
+        if (id >= bigs) return false;
+    } else {
+        id -= 8 * big_share;
+        if ((id >> 3) >= left_share) return false;
+        id = (id & 7) * left_share + (id >> 3) + bigs;
+        if (id >= bigs + lefts) return false;
+    }
     int base = 0;                          // full row blocks of the experts in front
     for (int c = 0; c < E; c += kWave) {
         const int n = rows_of(c), big = big_of(n);
@@ -119,7 +144,7 @@ __device__ __forceinline__ bool grouped_task(const int32_t* __restrict__ count, 
 }
 // What a grouped product does with its sums: one kernel each, so that a tile's code is a slab loop and one epilogue (with three of
 // them a kernel of several tiles is twice the instruction cache).
-enum : int { kSums = 0, kGelu = 2, kDeriv = 4 };      // sums or ReLU; GELU; the activation's derivative
+enum : int { kSums = 0, kGelu = 2, kSwiglu = 3, kDeriv = 4 };      // sums or ReLU; GELU; SwiGLU; the activation's derivative
 template <class T, int EPI>
 __device__ __forceinline__ void grouped_epilogue(const TaskPtrs& p, unsigned char* smem, f32x4 (&acc)[T::TM][T::TN]) {
     epilogue_full_n_impl<T, EPI == kDeriv ? 0 : EPI, NoHook, WholeTile, EPI == kDeriv>(p, smem, acc, NoHook());
@@ -142,12 +167,12 @@ __device__ __forceinline__ void grouped_tile(const TaskPtrs& p, unsigned char* s
     }
 }
 
-// Grouped GEMM on packed expert-major rows, outside the layer: out[r,:] = act(a[r,:] . w[e(r)]^T + bias[e(r)]) -- the
+// Grouped GEMM on packed expert-major rows: out[r,:] = act(a[r,:] . w[e(r)]^T + bias[e(r)]) -- the
 // reference's tile GEMM (mma.cuh:46-179) once per expert.  With the weight handed over in its K-major view this is the data
 // gradient of a projection (dX = dY . W).  DERIV: that of the down projection with the activation's derivative in its epilogue,
-// which hands on dU (and dG) instead of dH.  One workgroup per tile (grouped_task).
+// which hands on dU (and dG) instead of dH.  With gather and w1 the up projection of a layer.  One workgroup per tile (grouped_task).
 struct GroupedArgs {
-    const uint16_t* a_rows;
+    const uint16_t* a_rows;      // packed rows, or with gather the tokens
     const uint16_t* w;
     const uint16_t* bias;        // or null
     const uint16_t* u_rows;      // DERIV: the saved projections ...
@@ -158,32 +183,37 @@ struct GroupedArgs {
     const int32_t* offset;
     int E, N, K, act;            // act: the epilogue's activation (DERIV: the layer's hidden_act)
     uint32_t a_bytes;
+    // a layer's up projection:
+    const int32_t* gather;       // null, or the token of every packed row
+    const uint16_t* w1;          // SwiGLU: the gate's weights ...
+    const uint16_t* bias1;       // ... and biases, or null
 };
 template <class P, int EPI>
 __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a) {
-    constexpr bool DERIV = EPI == kDeriv;
+    constexpr bool DERIV = EPI == kDeriv, SWIGLU = EPI == kSwiglu;
+    constexpr int COLS = SWIGLU ? P::BN / 2 : P::BN;      // half of a SwiGLU tile's weight rows are gate rows
     extern __shared__ __align__(16) unsigned char smem[];
     const int N = a.N, K = a.K;
     GroupedTask t;
-    if (!grouped_task<P::BIG>(a.count, a.offset, a.E, (N + P::BN - 1) / P::BN, blockIdx.x, t)) return;
+    if (!grouped_task<P::BIG>(a.count, a.offset, a.E, (N + COLS - 1) / COLS, blockIdx.x, t)) return;
     const int64_t at = (int64_t)t.row0 * N;
     TaskPtrs p;
     p.a_base = a.a_rows;
-    p.gather = nullptr;
-    p.a_row0 = t.row0;
+    p.gather = a.gather ? a.gather + t.row0 : nullptr;
+    p.a_row0 = a.gather ? 0 : t.row0;
     p.a_ld = K;
     p.b0 = a.w + (int64_t)t.expert * N * K;
-    p.b1 = nullptr;
+    p.b1 = SWIGLU ? a.w1 + (int64_t)t.expert * N * K : nullptr;
     p.b_ld = K;
     p.bias0 = a.bias ? a.bias + (int64_t)t.expert * N : nullptr;
-    p.bias1 = nullptr;
+    p.bias1 = SWIGLU && a.bias1 ? a.bias1 + (int64_t)t.expert * N : nullptr;
     p.c_base = a.out + at;
     p.N = N;
     p.K = K;
     p.rows = t.rows;
-    p.n0 = t.ctile * P::BN;
+    p.n0 = t.ctile * COLS;
     p.act = DERIV ? MOE_ACT_NONE : a.act;
-    p.swiglu = false;
+    p.swiglu = SWIGLU;
     p.publish = false;
     p.a_extent = a.a_bytes;
     p.b_extent = (uint32_t)((int64_t)N * K * 2);
@@ -556,7 +586,8 @@ static hipError_t launch_grouped(const GroupedArgs& g, int64_t A, hipStream_t st
     const auto kernel = &grouped_gemm_kernel<P, EPI>;
     hipError_t e = allow_lds(kernel, P::LDS_BYTES);
     if (e != hipSuccess) return e;
-    const int64_t blocks = (A / P::BIG + g.E) * ((g.N + P::BN - 1) / P::BN);      // no expert has more than rows / BIG + 1 row blocks
+    constexpr int COLS = EPI == kSwiglu ? P::BN / 2 : P::BN;
+    const int64_t blocks = (A / P::BIG + g.E) * ((g.N + COLS - 1) / COLS) + kShareSlack;      // no expert has more than rows / BIG + 1 row blocks
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     kernel<<<(unsigned)blocks, P::THREADS, P::LDS_BYTES, st>>>(g);
     return hipGetLastError();
@@ -573,7 +604,7 @@ static hipError_t launch_grouped_tile(const GroupedArgs& g, int tile, int64_t A,
 hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const int32_t* count,
                                   const int32_t* offset, int tile, int64_t A, int E, int N, int K, int act, bool f16, hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, (const uint16_t*)bias, nullptr, nullptr, (uint16_t*)out, nullptr,
-                        count, offset, E, N, K, act, (uint32_t)(A * K * 2)};
+                        count, offset, E, N, K, act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
     if (act == MOE_ACT_GELU) return f16 ? launch_grouped_tile<true, kGelu>(g, tile, A, st) : launch_grouped_tile<false, kGelu>(g, tile, A, st);
     return f16 ? launch_grouped_tile<true, kSums>(g, tile, A, st) : launch_grouped_tile<false, kSums>(g, tile, A, st);
 }
@@ -583,8 +614,30 @@ hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const
                                         const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
                                         int hidden_act, bool f16, hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)du,
-                        (uint16_t*)dg, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2)};
+                        (uint16_t*)dg, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
     return f16 ? launch_grouped_tile<true, kDeriv>(g, tile, A, st) : launch_grouped_tile<false, kDeriv>(g, tile, A, st);
+}
+
+// A layer's two projections, a launch each: blocks of 256 rows and the 128-row tile for what an expert has left, or blocks of 128 rows.
+// Whole layers, us, the queue / two launches of it in the order of the row block table / this:
+//   128-row blocks: 12 experts of 1344 x 2752, GELU, 150 rows each 122 / 108 / 88, 250 rows 131 / 118 / 115; 64 of 2048 x 1408, SwiGLU,
+//   94 rows 278 / 295 / 264; 8 of 4096 x 14336, 128 rows 679 / 672 / 655; 16 of 2048 x 2048, 128 rows 130 / 112 / 110
+//   256-row blocks (queue / this): see resolved_ffn_mode
+template <class P>
+static hipError_t launch_ffn_split(const FfnArgs& a, hipStream_t st) {
+    const int64_t A = (int64_t)a.S * a.k;
+    GroupedArgs g{(const uint16_t*)a.x, (const uint16_t*)a.w_up, (const uint16_t*)a.b_up, nullptr, nullptr, (uint16_t*)a.h, nullptr,
+                  a.expert_count, a.expert_offset, a.E, a.I, a.H, a.act, a.x_bytes, a.token_indices, (const uint16_t*)a.w_gate, (const uint16_t*)a.b_gate};
+    const hipError_t e = a.act == MOE_ACT_SWIGLU ? launch_grouped<P, kSwiglu>(g, A, st)
+                         : a.act == MOE_ACT_GELU ? launch_grouped<P, kGelu>(g, A, st) : launch_grouped<P, kSums>(g, A, st);
+    if (e != hipSuccess) return e;
+    g = GroupedArgs{(const uint16_t*)a.h, (const uint16_t*)a.w_down, (const uint16_t*)a.b_down, nullptr, nullptr, (uint16_t*)a.y, nullptr,
+                    a.expert_count, a.expert_offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr};
+    return launch_grouped<P, kSums>(g, A, st);
+}
+hipError_t launch_ffn_split_16(const FfnArgs& a, int block_rows, bool f16, hipStream_t st) {
+    if (block_rows == 128) return f16 ? launch_ffn_split<RowSplit<true, 128>>(a, st) : launch_ffn_split<RowSplit<false, 128>>(a, st);
+    return f16 ? launch_ffn_split<RowSplit<true, 256>>(a, st) : launch_ffn_split<RowSplit<false, 256>>(a, st);
 }
 
 template <class T>
@@ -658,7 +711,7 @@ static hipError_t launch_grouped_kn(const GroupedArgs& g, int64_t A, hipStream_t
     using T = ProdTile<F16>;
     hipError_t e = allow_lds(&grouped_kn_kernel<T, EPI>, T::LDS_BYTES);
     if (e != hipSuccess) return e;
-    const int64_t tiles = (A / T::BM + g.E) * ((g.N + T::BN - 1) / T::BN);
+    const int64_t tiles = (A / T::BM + g.E) * ((g.N + T::BN - 1) / T::BN) + kShareSlack;
     if (tiles > INT32_MAX) return hipErrorInvalidValue;
     grouped_kn_kernel<T, EPI><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(g);
     return hipGetLastError();
@@ -668,7 +721,7 @@ hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const vo
                                      const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)out,
-                        (uint16_t*)out1, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2)};
+                        (uint16_t*)out1, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
     if (u) return f16 ? launch_grouped_kn<true, kDeriv>(g, A, st) : launch_grouped_kn<false, kDeriv>(g, A, st);
     return f16 ? launch_grouped_kn<true, kSums>(g, A, st) : launch_grouped_kn<false, kSums>(g, A, st);
 }

@@ -79,6 +79,8 @@ struct CombineState {
 struct FfnArgs {
     const void* x;              // [S,H]
     const int32_t* token_indices;
+    const int32_t* expert_count;   // [E] rows kept of every expert, and where they begin among the packed ones
+    const int32_t* expert_offset;
     const void* w_up;           // [E,I,H]
     const void* w_gate;         // [E,I,H] or null
     const void* w_down;         // [E,H,I]
@@ -190,6 +192,7 @@ struct FfnArgs;
 int stream16_block_m(int form);
 int stream16_block_n(int form);
 int ffn_persistent_occupancy_stream16(int form);
+hipError_t launch_ffn_split_16(const FfnArgs& a, int block_rows, bool f16, hipStream_t st);   // ffn_bf16_grouped.hip
 hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st);
 struct FfnPlan {
     int kernel_dtype;   // the dtype whose kernels run: the layer's, or bf16 for an e4m3 layer whose weights are widened

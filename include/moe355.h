@@ -307,8 +307,9 @@ int moe_get_stage_ms(moe_handle* h, int stage, float* ms, int32_t* calls);
 int moe_get_stage_samples(moe_handle* h, int stage, float* ms, int32_t capacity, int32_t* count);
 
 /* How evenly the task queue of the last moe_forward kept its workgroups busy (task-queue FFN only; MOE_ERR_UNSUPPORTED
- * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers and for single experts:
- * moe_get_ffn_mode tells).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
+ * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers, for single experts and,
+ * in 16-bit layers, for up to about 192 rows per expert or many rounds of short tasks: moe_get_ffn_mode tells, moe_set_ffn_mode asks
+ * for the queue).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
  * the queue kernel: span_us = first entry to last exit, mean_active_us = mean of (exit - entry), mean_tail_idle_us =
  * mean of (last exit - own exit), i.e. the time a workgroup had nothing left to pop while others still worked.
  * Synchronises `stream`.  No counterpart in the reference, whose scheduler keeps no statistics. */

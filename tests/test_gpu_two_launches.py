@@ -1,0 +1,64 @@
+"""The two launches of a 16-bit layer on row blocks and remainders (csrc/ffn_bf16_grouped.hip: grouped_task,
+launch_ffn_split_16): every tile is taken once, by the same arithmetic as on the task queue, so the bits are the queue's."""
+import numpy as np
+import pytest
+
+from oracle import binding as ob
+from helpers import OUT_TOL, from_device, max_rel_err, product_config, upload_inputs
+from test_gpu_layer import FFN_PERSISTENT, FFN_TILED, check_routing
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    # more experts than a wavefront has lanes, most of them with a few rows, some with none; one column tile and a ragged one
+    "many_experts": (ob.Cfg(S=200, H=128, I=320, E=150, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=0), False),
+    # remainders of every kind, ragged columns, biases
+    "ragged_gelu": (ob.Cfg(S=1531, H=448, I=704, E=9, k=3, act=ob.ACT_GELU, dtype=ob.F16, gate_fn=ob.GATE_SIGMOID, drop=0), True),
+    "ragged_swiglu": (ob.Cfg(S=1100, H=320, I=448, E=5, k=2, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SIGMOID, drop=0), True),
+    # capacities that are no whole row blocks, and ones that are: 384 rows are a block and a full remainder
+    "capped": (ob.Cfg(S=1536, H=256, I=256, E=8, k=2, act=ob.ACT_RELU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=1, capacity_factor=0.7), False),
+    "capped_blocks": (ob.Cfg(S=1536, H=256, I=256, E=8, k=2, act=ob.ACT_GELU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=1, capacity_factor=1.0), False),
+    "one_token": (ob.Cfg(S=1, H=256, I=512, E=4, k=1, act=ob.ACT_GELU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=0), False),
+}
+
+
+def _forward(cfg, dev, mode, tile):
+    import torch
+    import cuplayground_amd as moe
+    layer = moe.MoELayer(product_config(cfg), ffn_mode=mode, options={"tile16": tile})
+    routing = layer.new_routing()
+    out = torch.full((cfg.S, cfg.H), float("nan"), dtype=layer.act_dtype, device="cuda")
+    layer.forward(dev["x"], dev, out=out, routing=routing)
+    torch.cuda.synchronize()
+    layer.task_counts()
+    res = {k: from_device(v) for k, v in routing.items()}
+    res["out"] = from_device(out)
+    layer.close()
+    return res
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_same_bits_as_the_queue(name, tile):
+    cfg, bias = SHAPES[name]
+    inp = ob.make_inputs(cfg, seed=5, with_bias=bias)
+    want = ob.forward(cfg, inp)
+    dev = upload_inputs(cfg, inp)
+    got = _forward(cfg, dev, FFN_TILED, tile)
+    check_routing(got, want)
+    assert max_rel_err(ob.to_f32(got["out"], cfg.act_dtype), ob.to_f32(want["out"], cfg.act_dtype)) <= OUT_TOL[cfg.dtype]
+    assert np.array_equal(got["out"], _forward(cfg, dev, FFN_PERSISTENT, tile)["out"])
+
+
+@pytest.mark.parametrize("rows, experts, tokens, queue", [(64, 16, 512, False), (192, 64, 2048, False), (200, 64, 2134, True)])
+def test_mode_that_is_chosen(rows, experts, tokens, queue):
+    """Few rows per expert: two launches, also where there are many tasks; options and reports of the queue keep it."""
+    import cuplayground_amd as moe
+    cfg = ob.Cfg(S=tokens, H=2048, I=1408, E=experts, k=6 if experts == 64 else 2, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=0)
+    layer = moe.MoELayer(product_config(cfg))
+    assert (layer.ffn_mode == FFN_PERSISTENT) == queue
+    if experts == 64:
+        layer.enable_task_trace(1 << 10)
+        assert layer.ffn_mode == FFN_PERSISTENT
+        layer.disable_task_trace()
+    layer.close()

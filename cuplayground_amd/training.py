@@ -256,8 +256,9 @@ class MoE355Train(torch.nn.Module):
     def _routed(self, x):
         """Whether the router's gradients have kernels for this call; else the gate weights are torch ops.  Not under autocast,
         which computes the logits in 16 bits, not with a route or gate weights of a subclass's own, and not for a softmax that is
-        not normalised over the chosen experts (every logit has a gradient there)."""
-        return (isinstance(self.layer, api.MoELayer) and x.is_cuda and x.dim() == 2 and x.shape[0] >= self.cfg.tokens
+        not normalised over the chosen experts (every logit has a gradient there).  A single expert's normalised weight is one and
+        the router's gradient nothing but the rounding of w / w: it stays what the torch expression gives."""
+        return (not (self.cfg.expert_top_k == 1 and self.cfg.norm_topk_prob) and isinstance(self.layer, api.MoELayer) and x.is_cuda and x.dim() == 2 and x.shape[0] >= self.cfg.tokens
                 and x.shape[1] == self.cfg.hidden_size and x.dtype == self.gate_w.dtype == self.layer.act_dtype
                 and getattr(self.route, "__func__", None) is _ROUTE and getattr(self.gate_weights, "__func__", None) is _GATE_WEIGHTS
                 and not torch.is_autocast_enabled("cuda") and self.layer.router_grad_bytes > 0)

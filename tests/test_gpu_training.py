@@ -258,3 +258,25 @@ def test_a_softmax_over_all_experts_keeps_its_torch_gate(moe):
     assert m.layer.router_grad_bytes == 0
     m(torch.randn(32, 64, device="cuda", dtype=torch.bfloat16)).float().sum().backward()
     assert bool((m.gate_w.grad.float().abs().sum(1) > 0).all())
+
+
+@pytest.mark.parametrize("gate_fn", [0, 1], ids=["softmax", "sigmoid"])
+def test_a_single_normalised_expert_keeps_its_torch_gate(moe, gate_fn):
+    """Its weight is one, and the router's gradient the rounding of torch's w / w: the same bits as with gate weights of the
+    caller's own, which are torch ops always."""
+    import torch
+    from cuplayground_amd import training
+
+    class Own(training.MoE355Train):
+        def gate_weights(self, x, idx):
+            return super().gate_weights(x, idx)
+
+    cfg = moe.MoEConfig(expert_top_k=1, hidden_act=1, hidden_size=128, intermediate_size=64, micro_batch=1, num_experts=4,
+                        sequence_len=97, torch_dtype=0, gate_fn=gate_fn, norm_topk_prob=1, is_training=1)
+    grads = []
+    for kind in (training.MoE355Train, Own):
+        m, g = kind(cfg, init_std=0.2, seed=2), torch.Generator(device="cuda").manual_seed(7)
+        x = torch.randn(97, 128, generator=g, device="cuda", requires_grad=True)
+        m(x).backward(torch.randn(97, 128, generator=g, device="cuda"))
+        grads.append([x.grad] + [p.grad for _, p in m.named_parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

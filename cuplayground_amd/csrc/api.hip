@@ -345,7 +345,7 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
-constexpr int kSplitComputeUnits = 256, kSplitRowsPerExpert = 192, kSplitRounds = 11;
+constexpr int kSplitComputeUnits = 256, kSplitRowsPerExpert = 192, kSplitRounds = 11, kSplitCappedRows = 48;
 int resolved_ffn_mode(const moe_handle* h) {
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
     if (h->d.plan.mfma8) return MOE_FFN_TILED;
@@ -378,9 +378,10 @@ int resolved_ffn_mode(const moe_handle* h) {
     // pops and written-through rows add up: 1536 rows 1707 / 1665, uneven and capped 728 / 720.  Between these the queue, which
     // starts the down projection under the up projection's last round: 750 rows 913 / 907, 375 rows 541 / 559; 16 of 2048 x 2048, 512
     // rows 214 / 223; 12 of 1344 x 2752, 1000 rows 259 / 289; 8 of 4096 x 14336, 256 rows 894 / 989, 2048 rows 4447 / 4463 (4 rounds down).
-    // (Options of the queue and its trace keep it.)
+    // (Options of the queue and its trace keep it.)  Layers that drop tokens at few rows per expert keep it too: 64 of 2048 x 1408, at most 29
+    // rows 234 / 243, 38 rows 237 / 247, 57 rows 248 / 248, 94 rows 249 / 240 (28 rows, none dropped: 284 / 267).
     if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && h->opt.queue_early != 1 && !h->task_trace) {
-        if (d.plan.tile == 2) return MOE_FFN_TILED;
+        if (d.plan.tile == 2 && !(h->cfg.drop_tokens && d.capacity <= kSplitCappedRows)) return MOE_FFN_TILED;
         const int64_t rounds = (d.A / d.plan.block_m) * std::min(d.plan.nnt0, d.plan.nnt1) / kSplitComputeUnits;
         if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || rounds >= kSplitRounds)) return MOE_FFN_TILED;
     }

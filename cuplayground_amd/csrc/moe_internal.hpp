@@ -192,6 +192,7 @@ struct FfnArgs;
 int stream16_block_m(int form);
 int stream16_block_n(int form);
 int ffn_persistent_occupancy_stream16(int form);
+bool ffn_split_16_keeps_table(const FfnArgs& a);
 hipError_t launch_ffn_split_16(const FfnArgs& a, int block_rows, bool f16, hipStream_t st);   // ffn_bf16_grouped.hip
 hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st);
 struct FfnPlan {

@@ -62,3 +62,30 @@ def test_mode_that_is_chosen(rows, experts, tokens, queue):
         assert layer.ffn_mode == FFN_PERSISTENT
         layer.disable_task_trace()
     layer.close()
+
+
+@pytest.mark.parametrize("S,H,I,E,k,tile", [(900, 1984, 3008, 20, 3, 2), (1300, 1984, 3008, 20, 3, 2), (2300, 2048, 2048, 16, 2, 1), (1000, 320, 448, 5, 2, 2)])
+def test_same_bits_whatever_blocks_the_rounds_choose(S, H, I, E, k, tile):
+    """Layers planned on 128-row blocks whose launches take 256-row blocks and remainders, layers that keep the table's order, and
+    ones on either side of the choice: an output is the same sum over k whichever tile holds it."""
+    import torch
+    import cuplayground_amd as moe
+    cfg = ob.Cfg(S=S, H=H, I=I, E=E, k=k, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SIGMOID, drop=0)
+    g = torch.Generator(device="cuda").manual_seed(S)
+
+    def normal(*shape):
+        return (torch.randn(*shape, generator=g, device="cuda") * 0.02).bfloat16()
+
+    dev = {"x": normal(S, H) * 50, "gate_w": normal(E, H), "w_up": normal(E, I, H), "w_gate": normal(E, I, H), "w_down": normal(E, H, I)}
+    got = _forward(cfg, dev, FFN_TILED, tile)["out"]
+    assert np.isfinite(ob.to_f32(got, cfg.act_dtype)).all()
+    assert np.array_equal(got, _forward(cfg, dev, FFN_PERSISTENT, tile)["out"])
+
+
+def test_capped_layers_of_few_rows_keep_the_queue():
+    import cuplayground_amd as moe
+    for factor, queue in ((1.0, True), (2.0, False)):
+        cfg = ob.Cfg(S=400, H=2048, I=1408, E=64, k=6, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=1, capacity_factor=factor)
+        layer = moe.MoELayer(product_config(cfg))
+        assert (layer.ffn_mode == FFN_PERSISTENT) == queue
+        layer.close()

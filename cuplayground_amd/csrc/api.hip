@@ -375,7 +375,7 @@ int resolved_ffn_mode(const moe_handle* h) {
     // Two launches on row blocks and remainders (launch_ffn_split_16) against the queue.  128-row blocks: always faster where that tile is
     // chosen (figures beside the launch).  256-row blocks, queue / two launches, us: few rows an expert, where remainders are most of the
     // work: 64 experts of 2048 x 1408, 141 rows each 323 / 311, 188 rows 346 / 328; and many rounds of short tasks, where the queue's
-    // pops and written-through rows add up: 1536 rows 1707 / 1665, uneven and capped 728 / 720.  Between these the queue, which
+    // pops and written-through rows add up: 1536 rows 1707 / 1665 (not where tokens are dropped: capped and uneven 712 / 730).  Between these the queue, which
     // starts the down projection under the up projection's last round: 750 rows 913 / 907, 375 rows 541 / 559; 16 of 2048 x 2048, 512
     // rows 214 / 223; 12 of 1344 x 2752, 1000 rows 259 / 289; 8 of 4096 x 14336, 256 rows 894 / 989, 2048 rows 4447 / 4463 (4 rounds down).
     // (Options of the queue and its trace keep it.)  Layers that drop tokens at few rows per expert keep it too: 64 of 2048 x 1408, at most 29
@@ -383,7 +383,7 @@ int resolved_ffn_mode(const moe_handle* h) {
     if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && h->opt.queue_early != 1 && !h->task_trace) {
         if (d.plan.tile == 2 && !(h->cfg.drop_tokens && d.capacity <= kSplitCappedRows)) return MOE_FFN_TILED;
         const int64_t rounds = (d.A / d.plan.block_m) * std::min(d.plan.nnt0, d.plan.nnt1) / kSplitComputeUnits;
-        if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || rounds >= kSplitRounds)) return MOE_FFN_TILED;
+        if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || (rounds >= kSplitRounds && !h->cfg.drop_tokens))) return MOE_FFN_TILED;
     }
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }

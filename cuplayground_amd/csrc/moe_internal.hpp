@@ -79,8 +79,6 @@ struct CombineState {
 struct FfnArgs {
     const void* x;              // [S,H]
     const int32_t* token_indices;
-    const int32_t* expert_count;   // [E] rows kept of every expert, and where they begin among the packed ones
-    const int32_t* expert_offset;
     const void* w_up;           // [E,I,H]
     const void* w_gate;         // [E,I,H] or null
     const void* w_down;         // [E,H,I]
@@ -131,6 +129,10 @@ struct FfnArgs {
     float* sx;                  // [S, H / 128]
     uint8_t* hq;                // [A, I]
     float* sh;                  // [A, I / 128]
+    // (Last, so that what the kernels of small layers read lies as it did: the weight streamer on 20 rows of 16 experts of 2048 x 2048,
+    // SwiGLU, took 91.7 us with these in front of the weights and 88.9 without.)
+    const int32_t* expert_count;   // [E] rows kept of every expert, and where they begin among the packed ones
+    const int32_t* expert_offset;
 };
 constexpr int kMaxQueueWorkgroups = 4096;   // workgroups of a queue kernel that get a slot in wg_clock
 

@@ -89,6 +89,13 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _own(t, given):
+    """What a node keeps of `given`, a tensor of the caller's, of which `t` is the aligned form: 16-bit operands as a copy, so that
+    adding the layer's output onto its input in place, or a step of the router's weights, may come before the backward (as with gate
+    weights in torch, which reads them as fp32 copies; fp32 ones autograd keeps itself, and refuses them once they are changed)."""
+    return t.clone() if t.dtype != torch.float32 and t.data_ptr() == given.data_ptr() else t
+
+
 def _as_stored(layer, w):
     """Whether a data gradient [rows, K] . w[e] takes the weight w [E, K, N] as it is (else: a transposed copy)."""
     return isinstance(layer, api.MoELayer) and w.data_ptr() % 16 == 0 and layer.gemm_kn_supported(w.shape[2], w.shape[1]) == 2
@@ -189,18 +196,20 @@ class _RoutedExperts(torch.autograd.Function):
     benchmark table), 1302 -> 1172 us (SwiGLU), 720 -> 330 us for a few hundred tokens, where launches are the time."""
 
     @staticmethod
-    def forward(ctx, x, w_up, w_gate, w_down, gate_w, layer):
+    def forward(ctx, x, w_up, w_gate, w_down, gate_w, layer, grad_enabled):
+        given = x, gate_w
         x, gate_w, w_up, w_down = _aligned(x), _aligned(gate_w), w_up.contiguous(), w_down.contiguous()
         w_gate = None if w_gate is None else w_gate.contiguous()
         c = layer.cfg
-        need_router = ctx.needs_input_grad[0] or ctx.needs_input_grad[4]
+        need_x, need_gate_w = (grad_enabled and ctx.needs_input_grad[i] for i in (0, 4))
+        need_router = need_x or need_gate_w
         gate = layer.gate(x, gate_w, want_logits=need_router and c.gate_fn != api.GATE_SOFTMAX and bool(c.norm_topk_prob))
         idx, topk_w, logits = gate if len(gate) == 3 else (*gate, None)
         r = layer.route(idx)
         pair_row, count, offset = r["pair_row"], r["expert_count"], r["expert_offset"]
         rows, u, g, h, y = _expert_rows(x, w_up, w_gate, w_down, layer, r["token_indices"], count, offset)
         ctx.save_for_backward(*_kept(ctx.needs_input_grad[:4], rows, u, g, h, w_up, w_gate, w_down), y, topk_w, pair_row, count, offset,
-                              x if ctx.needs_input_grad[4] else None, gate_w if ctx.needs_input_grad[0] else None, idx, logits)
+                              _own(x, given[0]) if need_gate_w else None, _own(gate_w, given[1]) if need_x else None, idx, logits)
         ctx.layer = layer
         return api.combine(y, pair_row, topk_w)
 
@@ -217,7 +226,7 @@ class _RoutedExperts(torch.autograd.Function):
         da, db, dup, dgate, ddown = _expert_gradients(layer, needs, dy, kept, count, offset)
         dx = layer.dispatch_router_backward(da, db, pair_row, idx, router, gate_w) if needs[0] else None
         dgate_w = layer.gate_wgrad(x, router) if ctx.needs_input_grad[4] else None
-        return dx, dup, dgate, ddown, dgate_w, None
+        return dx, dup, dgate, ddown, dgate_w, None, None
 
 
 class MoE355Train(torch.nn.Module):
@@ -267,7 +276,7 @@ class MoE355Train(torch.nn.Module):
         c = self.cfg
         if self._routed(x):
             rows = x if x.shape[0] == c.tokens else x[:c.tokens]
-            return _RoutedExperts.apply(rows, self.w_up, self.w_gate, self.w_down, self.gate_w, self.layer)
+            return _RoutedExperts.apply(rows, self.w_up, self.w_gate, self.w_down, self.gate_w, self.layer, torch.is_grad_enabled())
         idx, r = self.route(x)
         count, offset = r["expert_count"], r["expert_offset"]
         # fp32 whatever gate_weights computed in: the combine reads fp32 (under autocast the logits, and with them a sigmoid's

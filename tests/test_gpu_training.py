@@ -280,3 +280,31 @@ def test_a_single_normalised_expert_keeps_its_torch_gate(moe, gate_fn):
         m(x).backward(torch.randn(97, 128, generator=g, device="cuda"))
         grads.append([x.grad] + [p.grad for _, p in m.named_parameters()])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("dtype", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("gate_fn,norm", [(0, 1), (1, 0)], ids=["softmax", "sigmoid"])
+def test_input_and_router_may_change_before_the_backward(moe, gate_fn, norm, dtype):
+    """The layer's output added onto its input in place, and the router's weights stepped, between forward and backward: the
+    gradients are those of the values that the forward read, to the bit."""
+    import torch
+    from cuplayground_amd import training
+    cfg = moe.MoEConfig(expert_top_k=2, hidden_act=1, hidden_size=128, intermediate_size=64, micro_batch=1, num_experts=5,
+                        sequence_len=131, torch_dtype=dtype, gate_fn=gate_fn, norm_topk_prob=norm, is_training=1)
+    grads = []
+    for change in (False, True):
+        m, g = training.MoE355Train(cfg, init_std=0.2, seed=2), torch.Generator(device="cuda").manual_seed(7)
+        assert m.layer.router_grad_bytes > 0
+        x = torch.randn(131, 128, generator=g, device="cuda").to(m.layer.act_dtype).requires_grad_(True)
+        dout = torch.randn(131, 128, generator=g, device="cuda").to(m.layer.act_dtype)
+        h = x * 1
+        y = m(h)
+        if change:
+            h += y
+            with torch.no_grad():
+                m.gate_w.mul_(0.5)
+        else:
+            h = h + y
+        h.backward(dout)
+        grads.append([x.grad] + [p.grad for _, p in m.named_parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

@@ -96,6 +96,11 @@ def _own(t, given):
     return t.clone() if t.dtype != torch.float32 and t.data_ptr() == given.data_ptr() else t
 
 
+def _unpacked(ctx):
+    """The saved tensors as the kernels take them: a saved-tensor hook may hand back views at any address."""
+    return [None if t is None else _aligned(t) for t in ctx.saved_tensors]
+
+
 def _as_stored(layer, w):
     """Whether a data gradient [rows, K] . w[e] takes the weight w [E, K, N] as it is (else: a transposed copy)."""
     return isinstance(layer, api.MoELayer) and w.data_ptr() % 16 == 0 and layer.gemm_kn_supported(w.shape[2], w.shape[1]) == 2
@@ -178,7 +183,7 @@ class _Experts(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        *kept, y, topk_w, pair_row, count, offset = ctx.saved_tensors
+        *kept, y, topk_w, pair_row, count, offset = _unpacked(ctx)
         layer, needs = ctx.layer, ctx.needs_input_grad[:4]
         dy, dtopk = layer.combine_backward(_aligned(dout), y, pair_row, topk_w, dy=torch.empty_like(y))
         da, db, dup, dgate, ddown = _expert_gradients(layer, needs, dy, kept, count, offset)
@@ -215,7 +220,7 @@ class _RoutedExperts(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        *kept, y, topk_w, pair_row, count, offset, x, gate_w, idx, logits = ctx.saved_tensors
+        *kept, y, topk_w, pair_row, count, offset, x, gate_w, idx, logits = _unpacked(ctx)
         layer, needs = ctx.layer, ctx.needs_input_grad[:4]
         dout, dy, router = _aligned(dout), torch.empty_like(y), None
         if needs[0] or ctx.needs_input_grad[4]:

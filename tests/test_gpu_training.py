@@ -308,3 +308,33 @@ def test_input_and_router_may_change_before_the_backward(moe, gate_fn, norm, dty
         h.backward(dout)
         grads.append([x.grad] + [p.grad for _, p in m.named_parameters()])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("act,dtype,gate_fn,norm,k", [(2, 2, 0, 1, 2), (1, 3, 1, 1, 3), (0, 2, 1, 0, 1), (2, 0, 0, 1, 2), (1, 2, 0, 0, 2)])
+def test_saved_tensors_may_come_back_at_any_address(moe, act, dtype, gate_fn, norm, k):
+    """Saved-tensor hooks that keep what a step saves as one odd element into a buffer of their own: the same gradients."""
+    import torch
+    from cuplayground_amd import training
+    cfg = moe.MoEConfig(expert_top_k=k, hidden_act=act, hidden_size=128, intermediate_size=192, micro_batch=1, num_experts=5,
+                        sequence_len=131, torch_dtype=dtype, gate_fn=gate_fn, norm_topk_prob=norm, is_training=1)
+    m, g = training.MoE355Train(cfg, init_std=0.2, seed=2), torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(131, 128, generator=g, device="cuda").to(m.layer.act_dtype).requires_grad_(True)
+    dout = torch.randn(131, 128, generator=g, device="cuda").to(m.layer.act_dtype)
+
+    def pack(t):
+        buf = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+        buf[1:] = t.detach().reshape(-1)
+        return buf[1:].view(t.shape)
+
+    grads = []
+    for hooked in (False, True):
+        x.grad = None
+        m.zero_grad(set_to_none=True)
+        if hooked:
+            with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+                out = m(x)
+        else:
+            out = m(x)
+        out.backward(dout)
+        grads.append([x.grad] + [p.grad for _, p in m.named_parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

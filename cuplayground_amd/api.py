@@ -580,11 +580,13 @@ class MoELayer:
         Rows of no expert are not written."""
         import torch
         K, N = w.shape[1], w.shape[2]
-        for name, t in (("a_rows", a_rows), ("w", w)):
-            _operand(name, t, self.act_dtype)
+        _operand("a_rows", a_rows, self.act_dtype, a_rows.shape[0] * K)
+        _operand("w", w, self.act_dtype, self.E * K * N)
         for name, t in (("u_rows", u_rows), ("g_rows", g_rows)):
             if t is not None:
                 _operand(name, t, self.act_dtype, a_rows.shape[0] * N)
+        for name, t in (("expert_count", expert_count), ("expert_offset", expert_offset)):
+            _operand(name, t, torch.int32, self.E)
         out = torch.empty(a_rows.shape[0], N, dtype=a_rows.dtype, device=a_rows.device)
         out1 = None if g_rows is None else torch.empty_like(out)
         _check(self.L.moe_expert_gemm_kn(self._h, _ptr(a_rows), _ptr(w), _ptr(u_rows), _ptr(g_rows), _ptr(expert_count),
@@ -666,7 +668,6 @@ class MoELayer:
                                            _ptr(dw), _stream()), "moe_combine_backward")
         return dy, dw
 
-
     # the router's share of a training step
     @property
     def router_grad_bytes(self) -> int:
@@ -674,13 +675,22 @@ class MoELayer:
         n = C.c_size_t(0)
         return n.value if self.L.moe_router_grad_bytes(self._h, C.byref(n)) == 0 else 0
 
+    def _router_operands(self, router_grad, **int_tables):
+        """The router's gradient buffer and the [S, k] tables that go with it."""
+        import torch
+        _operand("router_grad", router_grad, torch.uint8, self.router_grad_bytes)
+        for name, t in int_tables.items():
+            _operand(name, t, torch.int32, self.S * self.k)
+
     def combine_router_backward(self, dout, y_rows, pair_row, topk_w, topk_idx, logits, dy, router_grad):
+        import torch
         _operand("dout", dout, self.act_dtype, self.S * self.H)
         _operand("y_rows", y_rows, self.act_dtype)
-        for name, t, dt in (("pair_row", pair_row, _i32()), ("topk_idx", topk_idx, _i32()), ("topk_w", topk_w, _f32())):
-            _operand(name, t, dt, self.S * self.k)
+        _operand("dy", dy, self.act_dtype, y_rows.numel())
+        _operand("topk_w", topk_w, torch.float32, self.S * self.k)
         if logits is not None:
-            _operand("logits", logits, _f32(), self.S * self.E)
+            _operand("logits", logits, torch.float32, self.S * self.E)
+        self._router_operands(router_grad, pair_row=pair_row, topk_idx=topk_idx)
         _check(self.L.moe_combine_router_backward(self._h, _ptr(dout), _ptr(y_rows), _ptr(pair_row), _ptr(topk_w), _ptr(topk_idx),
                                                   _ptr(logits), _ptr(dy), _ptr(router_grad), _stream()), "moe_combine_router_backward")
 
@@ -690,6 +700,7 @@ class MoELayer:
         if db_rows is not None:
             _operand("db_rows", db_rows, self.act_dtype, da_rows.numel())
         _operand("gate_w", gate_w, self.act_dtype, self.E * self.H)
+        self._router_operands(router_grad, pair_row=pair_row, topk_idx=topk_idx)
         dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
         _check(self.L.moe_dispatch_router_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(topk_idx),
                                                    _ptr(router_grad), _ptr(gate_w), _ptr(dx), _stream()), "moe_dispatch_router_backward")
@@ -698,20 +709,11 @@ class MoELayer:
     def gate_wgrad(self, x, router_grad):
         import torch
         _operand("x", x, self.act_dtype, self.S * self.H)
+        self._router_operands(router_grad)
         sc = self.backward_scratch()
         dw = torch.empty(self.E, self.H, dtype=self.act_dtype, device=x.device)
         _check(self.L.moe_gate_wgrad(self._h, _ptr(x), _ptr(router_grad), _ptr(dw), _ptr(sc), sc.numel(), _stream()), "moe_gate_wgrad")
         return dw
-
-
-def _i32():
-    import torch
-    return torch.int32
-
-
-def _f32():
-    import torch
-    return torch.float32
 
 
 def transpose(src, out=None):

@@ -72,6 +72,40 @@ def test_row_passes_refuse_operands_of_another_type():
             call()
 
 
+def test_router_passes_and_stored_weight_products_refuse_operands_they_would_read_past(monkeypatch):
+    """Tables, the gradient buffer, results and weights of too few elements or another type: refused before the first launch."""
+    layer = api.MoELayer.__new__(api.MoELayer)
+    layer.cfg, layer.S, layer.k, layer.H, layer.E, layer.act_dtype, layer._h = _cfg(), 8, 2, 64, 4, torch.bfloat16, None
+    monkeypatch.setattr(api.MoELayer, "router_grad_bytes", 768)
+    bf16 = dict(dtype=torch.bfloat16)
+    x, rows, gate_w = torch.zeros(8, 64, **bf16), torch.zeros(16, 64, **bf16), torch.zeros(4, 64, **bf16)
+    pairs, w, router = torch.zeros(8, 2, dtype=torch.int32), torch.ones(8, 2), torch.zeros(768, dtype=torch.uint8)
+    wkn, count = torch.zeros(4, 64, 64, **bf16), torch.zeros(4, dtype=torch.int32)
+
+    def combine(**kw):
+        a = dict(dout=x, y_rows=rows, pair_row=pairs, topk_w=w, topk_idx=pairs, logits=None, dy=rows, router_grad=router)
+        return lambda: layer.combine_router_backward(**dict(a, **kw))
+
+    def dispatch(**kw):
+        a = dict(da_rows=rows, db_rows=None, pair_row=pairs, topk_idx=pairs, router_grad=router, gate_w=gate_w)
+        return lambda: layer.dispatch_router_backward(**dict(a, **kw))
+
+    def product(**kw):
+        a = dict(a_rows=rows, w=wkn, expert_count=count, expert_offset=count)
+        return lambda: layer.expert_gemm_kn(**dict(a, **kw))
+
+    for call in (combine(dy=rows.float()), combine(router_grad=w), combine(topk_idx=pairs.long()), dispatch(pair_row=pairs.long()),
+                 dispatch(topk_idx=pairs.long()), dispatch(router_grad=w), lambda: layer.gate_wgrad(x, w),
+                 product(expert_count=count.long()), product(expert_offset=count.float())):
+        with pytest.raises(TypeError):
+            call()
+    for call in (combine(dy=rows[:15]), combine(router_grad=router[1:]), combine(topk_idx=pairs[1:]), dispatch(pair_row=pairs[1:]),
+                 dispatch(topk_idx=pairs[1:]), dispatch(router_grad=router[1:]), lambda: layer.gate_wgrad(x, router[1:]),
+                 product(w=wkn[:3]), product(a_rows=rows[:, :32]), product(expert_count=count[:3]), product(expert_offset=count[:3])):
+        with pytest.raises(ValueError):
+            call()
+
+
 class _RowsLayer:
     """The passes of the expert node as plain torch expressions (one expert, one rank): enough to run the node on the CPU."""
     fused_act_backward = False

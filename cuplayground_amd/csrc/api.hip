@@ -21,7 +21,7 @@ int bf16_block_n0(int tile, int swiglu);
 int bf16_block_n1(int tile);
 int f32_block_m();
 int f32_block_n();
-hipError_t launch_ffn_tiled_bf16(const FfnArgs&, int tile, int max_mtiles, int nnt0, int nnt1, hipStream_t, bool f16);
+hipError_t launch_ffn_tiled_bf16(const FfnArgs&, const ExpertRows&, int tile, int max_mtiles, int nnt0, int nnt1, hipStream_t, bool f16);
 hipError_t launch_ffn_persistent_bf16(const FfnArgs&, int tile, int blocks, bool early, hipStream_t, bool f16);
 int ffn_persistent_occupancy_bf16(int tile);
 hipError_t launch_gemm_dense_bf16(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int,
@@ -818,7 +818,6 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
     FfnArgs fa{};        // every field starts null / zero: a member nobody sets must not reach a kernel as stack garbage
     fa.x = x;
     fa.token_indices = ra.token_indices;
-    fa.expert_count = ra.expert_count; fa.expert_offset = ra.expert_offset;
     fa.w_up = w->w_up; fa.w_gate = w->w_gate; fa.w_down = w->w_down;
     fa.b_up = w->b_up; fa.b_gate = w->b_gate; fa.b_down = w->b_down;
     fa.s_up = w->s_up; fa.s_gate = w->s_gate; fa.s_down = w->s_down;
@@ -885,7 +884,7 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
     } else if (mode == MOE_FFN_PERSISTENT) {
         e = launch_ffn_persistent(fa, kdt, d.plan, h->arch.persistent_blocks, h->opt.queue_early == 1, st);
     } else {
-        e = launch_ffn_tiled(fa, kdt, d.plan, d.max_mtiles, st);
+        e = launch_ffn_tiled(fa, ExpertRows{ra.expert_count, ra.expert_offset}, kdt, d.plan, d.max_mtiles, st);
     }
     if (e != hipSuccess) return hip_fail(h, e);
     if ((e = mark(3)) != hipSuccess) return hip_fail(h, e);
@@ -1332,11 +1331,11 @@ int moe_combine(const void* y_rows, const int32_t* pair_row, const float* topk_w
 
 namespace moe355 {
 
-hipError_t launch_ffn_tiled(const FfnArgs& a, int dtype, const FfnPlan& p, int max_mtiles, hipStream_t st) {
+hipError_t launch_ffn_tiled(const FfnArgs& a, const ExpertRows& rows, int dtype, const FfnPlan& p, int max_mtiles, hipStream_t st) {
     if (dtype == MOE_DTYPE_F32 || dtype == MOE_DTYPE_TF32)
         return p.tile == 1 ? launch_ffn_f32_tile(a, max_mtiles, p.nnt0, p.nnt1, 0, st)
                            : launch_ffn_tiled_f32(a, p.tile == kF32StreamTile, max_mtiles, p.nnt0, p.nnt1, st);
-    return launch_ffn_tiled_bf16(a, p.tile, max_mtiles, p.nnt0, p.nnt1, st, dtype == MOE_DTYPE_FP16);
+    return launch_ffn_tiled_bf16(a, rows, p.tile, max_mtiles, p.nnt0, p.nnt1, st, dtype == MOE_DTYPE_FP16);
 }
 
 hipError_t launch_ffn_persistent(const FfnArgs& a, int dtype, const FfnPlan& p, int blocks, bool early, hipStream_t st) {

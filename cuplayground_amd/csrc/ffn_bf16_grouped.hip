@@ -625,15 +625,15 @@ hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const
 //   94 rows 278 / 295 / 264; 8 of 4096 x 14336, 128 rows 679 / 672 / 655; 16 of 2048 x 2048, 128 rows 130 / 112 / 110
 //   256-row blocks (queue / this): see resolved_ffn_mode
 template <class P>
-static hipError_t launch_ffn_split(const FfnArgs& a, hipStream_t st) {
+static hipError_t launch_ffn_split(const FfnArgs& a, const ExpertRows& rows, hipStream_t st) {
     const int64_t A = (int64_t)a.S * a.k;
     GroupedArgs g{(const uint16_t*)a.x, (const uint16_t*)a.w_up, (const uint16_t*)a.b_up, nullptr, nullptr, (uint16_t*)a.h, nullptr,
-                  a.expert_count, a.expert_offset, a.E, a.I, a.H, a.act, a.x_bytes, a.token_indices, (const uint16_t*)a.w_gate, (const uint16_t*)a.b_gate};
+                  rows.count, rows.offset, a.E, a.I, a.H, a.act, a.x_bytes, a.token_indices, (const uint16_t*)a.w_gate, (const uint16_t*)a.b_gate};
     const hipError_t e = a.act == MOE_ACT_SWIGLU ? launch_grouped<P, kSwiglu>(g, A, st)
                          : a.act == MOE_ACT_GELU ? launch_grouped<P, kGelu>(g, A, st) : launch_grouped<P, kSums>(g, A, st);
     if (e != hipSuccess) return e;
     g = GroupedArgs{(const uint16_t*)a.h, (const uint16_t*)a.w_down, (const uint16_t*)a.b_down, nullptr, nullptr, (uint16_t*)a.y, nullptr,
-                    a.expert_count, a.expert_offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr};
+                    rows.count, rows.offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr};
     return launch_grouped<P, kSums>(g, A, st);
 }
 // Rounds of the compute units that a launch of `full` 256-row tiles and, behind them, `left` tiles of 128 rows takes, in units of the
@@ -688,10 +688,10 @@ bool ffn_split_16_keeps_table(const FfnArgs& a) {
     return n.left >= 0.75 * a.E && n.full <= 1.25 * a.E && n.full * up >= 0.9 * 256 && rounds(n.table * up) <= 2 &&
            rounds(n.table * down) <= std::ceil(split_rounds(n.full * down, n.left * down) - 0.5);
 }
-hipError_t launch_ffn_split_16(const FfnArgs& a, int block_rows, bool f16, hipStream_t st) {
+hipError_t launch_ffn_split_16(const FfnArgs& a, const ExpertRows& rows, int block_rows, bool f16, hipStream_t st) {
     if (block_rows == 128 && split_on_256(a)) block_rows = 256;
-    if (block_rows == 128) return f16 ? launch_ffn_split<RowSplit<true, 128>>(a, st) : launch_ffn_split<RowSplit<false, 128>>(a, st);
-    return f16 ? launch_ffn_split<RowSplit<true, 256>>(a, st) : launch_ffn_split<RowSplit<false, 256>>(a, st);
+    if (block_rows == 128) return f16 ? launch_ffn_split<RowSplit<true, 128>>(a, rows, st) : launch_ffn_split<RowSplit<false, 128>>(a, rows, st);
+    return f16 ? launch_ffn_split<RowSplit<true, 256>>(a, rows, st) : launch_ffn_split<RowSplit<false, 256>>(a, rows, st);
 }
 
 template <class T>

@@ -129,10 +129,11 @@ struct FfnArgs {
     float* sx;                  // [S, H / 128]
     uint8_t* hq;                // [A, I]
     float* sh;                  // [A, I / 128]
-    // (Last, so that what the kernels of small layers read lies as it did: the weight streamer on 20 rows of 16 experts of 2048 x 2048,
-    // SwiGLU, took 91.7 us with these in front of the weights and 88.9 without.)
-    const int32_t* expert_count;   // [E] rows kept of every expert, and where they begin among the packed ones
-    const int32_t* expert_offset;
+};
+// The packed rows by expert: what the launches that find their row blocks themselves read instead of FfnArgs's tables.
+struct ExpertRows {
+    const int32_t* count;       // [E] rows kept of every expert
+    const int32_t* offset;      // [E] where they begin
 };
 constexpr int kMaxQueueWorkgroups = 4096;   // workgroups of a queue kernel that get a slot in wg_clock
 
@@ -190,12 +191,11 @@ hipError_t launch_combine(const void* y_rows, const int32_t* pair_row, const flo
 // FFN stage.  block_m / block_n are the tile sizes the routing stage must be told about.
 // FfnPlan::tile of a 16-bit layer from this value on: the weight streamer (ffn_stream16.hip) in its form tile - kStream16Tile.
 constexpr int kStream16Tile = 4;
-struct FfnArgs;
 int stream16_block_m(int form);
 int stream16_block_n(int form);
 int ffn_persistent_occupancy_stream16(int form);
 bool ffn_split_16_keeps_table(const FfnArgs& a);
-hipError_t launch_ffn_split_16(const FfnArgs& a, int block_rows, bool f16, hipStream_t st);   // ffn_bf16_grouped.hip
+hipError_t launch_ffn_split_16(const FfnArgs& a, const ExpertRows& rows, int block_rows, bool f16, hipStream_t st);   // ffn_bf16_grouped.hip
 hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st);
 struct FfnPlan {
     int kernel_dtype;   // the dtype whose kernels run: the layer's, or bf16 for an e4m3 layer whose weights are widened
@@ -214,7 +214,7 @@ hipError_t launch_widen_block128(const void* q, const float* scales, void* out, 
 // bf16 rows -> e4m3 codes + one fp32 scale per (row, 128 columns); limit: null, or a device word with the rows that matter
 hipError_t launch_quant_rows128(const void* x, void* q, float* scales, int64_t rows, int64_t K, const int32_t* limit,
                                 hipStream_t st);
-hipError_t launch_ffn_tiled(const FfnArgs& a, int dtype, const FfnPlan& p, int max_mtiles, hipStream_t st);
+hipError_t launch_ffn_tiled(const FfnArgs& a, const ExpertRows& rows, int dtype, const FfnPlan& p, int max_mtiles, hipStream_t st);
 hipError_t launch_ffn_persistent(const FfnArgs& a, int dtype, const FfnPlan& p, int blocks, bool early, hipStream_t st);
 int ffn_persistent_blocks(int dtype, int tile, int compute_units);
 

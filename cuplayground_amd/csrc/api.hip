@@ -242,6 +242,8 @@ struct moe_handle {
     int queue_groups;      // task queues of the FFN stage: one per XCD, or 1
     int queue_lag;         // experts of up-projection work between an expert's two projections in the queue
     int row_chunk;         // task order inside a queue segment (FfnArgs::row_chunk)
+    bool table_order;      // queue_groups or row_chunk differ from what AUTO gives: the launches keep the order they describe
+    bool queue_options;    // ... or another option of the queue does: AUTO keeps the queue
     int64_t* task_trace;   // the caller's device buffer for per-task records of the queue kernel, or null
     int task_trace_cap;    // records it holds
     int combine_mode;      // 0: a launch of its own, 1: arrival counters inside the FFN kernels, 2: tasks of the FFN queue
@@ -378,9 +380,9 @@ int resolved_ffn_mode(const moe_handle* h) {
     // pops and written-through rows add up: 1536 rows 1707 / 1665 (not where tokens are dropped: capped and uneven 712 / 730).  Between these the queue, which
     // starts the down projection under the up projection's last round: 750 rows 913 / 907, 375 rows 541 / 559; 16 of 2048 x 2048, 512
     // rows 214 / 223; 12 of 1344 x 2752, 1000 rows 259 / 289; 8 of 4096 x 14336, 256 rows 894 / 989, 2048 rows 4447 / 4463 (4 rounds down).
-    // (Options of the queue and its trace keep it.)  Layers that drop tokens at few rows per expert keep it too: 64 of 2048 x 1408, at most 29
+    // (Options of the queue and its trace keep it: queue_options and those below.)  Layers that drop tokens at few rows per expert keep it too: 64 of 2048 x 1408, at most 29
     // rows 234 / 243, 38 rows 237 / 247, 57 rows 248 / 248, 94 rows 249 / 240 (28 rows, none dropped: 284 / 267).
-    if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && h->opt.queue_early != 1 && !h->task_trace) {
+    if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && !h->queue_options && !h->task_trace) {
         if (d.plan.tile == 2 && !(h->cfg.drop_tokens && d.capacity <= kSplitCappedRows)) return MOE_FFN_TILED;
         const int64_t rounds = (d.A / d.plan.block_m) * std::min(d.plan.nnt0, d.plan.nnt1) / kSplitComputeUnits;
         if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || (rounds >= kSplitRounds && !h->cfg.drop_tokens))) return MOE_FFN_TILED;
@@ -533,13 +535,15 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
     snprintf(h->arch.name, sizeof h->arch.name, "%s", prop.gcnArchName);
     const int kdt = d.plan.kernel_dtype;
     const bool tile16 = kdt == MOE_DTYPE_BF16 || kdt == MOE_DTYPE_FP16;
-    int per_cu = ffn_persistent_blocks(kdt, d.plan.tile, 1);
+    const int auto_per_cu = ffn_persistent_blocks(kdt, d.plan.tile, 1);
+    int per_cu = auto_per_cu;
     if (opt->blocks_per_cu != MOE_OPT_AUTO) per_cu = opt->blocks_per_cu;    // resident workgroups per CU
     h->arch.persistent_blocks = prop.multiProcessorCount * per_cu;
     // One task queue per XCD for the MFMA-bound bf16 tiles, whose operand tiles are then shared in that XCD's L2;
     // so does the e4m3 tile GEMM; the fp32 kernels (the matrix-core tile measured 5 % faster on one queue than on eight)
     // and the weight streamers (no operand is shared between their workgroups) keep a single queue.
     h->queue_groups = ((tile16 && d.plan.tile < kStream16Tile) || (kdt == MOE_DTYPE_FP8_E4M3_B128 && d.plan.tile)) ? h->arch.xcds : 1;
+    const int auto_groups = h->queue_groups > h->arch.persistent_blocks ? 1 : h->queue_groups;
     if (opt->queue_groups != MOE_OPT_AUTO && opt->queue_groups <= h->arch.xcds) h->queue_groups = opt->queue_groups;   // never more queues than XCDs
     if (h->queue_groups > h->arch.persistent_blocks) h->queue_groups = 1;   // every queue needs a home workgroup
     // The e4m3 tile GEMM holds 64 workgroups per XCD on 128 x 128 tiles whose token rows (bf16) take twice the L2 space
@@ -547,14 +551,20 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
     // Mixtral shape with e4m3 weights: 6.57 ms against 6.96 with all row blocks of the expert at a time; 1: 6.62,
     // 4: 6.76, 8: 6.89).  The bf16 tiles are indifferent (within 1 %) and keep the plain order.
     h->row_chunk = (kdt == MOE_DTYPE_FP8_E4M3_B128 && d.plan.tile) ? 2 : 0;
+    const int auto_chunk = h->row_chunk;
     if (opt->row_chunk != MOE_OPT_AUTO) h->row_chunk = opt->row_chunk;
+    // (compared with the values AUTO gives, so that a handle made from moe_get_options runs as the one they came from)
+    h->table_order = h->queue_groups != auto_groups || h->row_chunk != auto_chunk;
+    h->queue_options = h->table_order || per_cu != auto_per_cu || (opt->queue_early == 1 && tile16 && d.plan.tile == 1) || opt->tail_round == 0;
     {   // phase-0 tasks an average expert contributes; enough experts of them to cover four tasks per workgroup
         const int64_t avg_mt = d.A / ((int64_t)d.E * d.plan.block_m) > 0 ? d.A / ((int64_t)d.E * d.plan.block_m) : 1;
         const int64_t per_expert = avg_mt * d.plan.nnt0;
         int64_t lag = (4 * (int64_t)h->arch.persistent_blocks + per_expert - 1) / per_expert;
         if (lag < 1) lag = 1;
+        const int64_t auto_lag = std::min<int64_t>(lag, d.E);
         if (opt->queue_lag != MOE_OPT_AUTO) lag = opt->queue_lag;
         if (lag > d.E) lag = d.E;
+        h->queue_options |= lag != auto_lag;
         h->queue_lag = (int)lag;
     }
     // Combine: a launch of its own unless asked otherwise.  Inside the FFN kernels by arrival counters it is bit-identical
@@ -884,7 +894,7 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
     } else if (mode == MOE_FFN_PERSISTENT) {
         e = launch_ffn_persistent(fa, kdt, d.plan, h->arch.persistent_blocks, h->opt.queue_early == 1, st);
     } else {
-        e = launch_ffn_tiled(fa, ExpertRows{ra.expert_count, ra.expert_offset}, kdt, d.plan, d.max_mtiles, st);
+        e = launch_ffn_tiled(fa, h->table_order ? ExpertRows{} : ExpertRows{ra.expert_count, ra.expert_offset}, kdt, d.plan, d.max_mtiles, st);
     }
     if (e != hipSuccess) return hip_fail(h, e);
     if ((e = mark(3)) != hipSuccess) return hip_fail(h, e);

@@ -449,8 +449,8 @@ template <class P> struct RunOccupancy {
 hipError_t launch_ffn_tiled_bf16(const FfnArgs& a, const ExpertRows& rows, int tile, int max_mtiles, int nnt0, int nnt1,
                                  hipStream_t st, bool f16) {
     if (tile >= kStream16Tile) return launch_ffn_stream16(a, tile - kStream16Tile, f16, max_mtiles, nnt0, nnt1, 0, st);
-    // (the combine inside the FFN kernels and partial sums: options, which the kernels on the row block table take)
-    if (tile >= 1 && tile <= 3 && !a.arrive && !a.split_cnt && !(tile == 1 && ffn_split_16_keeps_table(a))) return launch_ffn_split_16(a, rows, bf16_block_m(tile), f16, st);
+    // (the combine inside the FFN kernels, partial sums and orders of the table: options, which the kernels on the row block table take)
+    if (tile >= 1 && tile <= 3 && rows.count && !a.arrive && !a.split_cnt && !(tile == 1 && ffn_split_16_keeps_table(a))) return launch_ffn_split_16(a, rows, bf16_block_m(tile), f16, st);
     return for_plan<RunTiled>(tile, f16, a, max_mtiles, nnt0, nnt1, st);
 }
 

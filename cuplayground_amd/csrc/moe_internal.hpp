@@ -130,7 +130,8 @@ struct FfnArgs {
     uint8_t* hq;                // [A, I]
     float* sh;                  // [A, I / 128]
 };
-// The packed rows by expert: what the launches that find their row blocks themselves read instead of FfnArgs's tables.
+// The packed rows by expert: what the launches that find their row blocks themselves read instead of FfnArgs's tables (null: the
+// launches keep to the tables).
 struct ExpertRows {
     const int32_t* count;       // [E] rows kept of every expert
     const int32_t* offset;      // [E] where they begin

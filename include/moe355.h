@@ -308,8 +308,10 @@ int moe_get_stage_samples(moe_handle* h, int stage, float* ms, int32_t capacity,
 
 /* How evenly the task queue of the last moe_forward kept its workgroups busy (task-queue FFN only; MOE_ERR_UNSUPPORTED
  * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers, for single experts and,
- * in 16-bit layers, for up to about 192 rows per expert or many rounds of short tasks: moe_get_ffn_mode tells, moe_set_ffn_mode asks
- * for the queue).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
+ * in 16-bit layers, for up to about 192 rows per expert (more than 48 where tokens are dropped) and for many rounds of short tasks
+ * (where none are dropped): moe_get_ffn_mode tells, moe_set_ffn_mode asks for the queue, and a task trace or an option of the queue
+ * -- queue_groups, queue_lag, queue_early, row_chunk, blocks_per_cu, tail_round, combine, tail_split -- with another value than AUTO
+ * gives keeps it).  Every workgroup stamps the device's constant-rate clock when it enters and when it leaves
  * the queue kernel: span_us = first entry to last exit, mean_active_us = mean of (exit - entry), mean_tail_idle_us =
  * mean of (last exit - own exit), i.e. the time a workgroup had nothing left to pop while others still worked.
  * Synchronises `stream`.  No counterpart in the reference, whose scheduler keeps no statistics. */

@@ -52,7 +52,7 @@ def test_same_bits_as_the_queue(name, tile):
 
 @pytest.mark.parametrize("rows, experts, tokens, queue", [(64, 16, 512, False), (192, 64, 2048, False), (200, 64, 2134, True)])
 def test_mode_that_is_chosen(rows, experts, tokens, queue):
-    """Few rows per expert: two launches, also where there are many tasks; options and reports of the queue keep it."""
+    """Few rows per expert: two launches, also where there are many tasks; the queue's trace keeps it."""
     import cuplayground_amd as moe
     cfg = ob.Cfg(S=tokens, H=2048, I=1408, E=experts, k=6 if experts == 64 else 2, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=0)
     layer = moe.MoELayer(product_config(cfg))
@@ -62,6 +62,23 @@ def test_mode_that_is_chosen(rows, experts, tokens, queue):
         assert layer.ffn_mode == FFN_PERSISTENT
         layer.disable_task_trace()
     layer.close()
+
+
+@pytest.mark.parametrize("option", ["queue_groups", "queue_lag", "row_chunk", "blocks_per_cu", "tail_round", "queue_early"])
+@pytest.mark.parametrize("rows, tile", [(94, 2), (160, 1)])
+def test_options_of_the_queue_keep_it(rows, tile, option):
+    """Any option of the queue that differs from what AUTO gives; a handle made from another one's options runs as that one does."""
+    import cuplayground_amd as moe
+    cfg = ob.Cfg(S=rows * 64 // 6, H=2048, I=1408, E=64, k=6, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=0)
+    layer = moe.MoELayer(product_config(cfg))
+    assert layer.options["tile16"] == tile and layer.ffn_mode == FFN_TILED
+    same = moe.MoELayer(product_config(cfg), options=layer.options)
+    assert same.ffn_mode == FFN_TILED
+    value = {"queue_groups": 2, "queue_lag": 1, "row_chunk": 3, "blocks_per_cu": layer.options["blocks_per_cu"] + 1, "tail_round": 0, "queue_early": 1}
+    kept = moe.MoELayer(product_config(cfg), options={option: value[option]})
+    assert (kept.ffn_mode == FFN_PERSISTENT) == (option != "queue_early" or tile == 1)      # (an option of the 256 x 256 tile)
+    for l in (layer, same, kept):
+        l.close()
 
 
 @pytest.mark.parametrize("S,H,I,E,k,tile", [(900, 1984, 3008, 20, 3, 2), (1300, 1984, 3008, 20, 3, 2), (2300, 2048, 2048, 16, 2, 1), (1000, 320, 448, 5, 2, 2)])

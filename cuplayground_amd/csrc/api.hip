@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "moe_internal.hpp"
+#include "two_launches.hpp"
 
 namespace moe355 {
 
@@ -347,7 +348,6 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
-constexpr int kSplitComputeUnits = 256, kSplitRowsPerExpert = 192, kSplitRounds = 11, kSplitCappedRows = 48;
 int resolved_ffn_mode(const moe_handle* h) {
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
     if (h->d.plan.mfma8) return MOE_FFN_TILED;
@@ -374,19 +374,10 @@ int resolved_ffn_mode(const moe_handle* h) {
     // (the fp32 one: 1.26 against 1.02 ms, 16 tokens on 8 experts of 4096 x 14336; 2.89 against 2.21 for 128 tokens)
     if ((d.plan.kernel_dtype == MOE_DTYPE_F32 || d.plan.kernel_dtype == MOE_DTYPE_TF32) && d.plan.tile == kF32StreamTile) return MOE_FFN_TILED;
     if ((f32_tile || tile16) && d.E == 1) return MOE_FFN_TILED;
-    // Two launches on row blocks and remainders (launch_ffn_split_16) against the queue.  128-row blocks: always faster where that tile is
-    // chosen (figures beside the launch).  256-row blocks, queue / two launches, us: few rows an expert, where remainders are most of the
-    // work: 64 experts of 2048 x 1408, 141 rows each 323 / 311, 188 rows 346 / 328; and many rounds of short tasks, where the queue's
-    // pops and written-through rows add up: 1536 rows 1707 / 1665 (not where tokens are dropped: capped and uneven 712 / 730).  Between these the queue, which
-    // starts the down projection under the up projection's last round: 750 rows 913 / 907, 375 rows 541 / 559; 16 of 2048 x 2048, 512
-    // rows 214 / 223; 12 of 1344 x 2752, 1000 rows 259 / 289; 8 of 4096 x 14336, 256 rows 894 / 989, 2048 rows 4447 / 4463 (4 rounds down).
-    // (Options of the queue and its trace keep it: queue_options and those below.)  Layers that drop tokens at few rows per expert keep it too: 64 of 2048 x 1408, at most 29
-    // rows 234 / 243, 38 rows 237 / 247, 57 rows 248 / 248, 94 rows 249 / 240 (28 rows, none dropped: 284 / 267).
-    if (tile16 && h->combine_mode == 0 && d.plan.ksplit == 1 && !h->queue_options && !h->task_trace) {
-        if (d.plan.tile == 2 && !(h->cfg.drop_tokens && d.capacity <= kSplitCappedRows)) return MOE_FFN_TILED;
-        const int64_t rounds = (d.A / d.plan.block_m) * std::min(d.plan.nnt0, d.plan.nnt1) / kSplitComputeUnits;
-        if (d.plan.tile == 1 && (d.A <= (int64_t)d.E * kSplitRowsPerExpert || (rounds >= kSplitRounds && !h->cfg.drop_tokens))) return MOE_FFN_TILED;
-    }
+    // Two launches on row blocks and remainders against the queue: two_launches.hpp.  (Options of the queue and its trace keep it.)
+    if (tile16 && (d.plan.tile == 1 || d.plan.tile == 2) && h->combine_mode == 0 && d.plan.ksplit == 1 && !h->queue_options && !h->task_trace &&
+        two_launches_auto(TwoLaunchShape{d.A, d.E, d.H, d.I, h->cfg.hidden_act == MOE_ACT_SWIGLU}, d.plan.tile == 1, h->cfg.drop_tokens != 0, d.capacity))
+        return MOE_FFN_TILED;
     return est_tasks >= (f32_tile ? 4 : 2) * (int64_t)h->arch.persistent_blocks ? MOE_FFN_PERSISTENT : MOE_FFN_TILED;
 }
 

@@ -1,6 +1,5 @@
 // Products on the 16-bit tiles (ffn_bf16_tile.hpp): dense operands, packed rows by expert (a layer's two launches too), weight gradients.
 #include <algorithm>
-#include <cmath>
 
 #include "ffn_bf16_tile.hpp"
 
@@ -40,7 +39,8 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dense_kernel(const uint16_t* 
 }
 
 // The tiles a grouped product runs on.  256: blocks of 256 rows, and of 128 where an expert has no more than that many rows left
-// (the smaller tile takes 0.65 of the larger one's time; the other half of the larger one would multiply zeros).
+// (the smaller tile takes two thirds of the larger one's time at 16 slabs, three quarters at 32: tile_task_us; the other half of the
+// larger one would multiply zeros).
 template <bool F16_, int BIG_>
 struct RowSplit {
     static constexpr bool F16 = F16_, HAND = true;
@@ -623,7 +623,7 @@ hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const
 // Whole layers, us, the queue / two launches of it in the order of the row block table / this:
 //   128-row blocks: 12 experts of 1344 x 2752, GELU, 150 rows each 122 / 108 / 88, 250 rows 131 / 118 / 115; 64 of 2048 x 1408, SwiGLU,
 //   94 rows 278 / 295 / 264; 8 of 4096 x 14336, 128 rows 679 / 672 / 655; 16 of 2048 x 2048, 128 rows 130 / 112 / 110
-//   256-row blocks (queue / this): see resolved_ffn_mode
+//   256-row blocks, and which layers run so: two_launches.hpp
 template <class P>
 static hipError_t launch_ffn_split(const FfnArgs& a, const ExpertRows& rows, hipStream_t st) {
     const int64_t A = (int64_t)a.S * a.k;
@@ -636,60 +636,10 @@ static hipError_t launch_ffn_split(const FfnArgs& a, const ExpertRows& rows, hip
                     rows.count, rows.offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr};
     return launch_grouped<P, kSums>(g, A, st);
 }
-// Rounds of the compute units that a launch of `full` 256-row tiles and, behind them, `left` tiles of 128 rows takes, in units of the
-// former; a 128-row tile takes three quarters of it (it fetches three quarters of the bytes).
-static double split_rounds(double full, double left) {
-    constexpr double kUnits = 256, kLeft = 0.75;
-    const double whole = std::floor(full / kUnits), busy = full - whole * kUnits, idle = kUnits - busy;
-    double at_idle = whole, at_busy = whole + 1, end = busy > 0 ? whole + 1 : whole;
-    while (left > 0) {
-        const bool first = busy <= 0 || at_idle <= at_busy;
-        double& at = first ? at_idle : at_busy;
-        left -= first ? idle : busy;
-        at += kLeft;
-        end = std::max(end, at);
-    }
-    return end;
-}
-// Of `rows` packed rows per expert on average, an expert has about rows +- sqrt(rows): tiles per column tile of all experts.
-struct SplitBlocks {
-    double full = 0, left = 0, small = 0, table = 0;      // 256-row blocks and remainders; or 128-row blocks; or 256-row blocks alone
-    SplitBlocks(int64_t A, int E) {
-        const double rows = (double)A / E;
-        for (int i = -1; i <= 1; ++i) {
-            const double n = std::max(1.0, std::round(rows + i * std::sqrt(rows))), share = E * (i ? 0.25 : 0.5), f = std::floor((n + 127) / 256);
-            full += share * f;
-            left += n > 256 * f ? share : 0;
-            small += share * std::ceil(n / 128);
-            table += share * std::ceil(n / 256);
-        }
-    }
-};
-// Layers planned on 128-row blocks whose two launches take 256-row blocks and remainders after all: where many experts have just more than
-// 128 rows, second blocks of a few rows cost whole rounds.  Whole layers, us, 128-row blocks / these (the queue): 20 experts of 1984 x 3008,
-// SwiGLU, 135 rows each 296 / 217 (270); 18 of them, 150 rows 290 / 214 (264).  The estimate has to promise a tenth: 9 of 2048 x 3008, 289 rows
-// 187 / 177 is left, and so is where it would lose: 10 of 1024 x 2048, 330 rows 91 / 108; 20 of 1024 x 1024, 315 rows 81 / 92.
-static bool split_on_256(const FfnArgs& a) {
-    const SplitBlocks n((int64_t)a.S * a.k, a.E);
-    const double up = (a.I * (a.act == MOE_ACT_SWIGLU ? 2 : 1) + 255) / 256, down = (a.H + 255) / 256;
-    const double large = split_rounds(n.full * up, n.left * up) * a.H + split_rounds(n.full * down, n.left * down) * a.I;
-    const double small = split_rounds(0, n.small * up) * a.H + split_rounds(0, n.small * down) * a.I;
-    return large <= 0.9 * small;
-}
-// Layers whose full row blocks are a round of their own in the up projection, so that the remainders' round reads all weights from memory
-// again, and that take as many rounds on 256-row blocks alone: the order of the row block table, where the blocks of an expert meet
-// the same weight tile, is faster.  16 experts of 2048 x 2048, SwiGLU, us, table / remainders behind: 262 rows each 187 / 190, 287
-// rows 190 / 207, 325 rows 205 / 212; but 237 rows 202 / 181 (hardly a remainder), GELU (one round) 325 rows 155 / 144; 20 of
-// 2048 x 3072, ReLU, 290 rows (fewer rounds in the down projection) 311 / 274.  Above the rows and rounds of resolved_ffn_mode only.
-bool ffn_split_16_keeps_table(const FfnArgs& a) {
-    const SplitBlocks n((int64_t)a.S * a.k, a.E);
-    const double up = (a.I * (a.act == MOE_ACT_SWIGLU ? 2 : 1) + 255) / 256, down = (a.H + 255) / 256;
-    auto rounds = [](double tiles) { return std::ceil(tiles / 256); };
-    return n.left >= 0.75 * a.E && n.full <= 1.25 * a.E && n.full * up >= 0.9 * 256 && rounds(n.table * up) <= 2 &&
-           rounds(n.table * down) <= std::ceil(split_rounds(n.full * down, n.left * down) - 0.5);
-}
+static TwoLaunchShape two_launch_shape(const FfnArgs& a) { return TwoLaunchShape{(int64_t)a.S * a.k, a.E, a.H, a.I, a.act == MOE_ACT_SWIGLU}; }
+bool ffn_split_16_keeps_table(const FfnArgs& a) { return two_launches_keep_table(two_launch_shape(a)); }
 hipError_t launch_ffn_split_16(const FfnArgs& a, const ExpertRows& rows, int block_rows, bool f16, hipStream_t st) {
-    if (block_rows == 128 && split_on_256(a)) block_rows = 256;
+    if (block_rows == 128 && two_launches_on_256(two_launch_shape(a))) block_rows = 256;
     if (block_rows == 128) return f16 ? launch_ffn_split<RowSplit<true, 128>>(a, rows, st) : launch_ffn_split<RowSplit<false, 128>>(a, rows, st);
     return f16 ? launch_ffn_split<RowSplit<true, 256>>(a, rows, st) : launch_ffn_split<RowSplit<false, 256>>(a, rows, st);
 }

@@ -26,6 +26,7 @@
 
 #include "ffn_common.hpp"
 #include "act_deriv.hpp"
+#include "two_launches.hpp"
 
 namespace moe355 {
 namespace {
@@ -983,8 +984,7 @@ static bool hand_weights_ok(int64_t N, int64_t K) { return (N + 256) * K * 2 < k
 // The larger tile reads its operands half as often; the smaller one pads less behind an expert's last row and spreads few
 // rows over more compute units.  The estimate behind the choice, per projection: row blocks an expert is expected to have
 // (rows / height and a half, one if the expert's rows hardly ever reach the height) x column tiles, in rounds over the
-// compute units (at least one, and half a round of tail), x the time of a task: 1.3 us a slab + 10 us for 256 x 256,
-// 1.1 us + 3 us for 128 x 256 (cold weights; fill of the first slabs, epilogue and queue overhead in the constant).
+// compute units (at least one, and half a round of tail), x the time of a task (tile_task_us).
 // Measured, whole layer, 256 x 256 / 128 x 256 / the 128 x 128 tile of the general loop (better of queue and launches):
 //   12 experts of 1344 x 2752, GELU: 150 rows each 127 / 112 / 115 us, 444 176 / 168 / 199, 1000 269 / 293 / 350
 //   12 experts of 704 x 1152, SwiGLU, 296 rows 107 / 81 / 87;  5 of 1856 x 2112, 200 rows 108 / 78 / 87
@@ -997,8 +997,7 @@ static double projection_cost(bool large, int64_t pairs, int experts, int column
     const double rows = (double)pairs / experts, height = large ? 256 : 128;
     const double blocks = experts * (rows <= 0.75 * height ? 1.0 : rows / height + 0.5);
     const double rounds = blocks * column_tiles / 256;
-    const double slabs = (K + kBK - 1) / kBK;
-    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * (large ? 1.3 * slabs + 10.0 : 1.1 * slabs + 3.0);
+    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * tile_task_us(large, K);
 }
 static int columns256(int N) { return (N + 255) / 256; }
 

@@ -1,0 +1,104 @@
+// Which 16-bit layers on the hand-ordered tiles run as two launches (ffn_bf16_grouped.hip: launch_ffn_split_16) instead of on the task
+// queue, and on which row blocks.  Host arithmetic on the layer's shape only, so that a host program can test it.  "Queue / two" below
+// are whole layers, us, bf16, tokens from one seed, both modes of one handle's shape in turn on one card; "random layers" are 300 with
+// 4 to 64 experts, 60 to 500 rows each and dimensions of 512 to 4096 in steps of 64.
+#pragma once
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+
+namespace moe355 {
+
+// Time of one task of a grouped product, us, from its contraction's length: 256 x 256 (large) or 128 x 256 tile; cold weights; the fill of
+// the first slabs, epilogue and launch or queue overhead in the constant.
+inline double tile_task_us(bool large, int K) {
+    const double slabs = (K + 63) / 64;
+    return large ? 1.3 * slabs + 10.0 : 1.1 * slabs + 3.0;
+}
+
+struct TwoLaunchShape {
+    int64_t pairs;               // packed rows at most: tokens x experts per token
+    int experts, H, I;
+    bool swiglu;
+    int columns_up() const { return (I * (swiglu ? 2 : 1) + 255) / 256; }
+    int columns_down() const { return (H + 255) / 256; }
+};
+
+constexpr int kTaskUnits = 256;  // compute units: one task each at a time
+
+// AUTO on 128-row blocks (large = false): always, unless tokens are dropped and an expert takes at most kSplitCappedRows.
+//   Random layers: two launches are faster at 176 of 179, by 8 % in the mean.  The others: 32 of 2944 x 2688, GELU, 71 rows 8 % slower, 64
+//   of 2432 x 1664, SwiGLU, 101 rows 5 %, 9 of 2048 x 2112, SwiGLU, 388 rows (on 128-row blocks; it runs on 256-row ones).
+//   Dropping layers, 64 of 2048 x 1408: at most 29 rows 234 / 243, 38 rows 237 / 247, 57 rows 248 / 248, 94 rows 249 / 240 (28 rows, none
+//   dropped: 284 / 267).
+// On 256-row blocks the queue starts the down projection under the up projection's last round, which two launches have to make up for:
+//   few rows an expert, where remainders are most of the work and a remainder's task is shorter here: 64 of 2048 x 1408, 137 to 188 rows
+//   3 to 6 % faster, 197 rows of 32 of 3456 x 3264 6 % slower; at most 192 rows, random layers: faster at 25 of 26 (64 of 3072 x 1600, 125
+//   rows, 3 % slower);
+//   many rounds of short tasks, where the queue's pops and written-through rows add up: 64 of 2048 x 1408, 1434 rows 1606 / 1574, 1792
+//   rows 1985 / 1935.
+//   8 rounds of 64 of 2048 x 1408: 1167 / 1172.  Where tokens are dropped it depends on the routing, which is not known here (64 of
+//   2048 x 1408, 1434 rows at most, even 1587 / 1542, like 1 / rank^1.1 704 / 714): the queue.
+constexpr int kSplitRowsPerExpert = 192, kSplitRounds = 11, kSplitCappedRows = 48;
+inline bool two_launches_auto(const TwoLaunchShape& s, bool large, bool drops, int64_t capacity) {
+    if (!large) return !(drops && capacity <= kSplitCappedRows);
+    if (s.pairs <= (int64_t)s.experts * kSplitRowsPerExpert) return true;
+    const int64_t rounds = s.pairs / 256 * std::min(s.columns_up(), s.columns_down()) / kTaskUnits;
+    return rounds >= kSplitRounds && !drops;
+}
+
+// Time of a launch of `full` tasks of `large` each and, behind them, `left` tasks of `small`.
+inline double split_time(double full, double left, double large, double small) {
+    const double whole = std::floor(full / kTaskUnits), busy = full - whole * kTaskUnits, idle = kTaskUnits - busy;
+    double at_idle = whole * large, at_busy = (whole + 1) * large, end = busy > 0 ? at_busy : at_idle;
+    while (left > 0) {
+        const bool first = busy <= 0 || at_idle <= at_busy;
+        double& at = first ? at_idle : at_busy;
+        left -= first ? idle : busy;
+        at += small;
+        end = std::max(end, at);
+    }
+    return end;
+}
+// Of `pairs / experts` rows per expert on average, an expert has about that +- its root: tiles per column tile of all experts.
+struct SplitBlocks {
+    double full = 0, left = 0, small = 0, table = 0;      // 256-row blocks and remainders; or 128-row blocks; or 256-row blocks alone
+    SplitBlocks(int64_t pairs, int experts) {
+        const double rows = (double)pairs / experts;
+        for (int i = -1; i <= 1; ++i) {
+            const double n = std::max(1.0, std::round(rows + i * std::sqrt(rows))), share = experts * (i ? 0.25 : 0.5), f = std::floor((n + 127) / 256);
+            full += share * f;
+            left += n > 256 * f ? share : 0;
+            small += share * std::ceil(n / 128);
+            table += share * std::ceil(n / 256);
+        }
+    }
+};
+// Layers planned on 128-row blocks whose two launches take 256-row blocks and remainders after all: where a second block of an expert, or a
+// round of them, would be opened for a few rows.  128-row blocks / these: 18 of 1856 x 2944, SwiGLU, 157 rows 277 / 205; 17 of 2048 x 2048,
+// ReLU, 156 rows 187 / 138; 24 of 1536 x 1600, ReLU, 148 rows 131 / 109; 9 of 2048 x 2112, SwiGLU, 388 rows 14 % faster.
+// The estimate, in rounds with a 128-row tile at three quarters, has to promise a tenth.
+inline bool two_launches_on_256(const TwoLaunchShape& s) {
+    const SplitBlocks n(s.pairs, s.experts);
+    const double up = s.columns_up(), down = s.columns_down();
+    const double large = split_time(n.full * up, n.left * up, 1.0, 0.75) * s.H + split_time(n.full * down, n.left * down, 1.0, 0.75) * s.I;
+    const double small = split_time(0, n.small * up, 1.0, 0.75) * s.H + split_time(0, n.small * down, 1.0, 0.75) * s.I;
+    return large <= 0.9 * small;
+}
+// Layers on 256-row blocks whose full row blocks are a round of their own in the up projection, so that the remainders' round reads all
+// weights from memory again, and that take as many rounds on 256-row blocks alone: the order of the row block table, where the blocks
+// of an expert meet the same weight tile, is kept.  Table / remainders behind: 16 of 2048 x 2048, SwiGLU, 260 rows 187 / 193, 278 rows
+// 186 / 218, 300 rows 188 / 233, 325 rows 189 / 235; 32 of 1472 x 2048, GELU, 273 rows 225 / 231; but 237 rows 202 / 181 (hardly a
+// remainder), GELU (one round) 325 rows 155 / 144; 20 of 2048 x 3072, ReLU, 290 rows (fewer rounds in the down projection) 311 / 274.
+// The line is drawn from the first shape; where the up projection's full blocks fall short of the round by a few, it is not the faster
+// side always (the table is what such layers ran on before there was the other): 22 of 1216 x 2752, GELU, 309 rows 272 / 184; 11 of
+// 1856 x 2816, SwiGLU, 322 rows 220 / 197; 10 of 1920 x 2944, SwiGLU, 373 rows 188 / 198.
+inline bool two_launches_keep_table(const TwoLaunchShape& s) {
+    const SplitBlocks n(s.pairs, s.experts);
+    const double up = s.columns_up(), down = s.columns_down();
+    auto rounds = [](double tiles) { return std::ceil(tiles / kTaskUnits); };
+    return n.left >= 0.75 * s.experts && n.full <= 1.25 * s.experts && n.full * up >= 0.9 * kTaskUnits && rounds(n.table * up) <= 2 &&
+           rounds(n.table * down) <= std::ceil(split_time(n.full * down, n.left * down, 1.0, 0.75) - 0.5);      // (in rounds: a remainder is 0.74 at 32 slabs)
+}
+
+}  // namespace moe355

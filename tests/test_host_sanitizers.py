@@ -47,3 +47,20 @@ def test_queue_order_keeps_every_dependency_under_asan_and_ubsan(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=300)
     assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
     assert " 0 failed checks" in r.stdout and "with a rounded tail" in r.stdout and "with partial sums decoded id by id" in r.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_two_launch_rules_under_asan_and_ubsan(tmp_path):
+    """csrc/two_launches.hpp decides which 16-bit layers run as two launches and on which row blocks, where every choice gives
+    the same bits: its answers on both sides of each line, at layers that were measured both ways, and at the ends of the range."""
+    exe = str(tmp_path / "two_launches")
+    cmd = ["g++", "-std=c++17", "-O1", "-g", "-Wall", "-Werror", "-fno-omit-frame-pointer", "-fsanitize=address,undefined",
+           "-fno-sanitize-recover=all", "-static-libasan", "-I", os.path.join(ROOT, "cuplayground_amd", "csrc"), "-o", exe,
+           os.path.join(ROOT, "tests", "host", "two_launches.cpp")]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", UBSAN_OPTIONS="print_stacktrace=1")
+    env.pop("LD_PRELOAD", None)
+    r = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=120)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
+    assert " 0 failed checks" in r.stdout

@@ -35,16 +35,25 @@ constexpr int kTaskUnits = 256;  // compute units: one task each at a time
 //   few rows an expert, where remainders are most of the work and a remainder's task is shorter here: 64 of 2048 x 1408, 137 to 188 rows
 //   3 to 6 % faster, 197 rows of 32 of 3456 x 3264 6 % slower; at most 192 rows, random layers: faster at 25 of 26 (64 of 3072 x 1600, 125
 //   rows, 3 % slower);
-//   many rounds of short tasks, where the queue's pops and written-through rows add up: 64 of 2048 x 1408, 1434 rows 1606 / 1574, 1792
-//   rows 1985 / 1935.
+//   many rounds of tasks whose rows stay in the caches: the queue's pops and written-through rows add up, but each XCD works on an expert
+//   of its own, so that the rows of eight experts are read at a time, where the queue's workgroups share one expert's.  Bytes of eight
+//   experts' rows, 11 to 16 rounds, none dropped, queue / two:
+//     up to 78 MB: 64 of 2048 x 1408, 1434 rows 1606 / 1574, 1792 rows 1985 / 1935; 64 of 4096 x 1536, 956 rows 2239 / 2208; 64 of
+//     1536 x 1536, 1911 rows 1404 / 1363; 128 of 1024 x 1024, 1434 rows 1298 / 1264; routed like 1 / rank^0.5 and 1 / rank^1.1 0.5 % slower to
+//     16 % faster;
+//     94 to 161 MB: 32 of 2048 x 2048, 2867 rows 1646 / 1623 but like 1 / rank^1.1 1679 / 1724; 32 of 2048 x 2816, 3584 rows 3467 / 3426, 3477 / 3642;
+//     134 to 1600 MB: 16 of 3072 x 3072, 2731 rows 1542 / 1567; 8 of 4096 x 4096, 5734 rows 3607 / 3824; 8 of 4096 x 14336, 5734 rows
+//     12213 / 12609, 7168 rows 15209 / 16273.
 //   8 rounds of 64 of 2048 x 1408: 1167 / 1172.  Where tokens are dropped it depends on the routing, which is not known here (64 of
 //   2048 x 1408, 1434 rows at most, even 1587 / 1542, like 1 / rank^1.1 704 / 714): the queue.
 constexpr int kSplitRowsPerExpert = 192, kSplitRounds = 11, kSplitCappedRows = 48;
+constexpr int64_t kSplitRowBytes = 80 << 20;
 inline bool two_launches_auto(const TwoLaunchShape& s, bool large, bool drops, int64_t capacity) {
     if (!large) return !(drops && capacity <= kSplitCappedRows);
     if (s.pairs <= (int64_t)s.experts * kSplitRowsPerExpert) return true;
     const int64_t rounds = s.pairs / 256 * std::min(s.columns_up(), s.columns_down()) / kTaskUnits;
-    return rounds >= kSplitRounds && !drops;
+    const int64_t row_bytes = 8 * (s.pairs / s.experts) * std::max(s.H, s.I) * 2;
+    return rounds >= kSplitRounds && !drops && row_bytes <= kSplitRowBytes;
 }
 
 // Time of a launch of `full` tasks of `large` each and, behind them, `left` tasks of `small`.
@@ -90,9 +99,9 @@ inline bool two_launches_on_256(const TwoLaunchShape& s) {
 // of an expert meet the same weight tile, is kept.  Table / remainders behind: 16 of 2048 x 2048, SwiGLU, 260 rows 187 / 193, 278 rows
 // 186 / 218, 300 rows 188 / 233, 325 rows 189 / 235; 32 of 1472 x 2048, GELU, 273 rows 225 / 231; but 237 rows 202 / 181 (hardly a
 // remainder), GELU (one round) 325 rows 155 / 144; 20 of 2048 x 3072, ReLU, 290 rows (fewer rounds in the down projection) 311 / 274.
-// The line is drawn from the first shape; where the up projection's full blocks fall short of the round by a few, it is not the faster
-// side always (the table is what such layers ran on before there was the other): 22 of 1216 x 2752, GELU, 309 rows 272 / 184; 11 of
-// 1856 x 2816, SwiGLU, 322 rows 220 / 197; 10 of 1920 x 2944, SwiGLU, 373 rows 188 / 198.
+// The line is drawn from the first shape; where the up projection's full blocks fall a few short of the round, it is not always the faster
+// side (the table is what such layers ran on before there was the other): 10 of 1920 x 2944, SwiGLU, 373 rows 188 / 198, but 22 of
+// 1216 x 2752, GELU, 309 rows 272 / 184 and 11 of 1856 x 2816, SwiGLU, 322 rows 220 / 197.
 inline bool two_launches_keep_table(const TwoLaunchShape& s) {
     const SplitBlocks n(s.pairs, s.experts);
     const double up = s.columns_up(), down = s.columns_down();

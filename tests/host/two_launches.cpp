@@ -34,6 +34,10 @@ int main() {
     AUTO(false, true, true, 1434, 64, 2048, 1408, 1434, true);
     AUTO(true, true, false, 1 << 20, 64, 4096, 1536, 956, true);
     AUTO(true, true, false, 1 << 20, 128, 1024, 1024, 1434, false);
+    // ... and rows of eight experts that stay in the caches
+    AUTO(false, true, false, 1 << 20, 32, 2048, 2048, 2867, false);
+    AUTO(false, true, false, 1 << 20, 8, 4096, 14336, 5734, true);
+    AUTO(false, true, false, 1 << 20, 16, 3072, 3072, 3823, false);
     // 256-row blocks under a plan of 128-row ones
     ON256(true, 18, 1856, 2944, 157, true);
     ON256(true, 17, 2048, 2048, 156, false);

@@ -99,6 +99,16 @@ def test_same_bits_whatever_blocks_the_rounds_choose(S, H, I, E, k, tile):
     assert np.array_equal(got, _forward(cfg, dev, FFN_PERSISTENT, tile)["out"])
 
 
+@pytest.mark.parametrize("E,k,H,I,rows,drop,queue", [(64, 6, 2048, 1408, 1434, 0, False), (64, 6, 2048, 1408, 1434, 1, True), (64, 6, 2048, 1408, 1024, 0, True),
+                                                     (8, 2, 4096, 14336, 5734, 0, True), (32, 4, 2048, 2816, 2867, 0, True)])
+def test_many_rounds_leave_the_queue_where_their_rows_stay_in_the_caches(E, k, H, I, rows, drop, queue):
+    import cuplayground_amd as moe
+    cfg = ob.Cfg(S=rows * E // k, H=H, I=I, E=E, k=k, act=ob.ACT_SWIGLU, dtype=ob.BF16, gate_fn=ob.GATE_SOFTMAX, drop=drop)
+    layer = moe.MoELayer(product_config(cfg), allocate_workspace=False)
+    assert (layer.ffn_mode == FFN_PERSISTENT) == queue
+    layer.close()
+
+
 def test_capped_layers_of_few_rows_keep_the_queue():
     import cuplayground_amd as moe
     for factor, queue in ((1.0, True), (2.0, False)):

@@ -34,7 +34,7 @@ constexpr int kTaskUnits = 256;  // compute units: one task each at a time
 // On 256-row blocks the queue starts the down projection under the up projection's last round, which two launches have to make up for:
 //   few rows an expert, where remainders are most of the work and a remainder's task is shorter here: 64 of 2048 x 1408, 137 to 188 rows
 //   3 to 6 % faster, 197 rows of 32 of 3456 x 3264 6 % slower; at most 192 rows, random layers: faster at 25 of 26 (64 of 3072 x 1600, 125
-//   rows, 3 % slower);
+//   rows, 3 % slower; another, 32 of 3392 x 2560, ReLU, 166 rows, 8 %: 1.25 and 1.75 rounds, which two launches make two and two);
 //   many rounds of tasks whose rows stay in the caches: the queue's pops and written-through rows add up, but each XCD works on an expert
 //   of its own, so that the rows of eight experts are read at a time, where the queue's workgroups share one expert's.  Bytes of eight
 //   experts' rows, 11 to 16 rounds, none dropped, queue / two:
@@ -69,6 +69,7 @@ inline double split_time(double full, double left, double large, double small) {
     }
     return end;
 }
+inline double split_us(double full, double left, int K) { return split_time(full, left, tile_task_us(true, K), tile_task_us(false, K)); }
 // Of `pairs / experts` rows per expert on average, an expert has about that +- its root: tiles per column tile of all experts.
 struct SplitBlocks {
     double full = 0, left = 0, small = 0, table = 0;      // 256-row blocks and remainders; or 128-row blocks; or 256-row blocks alone
@@ -85,13 +86,15 @@ struct SplitBlocks {
 };
 // Layers planned on 128-row blocks whose two launches take 256-row blocks and remainders after all: where a second block of an expert, or a
 // round of them, would be opened for a few rows.  128-row blocks / these: 18 of 1856 x 2944, SwiGLU, 157 rows 277 / 205; 17 of 2048 x 2048,
-// ReLU, 156 rows 187 / 138; 24 of 1536 x 1600, ReLU, 148 rows 131 / 109; 9 of 2048 x 2112, SwiGLU, 388 rows 14 % faster.
-// The estimate, in rounds with a 128-row tile at three quarters, has to promise a tenth.
+// ReLU, 156 rows 187 / 138; 24 of 1536 x 1600, ReLU, 148 rows 131 / 109; 64 of 960 x 896, GELU, 212 rows 13 % faster.  The estimate has to
+// promise a tenth: of 219 layers planned on 128-row blocks it moves 29, 23 of them 6 to 26 % faster, 6 of them 1 to 10 % slower; of another
+// 110 that it moves 89 are up to 28 % faster, 21 are 1 to 13 % slower (9 of 1216 x 2688, ReLU, 649 rows).  With a 128-row tile at three
+// quarters of a round whatever the contraction's length it moves 43 of the 219, 19 of them up to 24 % slower (23 of 768 x 704, 143 rows 64 / 80).
 inline bool two_launches_on_256(const TwoLaunchShape& s) {
     const SplitBlocks n(s.pairs, s.experts);
     const double up = s.columns_up(), down = s.columns_down();
-    const double large = split_time(n.full * up, n.left * up, 1.0, 0.75) * s.H + split_time(n.full * down, n.left * down, 1.0, 0.75) * s.I;
-    const double small = split_time(0, n.small * up, 1.0, 0.75) * s.H + split_time(0, n.small * down, 1.0, 0.75) * s.I;
+    const double large = split_us(n.full * up, n.left * up, s.H) + split_us(n.full * down, n.left * down, s.I);
+    const double small = split_us(0, n.small * up, s.H) + split_us(0, n.small * down, s.I);
     return large <= 0.9 * small;
 }
 // Layers on 256-row blocks whose full row blocks are a round of their own in the up projection, so that the remainders' round reads all

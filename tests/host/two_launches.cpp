@@ -44,6 +44,12 @@ int main() {
     ON256(true, 9, 2048, 2112, 388, true);
     ON256(false, 64, 2048, 1408, 94, true);
     ON256(false, 16, 2048, 2048, 128, false);
+    ON256(true, 64, 960, 896, 212, false);
+    // ... the promised tenth, with a task's time from the length of its contraction
+    ON256(false, 10, 1536, 1344, 297, true);
+    ON256(false, 13, 1408, 1472, 212, true);
+    ON256(false, 23, 768, 704, 143, true);
+    ON256(false, 11, 1216, 768, 452, true);
     // the order of the row block table
     TABLE(true, 16, 2048, 2048, 262, true);
     TABLE(true, 16, 2048, 2048, 325, true);

@@ -14,6 +14,7 @@
 
 #include "moe_internal.hpp"
 #include "act_deriv.hpp"
+#include "product_choice.hpp"
 
 namespace moe355 {
 
@@ -24,9 +25,6 @@ hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void*
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
                            int64_t ld, bool f16, hipStream_t st);
 
-bool wgrad_rows_16_better(int64_t A, int E, int N, int K);
-bool grouped_kn_16_ok(int64_t A, int N, int K);
-bool grouped_kn_16_better(int64_t A, int E, int N, int K);
 hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
                                      const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st);
@@ -48,7 +46,6 @@ hipError_t launch_wgrad_f32_tile(const void* dyT, const void* aT, void* dw, cons
 
 namespace {
 
-constexpr int kWindowAlign = 128;   // columns an expert's window of a transposed operand is padded to
 
 // One workgroup: row blocks of `block_m` rows per expert (for the grouped GEMM) and the padded window offsets (for the
 // weight gradient).  Either table may be null.
@@ -605,7 +602,6 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 }  // namespace
 
-int64_t wgrad_ld(int64_t A, int E) { return (A + (int64_t)kWindowAlign * E + 127) / 128 * 128; }
 
 size_t backward_scratch_bytes(int64_t A, int E, int H, int I, int elem_bytes) {
     const size_t tables = align256(sizeof(int32_t)) + align256((size_t)(A / 64 + E + 1) * sizeof(MTile)) + align256((size_t)(E + 1) * 4);
@@ -645,7 +641,8 @@ ScratchTables scratch_tables(void* scratch, int64_t A, int E) {
 }
 }  // namespace
 
-// out_rows[r,:] = act(a_rows[r,:] . w[e(r)]^T + bias[e(r)]); scratch holds the row-block table.
+// out_rows[r,:] = act(a_rows[r,:] . w[e(r)]^T + bias[e(r)]); scratch: the row-block table of an fp32 product (16-bit ones
+// find their row blocks themselves).
 // dtype: the storage type of every operand (MOE_DTYPE_F32, _BF16 or _FP16).
 hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bias, const int32_t* count,
                               const int32_t* offset, int64_t A, int E, int N, int K, int act, int dtype,
@@ -703,22 +700,23 @@ hipError_t launch_expert_gemm_dact(const void* dy_rows, const void* w, const voi
 // out_rows[r,:] = a_rows[r,:] . w[e(r)] with w [E, K, N] as the other direction stores it, and with u_rows the derivative behind it
 // (launch_expert_gemm_dact): no transposed copy of the weight.  16-bit layers.
 int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
-    if (dtype == MOE_DTYPE_F32 || !grouped_kn_16_ok(A, N, K)) return 0;
-    return opt.grouped_tile == MOE_OPT_AUTO && grouped_kn_16_better(A, E, N, K) ? 2 : 1;
+    if (dtype == MOE_DTYPE_F32 || !stored_operands_ok(A, N, K)) return 0;
+    return opt.grouped_tile == MOE_OPT_AUTO && grouped_kn_as_stored(A, E, N, K) ? 2 : 1;
 }
 hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
                                  const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows, void* out1_rows,
                                  hipStream_t st) {
-    if (dtype == MOE_DTYPE_F32 || !grouped_kn_16_ok(A, N, K)) return hipErrorNotSupported;
+    if (dtype == MOE_DTYPE_F32 || !stored_operands_ok(A, N, K)) return hipErrorNotSupported;
     return launch_grouped_gemm_kn_16(a_rows, w, u_rows, g_rows, out_rows, out1_rows, count, offset, A, E, N, K, hidden_act, dtype == MOE_DTYPE_FP16, st);
 }
 
-// dw[e] [N,K] = dy_e^T . a_e, from the rows as they are or from transposed copies: scratch holds the window offsets and those.
+// dw[e] [N,K] = dy_e^T . a_e, from the rows as they are (product_choice.hpp; not where option grouped_tile asks for a tile) or from
+// transposed copies: scratch holds the window offsets and those.
 hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const int32_t* count, const int32_t* offset,
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st) {
     const bool aligned = ((uintptr_t)dy_rows | (uintptr_t)a_rows | (uintptr_t)dw) % 16 == 0;
-    if (dtype != MOE_DTYPE_F32 && aligned && wgrad_rows_16_better(A, E, N, K))
+    if (dtype != MOE_DTYPE_F32 && aligned && opt.grouped_tile == MOE_OPT_AUTO && wgrad_as_stored(A, E, N, K))
         return launch_wgrad_rows_16(dy_rows, a_rows, dw, count, offset, E, N, K, dtype == MOE_DTYPE_FP16, st);
     const ScratchTables t = scratch_tables(scratch, A, E);
     const int64_t ld = wgrad_ld(A, E);

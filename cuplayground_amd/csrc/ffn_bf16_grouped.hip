@@ -658,41 +658,10 @@ static hipError_t launch_wgrad(const void* dyT, const void* aT, void* dw, const 
 
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
                            int64_t ld, bool f16, hipStream_t st) {
-    const bool large = N >= 1024 && K >= 1024 && hand_weights_ok(N, ld) && hand_weights_ok(K, ld);
-    if (large) return f16 ? launch_wgrad<Tile256H>(dyT, aT, dw, poff, E, N, K, ld, st)
-                          : launch_wgrad<Tile256>(dyT, aT, dw, poff, E, N, K, ld, st);
+    if (wgrad_hand_ok(N, K, ld))
+        return f16 ? launch_wgrad<Tile256H>(dyT, aT, dw, poff, E, N, K, ld, st) : launch_wgrad<Tile256>(dyT, aT, dw, poff, E, N, K, ld, st);
     return f16 ? launch_wgrad<Tile128H>(dyT, aT, dw, poff, E, N, K, ld, st)
                : launch_wgrad<Tile128>(dyT, aT, dw, poff, E, N, K, ld, st);
-}
-
-// The 128 x 128 tiles that turn operands round, against the larger hand-ordered tile behind transposes.  An estimate of either, us;
-// constants and checks are measurements of whole calls (transposes and launches included, bf16, one card):
-//   hand-ordered: 1.3 us a slab of 64 and 8 us a task, rounds of 256 tasks and half a one; transposes at 4.5 TB/s read and written;
-//   these: 1.25 us a slab and round of 512 tasks (two on a compute unit share its time), 5 us a round.
-static double prod_us(double tiles, double slabs) {
-    const double rounds = tiles / 512;
-    return (rounds < 1.0 ? 1.0 : rounds) * (1.25 * slabs + 5.0);
-}
-static double hand_us(double tiles, double slabs, double transposed_bytes) {
-    const double rounds = tiles / 256;
-    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * (1.3 * slabs + 8.0) + 2.0 * transposed_bytes / 4.5e6 + 8.0;
-}
-static bool prod_operands_ok(int64_t rows, int N, int K) { return (rows + 128) * std::max(N, K) * 2 < kBufferLimit && (int64_t)(N + 128) * K * 2 < kBufferLimit && (int64_t)(K + 128) * N * 2 < kBufferLimit; }
-//   weight gradient, hand-ordered / these: 16 experts of 2048 x 2048, 512 rows each 120 / 111; 750 rows of 1408 x 2048 125 / 108; 136 of
-//   1280 x 1408 47 / 26; 19 of 1024 x 2560 49 / 21; 4 of 2048 x 2560, 4096 rows 225 / 212; 64 of 1408 x 2048, 1536 rows 903 / 761;
-//   16 of 2048 x 2560, 1024 rows 238 / 240; 8 of 4096 x 2048, 2048 rows 304 / 339; 8 of 4096 x 14336, 512 rows 664 / 790, 2048 rows 1680 / 2410
-bool wgrad_rows_16_better(int64_t A, int E, int N, int K) {
-    if (!prod_operands_ok(A, N, K)) return false;
-    const double rows = (double)A / std::max(E, 1);
-    return prod_us((double)E * ((N + 127) / 128) * ((K + 127) / 128), rows / 64 + 0.5) <
-           hand_us((double)E * columns256(N) * columns256(K), rows / 64 + 1.0, 2.0 * A * (N + K));
-}
-bool grouped_kn_16_ok(int64_t A, int N, int K) { return prod_operands_ok(A, N, K); }
-bool grouped_kn_16_better(int64_t A, int E, int N, int K) {
-    if (!prod_operands_ok(A, N, K)) return false;
-    const double rows = (double)A / std::max(E, 1);
-    const double blocks = E * (rows <= 96 ? 1.0 : rows / 128 + 0.5), big = E * (rows <= 192 ? 1.0 : rows / 256 + 0.25);
-    return prod_us(blocks * ((N + 127) / 128), K / 64.0) < hand_us(big * columns256(N), K / 64.0, 2.0 * E * N * K);
 }
 
 template <class T>

@@ -26,6 +26,7 @@
 
 #include "ffn_common.hpp"
 #include "act_deriv.hpp"
+#include "product_choice.hpp"
 #include "two_launches.hpp"
 
 namespace moe355 {
@@ -973,12 +974,6 @@ hipError_t allow_lds(K kernel, int bytes) {
                                bytes);
 }
 
-// The hand-ordered slab loop needs 32-bit buffer offsets: operands below 4 GiB (`pairs` bounds the token count), and for
-// the weights also the columns behind the last one that a ragged tile reaches.  Dimensions are multiples of 64
-// (moe_config_validate).
-constexpr int64_t kBufferLimit = (int64_t)1 << 32;
-static bool hand_weights_ok(int64_t N, int64_t K) { return (N + 256) * K * 2 < kBufferLimit; }
-
 // Which hand-ordered tile a grouped product runs on: the 256 x 256 one or the 128 x 256 one.
 //
 // The larger tile reads its operands half as often; the smaller one pads less behind an expert's last row and spreads few
@@ -999,7 +994,6 @@ static double projection_cost(bool large, int64_t pairs, int experts, int column
     const double rounds = blocks * column_tiles / 256;
     return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * tile_task_us(large, K);
 }
-static int columns256(int N) { return (N + 255) / 256; }
 
 }  // namespace
 }  // namespace moe355

@@ -1,0 +1,54 @@
+// Whether a 16-bit training product takes operands as they are stored (the 128 x 128 tiles of ffn_bf16_grouped.hip that turn them round on
+// the way) or transposed copies of them and the larger tiles.  Either way gives the same bits.  Host arithmetic only, so that a host
+// program can test it.  Estimates of either, us; constants and checks are measurements of whole calls (transposes and launches included,
+// bf16, one card):
+//   hand-ordered 256 x 256 tile: 1.3 us a slab of 64 and 8 us a task, rounds of 256 tasks and half a one; transposes at 4.5 TB/s read and
+//   written;  as stored: 1.25 us a slab and round of 512 tasks (two on a compute unit share its time), 5 us a round.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace moe355 {
+
+// The hand-ordered slab loop needs 32-bit buffer offsets: operands below 4 GiB, and for the weights also the columns behind the last one
+// that a ragged tile reaches.  Dimensions are multiples of 64 (moe_config_validate).
+constexpr int64_t kBufferLimit = (int64_t)1 << 32;
+inline bool hand_weights_ok(int64_t N, int64_t K) { return (N + 256) * K * 2 < kBufferLimit; }
+inline int columns256(int N) { return (N + 255) / 256; }
+
+// Transposed operands of a weight gradient: an expert's window of columns is padded to kWindowAlign, rows are wgrad_ld long.
+constexpr int kWindowAlign = 128;
+inline int64_t wgrad_ld(int64_t A, int E) { return (A + (int64_t)kWindowAlign * E + 127) / 128 * 128; }
+// They take the hand-ordered tile, else the 128 x 128 tile of the general loop.
+inline bool wgrad_hand_ok(int N, int K, int64_t ld) { return N >= 1024 && K >= 1024 && hand_weights_ok(N, ld) && hand_weights_ok(K, ld); }
+
+inline double stored_us(double tiles, double slabs) { return std::max(tiles / 512, 1.0) * (1.25 * slabs + 5.0); }
+inline double transposed_us(double tiles, double slabs, double transposed_bytes) {
+    const double rounds = tiles / 256;
+    return (rounds <= 1.0 ? 1.0 : rounds + 0.5) * (1.3 * slabs + 8.0) + 2.0 * transposed_bytes / 4.5e6 + 8.0;
+}
+inline bool stored_operands_ok(int64_t rows, int N, int K) {
+    return (rows + 128) * std::max(N, K) * 2 < kBufferLimit && (int64_t)(N + 128) * K * 2 < kBufferLimit && (int64_t)(K + 128) * N * 2 < kBufferLimit;
+}
+
+// Weight gradient [E, N, K] of A rows.  Transposed / as stored: 16 experts of 2048 x 2048, 512 rows each 124 / 105; 750 rows of 1408 x 2048
+// 127 / 98; 136 of 1280 x 1408 48 / 27; 19 of 1024 x 2560 48 / 22; 4 of 2048 x 2560, 4096 rows 231 / 201; 64 of 1408 x 2048, 1536 rows
+// 856 / 717; 16 of 2048 x 2560, 1024 rows 230 / 224 (estimated the other way round); 8 of 4096 x 2048, 2048 rows 305 / 330; 8 of 4096 x
+// 14336, 512 rows 641 / 721, 2048 rows 1710 / 2229.  Behind the general loop: 8 of 960 x 14336, 4096 rows 1494 / 1105; 64 of 960 x
+// 4096, 2048 rows 1945 / 1319; 12 of 512 x 512, 100 rows 18.5 / 9.1 (16 shapes in bf16 and fp16: as stored takes 0.44 to 0.77 of the time).
+inline bool wgrad_as_stored(int64_t A, int E, int N, int K) {
+    if (!stored_operands_ok(A, N, K)) return false;
+    if (!wgrad_hand_ok(N, K, wgrad_ld(A, E))) return true;
+    const double rows = (double)A / std::max(E, 1);
+    return stored_us((double)E * ((N + 127) / 128) * ((K + 127) / 128), rows / 64 + 0.5) <
+           transposed_us((double)E * columns256(N) * columns256(K), rows / 64 + 1.0, 2.0 * A * (N + K));
+}
+// Data gradient [A, N] from rows of K and the weight [E, K, N].
+inline bool grouped_kn_as_stored(int64_t A, int E, int N, int K) {
+    if (!stored_operands_ok(A, N, K)) return false;
+    const double rows = (double)A / std::max(E, 1);
+    const double blocks = E * (rows <= 96 ? 1.0 : rows / 128 + 0.5), big = E * (rows <= 192 ? 1.0 : rows / 256 + 0.25);
+    return stored_us(blocks * ((N + 127) / 128), K / 64.0) < transposed_us(big * columns256(N), K / 64.0, 2.0 * E * N * K);
+}
+
+}  // namespace moe355

@@ -52,7 +52,7 @@ CASES = [  # S, H, I, E, k, capacity factor, router skew
     (256, 256, 512, 8, 2, 1.0, 0.0),
     (512, 128, 320, 4, 1, 2.0, 0.7),        # skewed: one expert takes most rows, one may stay empty
     (2048, 512, 1024, 4, 2, 1.25, 0.0),     # 256-row blocks in the grouped product
-    (1024, 1024, 1024, 2, 2, 2.0, 0.0),     # 256 x 256 tiles in the weight gradient as well
+    (1024, 1024, 1024, 2, 2, 2.0, 0.0),     # 256 x 256 tiles in the weight gradient too, where it goes by transposed operands
     (700, 1088, 1216, 2, 1, 2.0, 0.2),      # the same, ragged in both dimensions
 ]
 
@@ -158,6 +158,52 @@ def test_weight_gradient_vs_oracle(moe, case, dtype):
                 assert not got[e].any()
             else:
                 assert max_rel_err(got[e], want[e]) <= OUT_TOL[dtype], (e, int(count[e]))
+
+
+@pytest.mark.parametrize("dtype", [ob.BF16, ob.F16])
+@pytest.mark.parametrize("case", CASES)
+def test_weight_gradient_of_transposed_operands(moe, case, dtype):
+    """The 16-bit weight gradient behind padded transposes (option grouped_tile, and where its larger tile is the faster way):
+    against the oracle, and bit for bit what the rows as they are give, an expert's rows being added up in the same order."""
+    S, H, I, E, k, cf, skew = case
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=5 * S + E, cf=cf, skew=skew)
+    count = count.copy()
+    count[E - 1] = 0                                           # and an expert without rows
+    auto, transposed = moe.MoELayer(product_config(cfg)), moe.MoELayer(product_config(cfg), options={"grouped_tile": 1})
+    kind = KIND[dtype]
+    dcount, doffset = to_device(count, "i32"), to_device(offset, "i32")
+    for (N, K) in ((H, I), (I, H)):
+        a, dy, _, _ = operands(rng, S * k, E, N, K, dtype)
+        want = ob.to_f32(ob.expert_wgrad(dy, a, count, offset, dtype), dtype)
+        args = to_device(dy, kind), to_device(a, kind), dcount, doffset
+        got = from_device(transposed.expert_wgrad(*args))
+        for e in range(E):
+            if count[e] == 0:
+                assert not ob.to_f32(got[e], dtype).any()
+            else:
+                assert max_rel_err(ob.to_f32(got[e], dtype), want[e]) <= OUT_TOL[dtype], (e, int(count[e]))
+        assert np.array_equal(got, from_device(auto.expert_wgrad(*args)))
+
+
+@pytest.mark.parametrize("tile", [None, 1], ids=["rows", "transposed"])
+def test_scratch_of_a_weight_gradient_may_hold_anything(moe, tile):
+    """All rows on one expert, then other splits through the same layer, its scratch filled with NaN in between."""
+    import torch
+    dtype, kind = ob.BF16, "bf16"
+    S, H, I, E = 256, 128, 256, 4
+    cfg = ob.Cfg(S=S, H=H, I=I, E=E, k=1, dtype=dtype, act=ob.ACT_RELU, drop=0)
+    layer = moe.MoELayer(product_config(cfg), options={} if tile is None else {"grouped_tile": tile})
+    rng = np.random.default_rng(9)
+    a, dy, _, _ = operands(rng, S, E, H, I, dtype)
+    for count in ([0, S, 0, 0], [100, 0, 29, 127], [0, 0, 0, 0]):
+        count = np.asarray(count, np.int32)
+        offset = np.concatenate([[0], np.cumsum(count)[:-1]]).astype(np.int32)
+        want = ob.to_f32(ob.expert_wgrad(dy, a, count, offset, dtype), dtype)
+        sc = layer.backward_scratch()
+        sc[:sc.numel() // 2 * 2].view(torch.bfloat16).fill_(float("nan"))
+        got = ob.to_f32(from_device(layer.expert_wgrad(to_device(dy, kind), to_device(a, kind),
+                                                       to_device(count, "i32"), to_device(offset, "i32"))), dtype)
+        assert np.abs(got - want).max() <= OUT_TOL[dtype] * max(np.abs(want).max(), 1.0)
 
 
 def test_empty_experts_and_second_call_reuse_scratch(moe):

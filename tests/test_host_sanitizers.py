@@ -50,13 +50,15 @@ def test_queue_order_keeps_every_dependency_under_asan_and_ubsan(tmp_path):
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_two_launch_rules_under_asan_and_ubsan(tmp_path):
-    """csrc/two_launches.hpp decides which 16-bit layers run as two launches and on which row blocks, where every choice gives
-    the same bits: its answers on both sides of each line, at layers that were measured both ways, and at the ends of the range."""
-    exe = str(tmp_path / "two_launches")
+@pytest.mark.parametrize("rules", ["two_launches", "product_choice"])
+def test_dispatch_rules_under_asan_and_ubsan(tmp_path, rules):
+    """csrc/two_launches.hpp decides which 16-bit layers run as two launches and on which row blocks, csrc/product_choice.hpp whether
+    a training product takes operands as stored; every choice gives the same bits.  Their answers on both sides of each line, at
+    shapes that were measured both ways, and at the ends of the range."""
+    exe = str(tmp_path / rules)
     cmd = ["g++", "-std=c++17", "-O1", "-g", "-Wall", "-Werror", "-fno-omit-frame-pointer", "-fsanitize=address,undefined",
            "-fno-sanitize-recover=all", "-static-libasan", "-I", os.path.join(ROOT, "cuplayground_amd", "csrc"), "-o", exe,
-           os.path.join(ROOT, "tests", "host", "two_launches.cpp")]
+           os.path.join(ROOT, "tests", "host", rules + ".cpp")]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", UBSAN_OPTIONS="print_stacktrace=1")

@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_gate_wgrad_rows", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -170,7 +170,7 @@ def load_library():
     L.moe_router_grad_bytes.argtypes = [vp, C.POINTER(C.c_size_t)]
     L.moe_combine_router_backward.argtypes = [vp] * 10
     L.moe_dispatch_router_backward.argtypes = [vp] * 9
-    L.moe_gate_wgrad.argtypes = [vp, vp, vp, vp, vp, C.c_size_t, vp]
+    L.moe_gate_wgrad.argtypes = L.moe_gate_wgrad_rows.argtypes = [vp, vp, vp, vp, vp, C.c_size_t, vp]
     L.moe_last_hip_error.argtypes = [vp]
     L.moe_status_string.argtypes = [C.c_int]; L.moe_status_string.restype = C.c_char_p
     L.moe_version.restype = C.c_int
@@ -672,14 +672,16 @@ class MoELayer:
     @property
     def router_grad_bytes(self) -> int:
         """Bytes of the router's gradient buffer; 0 where the gate has no such kernels (softmax not normalised over the chosen)."""
-        n = C.c_size_t(0)
-        return n.value if self.L.moe_router_grad_bytes(self._h, C.byref(n)) == 0 else 0
+        if getattr(self, "_router_grad_bytes", None) is None:      # the handle's shape says it all
+            n = C.c_size_t(0)
+            self._router_grad_bytes = n.value if self.L.moe_router_grad_bytes(self._h, C.byref(n)) == 0 else 0
+        return self._router_grad_bytes
 
-    def _router_operands(self, router_grad, **int_tables):
-        """The router's gradient buffer and the [S, k] tables that go with it."""
+    def _router_operands(self, router_grad, *int_tables):
+        """The router's gradient buffer and the [S, k] tables that go with it, as (name, tensor)."""
         import torch
         _operand("router_grad", router_grad, torch.uint8, self.router_grad_bytes)
-        for name, t in int_tables.items():
+        for name, t in int_tables:
             _operand(name, t, torch.int32, self.S * self.k)
 
     def combine_router_backward(self, dout, y_rows, pair_row, topk_w, topk_idx, logits, dy, router_grad):
@@ -690,7 +692,7 @@ class MoELayer:
         _operand("topk_w", topk_w, torch.float32, self.S * self.k)
         if logits is not None:
             _operand("logits", logits, torch.float32, self.S * self.E)
-        self._router_operands(router_grad, pair_row=pair_row, topk_idx=topk_idx)
+        self._router_operands(router_grad, ("pair_row", pair_row), ("topk_idx", topk_idx))
         _check(self.L.moe_combine_router_backward(self._h, _ptr(dout), _ptr(y_rows), _ptr(pair_row), _ptr(topk_w), _ptr(topk_idx),
                                                   _ptr(logits), _ptr(dy), _ptr(router_grad), _stream()), "moe_combine_router_backward")
 
@@ -700,19 +702,21 @@ class MoELayer:
         if db_rows is not None:
             _operand("db_rows", db_rows, self.act_dtype, da_rows.numel())
         _operand("gate_w", gate_w, self.act_dtype, self.E * self.H)
-        self._router_operands(router_grad, pair_row=pair_row, topk_idx=topk_idx)
+        self._router_operands(router_grad, ("pair_row", pair_row), ("topk_idx", topk_idx))
         dx = torch.empty(self.S, self.H, dtype=da_rows.dtype, device=da_rows.device)
         _check(self.L.moe_dispatch_router_backward(self._h, _ptr(da_rows), _ptr(db_rows), _ptr(pair_row), _ptr(topk_idx),
                                                    _ptr(router_grad), _ptr(gate_w), _ptr(dx), _stream()), "moe_dispatch_router_backward")
         return dx
 
-    def gate_wgrad(self, x, router_grad):
+    def gate_wgrad(self, x, router_grad, packed: bool = False):
+        """The gradient of the router's weights; packed: x are the rows of dispatch_rows instead of the tokens."""
         import torch
-        _operand("x", x, self.act_dtype, self.S * self.H)
+        _operand("x", x, self.act_dtype, self.S * self.H * (self.k if packed else 1))
         self._router_operands(router_grad)
         sc = self.backward_scratch()
         dw = torch.empty(self.E, self.H, dtype=self.act_dtype, device=x.device)
-        _check(self.L.moe_gate_wgrad(self._h, _ptr(x), _ptr(router_grad), _ptr(dw), _ptr(sc), sc.numel(), _stream()), "moe_gate_wgrad")
+        call = self.L.moe_gate_wgrad_rows if packed else self.L.moe_gate_wgrad
+        _check(call(self._h, _ptr(x), _ptr(router_grad), _ptr(dw), _ptr(sc), sc.numel(), _stream()), "moe_gate_wgrad")
         return dw
 
 

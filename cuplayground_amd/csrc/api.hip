@@ -1309,14 +1309,24 @@ int moe_dispatch_router_backward(moe_handle* h, const void* da_rows, const void*
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 
-int moe_gate_wgrad(moe_handle* h, const void* x, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream) {
+namespace {
+int gate_wgrad(moe_handle* h, const void* x, bool packed, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream) {
     if (!h || !x || !router_grad || !dgate_w) return MOE_ERR_BAD_ARGUMENT;
     if (!backward_dtype(h)) return MOE_ERR_UNSUPPORTED;
     if ((uintptr_t)x % 16 || (uintptr_t)router_grad % kAlign) return MOE_ERR_BAD_ARGUMENT;
     if (!scratch || (uintptr_t)scratch % kAlign || scratch_bytes < backward_scratch_bytes(h->d.A, h->d.E, h->d.H, h->d.I, (int)h->d.act_bytes))
         return MOE_ERR_WORKSPACE;
-    const hipError_t e = launch_gate_wgrad(x, router_grad, h->d.S, h->d.E, h->d.k, h->d.H, h->d.act_dtype, dgate_w, scratch, (hipStream_t)stream);
+    const hipError_t e = launch_gate_wgrad(x, packed, router_grad, h->d.S, h->d.E, h->d.k, h->d.H, h->d.act_dtype, dgate_w, scratch, (hipStream_t)stream);
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+}  // namespace
+
+int moe_gate_wgrad(moe_handle* h, const void* x, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream) {
+    return gate_wgrad(h, x, false, router_grad, dgate_w, scratch, scratch_bytes, stream);
+}
+
+int moe_gate_wgrad_rows(moe_handle* h, const void* x_rows, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream) {
+    return gate_wgrad(h, x_rows, true, router_grad, dgate_w, scratch, scratch_bytes, stream);
 }
 
 int moe_combine(const void* y_rows, const int32_t* pair_row, const float* topk_w, int32_t S, int32_t k, int32_t H,

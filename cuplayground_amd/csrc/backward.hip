@@ -327,13 +327,15 @@ struct RouterGrad {
     const float* logits;         // [S, E], read where the gate is a normalised sigmoid only
     float* dl;                   // [S, k]: of the chosen experts' logits (those of the others are zero)
     float* dl_dense;             // [S, ld]: the same as rows over the experts, zeros elsewhere
+    int32_t* row_of;             // [S]: a packed row that holds the token, -1 where all of its pairs were dropped (its dl are zeros)
     int E, ld, gate_fn, norm;
 };
 // The adjoint of the gate weights of one token (one wavefront; lane j < k holds dw of rank j), in fp32:
 //   softmax, normalised over the chosen: w = softmax of the chosen logits,  dl_j = w_j (dw_j - sum_m w_m dw_m);
 //   sigmoid: dl_j = s_j (1 - s_j) dw_j, s = w;  normalised: ds_j = (dw_j - sum_m w_m dw_m) / sum_m s_m, dl_j = s_j (1 - s_j) ds_j.
-__device__ __forceinline__ void router_grad_token(const RouterGrad& r, const float* __restrict__ topk_w, float dw, int t, int k) {
+__device__ __forceinline__ void router_grad_token(const RouterGrad& r, const float* __restrict__ topk_w, float dw, int row, int t, int k) {
     const int lane = threadIdx.x & 63;
+    if (lane == 0) r.row_of[t] = row;
     const bool have = lane < k;
     const int e = have ? r.topk_idx[(size_t)t * k + lane] : -1;
     const float w = have ? topk_w[(size_t)t * k + lane] : 0.0f;
@@ -368,10 +370,11 @@ __device__ __forceinline__ void router_grad_token(const RouterGrad& r, const flo
 
 // The router's weight gradient, dgate_w[e, :] = sum over tokens of dl[t, e] x[t, :], in fp32: a share of the tokens a wavefront,
 // 256 columns x 16 experts of sums in its registers, the coefficients as scalars; the four wavefronts' sums meet in LDS and the
-// workgroups' in gate_wgrad_sum_kernel, both in a fixed order.  grid = (columns / 256, shares, experts / 16).
+// workgroups' in gate_wgrad_sum_kernel, both in a fixed order.  grid = (columns / 256, shares, experts / 16).  row_of: null, or x are the
+// packed rows, and a token is read from the one that row_of names.
 constexpr int kGateShareMax = 64;      // partial sums of E * H * 4 bytes each: never more than the transposed operands the scratch is sized for
 template <class T16, class RAW = typename RawOf<T16>::type>
-__global__ __launch_bounds__(256) void gate_wgrad_kernel(const RAW* __restrict__ x, const float* __restrict__ dl, int S, int H, int E, int ld, float* __restrict__ part) {
+__global__ __launch_bounds__(256) void gate_wgrad_kernel(const RAW* __restrict__ x, const int32_t* __restrict__ row_of, const float* __restrict__ dl, int S, int H, int E, int ld, float* __restrict__ part) {
     __shared__ float red[4][64][64];   // [wavefront][expert * 4 + column of the lane][lane]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = blockIdx.x * 256 + 4 * lane, e0 = blockIdx.z * 16;
@@ -386,7 +389,9 @@ __global__ __launch_bounds__(256) void gate_wgrad_kernel(const RAW* __restrict__
     struct alignas(4 * sizeof(RAW)) Four { RAW e[4]; };
 #pragma unroll 4
     for (int t = t0; t < t1; ++t) {
-        const Four q = *reinterpret_cast<const Four*>(x + (size_t)t * H + c);
+        const int row = row_of ? row_of[t] : t;
+        Four q = *reinterpret_cast<const Four*>(x + (size_t)max(row, 0) * H + c);
+        if (row < 0) q = Four{};               // no packed row: whatever row 0 holds, infinities too, takes no part
         const float* d = dl + (size_t)t * ld + e0;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -433,6 +438,7 @@ __global__ __launch_bounds__(256) void combine_backward_kernel(const RAW* __rest
     const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= S) return;
     float mine = 0.0f;                 // lane j: dw[t, j]
+    int held = -1;                     // the token's first packed row
     for (int r0 = 0; r0 < k; r0 += 4) {
         int row[4];
         float w[4], acc[4];
@@ -465,11 +471,12 @@ __global__ __launch_bounds__(256) void combine_backward_kernel(const RAW* __rest
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) acc[j] += __shfl_xor(acc[j], off, 64);
             if (row[j] < 0) acc[j] = 0.0f;
+            else if (held < 0) held = row[j];
             if (lane == r0 + j) mine = acc[j];
             if (dw && lane == 0 && r0 + j < k) dw[(size_t)t * k + r0 + j] = acc[j];
         }
     }
-    if (router.dl) router_grad_token(router, topk_w, mine, t, k);
+    if (router.dl) router_grad_token(router, topk_w, mine, held, t, k);
 }
 
 // The same one element at a time, for operands that are not 16-byte aligned: one workgroup per token.
@@ -797,31 +804,36 @@ hipError_t launch_combine_backward(const void* dout, const void* y, const int32_
 
 // ---- the router's share of a backward pass ----
 static int router_ld(int E) { return (E + 15) / 16 * 16; }
-size_t router_grad_bytes(int S, int E, int k) { return align256((size_t)S * k * 4) + align256((size_t)S * router_ld(E) * 4); }
+size_t router_grad_bytes(int S, int E, int k) { return align256((size_t)S * k * 4) + align256((size_t)S * router_ld(E) * 4) + align256((size_t)S * 4); }
 static float* router_dense(void* grad, int S, int k) { return reinterpret_cast<float*>(static_cast<char*>(grad) + align256((size_t)S * k * 4)); }
+
+static int32_t* router_rows(void* grad, int S, int E, int k) {
+    return reinterpret_cast<int32_t*>(reinterpret_cast<char*>(router_dense(grad, S, k)) + align256((size_t)S * router_ld(E) * 4));
+}
 
 hipError_t launch_combine_backward_router(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w,
                                           const int32_t* topk_idx, const float* logits, int S, int E, int k, int H, int gate_fn, int norm,
                                           int dtype, void* dy, void* grad, hipStream_t st) {
-    const RouterGrad r{topk_idx, logits, static_cast<float*>(grad), router_dense(grad, S, k), E, router_ld(E), gate_fn, norm};
+    const RouterGrad r{topk_idx, logits, static_cast<float*>(grad), router_dense(grad, S, k), router_rows(grad, S, E, k), E, router_ld(E), gate_fn, norm};
     return combine_backward(dout, y, pair_row, topk_w, S, k, H, dtype, dy, nullptr, r, st);
 }
 
-hipError_t launch_gate_wgrad(const void* x, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st) {
+hipError_t launch_gate_wgrad(const void* x, bool packed, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st) {
     const float* dense = router_dense(const_cast<void*>(grad), S, k);
+    const int32_t* row_of = packed ? router_rows(const_cast<void*>(grad), S, E, k) : nullptr;
     // shares: 32 tokens a wavefront, at least enough workgroups for the compute units where there are tokens for them
     const int shares = std::min(std::max((S + 127) / 128, 1), kGateShareMax), n = E * H;
     const dim3 grid((unsigned)((H + 255) / 256), (unsigned)shares, (unsigned)(router_ld(E) / 16));
     float* part = static_cast<float*>(scratch);
     const unsigned sums = (unsigned)((n + 255) / 256);
     if (dtype == MOE_DTYPE_F32) {
-        gate_wgrad_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)x, row_of, dense, S, H, E, router_ld(E), part);
         gate_wgrad_sum_kernel<f32_s><<<sums, 256, 0, st>>>(part, shares, n, (float*)dgate_w);
     } else if (dtype == MOE_DTYPE_FP16) {
-        gate_wgrad_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, row_of, dense, S, H, E, router_ld(E), part);
         gate_wgrad_sum_kernel<f16_s><<<sums, 256, 0, st>>>(part, shares, n, (uint16_t*)dgate_w);
     } else {
-        gate_wgrad_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, dense, S, H, E, router_ld(E), part);
+        gate_wgrad_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)x, row_of, dense, S, H, E, router_ld(E), part);
         gate_wgrad_sum_kernel<bf16_s><<<sums, 256, 0, st>>>(part, shares, n, (uint16_t*)dgate_w);
     }
     return hipGetLastError();

@@ -253,7 +253,7 @@ size_t router_grad_bytes(int S, int E, int k);
 hipError_t launch_combine_backward_router(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w,
                                           const int32_t* topk_idx, const float* logits, int S, int E, int k, int H, int gate_fn, int norm,
                                           int dtype, void* dy, void* grad, hipStream_t st);
-hipError_t launch_gate_wgrad(const void* x, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st);
+hipError_t launch_gate_wgrad(const void* x, bool packed, const void* grad, int S, int E, int k, int H, int dtype, void* dgate_w, void* scratch, hipStream_t st);
 hipError_t launch_combine_backward(const void* dout, const void* y, const int32_t* pair_row, const float* topk_w, int S,
                                    int k, int H, int dtype, void* dy, float* dw, hipStream_t st);
 

@@ -90,15 +90,19 @@ def _aligned(t):
 
 
 def _own(t, given):
-    """What a node keeps of `given`, a tensor of the caller's, of which `t` is the aligned form: 16-bit operands as a copy, so that
-    adding the layer's output onto its input in place, or a step of the router's weights, may come before the backward (as with gate
-    weights in torch, which reads them as fp32 copies; fp32 ones autograd keeps itself, and refuses them once they are changed)."""
+    """What a node keeps of `given`, the caller's router weights, of which `t` is the aligned form: 16-bit ones as a copy, so that they may
+    be stepped before the backward (as with gate weights in torch, which reads fp32 copies of them; fp32 ones autograd keeps itself, and
+    refuses them once they are changed)."""
     return t.clone() if t.dtype != torch.float32 and t.data_ptr() == given.data_ptr() else t
 
 
 def _unpacked(ctx):
     """The saved tensors as the kernels take them: a saved-tensor hook may hand back views at any address."""
-    return [None if t is None else _aligned(t) for t in ctx.saved_tensors]
+    saved = ctx.saved_tensors
+    for t in saved:
+        if t is not None and (t.data_ptr() & 15 or not t.is_contiguous()):
+            return [None if t is None else _aligned(t) for t in saved]
+    return saved                       # (without hooks)
 
 
 def _as_stored(layer, w):
@@ -120,7 +124,7 @@ def _expert_rows(x, w_up, w_gate, w_down, layer, token_indices, count, offset):
     return rows, u, g, h, product(h, w_down)
 
 
-def _kept(needs, rows, u, g, h, w_up, w_gate, w_down):
+def _kept(needs, rows, u, g, h, w_up, w_gate, w_down, need_rows=False):
     """What of the forward pass the gradients that are asked for read (a step that trains the router alone reads y)."""
     need_x, need_up, need_gate, need_down = needs
     need_u = need_x or need_up or need_gate
@@ -128,7 +132,7 @@ def _kept(needs, rows, u, g, h, w_up, w_gate, w_down):
     def kept(needed, t):
         return t if needed else None
 
-    return (kept(need_up or need_gate, rows), kept(need_u, u), kept(need_u, g), kept(need_down, h),
+    return (kept(need_up or need_gate or need_rows, rows), kept(need_u, u), kept(need_u, g), kept(need_down, h),
             kept(need_x, w_up), kept(need_x, w_gate), kept(need_u, w_down))
 
 
@@ -196,41 +200,41 @@ class _RoutedExperts(torch.autograd.Function):
 
     The gate weights are the routing kernel's own and their adjoint rides in passes that run anyway: the combine's adjoint, one
     wavefront a token, goes on to the logits' gradients; the dispatch's adds their product with the router's weight rows to the
-    tokens' gradient in fp32; what is left is one pass over x for the router's weight gradient.  As torch ops the router took
+    tokens' gradient in fp32; what is left is one pass over the tokens' packed rows for the router's weight gradient.  As torch ops the router took
     about 25 launches and fp32 copies of x.  A bf16 step, before and after: 922 -> 786 us (GELU, the larger layer of the
     benchmark table), 1302 -> 1172 us (SwiGLU), 720 -> 330 us for a few hundred tokens, where launches are the time."""
 
     @staticmethod
     def forward(ctx, x, w_up, w_gate, w_down, gate_w, layer, grad_enabled):
-        given = x, gate_w
-        x, gate_w, w_up, w_down = _aligned(x), _aligned(gate_w), w_up.contiguous(), w_down.contiguous()
+        x, gate, w_up, w_down = _aligned(x), _aligned(gate_w), w_up.contiguous(), w_down.contiguous()
         w_gate = None if w_gate is None else w_gate.contiguous()
         c = layer.cfg
         need_x, need_gate_w = (grad_enabled and ctx.needs_input_grad[i] for i in (0, 4))
-        need_router = need_x or need_gate_w
-        gate = layer.gate(x, gate_w, want_logits=need_router and c.gate_fn != api.GATE_SOFTMAX and bool(c.norm_topk_prob))
-        idx, topk_w, logits = gate if len(gate) == 3 else (*gate, None)
+        want_logits = (need_x or need_gate_w) and c.gate_fn != api.GATE_SOFTMAX and bool(c.norm_topk_prob)
+        idx, topk_w, *logits = layer.gate(x, gate, want_logits=want_logits)
         r = layer.route(idx)
         pair_row, count, offset = r["pair_row"], r["expert_count"], r["expert_offset"]
         rows, u, g, h, y = _expert_rows(x, w_up, w_gate, w_down, layer, r["token_indices"], count, offset)
-        ctx.save_for_backward(*_kept(ctx.needs_input_grad[:4], rows, u, g, h, w_up, w_gate, w_down), y, topk_w, pair_row, count, offset,
-                              _own(x, given[0]) if need_gate_w else None, _own(gate_w, given[1]) if need_x else None, idx, logits)
+        # (the router's gradients read the tokens from their packed rows: x itself is not kept, and may change before the backward)
+        ctx.save_for_backward(*_kept(ctx.needs_input_grad[:4], rows, u, g, h, w_up, w_gate, w_down, need_rows=need_gate_w), y, topk_w, pair_row,
+                              count, offset, _own(gate, gate_w) if need_x else None, idx, *logits)
         ctx.layer = layer
         return api.combine(y, pair_row, topk_w)
 
     @staticmethod
     def backward(ctx, dout):
-        *kept, y, topk_w, pair_row, count, offset, x, gate_w, idx, logits = _unpacked(ctx)
+        rows, u, g, h, w_up, w_gate, w_down, y, topk_w, pair_row, count, offset, gate_w, idx, *logits = _unpacked(ctx)
         layer, needs = ctx.layer, ctx.needs_input_grad[:4]
         dout, dy, router = _aligned(dout), torch.empty_like(y), None
         if needs[0] or ctx.needs_input_grad[4]:
             router = torch.empty(layer.router_grad_bytes, dtype=torch.uint8, device=y.device)
-            layer.combine_router_backward(dout, y, pair_row, topk_w, idx, logits, dy, router)
+            layer.combine_router_backward(dout, y, pair_row, topk_w, idx, logits[0] if logits else None, dy, router)
         else:
             layer.combine_backward(dout, y, pair_row, topk_w, dy=dy)
+        kept = rows, u, g, h, w_up, w_gate, w_down
         da, db, dup, dgate, ddown = _expert_gradients(layer, needs, dy, kept, count, offset)
         dx = layer.dispatch_router_backward(da, db, pair_row, idx, router, gate_w) if needs[0] else None
-        dgate_w = layer.gate_wgrad(x, router) if ctx.needs_input_grad[4] else None
+        dgate_w = layer.gate_wgrad(rows, router, packed=True) if ctx.needs_input_grad[4] else None
         return dx, dup, dgate, ddown, dgate_w, None, None
 
 

@@ -453,6 +453,9 @@ int moe_combine_router_backward(moe_handle* h, const void* dout, const void* y_r
                                 const int32_t* topk_idx, const float* logits, void* dy_rows, void* router_grad, void* stream);
 int moe_dispatch_router_backward(moe_handle* h, const void* da_rows, const void* db_rows, const int32_t* pair_row, const int32_t* topk_idx,
                                  const void* router_grad, const void* gate_w, void* dx, void* stream);
+/* (moe_gate_wgrad_rows: the same sums from the packed rows of moe_dispatch_rows instead of the tokens, so that a training step need
+ * not keep both; router_grad says where each token lies.  A token that lost every pair takes no part.) */
+int moe_gate_wgrad_rows(moe_handle* h, const void* x_rows, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream);
 int moe_gate_wgrad(moe_handle* h, const void* x, const void* router_grad, void* dgate_w, void* scratch, size_t scratch_bytes, void* stream);
 /* The elementwise and reduction steps between those products (same layers; fp32 arithmetic, one rounding on store):
  * moe_act_backward: for the first `rows` packed rows of width I, du = dh * act'(u) for hidden_act ReLU (1 where u > 0)

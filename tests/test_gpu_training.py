@@ -240,6 +240,14 @@ def test_router_gradients(moe, S, H, E, k, gate_fn, norm, dtype, drop):
     got, ref, mag = layer.gate_wgrad(x, router).double(), dense.t() @ x.double(), dense.t().abs() @ x.double().abs()
     tiny = 2.0 ** -24 if dtype == 3 else 0.0           # fp16 below its normal range
     assert bool(((got - ref).abs() <= unit * ref.abs() + (S / 4 + 68) * 2.0 ** -24 * mag + tiny).all())
+    # the same sums from the packed rows, whatever the rows of no expert hold: a token without a row has no gradient to add
+    packed = torch.full((S * k, H), float("nan"), dtype=layer.act_dtype, device="cuda")
+    kept = (rows >= 0).nonzero()
+    packed[rows[rows >= 0].long()] = x[kept[:, 0]]
+    lost = (rows < 0).all(1)
+    assert bool((dl[lost] == 0).all())
+    x_kept = x.masked_fill(lost[:, None], 0)
+    assert torch.equal(layer.gate_wgrad(packed, router, packed=True), layer.gate_wgrad(x_kept, router))
     a, b = rand(S * k, H), rand(S * k, H)
     got = layer.dispatch_router_backward(a, b, rows, idx, router, gate_w).double()
     part = torch.where((rows >= 0)[..., None], a[rows.clamp(min=0).long()].double() + b[rows.clamp(min=0).long()].double(), 0.0).sum(1)

@@ -32,8 +32,8 @@ def test_trainable_layer_matches_torch_autograd(moe, act, dtype, drop, inter):
     g = torch.Generator(device="cuda").manual_seed(1)
     x = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype).requires_grad_(True)
     dout = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype)
-    # the activation's derivative rides in the epilogue of the down projection's data gradient where the layer has
-    # that kernel (16-bit, 256 | intermediate size), else the two building blocks run one after the other
+    # (the 16-bit cases' products take the weights as stored, with the activation's derivative in the epilogue; the branches of
+    # layers that go by transposed copies give the same bits: the test below)
     assert m.layer.fused_act_backward == (dtype in (2, 3) and inter % 256 == 0)
     out = m(x)
     out.backward(dout)
@@ -56,6 +56,32 @@ def test_trainable_layer_matches_torch_autograd(moe, act, dtype, drop, inter):
         assert rel(p.grad.float(), ps[n].grad) <= tol, n
     if drop:                                # some pairs were dropped in this configuration: the test covers that path
         assert int((m.route(x)[1]["pair_row"] < 0).sum()) > 0
+
+
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("act,dtype,drop,inter", [(2, 2, 0, 384), (1, 2, 1, 512), (0, 3, 0, 512), (2, 3, 1, 384), (2, 2, 1, 512)])
+def test_transposed_copies_and_operands_as_stored_give_the_same_step(moe, act, dtype, drop, inter, tile):
+    """Large layers' gradients go by transposed copies of the weights and rows -- with the activation's derivative in the epilogue where
+    the layer has that kernel, else as a pass of its own -- small ones' by the operands as stored.  Option grouped_tile takes a small
+    layer the first way: the same sums in the same order, so the same bits."""
+    import torch
+    from cuplayground_amd import training
+    cfg = moe.MoEConfig(capacity_factor=1.0, drop_tokens=drop, expert_top_k=2, hidden_act=act, hidden_size=256,
+                        intermediate_size=inter, micro_batch=1, num_experts=6, sequence_len=700,
+                        torch_dtype=dtype, gate_fn=0, norm_topk_prob=1, is_training=1)
+    steps = []
+    for options, stored in ((None, 2), ({"grouped_tile": tile}, 1)):
+        m, g = training.MoE355Train(cfg, init_std=0.05, seed=3), torch.Generator(device="cuda").manual_seed(1)
+        if options:
+            m.layer = moe.MoELayer(cfg, options=options)
+        for n, k in ((256, inter), (inter, 256)):
+            assert m.layer.gemm_kn_supported(n, k) == stored
+        assert m.layer.fused_act_backward == (inter % 256 == 0)
+        x = torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype).requires_grad_(True)
+        out = m(x)
+        out.backward(torch.randn(cfg.tokens, cfg.hidden_size, generator=g, device="cuda").to(m.layer.act_dtype))
+        steps.append([out.detach(), x.grad] + [p.grad for _, p in m.named_parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*steps))
 
 
 def test_e4m3_layers_are_refused(moe):

@@ -68,10 +68,11 @@ struct GroupedTask {
 // first, and the short ones fill the compute units that the last round of long ones leaves idle.  Workgroups go to the eight XCDs in
 // turn: each XCD takes an eighth of either list in a row, so that the tiles that share a weight tile or token rows share an L2.
 // Every wavefront works it out for itself, an expert a lane, which takes less time than a launch in front that writes tables.
-// 16 experts of 2048 x 2048, 512 rows each, bf16: 112 -> 93 us (320 tasks on 256 compute units, 64 of them remainders); 8 of
-// 4096 x 2048, 2048 rows 297 -> 258; 64 of 2048 x 1408, 94 rows 113 -> 106; 16 of 2048 x 1408, 750 rows, no remainders, 109 -> 110.
-// The share of an XCD in a row, against the list dealt out to them: whole layers, 8 experts of 4096 x 14336, 2048 rows 4825 -> 4463 us,
-// 1024 rows 2888 -> 2448; 64 of 2048 x 1408, 1536 rows 1862 -> 1665, 750 rows 1112 -> 907; 12 of 1344 x 2752, 444 rows 180 -> 166.
+// One product, bf16, the launch and table in front of 256-row blocks alone against this: 16 experts of 2048 x 2048, about 512 rows each
+// 109 -> 80 us; 8 of 4096 x 2048, 2048 rows 274 -> 234; 64 of 2048 x 1408, 94 rows 94 -> 89; 16 of 2048 x 1408, 750 rows 91 -> 73.
+// The share of an XCD in a row, against the list dealt out to them: whole layers as two launches, 8 experts of 4096 x 14336, 2048 rows
+// 4679 -> 4431 us, 1024 rows 2860 -> 2484; 64 of 2048 x 1408, 1536 rows 1863 -> 1662, 750 rows 1089 -> 907; 12 of 1344 x 2752, 444 rows
+// 174 -> 165, 150 rows 125 -> 107.
 template <int BIG>
 __device__ __forceinline__ bool grouped_task(const int32_t* __restrict__ count, const int32_t* __restrict__ offset, int E, int ncol, int id, GroupedTask& t) {
     constexpr int LEFT = BIG == 256 ? 128 : 0;          // rows up to which what is left of an expert is a block of its own kind
@@ -315,7 +316,8 @@ struct ProdJob {
 
 // The slab loop of one tile.  What bounds it: LDS (a 64 x 64 wavefront tile reads 16 KB of fragments a slab at 256 bytes a cycle,
 // the slab's 32 KB are written at 128), the address unit (64 bytes a cycle) and the matrix instructions, each about half of the
-// time; two workgroups share a compute unit and fill each other's waits.  0.9 PFLOP/s in 2048 rows an expert.  (Workgroups that stay and
+// time; two workgroups share a compute unit and fill each other's waits.  0.85 PFLOP/s with 4096 rows an expert (a weight
+// gradient of 4 x 2048 x 2560), 0.65 with 512 (of 16 x 2048 x 2048).  (Workgroups that stay and
 // request the next tile's first slabs under this one's last: no faster, what they save at the ends of tiles they lose in the
 // last round of an uneven number of tiles.)
 template <class T, bool TA, bool TB>
@@ -621,8 +623,8 @@ hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const
 
 // A layer's two projections, a launch each: blocks of 256 rows and the 128-row tile for what an expert has left, or blocks of 128 rows.
 // Whole layers, us, the queue / two launches of it in the order of the row block table / this:
-//   128-row blocks: 12 experts of 1344 x 2752, GELU, 150 rows each 122 / 108 / 88, 250 rows 131 / 118 / 115; 64 of 2048 x 1408, SwiGLU,
-//   94 rows 278 / 295 / 264; 8 of 4096 x 14336, 128 rows 679 / 672 / 655; 16 of 2048 x 2048, 128 rows 130 / 112 / 110
+//   128-row blocks: 12 experts of 1344 x 2752, GELU, 150 rows each 122 / 108 / 107, 250 rows 130 / 118 / 115; 64 of 2048 x 1408, SwiGLU,
+//   94 rows 294 / 306 / 282; 8 of 4096 x 14336, 128 rows 726 / 740 / 706; 16 of 2048 x 2048, 128 rows 130 / 113 / 109
 //   256-row blocks, and which layers run so: two_launches.hpp
 template <class P>
 static hipError_t launch_ffn_split(const FfnArgs& a, const ExpertRows& rows, hipStream_t st) {

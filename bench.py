@@ -40,11 +40,11 @@ WIDEN_SOURCES = BF16_SOURCES + ("quant.hip",)
 F32_TILE_SOURCES = ("ffn_f32_tile.hip", "ffn_common.hpp", "route.hip")
 FP8_MFMA_SOURCES = FP8_TILE_SOURCES + ("quant.hip",)
 MEASURED_TRAFFIC = {
-    "mixtral": {"bytes": 18.54e9, "sources": BF16_SOURCES, "kernel_digest": "8bf0c797b2f2",
+    "mixtral": {"bytes": 18.52e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
                 "profile": "profiles/ffn_persistent_kernel_bf16_mixtral_c3_hbm_traffic.txt"},
-    "mid": {"bytes": 0.8068e9, "sources": BF16_SOURCES, "kernel_digest": "8bf0c797b2f2",
+    "mid": {"bytes": 0.8063e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
             "profile": "profiles/ffn_persistent_kernel_bf16_mid_c2_hbm_traffic.txt"},
-    "finegrained": {"bytes": 3.353e9, "sources": BF16_SOURCES, "kernel_digest": "8bf0c797b2f2",
+    "finegrained": {"bytes": 3.355e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
                     "profile": "profiles/ffn_persistent_kernel_bf16_finegrained_c4_hbm_traffic.txt"},
     "decode_fp8": {"bytes": 9.907e9, "sources": FP8_SOURCES, "kernel_digest": "db57f455db60",
                    "profile": "profiles/ffn_persistent_fp8_kernel_decode_c5_hbm_traffic.txt"},
@@ -52,7 +52,7 @@ MEASURED_TRAFFIC = {
     "reference_default": {"bytes": 0.9174e9, "sources": F32_TILE_SOURCES, "kernel_digest": "18f0fced7a60", "ffn_mode": 1,
                           "profile": "profiles/ffn_tiled_f32_tile_kernel_reference_default_hbm_traffic.txt"},
     # the widening pass and the bf16 queue kernel together (what the layer's FFN stage launches by default) ...
-    "prefill_fp8": {"bytes": 22.97e9, "sources": WIDEN_SOURCES, "kernel_digest": "2bd72ccae054",
+    "prefill_fp8": {"bytes": 23.35e9, "sources": WIDEN_SOURCES, "kernel_digest": "1a74032c0fe0",
                     "profile": "profiles/widen_plus_ffn_persistent_kernel_prefill_fp8_hbm_traffic.txt"},
     # ... the e4m3 tile GEMM on the same layer (option fp8_widen = 0) ...
     "prefill_fp8/e4m3_tile": {"bytes": 26.44e9, "sources": FP8_TILE_SOURCES, "kernel_digest": "21f3a64c924d",

@@ -554,7 +554,8 @@ __global__ __launch_bounds__(256) void dispatch_rows_kernel(const uint4* __restr
 // dx[t, :] = sum over ranks r, ascending, of a[pair_row[t,r], :] + b[pair_row[t,r], :] (b may be null), and, with dl, behind
 // them of dl[t,r] gate_w[topk_idx[t,r], :], in fp32 and rounded once: the adjoint of the dispatch for one or two row gradients.  One wavefront per token and 64 16-byte pieces of its row,
 // the rows of four ranks in flight.  (torch's index_add backward of the same gather, 8192 rows x 2048 columns in bf16:
-// 55 us, behind two zero fills and, for two projections, two more sums over the rows.)
+// 55 us, behind two zero fills and, for two projections, two more sums over the rows.)  The router's share, a serial loop over the
+// ranks behind each 512 columns, costs 8 us of 19 for 4096 tokens x 2, 10 of 38 for 3000 x 4 with two row gradients.
 template <class T16, class RAW = typename RawOf<T16>::type>
 __global__ __launch_bounds__(256) void dispatch_backward_kernel(const RAW* __restrict__ a, const RAW* __restrict__ b,
                                                                 const int32_t* __restrict__ pair_row, int S, int k, int H,

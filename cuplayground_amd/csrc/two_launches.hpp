@@ -27,7 +27,7 @@ struct TwoLaunchShape {
 constexpr int kTaskUnits = 256;  // compute units: one task each at a time
 
 // AUTO on 128-row blocks (large = false): always, unless tokens are dropped and an expert takes at most kSplitCappedRows.
-//   Random layers: two launches are faster at 176 of 179, by 8 % in the mean.  The others: 32 of 2944 x 2688, GELU, 71 rows 8 % slower, 64
+//   Random layers: two launches are faster at 176 of 179, by a fifth in the mean.  The others: 32 of 2944 x 2688, GELU, 71 rows 8 % slower, 64
 //   of 2432 x 1664, SwiGLU, 101 rows 5 %, 9 of 2048 x 2112, SwiGLU, 388 rows (on 128-row blocks; it runs on 256-row ones).
 //   Dropping layers, 64 of 2048 x 1408: at most 29 rows 234 / 243, 38 rows 237 / 247, 57 rows 248 / 248, 94 rows 249 / 240 (28 rows, none
 //   dropped: 284 / 267).

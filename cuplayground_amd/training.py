@@ -2,13 +2,14 @@
 
 The reference declares a training knob (`is_training`, aristos_config.schema.json:20-23) that none of its code reads.
 Here it has a consumer: `MoE355Train` runs the expert projections through `moe_expert_gemm` and gets their gradients
-from `moe_expert_gemm` on the transposed weight (data gradient) and `moe_expert_wgrad` (weight gradient).  Routing
+from `moe_expert_gemm` on the transposed weight or `moe_expert_gemm_kn` on the weight as stored (data gradient) and
+`moe_expert_wgrad` (weight gradient).  Routing
 decisions (top-k indices, slots, capacity drops) come from the library's router and are not differentiated; the gate
 weights that scale the expert outputs are, by the router's own kernels (`_RoutedExperts`) or, where those do not exist, as
 torch ops on the same logits formula, so the router's weight matrix and the tokens receive gradients through them.
 Everything else -- dispatch, projections, activation, combine -- is one autograd node (`_Experts`, or that node with the
 router) whose backward runs the library's adjoints; the data gradient of the down projection
-carries the activation's derivative in its epilogue (`moe_expert_gemm_act_backward`) where the layer has that kernel,
+carries the activation's derivative in its epilogue (either product; `moe_expert_gemm_act_backward`) where the layer has that kernel,
 else `moe_expert_gemm` is followed by `moe_act_backward`.  `expert_linear` and `act_down` are the projections as nodes
 of their own, for layers composed in torch.  There is no CPU path: every tensor lives on the GPU.
 """

@@ -97,19 +97,22 @@ inline bool two_launches_on_256(const TwoLaunchShape& s) {
     const double small = split_us(0, n.small * up, s.H) + split_us(0, n.small * down, s.I);
     return large <= 0.9 * small;
 }
-// Layers on 256-row blocks whose full row blocks are a round of their own in the up projection, so that the remainders' round reads all
-// weights from memory again, and that take as many rounds on 256-row blocks alone: the order of the row block table, where the blocks
-// of an expert meet the same weight tile, is kept.  Table / remainders behind: 16 of 2048 x 2048, SwiGLU, 260 rows 187 / 193, 278 rows
-// 186 / 218, 300 rows 188 / 233, 325 rows 189 / 235; 32 of 1472 x 2048, GELU, 273 rows 225 / 231; but 237 rows 202 / 181 (hardly a
-// remainder), GELU (one round) 325 rows 155 / 144; 20 of 2048 x 3072, ReLU, 290 rows (fewer rounds in the down projection) 311 / 274.
-// The line is drawn from the first shape; where the up projection's full blocks fall a few short of the round, it is not always the faster
-// side (the table is what such layers ran on before there was the other): 10 of 1920 x 2944, SwiGLU, 373 rows 188 / 198, but 22 of
-// 1216 x 2752, GELU, 309 rows 272 / 184 and 11 of 1856 x 2816, SwiGLU, 322 rows 220 / 197.
+// Layers of 8 or 16 experts on 256-row blocks whose full row blocks are a round of their own in the up projection, so that the remainders'
+// round reads all weights from memory again, and that take as many rounds on 256-row blocks alone: the order of the row block table,
+// where the blocks of an expert meet the same weight tile, is kept.  Table / remainders behind: 16 of 2048 x 2048, SwiGLU, 260 rows 187 / 193,
+// 278 rows 186 / 218, 300 rows 188 / 233, 325 rows 189 / 235; but 237 rows 202 / 181 (hardly a remainder), GELU (one round) 325 rows 155 / 144.
+// 16 of 3904 x 1856, SwiGLU, 306 rows: the up projection fetches 0.95 GB with remainders behind, 0.50 in the table's order.  Of 16 random
+// layers of 8 or 16 experts with full blocks of 0.9 rounds and more 14 are up to 15 % faster, 2 are 0.2 and 3 % slower; of 11 with 0.8 to
+// 0.9 rounds of 32 slabs and more 10 are 4 to 13 % faster, one is 4 % slower, and 3 of fewer slabs are 2 to 9 % slower.  With other numbers of experts (an XCD's
+// share of the list then begins and ends inside an expert, and the table's columns are dealt out unevenly) remainders behind are faster at 27
+// of 30, by up to 30 %: 24 of 1600 x 2112, GELU, 370 rows fetch 0.31 GB against 0.39; 22 of 1216 x 2752, GELU, 309 rows 272 / 184; 24 of 1024 x
+// 2560, 303 rows 43 % more on the table; the other way round 10 of 1920 x 2944, SwiGLU, 373 rows 188 / 198, 12 of 3712 x 3904, 17 of 3456 x
+// 3776 and 29 of 1920 x 1984 2 to 3 %.
 inline bool two_launches_keep_table(const TwoLaunchShape& s) {
     const SplitBlocks n(s.pairs, s.experts);
     const double up = s.columns_up(), down = s.columns_down();
     auto rounds = [](double tiles) { return std::ceil(tiles / kTaskUnits); };
-    return n.left >= 0.75 * s.experts && n.full <= 1.25 * s.experts && n.full * up >= 0.9 * kTaskUnits && rounds(n.table * up) <= 2 &&
+    return s.experts % 8 == 0 && s.experts <= 16 && n.left >= 0.75 * s.experts && n.full <= 1.25 * s.experts && n.full * up >= (s.H >= 2048 ? 0.8 : 0.9) * kTaskUnits && rounds(n.table * up) <= 2 &&
            rounds(n.table * down) <= std::ceil(split_time(n.full * down, n.left * down, 1.0, 0.75) - 0.5);      // (in rounds: a remainder is 0.74 at 32 slabs)
 }
 

@@ -57,6 +57,19 @@ int main() {
     TABLE(false, 16, 2048, 2048, 325, false);
     TABLE(false, 20, 2048, 3072, 290, false);
     TABLE(false, 64, 2048, 1408, 262, true);
+    TABLE(true, 16, 3904, 1856, 306, true);
+    TABLE(true, 8, 4032, 3968, 375, true);
+    // ... nearly a round of long tasks
+    TABLE(true, 8, 3264, 3392, 291, true);
+    TABLE(true, 16, 4032, 3392, 356, false);
+    TABLE(false, 16, 1920, 3136, 352, false);
+    TABLE(false, 16, 1344, 3584, 316, false);
+    TABLE(false, 16, 3840, 2944, 354, false);
+    // ... with one or two experts an XCD only
+    TABLE(false, 22, 1216, 2752, 309, false);
+    TABLE(false, 24, 1024, 2560, 303, false);
+    TABLE(false, 17, 1792, 3776, 346, false);
+    TABLE(false, 48, 960, 1088, 297, false);
     // the ends of the range: every rule ends
     int answers = 0;
     for (int experts : {1, 512})

@@ -26,7 +26,7 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
                            int64_t ld, bool f16, hipStream_t st);
 
 hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
-                                     const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
+                                     const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st);
 hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K,
                                 bool f16, hipStream_t st);
@@ -266,6 +266,7 @@ __device__ __forceinline__ void act_backward_one(float d, float uv, float gv, in
     }
 }
 
+constexpr int kRowsPass = 2;           // 16-byte pieces a thread of the pass below has in flight of every operand
 // 16 bytes of every operand per thread and step (8 or 4 elements): the pass is a stream over five arrays at most and
 // has nothing else to wait for.  n is a multiple of the intermediate size, which is a multiple of 64; all pointers
 // 16-byte aligned (the launcher checks both).
@@ -286,6 +287,47 @@ __global__ __launch_bounds__(256) void act_backward_kernel(const RAW* __restrict
         for (int k = 0; k < VEC; ++k) {
             float a, b;
             act_backward_one<T16>(ld16<T16>(d.e, k), ld16<T16>(uu.e, k), ld16<T16>(gg.e, k), act, a, b);
+            oa.e[k] = st16<T16>(a);
+            ob.e[k] = st16<T16>(b);
+        }
+        reinterpret_cast<uint4*>(du)[i] = oa.q;
+        if (gated) reinterpret_cast<uint4*>(dg)[i] = ob.q;
+    }
+}
+
+// The same in place behind a data gradient of the rows that belong to an expert: du holds dh and becomes du.  Rows of no expert are
+// neither read nor written.  Behind the 256-row tiles this pass is faster than their epilogue with the derivative in it, whose
+// arithmetic (14 us a tile) the one wavefront of a SIMD hides behind nothing; behind the 128-row tile, two thirds of whose tasks share a
+// round with others, it is not.  SwiGLU, bf16, us, epilogue / pass: 256-row blocks, 16 experts of 2048 x 2048, 512 rows each 128 / 117; 4 of
+// 2048 x 2560, 4096 rows 244 / 221; 128-row blocks, 8 of 1280 x 1664, 250 rows 30 / 30; 16 of 1152 x 1920, 175 rows 32 / 34; 4 of
+// 1024 x 2560, 750 rows 30 / 36.
+template <class T16>
+__global__ __launch_bounds__(256) void act_backward_rows_kernel(const uint16_t* __restrict__ u, const uint16_t* __restrict__ g,
+                                                                const int32_t* __restrict__ count, const int32_t* __restrict__ offset,
+                                                                int E, int64_t A, int N, int act, uint16_t* du, uint16_t* __restrict__ dg) {
+    union Pack { uint4 q; uint16_t e[8]; };
+    const int64_t kept = offset[E - 1] + count[E - 1];
+    const size_t nv = (size_t)(kept < A ? kept : A) * N / 8;
+    const bool gated = act == MOE_ACT_SWIGLU;
+    const size_t i0 = (size_t)blockIdx.x * (256 * kRowsPass) + threadIdx.x;
+    Pack d[kRowsPass], uu[kRowsPass], gg[kRowsPass];
+#pragma unroll
+    for (int p = 0; p < kRowsPass; ++p) {
+        const size_t i = i0 + p * 256;
+        if (i >= nv) break;
+        d[p].q = reinterpret_cast<const uint4*>(du)[i];
+        uu[p].q = reinterpret_cast<const uint4*>(u)[i];
+        gg[p].q = gated ? reinterpret_cast<const uint4*>(g)[i] : uint4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int p = 0; p < kRowsPass; ++p) {
+        const size_t i = i0 + p * 256;
+        if (i >= nv) break;
+        Pack oa, ob;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float a, b;
+            act_backward_one<T16>(ld16<T16>(d[p].e, k), ld16<T16>(uu[p].e, k), ld16<T16>(gg[p].e, k), act, a, b);
             oa.e[k] = st16<T16>(a);
             ob.e[k] = st16<T16>(b);
         }
@@ -705,6 +747,9 @@ hipError_t launch_expert_gemm_dact(const void* dy_rows, const void* w, const voi
                                         dtype == MOE_DTYPE_FP16, st);
 }
 
+static bool overlap(const void* a, const void* b, int64_t bytes) {
+    return a && b && (uintptr_t)a < (uintptr_t)b + bytes && (uintptr_t)b < (uintptr_t)a + bytes;
+}
 // out_rows[r,:] = a_rows[r,:] . w[e(r)] with w [E, K, N] as the other direction stores it, and with u_rows the derivative behind it
 // (launch_expert_gemm_dact): no transposed copy of the weight.  16-bit layers.
 int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
@@ -715,7 +760,18 @@ hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* 
                                  const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows, void* out1_rows,
                                  hipStream_t st) {
     if (dtype == MOE_DTYPE_F32 || !stored_operands_ok(A, N, K)) return hipErrorNotSupported;
-    return launch_grouped_gemm_kn_16(a_rows, w, u_rows, g_rows, out_rows, out1_rows, count, offset, A, E, N, K, hidden_act, dtype == MOE_DTYPE_FP16, st);
+    const bool f16 = dtype == MOE_DTYPE_FP16, large = grouped_kn_large(A, E, N, K);
+    // (results on top of the saved projections: the epilogue reads those before it writes)
+    const bool in_place = u_rows && (overlap(out_rows, u_rows, A * N * 2) || overlap(out_rows, g_rows, A * N * 2) || overlap(out1_rows, u_rows, A * N * 2) ||
+                                     overlap(out1_rows, g_rows, A * N * 2));
+    if (!u_rows || !large || in_place)
+        return launch_grouped_gemm_kn_16(a_rows, w, u_rows, g_rows, out_rows, out1_rows, count, offset, large, A, E, N, K, hidden_act, f16, st);
+    const hipError_t e = launch_grouped_gemm_kn_16(a_rows, w, nullptr, nullptr, out_rows, nullptr, count, offset, large, A, E, N, K, hidden_act, f16, st);
+    if (e != hipSuccess) return e;
+    const unsigned grid = (unsigned)((A * N / 8 + 256 * kRowsPass - 1) / (256 * kRowsPass));
+    const auto pass = f16 ? &act_backward_rows_kernel<f16_s> : &act_backward_rows_kernel<bf16_s>;
+    pass<<<grid, 256, 0, st>>>((const uint16_t*)u_rows, (const uint16_t*)g_rows, count, offset, E, A, N, hidden_act, (uint16_t*)out_rows, (uint16_t*)out1_rows);
+    return hipGetLastError();
 }
 
 // dw[e] [N,K] = dy_e^T . a_e, from the rows as they are (product_choice.hpp; not where option grouped_tile asks for a tile) or from

@@ -41,19 +41,20 @@ __global__ __launch_bounds__(T::THREADS) void gemm_dense_kernel(const uint16_t* 
 // The tiles a grouped product runs on.  256: blocks of 256 rows, and of 128 where an expert has no more than that many rows left
 // (the smaller tile takes two thirds of the larger one's time at 16 slabs, three quarters at 32: tile_task_us; the other half of the
 // larger one would multiply zeros).
-template <bool F16_, int BIG_>
+// KN: the weights are stored with k as their slow index.
+template <bool F16_, int BIG_, bool KN_ = false>
 struct RowSplit {
-    static constexpr bool F16 = F16_, HAND = true;
+    static constexpr bool F16 = F16_, HAND = true, KN = KN_;
     static constexpr int BIG = BIG_, BN = 256, THREADS = 256;
-    using TB = typename std::conditional<BIG_ == 256, Tile<256, 256, 2, 2, 2, F16_>, Tile<128, 256, 1, 4, 2, F16_>>::type;
-    using TH = Tile<128, 256, 1, 4, 2, F16_>;
+    using TH = Tile<128, 256, 1, 4, 2, F16_, false, KN_>;
+    using TB = typename std::conditional<BIG_ == 256, Tile<256, 256, 2, 2, 2, F16_, false, KN_>, TH>::type;
     static constexpr int LDS_BYTES = TB::LDS_BYTES;
     static_assert(TH::LDS_BYTES <= LDS_BYTES, "one dynamic LDS block for both");
 };
 // The 128 x 128 tile of the general loop.
 template <bool F16_>
 struct PlainSplit {
-    static constexpr bool F16 = F16_, HAND = false;
+    static constexpr bool F16 = F16_, HAND = false, KN = false;
     using TB = Tile<128, 128, 2, 2, 2, F16_>;
     static constexpr int BIG = 128, BN = 128, THREADS = 256, LDS_BYTES = TB::LDS_BYTES;
 };
@@ -175,7 +176,7 @@ __device__ __forceinline__ void grouped_tile(const TaskPtrs& p, unsigned char* s
 // which hands on dU (and dG) instead of dH.  With gather and w1 the up projection of a layer.  One workgroup per tile (grouped_task).
 struct GroupedArgs {
     const uint16_t* a_rows;      // packed rows, or with gather the tokens
-    const uint16_t* w;
+    const uint16_t* w;           // [E, N, K] (KN: [E, K, N])
     const uint16_t* bias;        // or null
     const uint16_t* u_rows;      // DERIV: the saved projections ...
     const uint16_t* g_rows;      // ... and, with SwiGLU, the gate's
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
     p.b0 = a.w + (int64_t)t.expert * N * K;
     p.b1 = SWIGLU ? a.w1 + (int64_t)t.expert * N * K : nullptr;
     p.b_ld = K;
-    p.bias0 = a.bias ? a.bias + (int64_t)t.expert * N : nullptr;
+    p.bias0 = !DERIV && a.bias ? a.bias + (int64_t)t.expert * N : nullptr;
     p.bias1 = SWIGLU && a.bias1 ? a.bias1 + (int64_t)t.expert * N : nullptr;
     p.c_base = a.out + at;
     p.N = N;
@@ -219,6 +220,11 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
     p.publish = false;
     p.a_extent = a.a_bytes;
     p.b_extent = (uint32_t)((int64_t)N * K * 2);
+    if constexpr (P::KN) {
+        p.b0 += p.n0;
+        p.b_ld = N;
+        p.b_extent -= (uint32_t)p.n0 * 2;
+    }
     p.part = nullptr; p.part_cnt = nullptr; p.kparts = 1; p.kpart = 0; p.poison = false;
     p.deriv = DERIV ? 1 + a.act : 0;
     p.aux0 = DERIV ? a.u_rows + at : nullptr;
@@ -227,11 +233,10 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
     grouped_tile<P, EPI>(p, smem);
 }
 
-// ---- products whose operands may lie the other way round ----
+// ---- weight gradients from the packed rows as they lie ----
 //
-// C[i, j] = sum over k of A(i, k) B(j, k) on 128 x 128 tiles, where either operand may be stored with k as its slow index: the
-// weight as it is in a data gradient (dX = dY . W), both operands in a weight gradient (dW[e] = dY_e^T . X_e).  A transposed
-// operand is turned round on its way through the registers: a thread fetches 16 bytes of four consecutive k and writes, for each
+// C[i, j] = sum over k of A(i, k) B(j, k) on 128 x 128 tiles, both operands stored with k as the slow index (dW[e] = dY_e^T . X_e).
+// An operand is turned round on its way through the registers: a thread fetches 16 bytes of four consecutive k and writes, for each
 // of the eight i, the four values of k side by side (one byte permute a dword), so that LDS holds what it holds for the other
 // tiles and nothing else is ever written to memory.
 template <bool F16_>
@@ -246,57 +251,38 @@ struct ProdTile {
 // An operand of one tile: 128 rows i (or columns j) from `base` on.
 struct ProdOperand {
     const uint16_t* base;
-    int ld;                // elements between consecutive i (as it is) or consecutive k (transposed)
+    int ld;                // elements between consecutive k
     uint32_t extent;       // bytes from base that exist; loads behind read zeros
 };
 // LDS: 128-byte rows of 64 k, 16-byte piece c of row i at c ^ prod_swizzle(i).  The 16 rows of a fragment read meet all banks, and
 // so do eight rows that lie eight apart, which is what a transposed operand writes at a time.
 __device__ __forceinline__ int prod_swizzle(int i) { return ((i >> 1) ^ (i >> 4)) & 7; }
-template <bool TR>
 struct ProdLoads {
     uint32_t off[4];       // rows behind the operand's last one lie behind its extent, whatever the tile
     int put;
     __device__ __forceinline__ ProdLoads(int ld, int tid) {
-        if constexpr (TR) {
-            // Eight lanes in a row fetch 128 bytes in a row: the address unit takes four neighbouring lanes a cycle only where
-            // their addresses follow each other, else one (with the lanes of a row eight apart: 64 cycles a request, the unit busy
-            // 94 % of the time, 1.6 times the kernel's time).
-            const int lane = tid & 63, wave = tid >> 6;
-            const int kq = (lane >> 3) + 8 * (wave & 1), ig = (lane & 7) + 8 * (wave >> 1);
+        // Eight lanes in a row fetch 128 bytes in a row: the address unit takes four neighbouring lanes a cycle only where
+        // their addresses follow each other, else one (with the lanes of a row eight apart: 64 cycles a request, the unit busy
+        // 94 % of the time, 1.6 times the kernel's time).
+        const int lane = tid & 63, wave = tid >> 6;
+        const int kq = (lane >> 3) + 8 * (wave & 1), ig = (lane & 7) + 8 * (wave >> 1);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) off[q] = (uint32_t)((4 * kq + q) * ld + 8 * ig) * 2;
-            put = ig * 8 * kRowBytes + (((kq >> 1) ^ prod_swizzle(8 * ig)) << 4) + (kq & 1) * 8;
-        } else {
-            const int row = tid >> 3;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) off[q] = (uint32_t)((row + 32 * q) * ld + 8 * (tid & 7)) * 2;
-            put = row * kRowBytes + (((tid & 7) ^ prod_swizzle(row)) << 4);
-        }
+        for (int q = 0; q < 4; ++q) off[q] = (uint32_t)((4 * kq + q) * ld + 8 * ig) * 2;
+        put = ig * 8 * kRowBytes + (((kq >> 1) ^ prod_swizzle(8 * ig)) << 4) + (kq & 1) * 8;
     }
-    // slab s of 64 k.  Transposed: k behind the extent are zeros.
+    // slab s of 64 k; k behind the extent are zeros.
     __device__ __forceinline__ void load(const ProdOperand& o, int slab, u32x4 (&d)[4]) const {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(o.base), 0, (int)o.extent, 0x00020000);
-        if constexpr (TR) {
-            const uint32_t k = (uint32_t)(slab * kBK) * o.ld * 2;
+        const uint32_t k = (uint32_t)(slab * kBK) * o.ld * 2;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) d[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off[q] + k), 0, 0));
-        } else {
-            const int k = slab * kRowBytes;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) d[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[q], k, 0));
-        }
+        for (int q = 0; q < 4; ++q) d[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off[q] + k), 0, 0));
     }
     __device__ __forceinline__ void store(const u32x4 (&d)[4], unsigned char* st) const {
-        if constexpr (TR) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {      // row i = 8 ig + j: its swizzle differs from that of 8 ig by j >> 1
-                const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-                const u32x2 v = {__builtin_amdgcn_perm(d[1][j >> 1], d[0][j >> 1], sel), __builtin_amdgcn_perm(d[3][j >> 1], d[2][j >> 1], sel)};
-                *reinterpret_cast<u32x2*>(st + ((put ^ ((j >> 1) << 4)) + j * kRowBytes)) = v;
-            }
-        } else {                               // row + 32 q: by 2 q
-#pragma unroll
-            for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(st + ((put ^ (q << 5)) + q * 32 * kRowBytes)) = d[q];
+        for (int j = 0; j < 8; ++j) {      // row i = 8 ig + j: its swizzle differs from that of 8 ig by j >> 1
+            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+            const u32x2 v = {__builtin_amdgcn_perm(d[1][j >> 1], d[0][j >> 1], sel), __builtin_amdgcn_perm(d[3][j >> 1], d[2][j >> 1], sel)};
+            *reinterpret_cast<u32x2*>(st + ((put ^ ((j >> 1) << 4)) + j * kRowBytes)) = v;
         }
     }
 };
@@ -320,14 +306,14 @@ struct ProdJob {
 // gradient of 4 x 2048 x 2560), 0.65 with 512 (of 16 x 2048 x 2048).  (Workgroups that stay and
 // request the next tile's first slabs under this one's last: no faster, what they save at the ends of tiles they lose in the
 // last round of an uneven number of tiles.)
-template <class T, bool TA, bool TB>
+template <class T>
 __device__ __forceinline__ void prod_slabs(const ProdJob& job, unsigned char* smem, f32x4 (&acc)[T::TM][T::TN]) {
     constexpr int D = 2;                       // slabs on their way in registers
     typedef typename std::conditional<T::F16, f16x8, bf16x8>::type frag_t;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / T::WN, wn = wave % T::WN;
-    const ProdLoads<TA> la(job.a.ld, tid);
-    const ProdLoads<TB> lb(job.b.ld, tid);
+    const ProdLoads la(job.a.ld, tid);
+    const ProdLoads lb(job.b.ld, tid);
     const int slabs = job.slabs;
     const int frow = lane & 15, fk = lane >> 4, sw = (frow >> 1) & 7;
     int get_a[T::TM], get_b[T::TN];            // this lane's pieces of k half 0; those of half 1 lie 64 bytes up or down
@@ -395,13 +381,13 @@ __device__ __forceinline__ void prod_slabs(const ProdJob& job, unsigned char* sm
     if (slab < slabs) step(std::integral_constant<int, 0>{}, slab);
 }
 // Tiles: job(id, j) the operands of tile `id` (false: no such tile), finish(id, acc, smem) its epilogue.
-template <class T, bool TA, bool TB, class Tiles>
+template <class T, class Tiles>
 __device__ __forceinline__ void prod_tile(const Tiles& tiles, unsigned char* smem) {
     ProdJob job;
     if (!tiles.job(blockIdx.x, job)) return;
     job = ProdJob{prod_uniform(job.a), prod_uniform(job.b), __builtin_amdgcn_readfirstlane(job.slabs)};
     f32x4 acc[T::TM][T::TN];
-    prod_slabs<T, TA, TB>(job, smem, acc);
+    prod_slabs<T>(job, smem, acc);
     tiles.finish(blockIdx.x, acc, smem);
 }
 
@@ -456,44 +442,7 @@ struct WgradTiles {
 template <class T>
 __global__ __launch_bounds__(T::THREADS, 2) void wgrad_rows_kernel(WgradTiles<T> tiles) {
     extern __shared__ __align__(16) unsigned char smem[];
-    prod_tile<T, true, true>(tiles, smem);
-}
-
-// A grouped product with the weight as it is stored for the other direction: out[r, :] = a[r, :] . w[e(r)], w [E, K, N].
-template <class T, int EPI>
-struct GroupedTiles {
-    GroupedArgs g;
-    __device__ __forceinline__ bool place(int id, GroupedTask& t) const {
-        return grouped_task<T::BM>(g.count, g.offset, g.E, (g.N + T::BN - 1) / T::BN, id, t);
-    }
-    __device__ __forceinline__ bool job(int id, ProdJob& j) const {
-        GroupedTask t;
-        if (!place(id, t)) return false;
-        const int n0 = t.ctile * T::BN;
-        const uint16_t* w = g.w + (int64_t)t.expert * g.N * g.K;
-        j.a = ProdOperand{g.a_rows + (int64_t)t.row0 * g.K, g.K, (uint32_t)((int64_t)t.rows * g.K * 2)};
-        j.b = ProdOperand{w + n0, g.N, (uint32_t)(((int64_t)g.K * g.N - n0) * 2)};
-        j.slabs = g.K / kBK;
-        return true;
-    }
-    __device__ __forceinline__ void finish(int id, f32x4 (&acc)[T::TM][T::TN], unsigned char* smem) const {
-        GroupedTask t;
-        place(id, t);
-        const int64_t at = (int64_t)t.row0 * g.N;
-        TaskPtrs p = prod_epilogue(g.out + at, g.N, t.ctile * T::BN, t.rows);
-        if constexpr (EPI == kDeriv) {
-            p.deriv = 1 + g.act;
-            p.aux0 = g.u_rows + at;
-            p.aux1 = g.g_rows ? g.g_rows + at : nullptr;
-            p.c1_base = g.out1 ? g.out1 + at : nullptr;
-        }
-        grouped_epilogue<T, EPI>(p, smem, acc);
-    }
-};
-template <class T, int EPI>
-__global__ __launch_bounds__(T::THREADS, 2) void grouped_kn_kernel(GroupedArgs g) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    prod_tile<T, false, true>(GroupedTiles<T, EPI>{g}, smem);
+    prod_tile<T>(tiles, smem);
 }
 
 // Weight gradient of one projection: dw[e] [N, K] = dy_e^T . a_e, the sum running over the rows of expert e.  Both
@@ -682,23 +631,17 @@ hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const i
 }
 
 template <bool F16, int EPI>
-static hipError_t launch_grouped_kn(const GroupedArgs& g, int64_t A, hipStream_t st) {
-    using T = ProdTile<F16>;
-    hipError_t e = allow_lds(&grouped_kn_kernel<T, EPI>, T::LDS_BYTES);
-    if (e != hipSuccess) return e;
-    const int64_t tiles = (A / T::BM + g.E) * ((g.N + T::BN - 1) / T::BN) + kShareSlack;
-    if (tiles > INT32_MAX) return hipErrorInvalidValue;
-    grouped_kn_kernel<T, EPI><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(g);
-    return hipGetLastError();
+static hipError_t launch_grouped_kn(const GroupedArgs& g, bool large, int64_t A, hipStream_t st) {
+    return large ? launch_grouped<RowSplit<F16, 256, true>, EPI>(g, A, st) : launch_grouped<RowSplit<F16, 128, true>, EPI>(g, A, st);
 }
-// out = a . w[e], or, with u, du (and dg) = (a . w[e]) * act'(u, g).
+// out = a . w[e], or, with u, du (and dg) = (a . w[e]) * act'(u, g); large: on 256-row blocks and remainders.
 hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
-                                     const int32_t* count, const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, bool f16,
+                                     const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)out,
-                        (uint16_t*)out1, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
-    if (u) return f16 ? launch_grouped_kn<true, kDeriv>(g, A, st) : launch_grouped_kn<false, kDeriv>(g, A, st);
-    return f16 ? launch_grouped_kn<true, kSums>(g, A, st) : launch_grouped_kn<false, kSums>(g, A, st);
+                        (uint16_t*)out1, count, offset, E, N, K, u ? hidden_act : MOE_ACT_NONE, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
+    if (u) return f16 ? launch_grouped_kn<true, kDeriv>(g, large, A, st) : launch_grouped_kn<false, kDeriv>(g, large, A, st);
+    return f16 ? launch_grouped_kn<true, kSums>(g, large, A, st) : launch_grouped_kn<false, kSums>(g, large, A, st);
 }
 
 }  // namespace moe355

@@ -44,10 +44,11 @@ constexpr int kRowBytes = kBK * 2;
 
 // F16: operands and results are IEEE binary16 (torch_dtype 3) instead of bfloat16; same tile, same loops, the other
 // MFMA instruction and the other conversions.
-template <int BM_, int BN_, int WM_, int WN_, int NS_, bool F16_ = false>
+// TRA, TRB: the token / weight operand is stored with k as its slow index (hand-ordered tiles only; ring_load_one).
+template <int BM_, int BN_, int WM_, int WN_, int NS_, bool F16_ = false, bool TRA_ = false, bool TRB_ = false>
 struct Tile {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_;
-    static constexpr bool F16 = F16_;
+    static constexpr bool F16 = F16_, TRA = TRA_, TRB = TRB_;
     static constexpr int THREADS = WM * WN * kWave;
     static constexpr int TM = BM / WM / 16;       // 16x16 MFMA tiles per wavefront along tokens
     static constexpr int TN = BN / WN / 16;       // ... along weight rows
@@ -69,6 +70,8 @@ struct Tile {
     static_assert(TM >= 2 && TM % 2 == 0 && TN >= 2 && TN % 2 == 0, "a wavefront's tile is split in token halves; SwiGLU pairs weight-row halves");
     static_assert(RA >= 1 && RB >= 1, "tile too small for the workgroup");
     static_assert(NS == 2, "two LDS stages");
+    static_assert(HAND || !(TRA || TRB), "operands with k as their slow index: the hand-ordered tiles");
+    static_assert(TRB || !TRA, "slab orders exist for the weights alone or both operands");
 };
 
 // What one task needs, resolved to pointers.
@@ -449,23 +452,33 @@ __device__ __forceinline__ void epilogue_full_n_impl(const TaskPtrs& p, unsigned
     const uint32_t lane_off = (uint32_t)(rd_row * p.N + col0 + rd_chunk * 8);   // elements from the uniform row pointer
     const bool publish = p.publish;
     constexpr int NQ = 16 / ROWS_PER_PASS;
+    // (DERIV) the saved projections, requested kAhead row groups in front of the one that uses them: nothing else in flight on the
+    // SIMD hides their way from memory.  Against requests at the top of their own group, a SwiGLU data gradient on the 128 x 256
+    // tile: 16 experts of 2048 x 2048, 512 rows each 148 -> 137 us; of 2048 x 1408, 750 rows 131 -> 119; 16 of 1152 x 1920, 175 rows 33.8 -> 31.6.
+    constexpr int kAhead = T::RING ? 3 : 2;
+    u32x4 saved_u[DERIV ? kAhead + 1 : 1][NQ], saved_g[DERIV ? kAhead + 1 : 1][NQ];
+    auto saved_rows = [&](int i) {
+        if (i >= T::TM) return;
+        const int64_t group = (int64_t)(wm * 16 * T::TM + i * 16) * p.N;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            u32x4 &u = saved_u[i % (kAhead + 1)][q], &g = saved_g[i % (kAhead + 1)][q];
+            u = g = u32x4{0u, 0u, 0u, 0u};
+            if (i * 16 + q * ROWS_PER_PASS < rows_left) {
+                const int64_t at = group + (int64_t)(q * ROWS_PER_PASS) * p.N + lane_off;
+                u = *reinterpret_cast<const u32x4*>(p.aux0 + at);
+                if (p.deriv == 1 + MOE_ACT_SWIGLU) g = *reinterpret_cast<const u32x4*>(p.aux1 + at);
+            }
+        }
+    };
+    if constexpr (DERIV) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) saved_rows(i);
+    }
 #pragma unroll
     for (int i = 0; i < T::TM; ++i) {
         between(i);
-        // (DERIV) the saved projections of this row group's rows: requested here, used behind the staging round trip
-        u32x4 uu[DERIV ? NQ : 1], gg[DERIV ? NQ : 1];
-        if constexpr (DERIV) {
-            const int64_t group = (int64_t)(wm * 16 * T::TM + i * 16) * p.N;
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                uu[q] = gg[q] = u32x4{0u, 0u, 0u, 0u};
-                if (i * 16 + q * ROWS_PER_PASS < rows_left) {
-                    const int64_t at = group + (int64_t)(q * ROWS_PER_PASS) * p.N + lane_off;
-                    uu[q] = *reinterpret_cast<const u32x4*>(p.aux0 + at);
-                    if (p.deriv == 1 + MOE_ACT_SWIGLU) gg[q] = *reinterpret_cast<const u32x4*>(p.aux1 + at);
-                }
-            }
-        }
+        if constexpr (DERIV) saved_rows(i + kAhead);
         // Partial sums: the row group's sums of the other parts come back from memory (written through by their tasks,
         // read past this XCD's L2) and are added here -- two parts: own registers + the other part, which is the same
         // in either order; four parts: all four as stored, in the order of the parts, whichever of them runs this.
@@ -529,10 +542,11 @@ __device__ __forceinline__ void epilogue_full_n_impl(const TaskPtrs& p, unsigned
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     const float d0 = widen1<T>((uint16_t)(v[q][w] & 0xFFFFu)), d1 = widen1<T>((uint16_t)(v[q][w] >> 16));
-                    const float u0 = widen1<T>((uint16_t)(uu[q][w] & 0xFFFFu)), u1 = widen1<T>((uint16_t)(uu[q][w] >> 16));
+                    const u32x4 uu = saved_u[i % (kAhead + 1)][q], gg = saved_g[i % (kAhead + 1)][q];
+                    const float u0 = widen1<T>((uint16_t)(uu[w] & 0xFFFFu)), u1 = widen1<T>((uint16_t)(uu[w] >> 16));
                     float a0, a1, b0v = 0.0f, b1v = 0.0f;
                     if (gated) {
-                        const float g0 = widen1<T>((uint16_t)(gg[q][w] & 0xFFFFu)), g1 = widen1<T>((uint16_t)(gg[q][w] >> 16));
+                        const float g0 = widen1<T>((uint16_t)(gg[w] & 0xFFFFu)), g1 = widen1<T>((uint16_t)(gg[w] >> 16));
                         dswiglu16(d0, u0, g0, a0, b0v);
                         dswiglu16(d1, u1, g1, a1, b1v);
                     } else if (p.deriv == 1 + MOE_ACT_GELU) {
@@ -578,9 +592,35 @@ struct RingLoads {
     const void* base_b0;
     const void* base_b1;
     uint32_t a_extent, b_extent;
+    uint32_t a_slab, b_slab;         // TRA, TRB: bytes of a slab's 64 k
     int KT;                          // slabs of 64, >= 1
     int wrow;                        // first of the eight consecutive stage rows this wavefront's loads fill per pass
 };
+
+// Operands with k as their slow index (TRA, TRB).  A slab is 64 rows of k, each as long as the tile is wide (W elements), and goes
+// into the stage as it lies in memory.  What turns it round is the fragment read: ds_read_b64_tr_b16 gives lane i of sixteen the
+// i-th column of the 4 x 16 block whose rows its groups of four lanes address, so two of them make the eight k of a lane's
+// operand, the same k in the same places as from an operand stored the other way: same bits.  (Turning the operand in registers on
+// its way to LDS, 128 x 128 tiles on two workgroups a compute unit: ProdTile, ffn_bf16_grouped.hip.)
+// A wavefront's read meets rows of k that lie a multiple of 256 bytes apart, eight at a time; the 32-byte pieces of a row are
+// therefore permuted within every eight, by turned_swizzle, on the global side of the loads and in the addresses of the reads.
+__device__ __forceinline__ int turned_swizzle(int k) { return (k & 3) | ((k >> 1) & 4); }
+// Byte offsets of this thread's loads of a slab, from its first row of k on: load n of a wavefront fills 1 KiB of the stage.
+template <int W>
+__device__ __forceinline__ void turned_offsets(int ld, int tid, unsigned (&voff)[8]) {
+    constexpr int PITCH = W * 2;
+#pragma unroll
+    for (int n = 0; n < W / 32; ++n) {
+        const int at = n * 4096 + tid * 16, k = at / PITCH, piece = at % PITCH / 32;
+        voff[n] = (unsigned)(k * ld * 2 + (piece ^ turned_swizzle(k)) * 32 + (at & 16));
+    }
+}
+// This lane's place in the stage for its fragment `f` (sixteen columns) of k 0..31; the second four of its k lie 4 rows on.
+template <int W>
+__device__ __forceinline__ unsigned turned_fragment(int f, int lane) {
+    const int k = 8 * (lane >> 4) + ((lane >> 2) & 3);
+    return (unsigned)(k * (W * 2) + (f ^ turned_swizzle(k)) * 32 + (lane & 3) * 8);
+}
 
 // The part of a task's load state that needs no memory access: weight-row offsets, bases, extents.
 template <class T>
@@ -595,8 +635,9 @@ __device__ __forceinline__ RingLoads ring_prepare_weights(const TaskPtrs& p) {
     RingLoads L;
 #pragma unroll
     for (int n = 0; n < 8; ++n) L.voff_a[n] = L.voff_b[n] = p.a_extent;
+    if constexpr (T::TRB) turned_offsets<T::BN>(p.b_ld, tid, L.voff_b);
 #pragma unroll
-    for (int n = 0; n < T::RB; ++n) {
+    for (int n = 0; n < (T::TRB ? 0 : T::RB); ++n) {
         // SwiGLU: a wavefront's weight rows are the gate rows of its output columns followed by their up rows
         const int j = prow + n * T::ROWS_PER_PASS;
         const int col = p.swiglu ? p.n0 + (j / T::WB) * (T::WB / 2) + (j % (T::WB / 2)) : p.n0 + j;
@@ -615,6 +656,8 @@ __device__ __forceinline__ RingLoads ring_prepare_weights(const TaskPtrs& p) {
     L.base_b1 = uniform(p.swiglu ? p.b1 : p.b0);
     L.a_extent = p.a_extent;
     L.b_extent = p.b_extent;
+    L.a_slab = T::TRA ? (uint32_t)p.a_ld * kRowBytes : 0u;
+    L.b_slab = T::TRB ? (uint32_t)p.b_ld * kRowBytes : 0u;
     L.KT = p.K / kBK;
     L.wrow = __builtin_amdgcn_readfirstlane(prow & ~7);
     return L;
@@ -627,6 +670,10 @@ __device__ __forceinline__ void ring_prepare_tokens(const TaskPtrs& p, RingLoads
     asm volatile("" : "+v"(tid));
     const int prow = tid >> 3;
     const int chunk = (tid & 7) ^ ((prow >> 1) & 7);
+    if constexpr (T::TRA) {
+        turned_offsets<T::BM>(p.a_ld, tid, L.voff_a);
+        return;
+    }
 #pragma unroll
     for (int n = 0; n < T::RA; ++n) {
         // Padding rows are never stored.  Their loads are aimed behind the end of the buffer, which the hardware
@@ -654,7 +701,16 @@ __device__ __forceinline__ void ring_load_one(const RingLoads& L, unsigned char*
     unsigned char* base = smem + (slab & 1) * T::STAGE_BYTES;
     const int soff = slab * kRowBytes;
     const bool live = slab < L.KT;
-    if (n < T::RA) {
+    if (n < T::RA ? T::TRA : T::TRB) {
+        // the slab's rows of k: a buffer that begins at them and ends where the operand ends (rows behind it are zeros)
+        const bool a = n < T::RA;
+        const uint32_t at = (uint32_t)slab * (a ? L.a_slab : L.b_slab), extent = a ? L.a_extent : L.b_extent;
+        char* first = (char*)const_cast<void*>(a ? L.base_a : L.base_b0) + at;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)first, 0, live && at < extent ? (int)(extent - at) : 0, 0x00020000);
+        const unsigned voff = a ? L.voff_a[n & 7] : L.voff_b[(n - T::RA) & 7];
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(base + (a ? 0 : T::BM * kRowBytes) + (wrow + (a ? n : n - T::RA) * T::ROWS_PER_PASS) * kRowBytes),
+                                                 16, voff, 0, 0, 0);
+    } else if (n < T::RA) {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(L.base_a), 0, live ? (int)L.a_extent : 0, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(base + (wrow + n * T::ROWS_PER_PASS) * kRowBytes), 16,
                                                  L.voff_a[n], soff, 0, 0);
@@ -724,6 +780,7 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
         };
         U.base_a = unip(L.base_a); U.base_b0 = unip(L.base_b0); U.base_b1 = unip(L.base_b1);
         U.a_extent = uni(L.a_extent); U.b_extent = uni(L.b_extent);
+        U.a_slab = uni(L.a_slab); U.b_slab = uni(L.b_slab);
         U.KT = (int)uni((unsigned)L.KT); U.wrow = (int)uni((unsigned)L.wrow);
     }
     const int KT = U.KT;                        // an odd one runs one slab more, on the zeros that its loads fetch
@@ -744,16 +801,41 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
     const unsigned c0 = (unsigned)((fk ^ sw) << 4), c1 = (unsigned)(((4 + fk) ^ sw) << 4);
     const unsigned la0[2] = {a_row + c0, a_row + c1}, lb0[2] = {b_row + c0, b_row + c1};
     const unsigned la1[2] = {la0[0] + STAGE, la0[1] + STAGE}, lb1[2] = {lb0[0] + STAGE, lb0[1] + STAGE};
+    // ... and of its turned fragments: [stage][fragment], both k halves within the offset field's reach
+    unsigned lat[2][8], lbt[2][TN];
+    if constexpr (T::TRA) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) lat[1][i] = (lat[0][i] = lds0 + turned_fragment<BM>(wm * 8 + i, lane)) + STAGE;
+    }
+    if constexpr (T::TRB) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) lbt[1][j] = (lbt[0][j] = lds0 + BM * kRowBytes + turned_fragment<T::BN>(wn * TN + j, lane)) + STAGE;
+    }
     bf16x8 af[2][8], bfr[2][TN];
     int kt = 0;
 
+#define TURNED(frag, at, pitch, half)                                                                                     \
+    do {                                                                                                                 \
+        u32x2 lo_, hi_;                                                                                                  \
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo_) : "v"(at), "n"((half) * 32 * (pitch)));           \
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi_) : "v"(at), "n"((half) * 32 * (pitch) + 4 * (pitch))); \
+        frag = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo_, hi_, 0, 1, 2, 3));                                \
+    } while (0)
 #define MF(i, j, s)                                                                                                      \
     do {                                                                                                                 \
         if constexpr (T::F16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(bfr[s][j]), "v"(af[s][i])); \
         else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(bfr[s][j]), "v"(af[s][i]));                  \
     } while (0)
-#define RA(stg, half, idx) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(af[half][idx]) : "v"((stg) ? la1[half] : la0[half]), "n"((idx) * 16 * kRowBytes))
-#define RB(stg, half, j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(bfr[half][j]) : "v"((stg) ? lb1[half] : lb0[half]), "n"((j) * 16 * kRowBytes))
+#define RA(stg, half, idx)                                                                                               \
+    do {                                                                                                                 \
+        if constexpr (T::TRA) TURNED(af[half][idx], lat[stg][idx], BM * 2, half);                                        \
+        else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(af[half][idx]) : "v"((stg) ? la1[half] : la0[half]), "n"((idx) * 16 * kRowBytes)); \
+    } while (0)
+#define RB(stg, half, j)                                                                                                 \
+    do {                                                                                                                 \
+        if constexpr (T::TRB) TURNED(bfr[half][j], lbt[stg][j], T::BN * 2, half);                                        \
+        else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(bfr[half][j]) : "v"((stg) ? lb1[half] : lb0[half]), "n"((j) * 16 * kRowBytes)); \
+    } while (0)
 #define WL(n) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(n))
 #define BAR1 do { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); } while (0)
 #define BAR2(n) do { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory"); __builtin_amdgcn_s_barrier(); } while (0)
@@ -783,21 +865,13 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
             {
                 constexpr unsigned st = 0, sn = 1;
                 (void)st; (void)sn;
-                if constexpr (TN == 8) {
-#include "ffn_bf16_slab_steady.inc"
-                } else {
-#include "ffn_bf16_slab_half.inc"
-                }
+#include "ffn_bf16_slab.inc"
             }
             ++kt;
             {
                 constexpr unsigned st = 1, sn = 0;
                 (void)st; (void)sn;
-                if constexpr (TN == 8) {
-#include "ffn_bf16_slab_steady.inc"
-                } else {
-#include "ffn_bf16_slab_half.inc"
-                }
+#include "ffn_bf16_slab.inc"
             }
             --kt;
         }
@@ -823,20 +897,12 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
     for (; kt < KT; kt += 2) {
         {
             constexpr unsigned st = 0, sn = 1;
-                if constexpr (TN == 8) {
-#include "ffn_bf16_slab_steady.inc"
-                } else {
-#include "ffn_bf16_slab_half.inc"
-                }
+#include "ffn_bf16_slab.inc"
         }
         ++kt;
         {
             constexpr unsigned st = 1, sn = 0;
-                if constexpr (TN == 8) {
-#include "ffn_bf16_slab_steady.inc"
-                } else {
-#include "ffn_bf16_slab_half.inc"
-                }
+#include "ffn_bf16_slab.inc"
         }
         --kt;
     }
@@ -860,6 +926,7 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
 #undef BAR2
 #undef GL
 #undef TAIL
+#undef TURNED
     return true;
 }
 

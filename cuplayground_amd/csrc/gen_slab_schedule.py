@@ -41,6 +41,17 @@ BAR2_ROW = 13                         # MFMA row in front of which the next slab
 HALF = dict(nb=4, bar1=7, per_row=[3, 3, 2, 2, 2, 0, 0, 0], bar2=11, next_per_row=[3, 3, 2, 2, 2])
 FULL = dict(nb=8, bar1=BAR1_ROW, per_row=PER_ROW, bar2=BAR2_ROW, next_per_row=[6, 6, 4])
 
+# Operands stored with k as their slow index: a fragment is two transposing reads of four k each instead of one read of
+# eight, so that the waits count twice as many.  "kn": the weights (a data gradient), "rows": both operands (a weight gradient).
+SHAPES = {
+    "steady": FULL,
+    "half": HALF,
+    "steady_kn": dict(FULL, rb=2),
+    "half_kn": dict(HALF, rb=2),
+    "steady_rows": dict(FULL, ra=2, rb=2),
+    "half_rows": dict(HALF, ra=2, rb=2),
+}
+
 
 def build(variant, shape=FULL):
     nb, bar1, bar2 = shape["nb"], shape["bar1"], shape["bar2"]
@@ -91,15 +102,16 @@ def build(variant, shape=FULL):
 def emit(variant, shape=FULL):
     steady, cur = build("steady", shape), build(variant, shape)
     issued, last = 0, {}
+    reads = {"RA": shape.get("ra", 1), "RB": shape.get("rb", 1)}     # LDS reads a fragment
 
     def run(seq, out):
         nonlocal issued
         for op in seq:
             if op[0] == "RA":
-                issued += 1
+                issued += reads["RA"]
                 last[("a", op[2], op[3])] = issued
             elif op[0] == "RB":
-                issued += 1
+                issued += reads["RB"]
                 last[("b", op[2], op[3])] = issued
             if out is None:
                 continue
@@ -114,7 +126,7 @@ def emit(variant, shape=FULL):
     lines, prev, since = [], None, 0
     for op in out:
         if op[0] in ("RA", "RB"):
-            since += 1
+            since += reads[op[0]]
         if op[0] == "WL":
             if prev is not None and op[1] >= prev + since:
                 continue       # already implied by the previous wait
@@ -139,6 +151,6 @@ def emit(variant, shape=FULL):
 
 if __name__ == "__main__":
     here = os.path.dirname(os.path.abspath(__file__))
-    for name, shape in (("steady", FULL), ("half", HALF)):
+    for name, shape in SHAPES.items():
         with open(os.path.join(here, "ffn_bf16_slab_%s.inc" % name), "w") as f:
             f.write("// generated by gen_slab_schedule.py -- do not edit\n" + emit("steady", shape))

@@ -1,5 +1,5 @@
-// Whether a 16-bit training product takes operands as they are stored (the 128 x 128 tiles of ffn_bf16_grouped.hip that turn them round on
-// the way) or transposed copies of them and the larger tiles.  Either way gives the same bits.  Host arithmetic only, so that a host
+// Whether a 16-bit weight gradient takes its operands as they are stored (the 128 x 128 tiles of ffn_bf16_grouped.hip that turn them round on
+// the way) or transposed copies of them and the larger tiles, and which tile a data gradient takes.  Either way gives the same bits.  Host arithmetic only, so that a host
 // program can test it.  Estimates of either, us; constants and checks are measurements of whole calls (transposes and launches included,
 // bf16, one card):
 //   hand-ordered 256 x 256 tile: 1.3 us a slab of 64 and 8 us a task, rounds of 256 tasks and half a one; transposes at 4.5 TB/s read and
@@ -7,6 +7,8 @@
 #pragma once
 #include <algorithm>
 #include <cstdint>
+
+#include "two_launches.hpp"
 
 namespace moe355 {
 
@@ -43,12 +45,17 @@ inline bool wgrad_as_stored(int64_t A, int E, int N, int K) {
     return stored_us((double)E * ((N + 127) / 128) * ((K + 127) / 128), rows / 64 + 0.5) <
            transposed_us((double)E * columns256(N) * columns256(K), rows / 64 + 1.0, 2.0 * A * (N + K));
 }
-// Data gradient [A, N] from rows of K and the weight [E, K, N].
-inline bool grouped_kn_as_stored(int64_t A, int E, int N, int K) {
-    if (!stored_operands_ok(A, N, K)) return false;
-    const double rows = (double)A / std::max(E, 1);
-    const double blocks = E * (rows <= 96 ? 1.0 : rows / 128 + 0.5), big = E * (rows <= 192 ? 1.0 : rows / 256 + 0.25);
-    return stored_us(blocks * ((N + 127) / 128), K / 64.0) < transposed_us(big * columns256(N), K / 64.0, 2.0 * E * N * K);
+// Data gradient [A, N] from rows of K and the weight [E, K, N]: as stored wherever the offsets allow it -- the transposing fragment reads
+// (ffn_bf16_tile.hpp) run at the rate of the plain ones, and the transposed copy costs what it moves.
+inline bool grouped_kn_as_stored(int64_t A, int, int N, int K) { return stored_operands_ok(A, N, K); }
+// ... on 256-row blocks and remainders, or on 128-row blocks: the shorter by the estimate of a layer's launches (two_launches.hpp).
+// us, 256 / 128: 16 experts of 2048 x 2048, 512 rows each 81 / 86; of 1408 x 2048, 750 rows 77 / 90; 4 of 2560 x 2048, 4096 rows 133 / 157; 8 of
+// 1664 x 1280, 250 rows 40 / 25; 16 of 1920 x 1152, 175 rows 45 / 28; 8 of 2560 x 1024, 750 rows 59 / 40; 4 of them 55 / 34; 8 of 1536 x
+// 1920, 500 rows 41 / 46 (the 128 x 128 tiles that turned the operand round in registers: 107, 107, 230, 27, 41, 56, 37, 38).
+inline bool grouped_kn_large(int64_t A, int E, int N, int K) {
+    const SplitBlocks n(A, std::max(E, 1));
+    const double cols = columns256(N);
+    return split_us(n.full * cols, n.left * cols, K) < split_us(0, n.small * cols, K);
 }
 
 }  // namespace moe355

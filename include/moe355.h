@@ -434,8 +434,8 @@ int moe_expert_gemm_act_backward(moe_handle* h, const void* dy_rows, const void*
  * a projection's data gradient without a transposed copy of its weight; with u_rows (and, for a SwiGLU layer, g_rows and
  * out1_rows) what moe_expert_gemm_act_backward gives, N = intermediate_size and K = hidden_size.  The sums run in the same order of
  * k as in moe_expert_gemm: the same bits as behind moe_transpose.  *supported: 0 = no such kernel for this layer (fp32, operands of
- * 4 GiB and more), 1 = it exists, 2 = and is expected to be faster than a transpose and the k-contiguous product (few rows per
- * expert, small matrices; option grouped_tile asks for the latter).  Every pointer 16-byte aligned.  No scratch. */
+ * 4 GiB and more), 1 = it exists, 2 = and is expected to be faster than a transpose and the k-contiguous product (unless option
+ * grouped_tile asks for the latter).  Every pointer 16-byte aligned.  No scratch. */
 int moe_expert_gemm_kn_supported(const moe_handle* h, int32_t N, int32_t K, int32_t* supported);
 int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const void* u_rows, const void* g_rows,
                        const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K, void* out_rows,

@@ -1,0 +1,46 @@
+"""Products on operands as stored, on the hand-ordered tiles: row blocks of 256 and their remainders, of 128, ragged columns and odd slab
+counts, an expert without rows; the same bits as with a transposed copy of the weight.  (The fourth and fifth shape take 256-row blocks for one of the two gradients: grouped_kn_large.)"""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from oracle import binding as ob
+from helpers import product_config, to_device
+from test_gpu_backward import KIND, moe, routed_case  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [ob.BF16, ob.F16])
+@pytest.mark.parametrize("shape", [(1, 64, 64, 2, 1), (520, 576, 320, 2, 1), (1100, 2112, 448, 2, 2), (1900, 2112, 1088, 8, 2), (2000, 1152, 2112, 8, 2), (400, 320, 1088, 70, 2)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_data_gradients_on_weights_as_stored(moe, dtype, shape, gated):
+    import torch
+    import cuplayground_amd.api as api
+    S, H, I, E, k = shape
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=S, drop=0, skew=0.3)
+    if gated:
+        cfg = dataclasses.replace(cfg, act=ob.ACT_SWIGLU)
+    R = int(count.sum())
+    layer = moe.MoELayer(product_config(cfg))
+    assert layer.gemm_kn_supported(H, I) == 2 and layer.gemm_kn_supported(I, H) == 2
+    dev = lambda *s: to_device(ob.from_f32((rng.standard_normal(s) * 0.3).astype(np.float32), dtype), KIND[dtype])
+    dcount, doff = to_device(count, "i32"), to_device(offset, "i32")
+    rows = {n: dev(S * k, n) for n in (H, I)}
+    u, g = dev(S * k, I), dev(S * k, I)
+    for t in (rows[H], rows[I]):
+        t[R:] = float("nan")                     # rows of no expert must not reach a result
+    w_up, w_down = dev(E, I, H), dev(E, H, I)
+    da = layer.expert_gemm_kn(rows[I], w_up, dcount, doff)
+    assert torch.equal(da[:R], layer.expert_gemm(rows[I], api.transpose(w_up), None, dcount, doff, api.ACT_NONE)[:R])
+    dh = layer.expert_gemm(rows[H], api.transpose(w_down), None, dcount, doff, api.ACT_NONE)
+    want = layer.act_backward(dh, u, g if gated else None)
+    du, dg = layer.expert_gemm_kn(rows[H], w_down, dcount, doff, u, g if gated else None)
+    assert torch.equal(du[:R], want[0][:R]) and (not gated or torch.equal(dg[:R], want[1][:R]))
+    # results in the place of the saved projections, as a caller short of memory may have them
+    out = [u.clone(), g.clone()]
+    rc = layer.L.moe_expert_gemm_kn(layer._h, api._ptr(rows[H]), api._ptr(w_down), api._ptr(out[0]), api._ptr(out[1] if gated else None), api._ptr(dcount),
+                                    api._ptr(doff), I, H, api._ptr(out[0]), api._ptr(out[1] if gated else None), api._stream())
+    assert rc == 0 and torch.equal(out[0][:R], want[0][:R]) and (not gated or torch.equal(out[1][:R], want[1][:R]))
+    assert torch.equal(out[0][R:], u[R:])        # rows of no expert stay as they are

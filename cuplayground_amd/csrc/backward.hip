@@ -28,7 +28,7 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
 hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
                                      const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st);
-hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K,
+hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K,
                                 bool f16, hipStream_t st);
 hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* du, void* dg,
                                         const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
@@ -780,8 +780,8 @@ hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const in
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st) {
     const bool aligned = ((uintptr_t)dy_rows | (uintptr_t)a_rows | (uintptr_t)dw) % 16 == 0;
-    if (dtype != MOE_DTYPE_F32 && aligned && opt.grouped_tile == MOE_OPT_AUTO && wgrad_as_stored(A, E, N, K))
-        return launch_wgrad_rows_16(dy_rows, a_rows, dw, count, offset, E, N, K, dtype == MOE_DTYPE_FP16, st);
+    if (dtype != MOE_DTYPE_F32 && aligned && opt.grouped_tile == MOE_OPT_AUTO && stored_operands_ok(A, N, K))
+        return launch_wgrad_rows_16(dy_rows, a_rows, dw, count, offset, wgrad_large(A, E, N, K), E, N, K, dtype == MOE_DTYPE_FP16, st);
     const ScratchTables t = scratch_tables(scratch, A, E);
     const int64_t ld = wgrad_ld(A, E);
     const size_t eb = dtype == MOE_DTYPE_F32 ? 4 : 2;

@@ -242,7 +242,7 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
 template <bool F16_>
 struct ProdTile {
     static constexpr int BM = 128, BN = 128, WM = 2, WN = 2, NS = 2, THREADS = 256, TM = 4, TN = 4, WB = 64;
-    static constexpr bool F16 = F16_, RING = false, HALF = false, HAND = true;
+    static constexpr bool F16 = F16_, RING = false, HALF = false, HAND = true, TRA = false;
     static constexpr int STAGE_BYTES = (BM + BN) * kRowBytes;
     static constexpr int STAGING_BYTES = 4 * 16 * (TN * 32 + 16);
     static constexpr int LDS_BYTES = NS * STAGE_BYTES + STAGING_BYTES;
@@ -445,6 +445,50 @@ __global__ __launch_bounds__(T::THREADS, 2) void wgrad_rows_kernel(WgradTiles<T>
     prod_tile<T>(tiles, smem);
 }
 
+// The same on the hand-ordered 256 x 256 tile, both operands turned round by the fragment reads.  A tile's sum is short (8 slabs of 512
+// rows are 11 us) against what surrounds it, so the workgroups stay: the next tile's first two slabs are on their way while this
+// one's results are stored.  16 experts of 2048 x 2048, 512 rows each: a workgroup per tile 87 us, this 81 (the 128 x 128 tiles 101);
+// of 2048 x 1408, 750 rows 81 and 82 (96); 4 of 2048 x 2560, 4096 rows 174 and 174 (192), 1.72 PFLOP/s inside the slab loop.
+template <class T>
+__global__ __launch_bounds__(T::THREADS) void wgrad_ring_kernel(WgradTiles<T> w, int ids) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    auto find = [&](int id, TaskPtrs& p) {     // the first tile from `id` on, in steps of the grid
+        int e, n0, k0;
+        while (id < ids && !w.place(id, e, n0, k0)) id += gridDim.x;
+        if (id >= ids) return id;
+        ProdJob j;
+        w.job(id, j);
+        p = prod_epilogue(w.dw + ((int64_t)e * w.N + n0) * w.K, w.K, k0, min(T::BM, w.N - n0));
+        p.a_base = j.a.base;
+        p.a_ld = j.a.ld;
+        p.a_extent = j.a.extent;
+        p.b0 = j.b.base;
+        p.b_ld = j.b.ld;
+        p.b_extent = j.b.extent;
+        p.K = j.slabs * kBK;
+        return id;
+    };
+    TaskPtrs p;
+    int id = find(blockIdx.x, p);
+    if (id >= ids) return;
+    RingLoads L = ring_prepare<T>(p);
+    ring_first_loads<T>(L, smem);
+    while (true) {
+        f32x4 acc[T::TM][T::TN];
+        const bool mine = ring_slabs<T>(p.rows, L, smem, acc);
+        __builtin_amdgcn_s_barrier();          // every wavefront has read its last fragments (ring_slabs waits for them)
+        TaskPtrs next;
+        id = find(id + gridDim.x, next);
+        if (id < ids) {
+            L = ring_prepare<T>(next);
+            ring_first_loads<T>(L, smem);
+        }
+        if (mine) grouped_epilogue<T, kSums>(p, smem, acc);
+        if (id >= ids) return;
+        p = next;
+    }
+}
+
 // Weight gradient of one projection: dw[e] [N, K] = dy_e^T . a_e, the sum running over the rows of expert e.  Both
 // operands arrive transposed and padded: dyT [N, ld] and aT [K, ld] hold expert e's rows in columns
 // [poff[e], poff[e+1]) (zeros behind the last real row; every window is a multiple of 128 wide), so each expert is one
@@ -616,18 +660,30 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
 }
 
 template <class T>
-static hipError_t launch_wgrad_rows(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K, hipStream_t st) {
-    hipError_t e = allow_lds(&wgrad_rows_kernel<T>, T::LDS_BYTES);
-    if (e != hipSuccess) return e;
-    const int64_t tiles = ((int64_t)((K + T::BN - 1) / T::BN) * ((N + T::BM - 1) / T::BM) + 7) / 8 * 8 * E;
+static hipError_t launch_wgrad_rows(const WgradTiles<T>& w, hipStream_t st) {
+    const int64_t tiles = ((int64_t)((w.K + T::BN - 1) / T::BN) * ((w.N + T::BM - 1) / T::BM) + 7) / 8 * 8 * w.E;
     if (tiles > INT32_MAX) return hipErrorInvalidValue;
-    wgrad_rows_kernel<T><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(WgradTiles<T>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K});
+    if constexpr (T::TRA) {
+        hipError_t e = allow_lds(&wgrad_ring_kernel<T>, T::LDS_BYTES);
+        if (e != hipSuccess) return e;
+        wgrad_ring_kernel<T><<<(unsigned)std::min<int64_t>(tiles, kTaskUnits), T::THREADS, T::LDS_BYTES, st>>>(w, (int)tiles);
+    } else {
+        hipError_t e = allow_lds(&wgrad_rows_kernel<T>, T::LDS_BYTES);
+        if (e != hipSuccess) return e;
+        wgrad_rows_kernel<T><<<(unsigned)tiles, T::THREADS, T::LDS_BYTES, st>>>(w);
+    }
     return hipGetLastError();
 }
-hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, int E, int N, int K,
+template <bool F16>
+static hipError_t launch_wgrad_rows(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K, hipStream_t st) {
+    using Large = Tile<256, 256, 2, 2, 2, F16, true, true>;
+    if (large) return launch_wgrad_rows(WgradTiles<Large>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K}, st);
+    return launch_wgrad_rows(WgradTiles<ProdTile<F16>>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K}, st);
+}
+// large: on the 256 x 256 tile.
+hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K,
                                 bool f16, hipStream_t st) {
-    return f16 ? launch_wgrad_rows<ProdTile<true>>(dy, a, dw, count, offset, E, N, K, st)
-               : launch_wgrad_rows<ProdTile<false>>(dy, a, dw, count, offset, E, N, K, st);
+    return f16 ? launch_wgrad_rows<true>(dy, a, dw, count, offset, large, E, N, K, st) : launch_wgrad_rows<false>(dy, a, dw, count, offset, large, E, N, K, st);
 }
 
 template <bool F16, int EPI>

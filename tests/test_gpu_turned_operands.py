@@ -44,3 +44,24 @@ def test_data_gradients_on_weights_as_stored(moe, dtype, shape, gated):
                                     api._ptr(doff), I, H, api._ptr(out[0]), api._ptr(out[1] if gated else None), api._stream())
     assert rc == 0 and torch.equal(out[0][:R], want[0][:R]) and (not gated or torch.equal(out[1][:R], want[1][:R]))
     assert torch.equal(out[0][R:], u[R:])        # rows of no expert stay as they are
+
+
+@pytest.mark.parametrize("dtype", [ob.BF16, ob.F16])
+@pytest.mark.parametrize("shape", [(750, 2560, 1088, 5, 2), (2304, 2048, 1024, 24, 2), (700, 1152, 1920, 16, 4)])
+def test_weight_gradients_on_rows_as_stored(moe, dtype, shape):
+    """Workgroups with a tile each, with several in a row (and a ragged last round), and the 128 x 128 tiles (wgrad_large), experts
+    without rows and with odd slab counts: the bits that the transposed copies give."""
+    import torch
+    S, H, I, E, k = shape
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=S, drop=0, skew=0.2)
+    count[1] += count[0]                         # an expert without rows
+    offset[1], count[0] = offset[0], 0
+    R = int(count.sum())
+    layer, copies = moe.MoELayer(product_config(cfg)), moe.MoELayer(product_config(cfg), options={"grouped_tile": 1})
+    dev = lambda *s: to_device(ob.from_f32(rng.standard_normal(s).astype(np.float32), dtype), KIND[dtype])
+    dcount, doff = to_device(count, "i32"), to_device(offset, "i32")
+    a, b = dev(S * k, H), dev(S * k, I)
+    a[R:] = b[R:] = float("nan")
+    for x, y in ((a, b), (b, a)):
+        got, want = layer.expert_wgrad(x, y, dcount, doff), copies.expert_wgrad(x, y, dcount, doff)
+        assert torch.equal(got, want) and not got[0].any() and got[-1].any()

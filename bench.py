@@ -26,6 +26,7 @@ sys.path.insert(0, ROOT)
 
 PEAK_BF16_TFLOPS = 2500.0     # MI355X dense bf16 MFMA
 PEAK_F32_TFLOPS = 157.3
+PEAK_F32_PIECES_TFLOPS = PEAK_BF16_TFLOPS / 6      # fp32 products as six bf16 ones (ffn_f32_pieces.hip)
 PEAK_FP8_TFLOPS = 5000.0      # MI355X dense fp8 MFMA: what bounds a layer whose both GEMM operands are e4m3 (option fp8_mfma)
 PEAK_HBM_GBS = 8000.0         # MI355X HBM3E
 
@@ -195,7 +196,11 @@ def measure(name, steps, warmup, seed, ffn_mode, calibrate_copy=False, balanced_
     fp8 = c.torch_dtype == api.DTYPE_FP8
     widened = fp8 and layer.kernel_dtype != c.torch_dtype   # the FFN stage widens the weights, then runs the bf16 tiles
     # fp32 layers: the matrix-core tile (128-row blocks) or the vector-ALU kernel (64-row blocks)
+    # or, where the layer has the room for them, bf16 pieces
     f32_kind = "" if c.torch_dtype != api.DTYPE_F32 else ("_f32_tile" if layer.plan["block_rows"] == 128 else "_f32")
+    pieces = f32_kind == "_f32_tile" and layer.options["f32_tile"] == -1      # (no option names them)
+    if pieces:
+        f32_kind = "_f32_pieces"
     if w.bound == "hbm" and fp8:
         active = int((cnt > 0).sum())
         nbytes = wl.fp8_ffn_bytes(c, active, kept)
@@ -207,11 +212,12 @@ def measure(name, steps, warmup, seed, ffn_mode, calibrate_copy=False, balanced_
     else:
         e4m3_mfma = fp8 and layer.options.get("fp8_mfma") == 1
         roof = {"bound": "mfma", "achieved": flops / (ffn["mean"] * 1e-3) / 1e12,
-                "peak": PEAK_F32_TFLOPS if c.torch_dtype == api.DTYPE_F32 else (PEAK_FP8_TFLOPS if e4m3_mfma else PEAK_BF16_TFLOPS),
+                "peak": PEAK_F32_PIECES_TFLOPS if pieces else PEAK_F32_TFLOPS if c.torch_dtype == api.DTYPE_F32 else (PEAK_FP8_TFLOPS if e4m3_mfma else PEAK_BF16_TFLOPS),
                 "unit": "TFLOP/s",
                 "kernel": "quant_rows128_kernel x2 + ffn_tiled_fp8_mfma_kernel x2" if e4m3_mfma else
                           (("ffn_persistent_fp8_tile_kernel" if queue else "ffn_tiled_fp8_tile_kernel x2")
                            if fp8 and not widened else
+                           ("make_pieces_kernel + " if pieces else "") +
                            ("widen_block128_kernel x%d + " % (3 if c.hidden_act == api.ACT_SWIGLU else 2) if widened else "") +
                            ("ffn_persistent%s_kernel" if queue else "ffn_tiled%s_kernel x2") % f32_kind),
                 "algorithmic_flops": flops}
@@ -223,6 +229,8 @@ def measure(name, steps, warmup, seed, ffn_mode, calibrate_copy=False, balanced_
     plan = ""
     if fp8 and w.bound == "mfma" and not widened:
         plan = "/e4m3_mfma" if layer.options.get("fp8_mfma") == 1 else "/e4m3_tile"
+    if pieces:
+        plan = "/pieces"
     t = MEASURED_TRAFFIC.get(name + plan)
     digest = kernel_digest(t["sources"]) if t else None
     same_schedule = t is not None and t.get("ffn_mode", 2) == layer.ffn_mode

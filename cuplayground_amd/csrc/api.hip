@@ -43,6 +43,8 @@ int fp8_tile_block_n0(int swiglu);
 int fp8_tile_block_n1();
 int ffn_persistent_occupancy_fp8_tile();
 hipError_t launch_ffn_f32_tile(const FfnArgs&, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t);
+hipError_t launch_ffn_f32_pieces(const FfnArgs&, const ExpertRows&, void* x_pieces, void* w_pieces, void* h_pieces, int32_t* inexact,
+                                 int max_mtiles, int nnt0, int nnt1, hipStream_t);
 bool gemm_dense_f32_takes_tile(int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm_dense_f32_tile(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int,
                                       hipStream_t);
@@ -66,6 +68,7 @@ struct Derived {
     int64_t capacity;
     FfnPlan plan;
     int nblk;          // workgroups of the slot-assignment kernels
+    bool f32_pieces;   // fp32 layer that runs on bf16 pieces unless its mode or options ask for a schedule of the fp32 tile
     int wide_mats;     // weight matrices per expert (3 with SwiGLU, else 2)
     int max_mtiles;
 };
@@ -73,7 +76,7 @@ struct Derived {
 struct WsLayout {
     size_t logits, topk_idx, topk_w, slot, pair_row, token_indices, expert_count, expert_offset, rank_local,
         block_hist, mtiles, seg0, seg1, segq, qstate, cstate, done0, done1, pair_mt, wg_clock, arrive, stats_prob, stats_cnt, h, y,
-        wide, xq, sx, hq, sh, split_cnt, split_part, total;
+        wide, xq, sx, hq, sh, split_cnt, split_part, x_pieces, w_pieces, total;
 };
 
 // Storage type of activations (x, biases, h, y, out): the layer's own, except that tf32 -- fp32 storage with
@@ -90,6 +93,25 @@ int check_supported(const moe_config& c) {
         return MOE_ERR_UNSUPPORTED;     // one scale per 128 x 128 block of a weight matrix
     if (c.hidden_size > 16384) return MOE_ERR_UNSUPPORTED;   // the router keeps a token row in registers
     return MOE_OK;
+}
+
+WsLayout layout(const Derived& d);
+
+// Rows per expert from which an fp32 layer on the 128 x 128 matrix-core tile runs on bf16 pieces instead (ffn_f32_pieces.hip): below,
+// making the weights' pieces costs what the products save.  Whole layers, us, fp32 tile / pieces, and their distance (2-norm) from
+// float64: the reference's knob file (8192 rows, one expert of 1024 x 4096) 1053 / 712, 1.0e-6 / 3.7e-7; 2048 rows of it 429 / 385; 8
+// experts of 1024 x 2048, GELU, 512 rows each 561 / 432, 1.1e-6 / 3.6e-7; 16 of 2048 x 2048, 512 rows 1334 / 1256, 1.2e-6 / 4.4e-7; of
+// 2048 x 1408, SwiGLU, 2048 rows 4489 / 2979, 1.4e-6 / 5.0e-7; 8 of 512 x 1024, 2048 rows 440 / 342; 4 of 256 x 512, 4096 rows 184 / 155.
+constexpr int64_t kPiecesRowsPerExpert = 512, kPiecesExtraBytes = (int64_t)4 << 30;
+bool f32_pieces_ok(const Derived& d, const moe_options& o) {
+    if (d.act_dtype != MOE_DTYPE_F32 || d.plan.tile != 1 || o.f32_tile != MOE_OPT_AUTO || d.A < d.E * kPiecesRowsPerExpert) return false;
+    const int64_t lim = (int64_t)1 << 32, HI = (int64_t)std::max(d.H, d.I);
+    if (HI > 65536 || (int64_t)d.S * d.H * 6 >= lim || (int64_t)d.A * d.I * 6 >= lim || (HI + 256) * 6 * std::min(d.H, d.I) >= lim || (std::min(d.H, d.I) + 256) * 6 * HI >= lim) return false;
+    // what moe_forward_static took before it takes still, and nobody's workspace grows by more than kPiecesExtraBytes
+    Derived with = d;
+    with.f32_pieces = true;
+    const size_t before = layout(d).total, after = layout(with).total;
+    return after - before <= (size_t)kPiecesExtraBytes && (before > MOE355_STATIC_WORKSPACE_BYTES || after <= MOE355_STATIC_WORKSPACE_BYTES);
 }
 
 int derive(const moe_config& c, const moe_options& o, Derived* d) {
@@ -112,6 +134,8 @@ int derive(const moe_config& c, const moe_options& o, Derived* d) {
     d->wide_in_workspace = d->plan.widen && o.prepared_weights != 1;
     d->nblk = ceil_div(d->A, kRouteBlock);
     d->max_mtiles = ceil_div(d->A, d->plan.block_m) + d->E;
+    d->f32_pieces = false;
+    d->f32_pieces = f32_pieces_ok(*d, o);
     return MOE_OK;
 }
 
@@ -142,7 +166,7 @@ WsLayout layout(const Derived& d) {
     w.arrive = take((size_t)d.S * std::max(d.plan.nnt1, ceil_div(d.H, 128)) * 4);   // no smaller for a plan with wider column tiles
     w.stats_prob = take((size_t)kStatsBlocks * d.E * 8);
     w.stats_cnt = take((size_t)kStatsBlocks * d.E * 4);
-    w.h = take((size_t)d.A * d.I * d.act_bytes);
+    w.h = take((size_t)d.A * d.I * (d.f32_pieces ? 6 : d.act_bytes));      // in fp32 or as pieces
     w.y = take((size_t)d.A * d.H * d.act_bytes);
     // bf16 copies of an e4m3 layer's expert weights (up, down, gate), rewritten by every call of such a plan
     w.wide = take(d.wide_in_workspace ? (size_t)d.wide_mats * d.E * d.I * d.H * 2 : 0);
@@ -156,6 +180,8 @@ WsLayout layout(const Derived& d) {
     const size_t split_tiles = d.plan.ksplit > 1 ? (size_t)d.plan.tail_blocks * d.plan.nnt1 : 0;
     w.split_cnt = take(split_tiles * 4);
     w.split_part = take(split_tiles * d.plan.ksplit * ((size_t)d.plan.block_m * bf16_block_n1(d.plan.tile)) * 4);
+    w.x_pieces = take(d.f32_pieces ? (size_t)d.S * d.H * 6 : 0);
+    w.w_pieces = take(d.f32_pieces ? (size_t)d.wide_mats * d.E * d.I * d.H * 6 : 0);
     w.total = off;
     return w;
 }
@@ -348,7 +374,12 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
+// Whether this call's FFN stage runs on bf16 pieces: as two launches, whatever a queue would take.
+bool pieces_run(const moe_handle* h) {
+    return h->d.f32_pieces && h->ffn_mode == MOE_FFN_AUTO && h->combine_mode == 0 && !h->queue_options && !h->task_trace;
+}
 int resolved_ffn_mode(const moe_handle* h) {
+    if (pieces_run(h)) return MOE_FFN_TILED;
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
     if (h->d.plan.mfma8) return MOE_FFN_TILED;
     if (h->ffn_mode != MOE_FFN_AUTO) return h->ffn_mode;
@@ -603,7 +634,8 @@ int moe_get_options(const moe_handle* h, moe_options* opt) {
     if (!h || !opt) return MOE_ERR_BAD_ARGUMENT;
     *opt = h->opt;
     const int kdt = h->d.plan.kernel_dtype;
-    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && h->d.plan.tile == kF32StreamTile) opt->f32_tile = MOE_OPT_AUTO;
+    // (nor have fp32 layers on bf16 pieces)
+    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && (h->d.plan.tile == kF32StreamTile || h->d.f32_pieces)) opt->f32_tile = MOE_OPT_AUTO;
     return MOE_OK;
 }
 
@@ -877,7 +909,10 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
         for (int i = 0; i < d.wide_mats; ++i) *dst[i] = wide + (size_t)i * d.E * d.I * d.H * 2;
         fa.s_up = fa.s_gate = fa.s_down = nullptr;
     }
-    if (d.plan.mfma8) {
+    if (pieces_run(h)) {
+        e = launch_ffn_f32_pieces(fa, ExpertRows{ra.expert_count, ra.expert_offset}, at<char>(workspace, L.x_pieces), at<char>(workspace, L.w_pieces), fa.h,
+                                  ra.q->inexact, d.max_mtiles, d.plan.nnt0, d.plan.nnt1, st);
+    } else if (d.plan.mfma8) {
         e = launch_ffn_fp8_mfma(fa, d.S, d.A, d.max_mtiles, d.plan.nnt0, d.plan.nnt1, st);
     } else if (kdt == MOE_DTYPE_FP8_E4M3_B128) {
         e = (d.plan.tile ? launch_ffn_fp8_tile : launch_ffn_fp8)(fa, d.max_mtiles, d.plan.nnt0, d.plan.nnt1,

@@ -49,6 +49,7 @@ template <int BM_, int BN_, int WM_, int WN_, int NS_, bool F16_ = false, bool T
 struct Tile {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_;
     static constexpr bool F16 = F16_, TRA = TRA_, TRB = TRB_;
+    static constexpr bool PIECES = false;         // fp32 operands as three bf16 pieces (ffn_f32_pieces.hip)
     static constexpr int THREADS = WM * WN * kWave;
     static constexpr int TM = BM / WM / 16;       // 16x16 MFMA tiles per wavefront along tokens
     static constexpr int TN = BN / WN / 16;       // ... along weight rows
@@ -593,6 +594,7 @@ struct RingLoads {
     const void* base_b1;
     uint32_t a_extent, b_extent;
     uint32_t a_slab, b_slab;         // TRA, TRB: bytes of a slab's 64 k
+    uint32_t piece_slabs, piece_recip;   // PIECES: slabs of one piece, and 2^32 over it, rounded up
     int KT;                          // slabs of 64, >= 1
     int wrow;                        // first of the eight consecutive stage rows this wavefront's loads fill per pass
 };
@@ -659,6 +661,8 @@ __device__ __forceinline__ RingLoads ring_prepare_weights(const TaskPtrs& p) {
     L.a_slab = T::TRA ? (uint32_t)p.a_ld * kRowBytes : 0u;
     L.b_slab = T::TRB ? (uint32_t)p.b_ld * kRowBytes : 0u;
     L.KT = p.K / kBK;
+    L.piece_slabs = T::PIECES ? (uint32_t)L.KT / 6u : 0u;
+    L.piece_recip = T::PIECES ? 0xFFFFFFFFu / L.piece_slabs + 1u : 0u;
     L.wrow = __builtin_amdgcn_readfirstlane(prow & ~7);
     return L;
 }
@@ -692,6 +696,14 @@ __device__ __forceinline__ RingLoads ring_prepare(const TaskPtrs& p) {
     return L;
 }
 
+// fp32 operands as three bf16 pieces, a row one piece behind the other (ffn_f32_pieces.hip): the contraction runs over six pairs of
+// pieces, the smallest products first.
+constexpr uint32_t kPieceA = 2u | 0u << 2 | 1u << 4 | 1u << 6 | 0u << 8 | 0u << 10, kPieceB = 0u | 2u << 2 | 1u << 4 | 0u << 6 | 1u << 8 | 0u << 10;
+__device__ __forceinline__ int piece_offset(const RingLoads& L, int slab, uint32_t pieces) {
+    const uint32_t pair = __umulhi((uint32_t)slab, L.piece_recip);      // slab / piece_slabs (slab < 7 * 2^10)
+    return (int)((((pieces >> (2 * pair)) & 3u) * L.piece_slabs + ((uint32_t)slab - pair * L.piece_slabs)) * kRowBytes);
+}
+
 // Load n of slab `slab` of a task: n < RA token rows, else weight rows; the weight rows of pass m come from w_gate when
 // they lie in the first half of a wavefront's weight rows.  Raw buffers (stride 0) that end where the operand ends.  Slabs past the end of K go through descriptors of
 // zero length, which the hardware answers with zeros without touching memory (the stages they land in are never read).
@@ -699,7 +711,7 @@ template <class T>
 __device__ __forceinline__ void ring_load_one(const RingLoads& L, unsigned char* smem, int slab, int n) {
     const int wrow = L.wrow;
     unsigned char* base = smem + (slab & 1) * T::STAGE_BYTES;
-    const int soff = slab * kRowBytes;
+    const int soff = T::PIECES ? piece_offset(L, slab, n < T::RA ? kPieceA : kPieceB) : slab * kRowBytes;
     const bool live = slab < L.KT;
     if (n < T::RA ? T::TRA : T::TRB) {
         // the slab's rows of k: a buffer that begins at them and ends where the operand ends (rows behind it are zeros)
@@ -781,6 +793,7 @@ __device__ __forceinline__ bool ring_slabs(int rows, const RingLoads& L, unsigne
         U.base_a = unip(L.base_a); U.base_b0 = unip(L.base_b0); U.base_b1 = unip(L.base_b1);
         U.a_extent = uni(L.a_extent); U.b_extent = uni(L.b_extent);
         U.a_slab = uni(L.a_slab); U.b_slab = uni(L.b_slab);
+        U.piece_slabs = uni(L.piece_slabs); U.piece_recip = uni(L.piece_recip);
         U.KT = (int)uni((unsigned)L.KT); U.wrow = (int)uni((unsigned)L.wrow);
     }
     const int KT = U.KT;                        // an odd one runs one slab more, on the zeros that its loads fetch

@@ -245,9 +245,11 @@ __device__ __forceinline__ TileTaskF resolve_tile_f32(const FfnArgs& a, const Ta
     return p;
 }
 
-__global__ __launch_bounds__(GTHREADS) void ffn_tiled_f32_tile_kernel(FfnArgs a, int phase) {
+// only_if: null, or two device words; where both are zero there is nothing to do (ffn_f32_pieces.hip).
+__global__ __launch_bounds__(GTHREADS) void ffn_tiled_f32_tile_kernel(FfnArgs a, int phase, const int32_t* only_if) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_list[1 + GBM];
+    if (only_if && (only_if[0] | only_if[1]) == 0) return;
     if (phase == 0) zero_unrouted_rows(a, 4);
     Task t;
     if (!tiled_task(a, phase, blockIdx.x, t)) return;
@@ -394,16 +396,22 @@ hipError_t launch_wgrad_f32_tile(const void* dyT, const void* aT, void* dw, cons
     return hipGetLastError();
 }
 
+// One projection of the two launches, if one of the two words is set.
+hipError_t launch_ffn_f32_tile_if(const FfnArgs& a, int phase, const int32_t* only_if, int max_mtiles, int nnt, hipStream_t st) {
+    hipError_t e = allow_lds(&ffn_tiled_f32_tile_kernel);
+    if (e != hipSuccess) return e;
+    ffn_tiled_f32_tile_kernel<<<tiled_grid(max_mtiles, nnt, a.groups), GTHREADS, GLDS, st>>>(a, phase, only_if);
+    return hipGetLastError();
+}
+
 hipError_t launch_ffn_f32_tile(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
     if (blocks > 0) {
         hipError_t e = allow_lds(&ffn_persistent_f32_tile_kernel);
         if (e != hipSuccess) return e;
         ffn_persistent_f32_tile_kernel<<<blocks, GTHREADS, GLDS, st>>>(a);
     } else {
-        hipError_t e = allow_lds(&ffn_tiled_f32_tile_kernel);
-        if (e != hipSuccess) return e;
-        ffn_tiled_f32_tile_kernel<<<tiled_grid(max_mtiles, nnt0, a.groups), GTHREADS, GLDS, st>>>(a, 0);
-        ffn_tiled_f32_tile_kernel<<<tiled_grid(max_mtiles, nnt1, a.groups), GTHREADS, GLDS, st>>>(a, 1);
+        const hipError_t e = launch_ffn_f32_tile_if(a, 0, nullptr, max_mtiles, nnt0, st);
+        return e != hipSuccess ? e : launch_ffn_f32_tile_if(a, 1, nullptr, max_mtiles, nnt1, st);
     }
     return hipGetLastError();
 }

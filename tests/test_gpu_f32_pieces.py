@@ -1,0 +1,139 @@
+"""fp32 layers on bf16 pieces (csrc/ffn_f32_pieces.hip): no further from float64 than the fp32 matrix instructions, over both row block
+heights and every epilogue, and those instructions themselves wherever a value is not held by three pieces."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# S, H, I, E, k, activation, capacity factor (0: none dropped), biases
+SHAPES = {
+    "relu_one_expert": (4500, 512, 2048, 1, 1, 0, 0.0, False),              # a ragged last row block
+    "gelu_bias_drop": (4700, 640, 1920, 3, 1, 1, 0.9, True),                # ragged column tiles, odd slab counts a piece
+    "swiglu_bias": (2600, 896, 1152, 2, 2, 2, 0.0, True),
+    "relu_many_rounds": (9000, 256, 1024, 4, 2, 0, 1.0, False),
+}
+
+
+@pytest.fixture(scope="module")
+def moe():
+    import torch
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    import cuplayground_amd
+    return cuplayground_amd
+
+
+def _layers(moe, name):
+    import torch
+    S, H, I, E, k, act, cf, bias = SHAPES[name]
+    cfg = moe.MoEConfig(capacity_factor=cf or 1.0, drop_tokens=int(cf > 0), expert_top_k=k, is_training=0, hidden_act=act, hidden_size=H,
+                        intermediate_size=I, micro_batch=1, num_experts=E, sequence_len=S, torch_dtype=0, gate_fn=0, norm_topk_prob=0)
+    pieces, tile = moe.MoELayer(cfg, options={}), moe.MoELayer(cfg, options={"f32_tile": 1}, ffn_mode=moe.api.FFN_TILED)
+    assert pieces.workspace_bytes > tile.workspace_bytes + 6 * S * H          # the pieces have their place
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rnd = lambda *s, std=0.05: torch.randn(*s, generator=g, device="cuda") * std
+    w = {"gate_w": rnd(E, H), "w_up": rnd(E, I, H), "w_down": rnd(E, H, I)}
+    if act == 2:
+        w["w_gate"] = rnd(E, I, H)
+    if bias:
+        w.update(b_up=rnd(E, I), b_down=rnd(E, H), **({"b_gate": rnd(E, I)} if act == 2 else {}))
+    return cfg, pieces, tile, rnd(S, H, std=1.0), w
+
+
+def _float64(cfg, x, w, routing):
+    import torch
+    S, k, E = cfg.tokens, cfg.expert_top_k, cfg.num_experts
+    out = torch.zeros(S, cfg.hidden_size, dtype=torch.float64, device="cuda")
+    idx, slot, tw = (routing[n].reshape(S, k) for n in ("topk_idx", "slot", "topk_w"))
+    d = lambda n, e: w[n][e].double() if n in w else 0.0
+    for e in range(E):
+        for r in range(k):
+            m = ((idx[:, r] == e) & (slot[:, r] >= 0)).nonzero().flatten()
+            rows = x[m].double()
+            h = rows @ d("w_up", e).t() + d("b_up", e)
+            if cfg.hidden_act == 2:
+                h = torch.nn.functional.silu(rows @ d("w_gate", e).t() + d("b_gate", e)) * h
+            else:
+                h = torch.nn.functional.gelu(h) if cfg.hidden_act == 1 else torch.relu(h)
+            out[m] += (h @ d("w_down", e).t() + d("b_down", e)) * tw[m, r:r + 1].double()
+    return out
+
+
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_no_further_from_float64_than_the_fp32_tile(moe, name):
+    cfg, pieces, tile, x, w = _layers(moe, name)
+    routing = pieces.new_routing()
+    got, other = pieces.forward(x, w, routing=routing), tile.forward(x, w)
+    ref = _float64(cfg, x, w, routing)
+    far = lambda o: ((o.double() - ref).norm() / ref.norm()).item()
+    assert far(got) <= far(other) and far(got) < 1e-6, (far(got), far(other))
+    assert ((got.double() - ref).abs().max() <= (other.double() - ref).abs().max() * 1.5)      # single values: the tails of two distributions
+    pieces.close(), tile.close()
+
+
+@pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_huge", "w_tiny", "x_denormal", "h_huge", "h_tiny"])
+@pytest.mark.parametrize("name", ["gelu_bias_drop", "swiglu_bias"])
+def test_values_that_pieces_do_not_hold(moe, name, what):
+    """The whole call by the fp32 instructions, bit for bit (NaN in the same places)."""
+    import torch
+    cfg, pieces, tile, x, w = _layers(moe, name)
+    if what == "x_inf":
+        x[17, 5] = float("inf")
+    elif what == "x_nan":
+        x[cfg.tokens - 1, 0] = float("nan")
+    elif what == "w_huge":
+        w["w_down"][1, 3, 64] = 3e38
+    elif what == "w_tiny":
+        w["w_up"][0, 7, 9] = 2.0 ** -101
+    elif what == "x_denormal":
+        x[100, 11] = 1e-41
+    else:      # operands that pieces hold, results of the up projection that they do not
+        x *= 1.0 if what == "h_huge" else 1e-15
+        for n in ("w_up", "w_gate", "b_up", "b_gate"):
+            if n in w:
+                w[n] *= 0.0 if n[0] == "b" else 1e30 if what == "h_huge" else 1e-20
+    got, want = pieces.forward(x, w), tile.forward(x, w)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32)) or (torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()))
+    pieces.close(), tile.close()
+
+
+def test_smallest_and_largest_magnitudes_that_pieces_hold(moe):
+    """2^-100 and just below 2^100 as operands: all three pieces count."""
+    import torch
+    cfg, pieces, tile, x, w = _layers(moe, "relu_one_expert")
+    x *= 2.0 ** -90
+    x[x.abs() < 2.0 ** -100] = 2.0 ** -100
+    w["w_up"] *= 2.0 ** 60
+    routing = pieces.new_routing()
+    got, other = pieces.forward(x, w, routing=routing), tile.forward(x, w)
+    ref = _float64(cfg, x, w, routing)
+    far = lambda o: ((o.double() - ref).norm() / ref.norm()).item()
+    assert far(got) <= far(other) and not torch.equal(got, other)
+    pieces.close(), tile.close()
+
+
+def test_replays_of_a_graph_change_over(moe):
+    """One captured call on inputs that pieces hold and on others: every replay is the eager call."""
+    import torch
+    cfg, pieces, tile, x, w = _layers(moe, "relu_one_expert")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    out = torch.empty_like(x)
+    with torch.cuda.stream(side):
+        pieces.forward(x, w, out=out)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pieces.forward(x, w, out=out)
+    clean = x.clone()
+    for it in range(4):
+        x.copy_(clean * (it + 1))
+        if it % 2:
+            x[3, 3] = float("inf")
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got, want = out.clone(), pieces.forward(x, w)
+        assert torch.equal(got.nan_to_num(), want.nan_to_num()) and torch.equal(got.isnan(), want.isnan())
+        assert bool(torch.isfinite(got).all()) == (it % 2 == 0)
+    pieces.close(), tile.close()

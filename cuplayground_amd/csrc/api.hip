@@ -362,7 +362,8 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
     a.max_mtiles = d.max_mtiles;
     a.lag = h->queue_lag;
     a.groups = h->queue_groups;
-    a.tail_workgroups = h->opt.tail_round == 0 ? 0 : h->arch.persistent_blocks;
+    // (the queue's order is read by the queue kernels only)
+    a.tail_workgroups = h->opt.tail_round == 0 || resolved_ffn_mode(h) != MOE_FFN_PERSISTENT ? 0 : h->arch.persistent_blocks;
     if (d.plan.ksplit > 1) {
         a.tail_split = d.plan.ksplit;
         a.tail_blocks = d.plan.tail_blocks;

@@ -102,11 +102,16 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave, int* tot
     return base + inc - v;
 }
 
-// One workgroup of kMaxExperts threads: thread e owns expert e.
+// One workgroup of kMaxExperts threads: thread e owns expert e.  (The groups that share an expert's histograms are at most kScanParts,
+// because every thread walks their sums, and the row blocks are written a thread each: with one expert of 8192 rows, 512 groups and all
+// blocks by its thread, the scan took 18.5 us, so 7; no difference from 12 experts on.)
+constexpr int kScanParts = 32;
 struct ScanShared {
     int wave[kMaxExperts / kWave];
     int nmt[kMaxExperts];
     int mt0[kMaxExperts];
+    int off[kMaxExperts];
+    int kept[kMaxExperts];
     int part[kMaxExperts];
     int total[kMaxExperts];
     // the segment tables while one thread rearranges them (split_tail): in LDS, where its dependent accesses cost cycles,
@@ -126,10 +131,10 @@ __device__ __forceinline__ void route_scan_body(const RouteArgs& a, ScanShared& 
     // `parts` groups that each take a contiguous run of workgroups (two passes over block_hist)
     int epad = 1;
     while (epad < a.E) epad <<= 1;
-    const int parts = kMaxExperts / epad;
+    const int parts = min(min(kMaxExperts / epad, kScanParts), a.nblk);
     const int pe = threadIdx.x % epad, part = threadIdx.x / epad;
     const int chunk = (a.nblk + parts - 1) / parts;
-    const int b0 = min(a.nblk, part * chunk), b1 = min(a.nblk, b0 + chunk);
+    const int b0 = part < parts ? min(a.nblk, part * chunk) : a.nblk, b1 = min(a.nblk, b0 + chunk);
     int sum = 0;
     if (pe < a.E) {
 #pragma unroll 4
@@ -165,6 +170,8 @@ __device__ __forceinline__ void route_scan_body(const RouteArgs& a, ScanShared& 
     const int mt0 = block_exclusive_scan(nmt, s_wave, &total_mt);
     s_nmt[e] = nmt;
     s_mt0[e] = mt0;
+    sh.off[e] = off;
+    sh.kept[e] = kept;
     __syncthreads();
     // the merged queue: thread t owns segments 2t and 2t+1.  A phase-1 task must not be popped while the
     // phase-0 tasks it depends on are still running, or its workgroup idles: `lag` experts of phase-0 work
@@ -243,15 +250,21 @@ __device__ __forceinline__ void route_scan_body(const RouteArgs& a, ScanShared& 
         a.q->nseg = nseg_final;
         a.expert_offset[a.E] = total_rows;
     }
-    if (e < a.E) {          // (behind the tail's one-thread section: the other threads get on with this meanwhile)
-        for (int i = 0; i < nmt; ++i) {
-            MTile t;
-            t.expert = e;
-            t.row0 = off + i * a.block_m;
-            t.rows = min(a.block_m, kept - i * a.block_m);
-            t.pad = 0;
-            a.mtiles[mt0 + i] = t;
+    // (behind the tail's one-thread section: the other threads get on with this meanwhile.)  A row block a thread: its expert is
+    // the last one whose blocks begin at or before it.
+    for (int i = threadIdx.x; i < total_mt; i += blockDim.x) {
+        int lo = 0, hi = a.E - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s_mt0[mid] <= i) lo = mid; else hi = mid - 1;
         }
+        const int first = (i - s_mt0[lo]) * a.block_m;
+        MTile t;
+        t.expert = lo;
+        t.row0 = sh.off[lo] + first;
+        t.rows = min(a.block_m, sh.kept[lo] - first);
+        t.pad = 0;
+        a.mtiles[i] = t;
     }
     for (int i = threadIdx.x; i < a.max_mtiles; i += blockDim.x) a.done0[i] = 0;
     if (a.done1)

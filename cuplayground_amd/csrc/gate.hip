@@ -8,6 +8,7 @@
 // lane l of a wavefront owns partial sum l and takes, in ascending k, every k with (k/8) % 64 == l using
 // one fmaf per element; the 64 partials are folded by an xor butterfly (32,16,8,4,2,1); the bias is added
 // last.  Top-k is taken on the logits (softmax and sigmoid are monotone), ties to the lower expert index.
+#include <algorithm>
 #include <type_traits>
 #include <cstdlib>
 
@@ -372,142 +373,181 @@ hipError_t launch_gate_tiled(const void* x, const void* gate_w, const float* gat
 //
 // v_mfma_f32_16x16x1_4b_f32 is four independent 16 x 16 outer products with k = 1: D_b[i][j] = C_b[i][j] + A_b[i] B_b[j],
 // one multiply-add per element -- and the product of two bf16 (or fp16) values is exact in fp32, so each element sees
-// exactly the fmaf the kernels above perform, at the full fp32 rate of the matrix pipe (twice the unpacked vector rate)
-// with the widening running beside it on the vector ALU.  A pair of wavefronts owns 16 tokens x 16 experts.  Block b of
-// accumulator g carries partial sum p = 4 g + b of every pair of the tile: lane 16 b + i loads the 16-byte chunk
-// p + 64 j of token row i (and of expert row i) -- the chunk partial sum p takes in step j, i.e. elements
-// 32 (16 j + g) + 8 b onwards -- and its 8 elements go through 8 MFMAs in ascending k.  The even g belong to one
-// wavefront of the pair and the odd g to the other (8 accumulators = 128 registers each, so two wavefronts fit a
-// SIMD and one's loads and widening hide behind the other's MFMAs).  The 32 partial sums a wavefront holds of a pair
-// sit in one lane (accumulator g, register 4 b + r: token 4 (lane / 16) + r, expert lane % 16): p is folded with
-// p + 32, 16 and 8 (g with g + 8, 4, 2) in the lane, with p + 4 (g with g + 1) across the two wavefronts through LDS,
-// then with p + 2 and p + 1 (b) in the lane again -- the pairings of fold16, so the logits are bit-identical.
+// exactly the fmaf the kernels above perform, at the full fp32 rate of the matrix pipe (twice the unpacked vector rate).
+// A tile is 16 tokens x 16 experts.  Block b of accumulator g carries partial sum p = 4 g + b of every pair of the tile: lane
+// 16 b + i reads the 16-byte chunk p + 64 j of token row i (and of expert row i) -- the chunk partial sum p takes in step j, i.e.
+// elements 32 (16 j + g) + 8 b onwards -- and its 8 elements go through 8 MFMAs in ascending k.  The even g belong to one
+// wavefront of a pair and the odd g to the other (8 accumulators = 128 registers each, so two wavefronts fit a SIMD).  The 32
+// partial sums a wavefront holds of a pair sit in one lane (accumulator g, register 4 b + r: token 4 (lane / 16) + r, expert
+// lane % 16): p is folded with p + 32, 16 and 8 (g with g + 8, 4, 2) in the lane, with p + 4 (g with g + 1) across the two
+// wavefronts through LDS, then with p + 2 and p + 1 (b) in the lane again -- the pairings of fold16, so the logits are bit-identical.
+//
+// A workgroup holds 2 x 2 tiles (32 tokens x 32 experts).  A step's 64 rows of 1 KiB go from memory straight into one of two stages,
+// requested two steps ahead and across the end of a tile too: the workgroups stay, `tiles` of them in steps of the grid.  What bounds
+// it: a SIMD's two wavefronts share the pipe, and the two widening operations an MFMA needs do not run beside fp32 MFMAs (measured on
+// registers: 36 cycles an MFMA without, 48 with them; 64 here).  16384 tokens x 64 experts of 2048, selection included, 83.5 -> 74.5 us
+// against rows fetched into registers, 64 bytes of each of 16 a request, one tile's column of 32 experts a workgroup; 4000 tokens 32.4 -> 23.5.
 typedef float gate_f32x16 __attribute__((ext_vector_type(16)));
 
-// PAIRS wavefront pairs per workgroup, 16 expert columns each.  FUSE: the workgroup's columns cover every expert
-// (grid.y == 1) and the selection follows right behind the sums, as in gate_tile_kernel.
-template <typename T, int PAIRS, bool FUSE>
-__global__ __launch_bounds__(PAIRS * 128) __attribute__((amdgpu_waves_per_eu(2, 2))) void gate_mfma_kernel(const T* __restrict__ x, const T* __restrict__ gate_w,
-                                                        const float* __restrict__ gate_bias, float* __restrict__ logits,
-                                                        int S, int H, int E, GateTopk tk) {
+template <typename T>
+struct GateStage {
+    static constexpr int TT = 2, ET = 2;                     // tiles of a workgroup: tokens, experts
+    static constexpr int WAVES = TT * ET * 2, THREADS = WAVES * 64, ROWS = (TT + ET) * 16, PER = ROWS / WAVES;
+    static constexpr int STAGE_BYTES = ROWS * 1024, FOLD = 8, FOLD_BYTES = WAVES * FOLD * 64 * 4;
+    static constexpr int LDS_BYTES = 2 * STAGE_BYTES + FOLD_BYTES;
+    static_assert(LDS_BYTES <= 160 * 1024 && ROWS % WAVES == 0, "two stages and the folds");
+};
+typedef __attribute__((address_space(3))) void gate_lds_void;
+typedef const __attribute__((address_space(1))) void gate_gbl_void;
+
+template <typename T>
+__global__ __launch_bounds__(GateStage<T>::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void gate_mfma_kernel(
+    const T* __restrict__ x, const T* __restrict__ gate_w, const float* __restrict__ gate_bias, float* __restrict__ logits, int S, int H, int E,
+    int etiles, int tiles) {
+    using G = GateStage<T>;
     typedef typename RawChunk<T>::type raw_t;
-    constexpr int ECOLS = PAIRS * 16;
-    __shared__ float s_odd[PAIRS][16][64];      // [pair][4 b + r][lane]: the odd wavefront's sums over its g
-    __shared__ float s_log[FUSE ? 16 * ECOLS : 1];   // [token of the tile][expert]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int pair = wave >> 1, odd = wave & 1;
+    constexpr int TT = G::TT, ET = G::ET, NG = 8, ECOLS = ET * 16;
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* s_fold = reinterpret_cast<float*>(smem + 2 * G::STAGE_BYTES);                       // [wavefront][2 b + r][lane]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = wave % 2, ei = wave / 2 % ET, ti = wave / (2 * ET);      // q: this wavefront's parity of g
     const int b = lane >> 4, i = lane & 15;
-    const int t0 = blockIdx.x * 16, e0 = (blockIdx.y * PAIRS + pair) * 16;
-    const bool live = e0 < E;                   // an expert tile past the last one: nothing to do, but meet the barrier
-    gate_f32x16 acc[8];
+    const int nstep = H / 512;
+    // Tile id -> token tile and expert tile: the expert tiles of the same tokens are eight ids apart, on one XCD and close in time.
+    auto place = [&](int id, int& t0, int& e0) {
+        const int group = id >> 3, tt = group / etiles * 8 + (id & 7);
+        t0 = tt * TT * 16;
+        e0 = group % etiles * ECOLS;
+        return t0 < S;
+    };
+    auto next_tile = [&](int id, int& t0, int& e0) {
+        while (id < tiles && !place(id, t0, e0)) id += gridDim.x;
+        return id;
+    };
+    // Row r of a stage: its 16-byte chunk c lies at c ^ (r & 15), so that the sixteen rows of a fragment read meet all banks.
+    auto request = [&](int t0, int e0, int step, int stage) {
 #pragma unroll
-    for (int g = 0; g < 8; ++g)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[g][v] = 0.f;
-    if (live) {
-        // this wavefront's chunks: g = 2 gg + odd
-        const T* xrow = x + (size_t)min(t0 + i, S - 1) * H + 8 * b + 32 * odd;
-        const T* wrow = gate_w + (size_t)min(e0 + i, E - 1) * H + 8 * b + 32 * odd;
-        raw_t xn[8], wn[8];
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            xn[g] = *reinterpret_cast<const raw_t*>(xrow + 64 * g);
-            wn[g] = *reinterpret_cast<const raw_t*>(wrow + 64 * g);
+        for (int n = 0; n < G::PER; ++n) {
+            const int r = wave + n * G::WAVES;
+            const T* row = r < TT * 16 ? x + (size_t)min(t0 + r, S - 1) * H : gate_w + (size_t)min(e0 + r - TT * 16, E - 1) * H;
+            __builtin_amdgcn_global_load_lds((gate_gbl_void*)(row + step * 512 + ((lane ^ (r & 15)) << 3)),
+                                             (gate_lds_void*)(smem + stage * G::STAGE_BYTES + r * 1024), 16, 0, 0);
         }
-        // One step = 512 elements of every row.  The chunks of the next step are requested as soon as this step's have
-        // been widened, each into the registers it will be used from, and the last step is a copy of the loop body
-        // without requests: with a condition around the requests the chunks reach their registers through copies at the
-        // end of the loop body, and the wait in front of those copies exposes the latency of the requests issued last
-        // in every step (2.5 us of a step's 3.6 on a 64-expert layer).
-        auto step = [&](const T* xnext, const T* wnext, auto more) {
+    };
+    const unsigned lds0 = (unsigned)(__UINTPTR_TYPE__)(gate_lds_void*)smem;
+    const unsigned xa = lds0 + (ti * 16 + i) * 1024 + ((b ^ i) << 4), wa = lds0 + ((TT + ei) * 16 + i) * 1024 + ((b ^ i) << 4);
+
+    int t0, e0, id = next_tile(blockIdx.x, t0, e0);
+    if (id >= tiles) return;
+    // the step that is requested next
+    int rt0 = t0, re0 = e0, rid = id, rstep = 0;
+    auto advance = [&]() {
+        if (++rstep == nstep) {
+            rstep = 0;
+            rid = next_tile(rid + gridDim.x, rt0, re0);
+        }
+    };
+    int stage = 0, on_the_way = 0;
+    for (; on_the_way < 2 && rid < tiles; ++on_the_way) {
+        request(rt0, re0, rstep, on_the_way);
+        advance();
+    }
+    while (true) {
+        gate_f32x16 acc[NG];
 #pragma unroll
-            for (int g = 0; g < 8; g += 2) {    // two accumulators at a time: consecutive MFMAs are independent
-                float xv[2][8], wv[2][8];
+        for (int m = 0; m < NG; ++m)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    widen8<T>(xn[g + h], xv[h]);
-                    widen8<T>(wn[g + h], wv[h]);
-                    if constexpr (decltype(more)::value) {
-                        xn[g + h] = *reinterpret_cast<const raw_t*>(xnext + 64 * (g + h));
-                        wn[g + h] = *reinterpret_cast<const raw_t*>(wnext + 64 * (g + h));
-                    }
+            for (int v = 0; v < 16; ++v) acc[m][v] = 0.f;
+        for (int j = 0; j < nstep; ++j) {
+            // (stores of the tile before are younger than both steps' requests: they only make the wait more cautious)
+            if (on_the_way < 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER) : "memory");
+            __builtin_amdgcn_s_barrier();
+            const unsigned at = stage * G::STAGE_BYTES;
+#pragma unroll
+            for (int m = 0; m < NG; m += 4) {       // four accumulators at a time: consecutive MFMAs are independent
+                raw_t xr[4], wr[4];
+                unsigned ax[4], aw[4];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const unsigned g = (q + 2 * (m + h)) << 6;
+                    ax[h] = (xa ^ g) + at;
+                    aw[h] = (wa ^ g) + at;
+                }
+                asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+                             "ds_read_b128 %4, %12\n\tds_read_b128 %5, %13\n\tds_read_b128 %6, %14\n\tds_read_b128 %7, %15\n\ts_waitcnt lgkmcnt(0)"
+                             : "=&v"(xr[0]), "=&v"(wr[0]), "=&v"(xr[1]), "=&v"(wr[1]), "=&v"(xr[2]), "=&v"(wr[2]), "=&v"(xr[3]), "=&v"(wr[3])
+                             : "v"(ax[0]), "v"(aw[0]), "v"(ax[1]), "v"(aw[1]), "v"(ax[2]), "v"(aw[2]), "v"(ax[3]), "v"(aw[3])
+                             : "memory");
+                float xv[4][8], wv[4][8];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    widen8<T>(xr[h], xv[h]);
+                    widen8<T>(wr[h], wv[h]);
                 }
 #pragma unroll
                 for (int v = 0; v < 8; ++v)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        acc[g + h] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[h][v], wv[h][v], acc[g + h], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);      // or the scheduler gathers every request of the step behind its last MFMA
+                    for (int h = 0; h < 4; ++h) acc[m + h] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[h][v], wv[h][v], acc[m + h], 0, 0, 0);
             }
-        };
-        const int nstep = H / 512;
-        for (int j = 1; j < nstep; ++j) step(xrow + 512 * j, wrow + 512 * j, std::true_type{});
-        step(xrow, wrow, std::false_type{});
-    }
-    // acc[gg] holds g = 2 gg + odd: g + 8, g + 4, g + 2 are gg + 4, gg + 2, gg + 1
-    float u[16];
+            __builtin_amdgcn_s_barrier();           // the stage is free
+            if (rid < tiles) {
+                request(rt0, re0, rstep, stage);
+                advance();
+            } else {
+                --on_the_way;
+            }
+            stage ^= 1;
+        }
+        // acc[m] holds g = 2 m + q: g + 8, g + 4, g + 2 are m + 4, m + 2, m + 1
+        float u[16];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const float s0 = acc[0][v] + acc[4][v], s1 = acc[1][v] + acc[5][v], s2 = acc[2][v] + acc[6][v],
-                    s3 = acc[3][v] + acc[7][v];                                        // p with p + 32
-        u[v] = (s0 + s2) + (s1 + s3);                                                  // ... p + 16, then p + 8
-    }
-    if (odd) {
+        for (int v = 0; v < 16; ++v)      // p with p + 32, then p + 16, then p + 8
+            u[v] = ((acc[0][v] + acc[4][v]) + (acc[2][v] + acc[6][v])) + ((acc[1][v] + acc[5][v]) + (acc[3][v] + acc[7][v]));
+        // each wavefront of the pair goes on with two of the four tokens r of every lane
+        float* mine = s_fold + wave * G::FOLD * 64 + lane;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) s_odd[pair][v][lane] = u[v];
-    }
-    __syncthreads();
-    if (!FUSE && (odd || !live)) return;
-    if (!odd && live) {
-        const int e = e0 + i;
+        for (int bb = 0; bb < 4; ++bb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float q[4];
+            for (int rr = 0; rr < 2; ++rr) mine[(2 * bb + rr) * 64] = q ? u[4 * bb + rr] : u[4 * bb + 2 + rr];
+        __syncthreads();
+        const float* other = s_fold + (wave ^ 1) * G::FOLD * 64 + lane;
 #pragma unroll
-            for (int bb = 0; bb < 4; ++bb) q[bb] = u[4 * bb + r] + s_odd[pair][4 * bb + r][lane];     // ... p + 4
-            const float sum = (q[0] + q[2]) + (q[1] + q[3]);                                           // ... p + 2, p + 1
-            const int t = t0 + 4 * b + r;
+        for (int rr = 0; rr < 2; ++rr) {
+            const int r = q * 2 + rr;
+            float s[4];
+#pragma unroll
+            for (int bb = 0; bb < 4; ++bb) s[bb] = (q ? u[4 * bb + 2 + rr] : u[4 * bb + rr]) + other[(2 * bb + rr) * 64];     // ... p + 4
+            const float sum = (s[0] + s[2]) + (s[1] + s[3]);                                                       // ... p + 2, p + 1
+            const int t = t0 + ti * 16 + 4 * b + r, e = e0 + ei * 16 + i;
             if (t < S && e < E) {
                 const float val = gate_bias ? sum + gate_bias[e] : sum;
-                if (!FUSE || logits) logits[(size_t)t * E + e] = val;
-                if (FUSE) s_log[(4 * b + r) * ECOLS + e] = val;                       // grid.y == 1: e < ECOLS
+                logits[(size_t)t * E + e] = val;
             }
         }
-    }
-    if constexpr (FUSE) {
-        __syncthreads();
-        for (int q = wave; q < 16; q += 2 * PAIRS) {      // this wavefront's share of the tile's tokens
-            const int t = t0 + q;
-            if (t < S) topk_one_token<1>(s_log + q * ECOLS, t, E, tk.k, tk.gate_fn, tk.norm, tk.idx, tk.w, lane);
-        }
+        id = next_tile(id + gridDim.x, t0, e0);
+        if (id >= tiles) return;
+        __syncthreads();                            // the folds have been read
     }
 }
-
-// The matrix-core kernel takes 16-bit layers whose rows split into full steps of 512 elements, when the experts fill
-// most of its 16 columns and there are enough 16 x 16 tiles for every SIMD of the chip to get several.  With at most 64
-// experts one workgroup holds them all (two or four wavefront pairs) and selects as well (*fused).
+// The matrix-core kernel takes 16-bit layers whose rows split into full steps of 512 elements, from 150 workgroups' tiles on that the
+// experts fill to three quarters, or where they are many and the experts fill most of 16 columns.  This / the best other kernel, us,
+// selection included, rows of 2048: 64 experts, 2500 tokens (158) 22.4 / 24.3, 2000 (126) 21.0 / 19.8; 32 experts, 8192 tokens (256) 24.7 /
+// 33.7, 4096 (128) 21.2 / 19.5; 24 experts, 16384 (512) 44.8 / 54.3; 128, 4096 (512) 40.9 / 45.7; 256 experts of 7168, 1024 tokens (256)
+// 55.2 / 76.9, 512 (128) 54.2 / 44.7; 16 experts, 8192 tokens (256, half filled) 23.2 / 22.6, 32768 73.4 / 74.0, 12 of 1024 49.8 / 53.4.
+// (The selection in the same launch, where a workgroup holds every expert: 27.5 against 24.7 us with 32 experts and 8192 tokens.)
 template <typename T>
-bool launch_gate_mfma(const void* x, const void* gate_w, const float* gate_bias, float* logits, bool keep_logits, int S,
-                      int H, int E, int opt_mfma, const GateTopk* tk, bool wide_fusion, bool* fused, hipStream_t st,
-                      hipError_t* err) {
+bool launch_gate_mfma(const void* x, const void* gate_w, const float* gate_bias, float* logits, int S, int H, int E, int opt_mfma, hipStream_t st, hipError_t* err) {
+    using G = GateStage<T>;
     if (H % 512 != 0) return false;
-    const int et = (E + 15) / 16;
-    bool use = et * 16 * 3 <= E * 4 && (int64_t)((S + 15) / 16) * et >= 2048;
+    const int et = (E + 15) / 16, etiles = (E + G::ET * 16 - 1) / (G::ET * 16), ttiles = (S + G::TT * 16 - 1) / (G::TT * 16);
+    bool use = (etiles * G::ET * 16 * 3 <= E * 4 && (int64_t)ttiles * etiles >= 150) || (et * 16 * 3 <= E * 4 && (int64_t)((S + 15) / 16) * et >= 2048);
     if (opt_mfma != MOE_OPT_AUTO) use = opt_mfma != 0;
-    if (!use) return false;
-    const unsigned tiles = (unsigned)((S + 15) / 16);
-    if (tk && et <= 2) {
-        gate_mfma_kernel<T, 2, true><<<dim3(tiles, 1), 256, 0, st>>>((const T*)x, (const T*)gate_w, gate_bias,
-                                                                    keep_logits ? logits : nullptr, S, H, E, *tk);
-        *fused = true;
-    } else if (tk && et <= 4 && wide_fusion) {   // on request only: the 512-thread form measured 17 us slower than two launches
-        gate_mfma_kernel<T, 4, true><<<dim3(tiles, 1), 512, 0, st>>>((const T*)x, (const T*)gate_w, gate_bias,
-                                                                    keep_logits ? logits : nullptr, S, H, E, *tk);
-        *fused = true;
-    } else {
-        gate_mfma_kernel<T, 2, false><<<dim3(tiles, (et + 1) / 2), 256, 0, st>>>((const T*)x, (const T*)gate_w, gate_bias,
-                                                                                logits, S, H, E, GateTopk{});
-    }
+    const int64_t tiles = (int64_t)(ttiles + 7) / 8 * 8 * etiles;
+    if (!use || tiles > INT32_MAX - 65536) return false;
+    *err = hipFuncSetAttribute(reinterpret_cast<const void*>(&gate_mfma_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS_BYTES);
+    if (*err != hipSuccess) return true;
+    gate_mfma_kernel<T><<<(unsigned)std::min<int64_t>(tiles, 256), G::THREADS, G::LDS_BYTES, st>>>((const T*)x, (const T*)gate_w, gate_bias, logits, S, H, E, etiles, (int)tiles);
     *err = hipGetLastError();
     return true;
 }
@@ -521,6 +561,85 @@ __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ log
     const int t = blockIdx.x * 4 + wave;
     if (t >= S) return;
     topk_one_token<J>(logits + (size_t)t * E, t, E, k, gate_fn, norm, topk_idx, topk_w, lane);
+}
+
+// The same for up to 64 experts, sixteen lanes to a token: lane l of a row of sixteen keeps the logits of experts l, l + 16, l + 32 and
+// l + 48, so that a candidate travels through four DPP moves instead of four and three lane reads, and a wavefront selects for four tokens
+// at a time.  The softmax's sum pairs the experts as the wavefront's butterfly does (e with e + 32, then + 16 in the lane, 8, 4, 2, 1
+// between them): the same bits.  64 experts, k 6, logits included, a token a wavefront / this: 16384 tokens 79 / 69 us, 8192 43 / 39, 4000
+// 24.0 / 22.5, up to 1000 no difference.
+struct Cand16 {
+    float key, v;
+    int i;
+};
+template <int CTRL>
+__device__ __forceinline__ void better16(Cand16& c) {
+    Cand16 o;
+    o.key = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c.key), CTRL, 0xF, 0xF, false));
+    o.v = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c.v), CTRL, 0xF, 0xF, false));
+    o.i = __builtin_amdgcn_update_dpp(0, c.i, CTRL, 0xF, 0xF, false);
+    if (o.key > c.key || (o.key == c.key && o.i < c.i)) c = o;
+}
+__global__ __launch_bounds__(256) void topk16_kernel(const float* __restrict__ logits, int S, int E, int k, int gate_fn, int norm,
+                                                     int32_t* __restrict__ topk_idx, float* __restrict__ topk_w) {
+    const int lane = threadIdx.x & 15, t = blockIdx.x * 16 + (threadIdx.x >> 4);
+    const bool live = t < S;                       // (a token past the end keeps the lane exchanges company)
+    const float* row = logits + (size_t)min(t, S - 1) * E;
+    float v[4];
+    unsigned avail = 0;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int e = 16 * m + lane;
+        v[m] = 0.0f;
+        if (e < E) {
+            v[m] = row[e];
+            avail |= 1u << m;
+        }
+    }
+    const unsigned valid = avail;
+    float my_l = 0.0f, top_l = 0.0f;
+    int my_i = 0;
+    for (int r = 0; r < k; ++r) {
+        Cand16 c{-INFINITY, 0.0f, 0x7FFFFFFF};
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const float key = v[m] != v[m] ? -INFINITY : v[m];
+            const int i = 16 * m + lane;
+            if (((avail >> m) & 1u) && (key > c.key || (key == c.key && i < c.i))) c = Cand16{key, v[m], i};
+        }
+        better16<0xB1>(c);                         // quad_perm [1,0,3,2]: lane ^ 1
+        better16<0x4E>(c);                         // quad_perm [2,3,0,1]: lane ^ 2
+        better16<0x141>(c);                        // row_half_mirror: i <-> 7 - i within 8 lanes
+        better16<0x140>(c);                        // row_mirror: i <-> 15 - i
+        if ((c.i & 15) == lane) avail &= ~(1u << ((c.i >> 4) & 31));
+        if (lane == r) { my_l = c.v; my_i = c.i; }
+        if (r == 0) top_l = c.v;
+    }
+    float p = 0.0f;
+    if (gate_fn == MOE_GATE_SOFTMAX) {
+        float e[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            e[m] = (valid >> m) & 1u ? expf(v[m] - top_l) : 0.0f;
+            asm volatile("" : "+v"(e[m]));         // a value of its own: the library's last product must not melt into the sum
+        }
+        float part = (e[0] + e[2]) + (e[1] + e[3]);
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) part = part + __shfl_xor(part, off, 16);
+        if (lane < k) p = expf(my_l - top_l) / part;
+    } else {
+        if (lane < k) p = 1.0f / (1.0f + expf(-my_l));
+    }
+    if (norm) {
+        float sum = p;
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) sum = sum + __shfl_xor(sum, off, 16);
+        p = p / sum;
+    }
+    if (live && lane < k) {
+        topk_idx[(size_t)t * k + lane] = my_i;
+        topk_w[(size_t)t * k + lane] = p;
+    }
 }
 
 // Router statistics for a load-balancing loss.  Block b, wavefront w takes tokens (4b + w) + 4*gridDim.x*i; a lane
@@ -628,8 +747,8 @@ static hipError_t launch_gate_logits(const void* x, const void* gate_w, const fl
     if (act_dtype != MOE_DTYPE_F32) {
         hipError_t e = hipSuccess;
         const bool taken = act_dtype == MOE_DTYPE_FP16
-            ? launch_gate_mfma<f16_s>(x, gate_w, gate_bias, logits, keep_logits, S, H, E, opt.gate_mfma, tk, opt.gate_fused_topk == 1, fused, st, &e)
-            : launch_gate_mfma<bf16_s>(x, gate_w, gate_bias, logits, keep_logits, S, H, E, opt.gate_mfma, tk, opt.gate_fused_topk == 1, fused, st, &e);
+            ? launch_gate_mfma<f16_s>(x, gate_w, gate_bias, logits, S, H, E, opt.gate_mfma, st, &e)
+            : launch_gate_mfma<bf16_s>(x, gate_w, gate_bias, logits, S, H, E, opt.gate_mfma, st, &e);
         if (taken) return e;
     }
     bool rows_in_registers = E >= 32 && (int64_t)S * E >= ((int64_t)1 << 19);
@@ -647,7 +766,7 @@ static hipError_t launch_gate_logits(const void* x, const void* gate_w, const fl
 static hipError_t launch_topk(const float* logits, int S, int E, int k, int gate_fn, int norm, int32_t* topk_idx,
                        float* topk_w, hipStream_t st) {
     const unsigned grid = (unsigned)((S + 3) / 4);
-    if (E <= 64) topk_kernel<1><<<grid, 256, 0, st>>>(logits, S, E, k, gate_fn, norm, topk_idx, topk_w);
+    if (E <= 64) topk16_kernel<<<(unsigned)((S + 15) / 16), 256, 0, st>>>(logits, S, E, k, gate_fn, norm, topk_idx, topk_w);
     else if (E <= 128) topk_kernel<2><<<grid, 256, 0, st>>>(logits, S, E, k, gate_fn, norm, topk_idx, topk_w);
     else if (E <= 256) topk_kernel<4><<<grid, 256, 0, st>>>(logits, S, E, k, gate_fn, norm, topk_idx, topk_w);
     else topk_kernel<kMaxExperts / kWave><<<grid, 256, 0, st>>>(logits, S, E, k, gate_fn, norm, topk_idx, topk_w);

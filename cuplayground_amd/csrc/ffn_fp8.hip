@@ -9,14 +9,18 @@
 // the kernel is a weight streamer.  A task is (expert, 16-token row block, chunk of weight rows -- 64 gate + 64 up rows
 // per sub-tile of a SwiGLU up projection, 128 rows of one matrix otherwise):
 //   * v_mfma_f32_16x16x32_bf16 with the weights as the "A" operand (16 weight rows) and up to 16 token rows
-//     as "B"; e4m3 bytes are widened to bf16 in registers (exact) right before the MFMA;
-//   * each lane fetches 16 contiguous weight bytes per 64-wide k slab, so a wavefront load covers 64
-//     contiguous bytes of 16 rows and the four wavefronts of a workgroup, which interleave 128-wide k
+//     as "B"; e4m3 bytes are widened to bf16 in registers (exact) right before the MFMA, two an instruction (by way of fp32 and
+//     byte masks, five operations for two, the vector ALU bounded every task: whole layers with the lines' twelve moves for 2 KB,
+//     us, that / this: 256 experts of 7168 x 2048, one token 278 / 188, 64 tokens 1532 / 1527; 8 of 4096 x 14336, 20 tokens 377 / 264;
+//     before either: 245, 1665, 339);
+//   * each lane fetches 16 contiguous weight bytes of a 128-wide k block an instruction, so that a wavefront's load covers whole
+//     lines of eight rows (stream_lines.hpp), and the four wavefronts of a workgroup, which interleave the k
 //     blocks, together sweep 512 contiguous bytes of each row;
 //   * each wavefront multiplies its k blocks against all 8 row groups of the task (activation fragments are
 //     reused 8 times), scales the 128-deep partial sums by the block scale in fp32, and the four
 //     wavefronts' sums meet in LDS for the epilogue (bias, SwiGLU, bf16 store).
 #include "ffn_common.hpp"
+#include "stream_lines.hpp"
 
 namespace moe355 {
 namespace {
@@ -44,18 +48,16 @@ union Frag {
     uint4 q;
 };
 
-// 8 e4m3 bytes -> 8 bf16.  Every e4m3 value is exactly representable in bf16, so truncating the fp32
-// conversion result is exact.
+// 8 e4m3 bytes -> 8 bf16 (exact), two an instruction.
 __device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+    const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
     Frag f;
-    const uint32_t w[2] = {lo, hi};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], false);
-        const f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], true);
-        f.u[2 * i] = (__float_as_uint(a[0]) >> 16) | (__float_as_uint(a[1]) & 0xFFFF0000u);
-        f.u[2 * i + 1] = (__float_as_uint(b[0]) >> 16) | (__float_as_uint(b[1]) & 0xFFFF0000u);
-    }
+    f.u[0] = __builtin_bit_cast(uint32_t, a);
+    f.u[1] = __builtin_bit_cast(uint32_t, b);
+    f.u[2] = __builtin_bit_cast(uint32_t, c);
+    f.u[3] = __builtin_bit_cast(uint32_t, d);
     return f.v;
 }
 
@@ -73,6 +75,8 @@ struct Fp8Task {
     bool publish;   // rows are read by other workgroups of the same launch
 };
 
+// COLD: the weights are too many for the caches, and hardly an expert has more rows than a block: fetched once and not kept.
+template <bool COLD>
 __device__ __forceinline__ void fp8_tile(const Fp8Task& t, float* red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int idx = lane & 15, kg = lane >> 4;
@@ -82,20 +86,21 @@ __device__ __forceinline__ void fp8_tile(const Fp8Task& t, float* red) {
     const int64_t src_row = t.gather ? (int64_t)t.gather[ar] : t.a_row0 + ar;
     const uint16_t* xp = t.a_base + src_row * t.K + 16 * kg;
 
-    // weight rows of this lane, one per group
+    // the 16 weight rows of every group
     const uint8_t* wp[QGROUPS];
+    const int64_t first = line_first(lane, t.K), second = line_second(lane, t.K);
 #pragma unroll
     for (int g = 0; g < QGROUPS; ++g) {
         int n;
         const uint8_t* base;
         if (t.paired) {
-            n = t.c0 + (g & 3) * 16 + idx;
+            n = t.c0 + (g & 3) * 16;
             base = t.w[g >> 2];
         } else {
-            n = t.c0 + g * 16 + idx;
+            n = t.c0 + g * 16;
             base = t.w[0];
         }
-        wp[g] = base + (int64_t)n * t.K + 16 * kg;
+        wp[g] = base + (int64_t)n * t.K + first;
     }
 
     f32x4 acc[QGROUPS];
@@ -105,11 +110,12 @@ __device__ __forceinline__ void fp8_tile(const Fp8Task& t, float* red) {
     const int KB = t.K >> 7;
     for (int kb = wave; kb < KB; kb += QWAVES) {
         const int k0 = kb << 7;
-        uint4 wv[QGROUPS][2];
+        line_u32x4 wv[QGROUPS][2];
 #pragma unroll
-        for (int g = 0; g < QGROUPS; ++g)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) wv[g][s] = *reinterpret_cast<const uint4*>(wp[g] + k0 + 64 * s);
+        for (int g = 0; g < QGROUPS; ++g) {
+            wv[g][0] = load_piece<COLD>(wp[g] + k0);
+            wv[g][1] = load_piece<COLD>(wp[g] + k0 + second);
+        }
         Frag xa[2][2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -119,6 +125,7 @@ __device__ __forceinline__ void fp8_tile(const Fp8Task& t, float* red) {
         const float sc0 = t.s[0][kb], sc1 = t.s[1][kb];
 #pragma unroll
         for (int g = 0; g < QGROUPS; ++g) {
+            line_pieces(wv[g][0], wv[g][1], wv[g][0], wv[g][1]);
             f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
@@ -236,6 +243,7 @@ __device__ __forceinline__ Fp8Task resolve_fp8(const FfnArgs& a, const Task& t, 
     return p;
 }
 
+template <bool COLD>
 __global__ __launch_bounds__(256) void ffn_tiled_fp8_kernel(FfnArgs a, int phase) {
     __shared__ float red[QWAVES * QGROUPS * 4 * 64];
     __shared__ int s_list[1 + QBM];
@@ -244,11 +252,12 @@ __global__ __launch_bounds__(256) void ffn_tiled_fp8_kernel(FfnArgs a, int phase
     if (!tiled_task(a, phase, blockIdx.x, t)) return;
     for (int sub = 0; sub < (phase ? QSUB1 : QSUB); ++sub) {
         const Fp8Task p = resolve_fp8(a, t, sub, phase == 1 && a.arrive);
-        if (p.c0 < p.N) fp8_tile(p, red);
+        if (p.c0 < p.N) fp8_tile<COLD>(p, red);
     }
     if (phase == 1 && a.arrive) combine_arrivals<bf16_s>(combine_args(a), t.row0, t.rows, t.ntile, t.ntile * QSUB1 * QN1, QSUB1 * QN1, s_list);
 }
 
+template <bool COLD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ffn_persistent_fp8_kernel(FfnArgs a) {
     __shared__ float red[QWAVES * QGROUPS * 4 * 64];
     __shared__ int s_task, s_ok;
@@ -269,7 +278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         for (int sub = 0; sub < (t.phase ? QSUB1 : QSUB); ++sub) {
             const Fp8Task p = resolve_fp8(a, t, sub, t.phase == 0 || publish_y(a));
             if (p.c0 >= p.N) continue;
-            if (ok) fp8_tile(p, red);
+            if (ok) fp8_tile<COLD>(p, red);
             else poison_tile(p.c_base, p.rows, p.N, p.c0, QN1, 2);
         }
         if (a.task_trace) trace_task(a.task_trace, a.task_trace_cap, t.phase, t.expert, t.mtile, t.ntile, t.rows, started);
@@ -288,20 +297,27 @@ int fp8_block_n1() { return QN1 * QSUB1; }
 
 int ffn_persistent_occupancy_fp8() {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&ffn_persistent_fp8_kernel), 256,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&ffn_persistent_fp8_kernel<true>), 256,
                                                      0) != hipSuccess || n < 1)
         n = 1;
     return n;
 }
 
-hipError_t launch_ffn_fp8(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
+template <bool COLD>
+static hipError_t launch_streamer(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
     if (blocks > 0) {
-        ffn_persistent_fp8_kernel<<<blocks, 256, 0, st>>>(a);
+        ffn_persistent_fp8_kernel<COLD><<<blocks, 256, 0, st>>>(a);
     } else {
-        ffn_tiled_fp8_kernel<<<tiled_grid(max_mtiles, nnt0, a.groups), 256, 0, st>>>(a, 0);
-        ffn_tiled_fp8_kernel<<<tiled_grid(max_mtiles, nnt1, a.groups), 256, 0, st>>>(a, 1);
+        ffn_tiled_fp8_kernel<COLD><<<tiled_grid(max_mtiles, nnt0, a.groups), 256, 0, st>>>(a, 0);
+        ffn_tiled_fp8_kernel<COLD><<<tiled_grid(max_mtiles, nnt1, a.groups), 256, 0, st>>>(a, 1);
     }
     return hipGetLastError();
+}
+hipError_t launch_ffn_fp8(const FfnArgs& a, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
+    // Experts of more rows than a block read their weights again for every block: with 25 rows each (8 experts of 4096 x 14336, 100 tokens)
+    // kept / not kept 477 / 522 us, with 8 rows (256 of 7168 x 2048, 256 tokens) 1974 / 1825.
+    const bool cold = stream_cold(a, 1) && (int64_t)a.S * a.k <= (int64_t)a.E * (QBM / 2);
+    return cold ? launch_streamer<true>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch_streamer<false>(a, max_mtiles, nnt0, nnt1, blocks, st);
 }
 
 }  // namespace moe355

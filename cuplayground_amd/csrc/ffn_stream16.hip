@@ -7,8 +7,8 @@
 //   * it owns 16 * CG output columns -- as many weight rows, or gate and up rows with SwiGLU -- over the whole contraction
 //     dimension, as the "A" operand of v_mfma_f32_16x16x32; the "B" operand is up to NT groups of 16 token rows, read through
 //     the caches that the neighbouring wavefronts read them through.  No LDS, no barrier;
-//   * weights go from memory into the fragment registers in which the matrix instruction wants them (16 bytes a lane, 64
-//     contiguous bytes of 16 rows an instruction, 8 KB in flight while the 8 KB before are multiplied);
+//   * weights go from memory into the fragment registers in which the matrix instruction wants them (whole lines of eight rows
+//     an instruction, two of which trade halves: stream_lines.hpp; 8 KB in flight while the 8 KB before are multiplied);
 //   * one accumulator per output element, added to in the order of k as in the tiles: the same bits as theirs, and no sums
 //     to bring together.
 // A workgroup is four wavefronts on neighbouring columns of one row block.
@@ -23,8 +23,9 @@
 //   12 of 1344 x 2752, GELU: 2 rows 105 / 63 / 69 / 76, 8 107 / 74 / 82 / 92, 16 106 / 102 / 92 / 99, 24 107 / 117 / 104 / 107
 // (4 rows of the first: 5.7 TB/s of weights behind about 30 us of routing, launches and combine.)  An expert with more rows
 // than a block had its weights read again for every block in these, which is where the steps upwards come from.  NT 4 was behind
-// the tile from 24 rows on the first and the third of these.  Non-temporal weight loads lose 1 to 15 % (an instruction takes half of a 128-byte
-// line; its other half must still be in the cache for the next one).  The task queue with its written-through rows and pops
+// the tile from 24 rows on the first and the third of these.  Since then the weights come in whole lines and, where they are more than
+// the memory-side cache holds, are not kept (stream_lines.hpp), us, before / this: 8 of 4096 x 14336, 0.25 rows each 177 / 171, 4 525 / 484, 10 586 /
+// 509, 16 618 / 541; 64 of 2048 x 1408, 1.5 rows 193 / 175, 9 251 / 213, 16 269 / 231; 16 of 2048 x 2048, 2 rows 68 / 66.  The task queue with its written-through rows and pops
 // of this much shorter tasks costs more than the overlap of the projections gives: 645 us against 520 (4 rows of the first),
 // 158 against 81 (4 of the second).
 //
@@ -41,6 +42,7 @@
 // What is left behind the tile are routers that send nearly every one of 96 tokens and more to the same few of many experts.
 #include "act_deriv.hpp"
 #include "ffn_common.hpp"
+#include "stream_lines.hpp"
 
 namespace moe355 {
 namespace {
@@ -53,9 +55,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int STHREADS = 256;
 constexpr int kGroupRows = 64, kGroupStage = kGroupRows * 128;      // rows of a group, bytes of 64 values of k of theirs
 
-template <class ET, int NT, int CG>
+// COLD: the weights are too many for the caches: they are fetched once and not kept.
+template <class ET, int NT, int CG, bool COLD_>
 struct Stream {
     using Elem = ET;
+    static constexpr bool COLD = COLD_;
     static constexpr bool F16 = std::is_same<ET, f16_s>::value;
     static constexpr int T = NT;             // groups of 16 token rows
     static constexpr int BM = 16 * NT;
@@ -147,9 +151,10 @@ __device__ __forceinline__ void stream_tile(const StreamTask& t) {
     const int c0 = t.n0 + 16 * CG * wave;
     if (c0 >= t.N) return;
 
-    const uint16_t* wp[G];
+    const char* wp[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) wp[g] = t.w[g / CG] + (int64_t)(c0 + 16 * (g % CG) + idx) * t.K + 8 * kg;
+    for (int g = 0; g < G; ++g) wp[g] = reinterpret_cast<const char*>(t.w[g / CG] + (int64_t)(c0 + 16 * (g % CG)) * t.K) + line_first(lane, 2 * (int64_t)t.K);
+    const int64_t second = line_second(lane, 2 * (int64_t)t.K);
     // rows behind the block's last one read row 0 again and are never stored
     const uint16_t* xp[NT];
 #pragma unroll
@@ -169,11 +174,18 @@ __device__ __forceinline__ void stream_tile(const StreamTask& t) {
     // slabs behind the last one read it again (and are not multiplied)
     auto load_w = [&](u32x4 (&d)[G][U], int s0) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = min(s0 + u, slabs - 1) << 5;
+        for (int u = 0; u < U; u += 2) {       // (a line is two slabs; K is a multiple of 64, U even)
+            const int k = min(s0 + u, slabs - 2) << 6;
 #pragma unroll
-            for (int g = 0; g < G; ++g) d[g][u] = *reinterpret_cast<const u32x4*>(wp[g] + k);
+            for (int g = 0; g < G; ++g) {
+                d[g][u] = load_piece<P::COLD>(wp[g] + k);
+                d[g][u + 1] = load_piece<P::COLD>(wp[g] + k + second);
+            }
         }
+    };
+    auto settle = [&](int u) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) line_pieces(w[g][u], w[g][u + 1], w[g][u], w[g][u + 1]);
     };
     auto load_x = [&](int s0) {
 #pragma unroll
@@ -196,7 +208,11 @@ __device__ __forceinline__ void stream_tile(const StreamTask& t) {
         if ((c + 1) * U < slabs) load_w(wn, (c + 1) * U);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < U; ++u) multiply(u);
+        for (int u = 0; u < U; u += 2) {
+            settle(u);
+            multiply(u);
+            multiply(u + 1);
+        }
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -205,8 +221,12 @@ __device__ __forceinline__ void stream_tile(const StreamTask& t) {
     if (left) {
         load_x(full * U);
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (u < left) multiply(u);
+        for (int u = 0; u < U; u += 2)
+            if (u < left) {
+                settle(u);
+                multiply(u);
+                multiply(u + 1);
+            }
     }
 
     stream_store<P, MATS, NT>(t, c0, acc);
@@ -261,7 +281,7 @@ __device__ __forceinline__ void stream_group(const StreamTask& t, unsigned char*
     const int c0 = t.n0 + 16 * CG * wave;
     const bool live = c0 < t.N;                  // a wavefront without columns helps to bring the rows
     // 32-bit offsets from bases that are the same in every lane: operands are below 4 GiB (large_tile_ok)
-    const uint32_t w_off = (uint32_t)(idx * t.K + 8 * kg) * 2;
+    const uint32_t w_off = (uint32_t)line_first(lane, 2 * (int64_t)t.K), w_second = w_off + (uint32_t)line_second(lane, 2 * (int64_t)t.K);
     uint32_t x_off[PASSES];
 #pragma unroll
     for (int n = 0; n < PASSES; ++n) {
@@ -291,8 +311,8 @@ __device__ __forceinline__ void stream_group(const StreamTask& t, unsigned char*
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const char* base = reinterpret_cast<const char*>(t.w[g / CG] + (int64_t)((live ? c0 : 0) + 16 * (g % CG)) * t.K + k);
-#pragma unroll
-            for (int u = 0; u < 2; ++u) d[g][u] = *reinterpret_cast<const u32x4*>(base + 64 * u + w_off);
+            d[g][0] = load_piece<P::COLD>(base + w_off);
+            d[g][1] = load_piece<P::COLD>(base + w_second);
         }
     };
     auto put_x = [&](const u32x4 (&d)[PASSES], int stage) {
@@ -302,6 +322,8 @@ __device__ __forceinline__ void stream_group(const StreamTask& t, unsigned char*
     // slab's rows lie in stage S; its successor's go into the other one, which was last read in front of the last barrier
     auto step = [&](auto S, int slab) {
         constexpr int st = decltype(S)::value;
+#pragma unroll
+        for (int g = 0; g < G; ++g) line_pieces(w[st][g][0], w[st][g][1], w[st][g][0], w[st][g][1]);
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -428,17 +450,22 @@ int occupancy() {
 }  // namespace
 
 // The two forms: 0 = blocks of 16 rows, tasks of 64 columns; 1 = 32 rows, 128 columns.
-template <class ET> using Narrow = Stream<ET, 1, 1>;
-template <class ET> using Wide = Stream<ET, 2, 2>;
+template <class ET, bool COLD> using Narrow = Stream<ET, 1, 1, COLD>;
+template <class ET, bool COLD> using Wide = Stream<ET, 2, 2, COLD>;
 
-int stream16_block_m(int form) { return form ? Wide<bf16_s>::BM : Narrow<bf16_s>::BM; }
-int stream16_block_n(int form) { return form ? Wide<bf16_s>::BN : Narrow<bf16_s>::BN; }
-int ffn_persistent_occupancy_stream16(int form) { return form ? occupancy<Wide<bf16_s>>() : occupancy<Narrow<bf16_s>>(); }
+int stream16_block_m(int form) { return form ? Wide<bf16_s, true>::BM : Narrow<bf16_s, true>::BM; }
+int stream16_block_n(int form) { return form ? Wide<bf16_s, true>::BN : Narrow<bf16_s, true>::BN; }
+int ffn_persistent_occupancy_stream16(int form) { return form ? occupancy<Wide<bf16_s, true>>() : occupancy<Narrow<bf16_s, true>>(); }
 
+template <class ET, bool COLD>
+static hipError_t launch_form(const FfnArgs& a, int form, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
+    return form ? launch<Wide<ET, COLD>>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch<Narrow<ET, COLD>>(a, max_mtiles, nnt0, nnt1, blocks, st);
+}
 // blocks > 0: workgroups of the task queue; 0: a launch per projection.
 hipError_t launch_ffn_stream16(const FfnArgs& a, int form, bool f16, int max_mtiles, int nnt0, int nnt1, int blocks, hipStream_t st) {
-    if (f16) return form ? launch<Wide<f16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch<Narrow<f16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st);
-    return form ? launch<Wide<bf16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st) : launch<Narrow<bf16_s>>(a, max_mtiles, nnt0, nnt1, blocks, st);
+    const bool cold = stream_cold(a, 2);
+    if (f16) return cold ? launch_form<f16_s, true>(a, form, max_mtiles, nnt0, nnt1, blocks, st) : launch_form<f16_s, false>(a, form, max_mtiles, nnt0, nnt1, blocks, st);
+    return cold ? launch_form<bf16_s, true>(a, form, max_mtiles, nnt0, nnt1, blocks, st) : launch_form<bf16_s, false>(a, form, max_mtiles, nnt0, nnt1, blocks, st);
 }
 
 }  // namespace moe355

@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_gate_wgrad_rows", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_gemm_pair", "moe_expert_gemm_kn_pair", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_gate_wgrad_rows", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -160,6 +160,8 @@ def load_library():
     L.moe_expert_gemm_act_backward.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp, C.c_size_t, vp]
     L.moe_expert_gemm_act_backward_supported.argtypes = [vp, C.POINTER(C.c_int32)]
     L.moe_expert_gemm_kn.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp]
+    L.moe_expert_gemm_pair.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp, C.c_size_t, vp]
+    L.moe_expert_gemm_kn_pair.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp]
     L.moe_expert_gemm_kn_supported.argtypes = [vp, i32, i32, C.POINTER(C.c_int32)]
     L.moe_act_backward.argtypes = [vp, vp, vp, vp, i64, vp, vp, vp]
     L.moe_bias_grad.argtypes = [vp, vp, vp, vp, i32, vp, vp]
@@ -592,6 +594,34 @@ class MoELayer:
         _check(self.L.moe_expert_gemm_kn(self._h, _ptr(a_rows), _ptr(w), _ptr(u_rows), _ptr(g_rows), _ptr(expert_count),
                                          _ptr(expert_offset), N, K, _ptr(out), _ptr(out1), _stream()), "moe_expert_gemm_kn")
         return out if u_rows is None else (out, out1)
+
+    def expert_gemm_pair(self, a_rows, w0, w1, expert_count, expert_offset):
+        """(a_rows[r] . w0[e(r)]^T, a_rows[r] . w1[e(r)]^T), w0 and w1 [E,N,K].  Rows of no expert are not written."""
+        import torch
+        N, K = w0.shape[1], w0.shape[2]
+        _operand("a_rows", a_rows, self.act_dtype, self.S * self.k * K)
+        for name, t in (("w0", w0), ("w1", w1)):
+            _operand(name, t, self.act_dtype, self.E * N * K)
+        out = [torch.empty(a_rows.shape[0], N, dtype=a_rows.dtype, device=a_rows.device) for _ in range(2)]
+        sc = self.backward_scratch()
+        _check(self.L.moe_expert_gemm_pair(self._h, _ptr(a_rows), _ptr(w0), _ptr(w1), _ptr(expert_count), _ptr(expert_offset), N, K, _ptr(out[0]),
+                                           _ptr(out[1]), _ptr(sc), sc.numel(), _stream()), "moe_expert_gemm_pair")
+        return out
+
+    def expert_gemm_kn_pair(self, a0_rows, a1_rows, w0, w1, expert_count, expert_offset):
+        """(a0_rows[r] . w0[e(r)], a1_rows[r] . w1[e(r)]), w0 and w1 [E,K,N].  Rows of no expert are not written."""
+        import torch
+        K, N = w0.shape[1], w0.shape[2]
+        for name, t in (("a0_rows", a0_rows), ("a1_rows", a1_rows)):
+            _operand(name, t, self.act_dtype, self.S * self.k * K)
+        for name, t in (("w0", w0), ("w1", w1)):
+            _operand(name, t, self.act_dtype, self.E * K * N)
+        for name, t in (("expert_count", expert_count), ("expert_offset", expert_offset)):
+            _operand(name, t, torch.int32, self.E)
+        out = [torch.empty(a0_rows.shape[0], N, dtype=a0_rows.dtype, device=a0_rows.device) for _ in range(2)]
+        _check(self.L.moe_expert_gemm_kn_pair(self._h, _ptr(a0_rows), _ptr(a1_rows), _ptr(w0), _ptr(w1), _ptr(expert_count), _ptr(expert_offset), N, K,
+                                              _ptr(out[0]), _ptr(out[1]), _stream()), "moe_expert_gemm_kn_pair")
+        return out
 
     def expert_wgrad(self, dy_rows, a_rows, expert_count, expert_offset, out=None):
         """dw[e] [N,K] = sum over expert e's rows of dy_rows[r,:N]^T a_rows[r,:K]."""

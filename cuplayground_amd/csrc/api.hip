@@ -1235,6 +1235,30 @@ int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const v
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 
+int moe_expert_gemm_pair(moe_handle* h, const void* a_rows, const void* w0, const void* w1, const int32_t* expert_count,
+                         const int32_t* expert_offset, int32_t N, int32_t K, void* out0_rows, void* out1_rows, void* scratch, size_t scratch_bytes,
+                         void* stream) {
+    if (!h || !a_rows || !w0 || !w1 || !expert_count || !expert_offset || !out0_rows || !out1_rows) return MOE_ERR_BAD_ARGUMENT;
+    const int rc = check_backward_call(h, N, K, scratch, scratch_bytes);
+    if (rc) return rc;
+    const hipError_t e = launch_expert_gemm_pair(a_rows, w0, w1, expert_count, expert_offset, h->d.A, h->d.E, N, K, h->d.act_dtype, h->opt, out0_rows,
+                                                 out1_rows, scratch, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
+int moe_expert_gemm_kn_pair(moe_handle* h, const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* expert_count,
+                            const int32_t* expert_offset, int32_t N, int32_t K, void* out0_rows, void* out1_rows, void* stream) {
+    if (!h || !a0_rows || !a1_rows || !w0 || !w1 || !expert_count || !expert_offset || !out0_rows || !out1_rows) return MOE_ERR_BAD_ARGUMENT;
+    if (((uintptr_t)a0_rows | (uintptr_t)a1_rows | (uintptr_t)w0 | (uintptr_t)w1 | (uintptr_t)out0_rows | (uintptr_t)out1_rows) % 16) return MOE_ERR_BAD_ARGUMENT;
+    int32_t supported = 0;
+    const int rc = moe_expert_gemm_kn_supported(h, N, K, &supported);
+    if (rc) return rc;
+    if (!supported) return MOE_ERR_UNSUPPORTED;
+    const hipError_t e = launch_expert_gemm_kn_pair(a0_rows, a1_rows, w0, w1, expert_count, expert_offset, h->d.A, h->d.E, N, K, h->d.act_dtype, out0_rows,
+                                                    out1_rows, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
 int moe_expert_wgrad(moe_handle* h, const void* dy_rows, const void* a_rows, const int32_t* expert_count,
                      const int32_t* expert_offset, int32_t N, int32_t K, void* dw, void* scratch, size_t scratch_bytes,
                      void* stream) {

@@ -19,7 +19,11 @@
 namespace moe355 {
 
 bool grouped_hand_ok(int64_t A, int N, int K);
-int grouped_gemm_tile_16(int64_t A, int E, int N, int K);
+int grouped_gemm_tile_16(int64_t A, int E, int N, int K, int products);
+hipError_t launch_grouped_gemm_pair_16(const void* a_rows, const void* w, const void* w1, void* out, void* out1, const int32_t* count,
+                                       const int32_t* offset, int tile, int64_t A, int E, int N, int K, bool f16, hipStream_t st);
+hipError_t launch_grouped_gemm_kn_pair_16(const void* a_rows, const void* a1_rows, const void* w, const void* w1, void* out, void* out1,
+                                          const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, bool f16, hipStream_t st);
 hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const int32_t* count,
                                   const int32_t* offset, int tile, int64_t A, int E, int N, int K, int act, bool f16, hipStream_t st);
 hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int32_t* poff, int E, int N, int K,
@@ -691,6 +695,13 @@ ScratchTables scratch_tables(void* scratch, int64_t A, int E) {
 }
 }  // namespace
 
+// Tile of 16-bit products: 1: 256 x 256, 2: 128 x 256, 0: 128 x 128.
+static int product_tile(int64_t A, int E, int N, int K, int products, const moe_options& opt) {
+    const int v = opt.grouped_tile;
+    if (v == 0) return 0;
+    return (v == 1 || v == 2) && grouped_hand_ok(A, N, K) ? v : grouped_gemm_tile_16(A, E, N, K, products);
+}
+
 // out_rows[r,:] = act(a_rows[r,:] . w[e(r)]^T + bias[e(r)]); scratch: the row-block table of an fp32 product (16-bit ones
 // find their row blocks themselves).
 // dtype: the storage type of every operand (MOE_DTYPE_F32, _BF16 or _FP16).
@@ -709,13 +720,18 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
         return (mfma ? launch_grouped_gemm_f32_tile : launch_grouped_gemm_f32)(a_rows, w, bias, out_rows, t.mtiles,
                                                                                t.num_mtiles, max_mtiles, N, K, act, st);
     }
-    int tile = grouped_gemm_tile_16(A, E, N, K);                       // 1: 256 x 256, 2: 128 x 256, 0: 128 x 128
-    if (opt.grouped_tile != MOE_OPT_AUTO) {
-        const int v = opt.grouped_tile;
-        if ((v == 1 || v == 2) && grouped_hand_ok(A, N, K)) tile = v;
-        if (v == 0) tile = 0;
-    }
+    const int tile = product_tile(A, E, N, K, 1, opt);
     return launch_grouped_gemm_16(a_rows, w, bias, out_rows, count, offset, tile, A, E, N, K, act, dtype == MOE_DTYPE_FP16, st);
+}
+
+// out0 = a_rows . w0[e]^T and out1 = a_rows . w1[e]^T: one launch on the hand-ordered tiles, else two calls.
+hipError_t launch_expert_gemm_pair(const void* a_rows, const void* w0, const void* w1, const int32_t* count, const int32_t* offset, int64_t A,
+                                   int E, int N, int K, int dtype, const moe_options& opt, void* out0, void* out1, void* scratch, hipStream_t st) {
+    const int tile = dtype == MOE_DTYPE_F32 ? 0 : product_tile(A, E, N, K, 2, opt);
+    if (tile) return launch_grouped_gemm_pair_16(a_rows, w0, w1, out0, out1, count, offset, tile, A, E, N, K, dtype == MOE_DTYPE_FP16, st);
+    const hipError_t e = launch_expert_gemm(a_rows, w0, nullptr, count, offset, A, E, N, K, MOE_ACT_NONE, dtype, opt, out0, scratch, st);
+    if (e != hipSuccess) return e;
+    return launch_expert_gemm(a_rows, w1, nullptr, count, offset, A, E, N, K, MOE_ACT_NONE, dtype, opt, out1, scratch, st);
 }
 
 // The tile the fused data gradient (product + activation derivative) runs on: 1 or 2 (the hand-ordered tiles), or 0 where
@@ -725,7 +741,7 @@ hipError_t launch_expert_gemm(const void* a_rows, const void* w, const void* bia
 int expert_gemm_dact_tile(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
     if (dtype != MOE_DTYPE_BF16 && dtype != MOE_DTYPE_FP16) return 0;
     const bool hand_ok = N % 256 == 0 && K % 128 == 0 && grouped_hand_ok(A, N, K);
-    int tile = hand_ok ? grouped_gemm_tile_16(A, E, N, K) : 0;
+    int tile = hand_ok ? grouped_gemm_tile_16(A, E, N, K, 1) : 0;
     if (opt.grouped_tile != MOE_OPT_AUTO) {
         const int v = opt.grouped_tile;
         if ((v == 1 || v == 2) && hand_ok) tile = v;
@@ -772,6 +788,14 @@ hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* 
     const auto pass = f16 ? &act_backward_rows_kernel<f16_s> : &act_backward_rows_kernel<bf16_s>;
     pass<<<grid, 256, 0, st>>>((const uint16_t*)u_rows, (const uint16_t*)g_rows, count, offset, E, A, N, hidden_act, (uint16_t*)out_rows, (uint16_t*)out1_rows);
     return hipGetLastError();
+}
+
+// out0_rows = a0_rows . w0[e] and out1_rows = a1_rows . w1[e] in one launch, both as launch_expert_gemm_kn gives them.
+hipError_t launch_expert_gemm_kn_pair(const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* count,
+                                      const int32_t* offset, int64_t A, int E, int N, int K, int dtype, void* out0_rows, void* out1_rows, hipStream_t st) {
+    if (dtype == MOE_DTYPE_F32 || !stored_operands_ok(A, N, K)) return hipErrorNotSupported;
+    return launch_grouped_gemm_kn_pair_16(a0_rows, a1_rows, w0, w1, out0_rows, out1_rows, count, offset, grouped_kn_large(A, E, N, K, 2), A, E, N, K,
+                                          dtype == MOE_DTYPE_FP16, st);
 }
 
 // dw[e] [N,K] = dy_e^T . a_e, from the rows as they are (product_choice.hpp; not where option grouped_tile asks for a tile) or from

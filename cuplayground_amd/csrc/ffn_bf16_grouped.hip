@@ -89,6 +89,10 @@ __device__ __forceinline__ void grouped_tile(const TaskPtrs& p, unsigned char* s
 // reference's tile GEMM (mma.cuh:46-179) once per expert.  With the weight handed over in its K-major view this is the data
 // gradient of a projection (dX = dY . W).  DERIV: that of the down projection with the activation's derivative in its epilogue,
 // which hands on dU (and dG) instead of dH.  With gather and w1 the up projection of a layer.  One workgroup per tile (grouped_task).
+// Two products of one shape (a training step's up and gate projections, and their data gradients) share a launch as one of twice the
+// columns, the second product's behind the first's: each would end in a round of few tasks.  Two launches / one, us, projections and
+// data gradients: 16 experts of 2048 x 1408, 750 rows each 191 / 156 and 161 / 143; 4 of 2048 x 2560, 4096 rows 297 / 268, 283 / 269; 8 of
+// 1280 x 1664, 256 rows 42 / 33, 48 / 26; 16 of 1152 x 1920, 175 rows 46 / 36, 53 / 44; 16 of 1024 x 2560, 62 rows 39 / 40, 62 / 34.
 struct GroupedArgs {
     const uint16_t* a_rows;      // packed rows, or with gather the tokens
     const uint16_t* w;           // [E, N, K] (KN: [E, K, N])
@@ -105,6 +109,7 @@ struct GroupedArgs {
     const int32_t* gather;       // null, or the token of every packed row
     const uint16_t* w1;          // SwiGLU: the gate's weights ...
     const uint16_t* bias1;       // ... and biases, or null
+    const uint16_t* a1_rows;     // kSums with out1: a second product of the same shape, a1_rows and w1 into out1
 };
 template <class P, int EPI>
 __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a) {
@@ -112,20 +117,24 @@ __global__ __launch_bounds__(P::THREADS) void grouped_gemm_kernel(GroupedArgs a)
     constexpr int COLS = SWIGLU ? P::BN / 2 : P::BN;      // half of a SwiGLU tile's weight rows are gate rows
     extern __shared__ __align__(16) unsigned char smem[];
     const int N = a.N, K = a.K;
+    const int cols = (N + COLS - 1) / COLS;
+    const bool two = EPI == kSums && a.out1;
     GroupedTask t;
-    if (!grouped_task<P::BIG>(a.count, a.offset, a.E, (N + COLS - 1) / COLS, blockIdx.x, t)) return;
+    if (!grouped_task<P::BIG>(a.count, a.offset, a.E, two ? 2 * cols : cols, blockIdx.x, t)) return;
+    const bool second = two && t.ctile >= cols;
+    if (second) t.ctile -= cols;
     const int64_t at = (int64_t)t.row0 * N;
     TaskPtrs p;
-    p.a_base = a.a_rows;
+    p.a_base = second ? a.a1_rows : a.a_rows;
     p.gather = a.gather ? a.gather + t.row0 : nullptr;
     p.a_row0 = a.gather ? 0 : t.row0;
     p.a_ld = K;
-    p.b0 = a.w + (int64_t)t.expert * N * K;
+    p.b0 = (second ? a.w1 : a.w) + (int64_t)t.expert * N * K;
     p.b1 = SWIGLU ? a.w1 + (int64_t)t.expert * N * K : nullptr;
     p.b_ld = K;
     p.bias0 = !DERIV && a.bias ? a.bias + (int64_t)t.expert * N : nullptr;
     p.bias1 = SWIGLU && a.bias1 ? a.bias1 + (int64_t)t.expert * N : nullptr;
-    p.c_base = a.out + at;
+    p.c_base = (second ? a.out1 : a.out) + at;
     p.N = N;
     p.K = K;
     p.rows = t.rows;
@@ -485,11 +494,11 @@ hipError_t launch_gemm_dense_bf16(const void* A, const void* B, const void* bias
 
 // ---- building blocks of the backward pass (callers: csrc/backward.hip) ----
 bool grouped_hand_ok(int64_t A, int N, int K) { return A * K * 2 < kBufferLimit && hand_weights_ok(N, K); }
-// Tile of one grouped product, as for a layer: 1, 2, or 0 when an operand has 4 GiB or more.
-int grouped_gemm_tile_16(int64_t A, int E, int N, int K) {
+// Tile of one grouped product (or of `products` that share a launch), as for a layer: 1, 2, or 0 when an operand has 4 GiB or more.
+int grouped_gemm_tile_16(int64_t A, int E, int N, int K, int products) {
     if (!grouped_hand_ok(A, N, K)) return 0;
-    const int e = E > 0 ? E : 1;
-    return projection_cost(true, A, e, columns256(N), K) <= projection_cost(false, A, e, columns256(N), K) ? 1 : 2;
+    const int e = E > 0 ? E : 1, cols = products * columns256(N);
+    return projection_cost(true, A, e, cols, K) <= projection_cost(false, A, e, cols, K) ? 1 : 2;
 }
 
 template <class P, int EPI>
@@ -498,7 +507,8 @@ static hipError_t launch_grouped(const GroupedArgs& g, int64_t A, hipStream_t st
     hipError_t e = allow_lds(kernel, P::LDS_BYTES);
     if (e != hipSuccess) return e;
     constexpr int COLS = EPI == kSwiglu ? P::BN / 2 : P::BN;
-    const int64_t blocks = (A / P::BIG + g.E) * ((g.N + COLS - 1) / COLS) + kShareSlack;      // no expert has more than rows / BIG + 1 row blocks
+    const int64_t cols = (int64_t)((g.N + COLS - 1) / COLS) * (EPI == kSums && g.out1 ? 2 : 1);
+    const int64_t blocks = (A / P::BIG + g.E) * cols + kShareSlack;      // no expert has more than rows / BIG + 1 row blocks
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     kernel<<<(unsigned)blocks, P::THREADS, P::LDS_BYTES, st>>>(g);
     return hipGetLastError();
@@ -511,11 +521,19 @@ static hipError_t launch_grouped_tile(const GroupedArgs& g, int tile, int64_t A,
     return hipErrorInvalidValue;
 }
 
+// out = a_rows . w[e]^T and out1 = a_rows . w1[e]^T in one launch; tile: 1 or 2.
+hipError_t launch_grouped_gemm_pair_16(const void* a_rows, const void* w, const void* w1, void* out, void* out1, const int32_t* count,
+                                       const int32_t* offset, int tile, int64_t A, int E, int N, int K, bool f16, hipStream_t st) {
+    const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, nullptr, nullptr, (uint16_t*)out, (uint16_t*)out1,
+                        count, offset, E, N, K, MOE_ACT_NONE, (uint32_t)(A * K * 2), nullptr, (const uint16_t*)w1, nullptr, (const uint16_t*)a_rows};
+    return f16 ? launch_grouped_tile<true, kSums>(g, tile, A, st) : launch_grouped_tile<false, kSums>(g, tile, A, st);
+}
+
 // tile: 1 (256-row blocks), 2 (128-row blocks) or 0 (the 128 x 128 tile of the general loop).
 hipError_t launch_grouped_gemm_16(const void* a_rows, const void* w, const void* bias, void* out, const int32_t* count,
                                   const int32_t* offset, int tile, int64_t A, int E, int N, int K, int act, bool f16, hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, (const uint16_t*)bias, nullptr, nullptr, (uint16_t*)out, nullptr,
-                        count, offset, E, N, K, act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
+                        count, offset, E, N, K, act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr, nullptr};
     if (act == MOE_ACT_GELU) return f16 ? launch_grouped_tile<true, kGelu>(g, tile, A, st) : launch_grouped_tile<false, kGelu>(g, tile, A, st);
     return f16 ? launch_grouped_tile<true, kSums>(g, tile, A, st) : launch_grouped_tile<false, kSums>(g, tile, A, st);
 }
@@ -525,7 +543,7 @@ hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const
                                         const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
                                         int hidden_act, bool f16, hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)du,
-                        (uint16_t*)dg, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
+                        (uint16_t*)dg, count, offset, E, N, K, hidden_act, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr, nullptr};
     return f16 ? launch_grouped_tile<true, kDeriv>(g, tile, A, st) : launch_grouped_tile<false, kDeriv>(g, tile, A, st);
 }
 
@@ -538,12 +556,12 @@ template <class P>
 static hipError_t launch_ffn_split(const FfnArgs& a, const ExpertRows& rows, hipStream_t st) {
     const int64_t A = (int64_t)a.S * a.k;
     GroupedArgs g{(const uint16_t*)a.x, (const uint16_t*)a.w_up, (const uint16_t*)a.b_up, nullptr, nullptr, (uint16_t*)a.h, nullptr,
-                  rows.count, rows.offset, a.E, a.I, a.H, a.act, a.x_bytes, a.token_indices, (const uint16_t*)a.w_gate, (const uint16_t*)a.b_gate};
+                  rows.count, rows.offset, a.E, a.I, a.H, a.act, a.x_bytes, a.token_indices, (const uint16_t*)a.w_gate, (const uint16_t*)a.b_gate, nullptr};
     const hipError_t e = a.act == MOE_ACT_SWIGLU ? launch_grouped<P, kSwiglu>(g, A, st)
                          : a.act == MOE_ACT_GELU ? launch_grouped<P, kGelu>(g, A, st) : launch_grouped<P, kSums>(g, A, st);
     if (e != hipSuccess) return e;
     g = GroupedArgs{(const uint16_t*)a.h, (const uint16_t*)a.w_down, (const uint16_t*)a.b_down, nullptr, nullptr, (uint16_t*)a.y, nullptr,
-                    rows.count, rows.offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr};
+                    rows.count, rows.offset, a.E, a.H, a.I, MOE_ACT_NONE, a.h_bytes, nullptr, nullptr, nullptr, nullptr};
     return launch_grouped<P, kSums>(g, A, st);
 }
 static TwoLaunchShape two_launch_shape(const FfnArgs& a) { return TwoLaunchShape{(int64_t)a.S * a.k, a.E, a.H, a.I, a.act == MOE_ACT_SWIGLU}; }
@@ -610,8 +628,15 @@ hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const vo
                                      const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st) {
     const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, (const uint16_t*)u, (const uint16_t*)g_rows, (uint16_t*)out,
-                        (uint16_t*)out1, count, offset, E, N, K, u ? hidden_act : MOE_ACT_NONE, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr};
+                        (uint16_t*)out1, count, offset, E, N, K, u ? hidden_act : MOE_ACT_NONE, (uint32_t)(A * K * 2), nullptr, nullptr, nullptr, nullptr};
     if (u) return f16 ? launch_grouped_kn<true, kDeriv>(g, large, A, st) : launch_grouped_kn<false, kDeriv>(g, large, A, st);
+    return f16 ? launch_grouped_kn<true, kSums>(g, large, A, st) : launch_grouped_kn<false, kSums>(g, large, A, st);
+}
+// out = a . w[e] and out1 = a1 . w1[e] in one launch.
+hipError_t launch_grouped_gemm_kn_pair_16(const void* a_rows, const void* a1_rows, const void* w, const void* w1, void* out, void* out1,
+                                          const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, bool f16, hipStream_t st) {
+    const GroupedArgs g{(const uint16_t*)a_rows, (const uint16_t*)w, nullptr, nullptr, nullptr, (uint16_t*)out, (uint16_t*)out1,
+                        count, offset, E, N, K, MOE_ACT_NONE, (uint32_t)(A * K * 2), nullptr, (const uint16_t*)w1, nullptr, (const uint16_t*)a1_rows};
     return f16 ? launch_grouped_kn<true, kSums>(g, large, A, st) : launch_grouped_kn<false, kSums>(g, large, A, st);
 }
 

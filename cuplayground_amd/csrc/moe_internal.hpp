@@ -236,6 +236,10 @@ int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const mo
 hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
                                  const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows,
                                  void* out1_rows, hipStream_t st);
+hipError_t launch_expert_gemm_pair(const void* a_rows, const void* w0, const void* w1, const int32_t* count, const int32_t* offset, int64_t A,
+                                   int E, int N, int K, int dtype, const moe_options& opt, void* out0, void* out1, void* scratch, hipStream_t st);
+hipError_t launch_expert_gemm_kn_pair(const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* count,
+                                      const int32_t* offset, int64_t A, int E, int N, int K, int dtype, void* out0_rows, void* out1_rows, hipStream_t st);
 hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const int32_t* count, const int32_t* offset,
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st);

@@ -65,9 +65,9 @@ inline bool grouped_kn_as_stored(int64_t A, int, int N, int K) { return stored_o
 // us, 256 / 128: 16 experts of 2048 x 2048, 512 rows each 81 / 86; of 1408 x 2048, 750 rows 77 / 90; 4 of 2560 x 2048, 4096 rows 133 / 157; 8 of
 // 1664 x 1280, 250 rows 40 / 25; 16 of 1920 x 1152, 175 rows 45 / 28; 8 of 2560 x 1024, 750 rows 59 / 40; 4 of them 55 / 34; 8 of 1536 x
 // 1920, 500 rows 41 / 46 (the 128 x 128 tiles that turned the operand round in registers: 107, 107, 230, 27, 41, 56, 37, 38).
-inline bool grouped_kn_large(int64_t A, int E, int N, int K) {
+inline bool grouped_kn_large(int64_t A, int E, int N, int K, int products = 1) {      // (`products` of this shape in one launch)
     const SplitBlocks n(A, std::max(E, 1));
-    const double cols = columns256(N);
+    const double cols = products * columns256(N);
     return split_us(n.full * cols, n.left * cols, K) < split_us(0, n.small * cols, K);
 }
 

@@ -119,8 +119,12 @@ def _expert_rows(x, w_up, w_gate, w_down, layer, token_indices, count, offset):
         out = torch.empty(a.shape[0], w.shape[1], dtype=a.dtype, device=a.device)
         return layer.expert_gemm(a, w, None, count, offset, api.ACT_NONE, out=out)
 
-    u = product(rows, w_up)
-    g = None if w_gate is None else product(rows, w_gate)
+    if w_gate is None:
+        u, g = product(rows, w_up), None
+    elif isinstance(layer, api.MoELayer):
+        u, g = layer.expert_gemm_pair(rows, w_up, w_gate, count, offset)
+    else:
+        u, g = product(rows, w_up), product(rows, w_gate)
     h = layer.act_forward(u, g, count, offset)
     return rows, u, g, h, product(h, w_down)
 
@@ -161,8 +165,11 @@ def _expert_gradients(layer, needs, dy, kept, count, offset):
             def data_gradient(d, w):                                                               # dA = dU . W_up
                 return layer.expert_gemm_kn(d, w, count, offset) if _as_stored(layer, w) else product(d, api.transpose(w))
 
-            da = data_gradient(du, w_up)
-            db = None if g is None else data_gradient(dg, w_gate)
+            if g is not None and _as_stored(layer, w_up) and _as_stored(layer, w_gate):
+                da, db = layer.expert_gemm_kn_pair(du, dg, w_up, w_gate, count, offset)
+            else:
+                da = data_gradient(du, w_up)
+                db = None if g is None else data_gradient(dg, w_gate)
         if need_up:
             dup = layer.expert_wgrad(du, rows, count, offset)                                      # dW[e] = dU_e^T . A_e
         if need_gate:

@@ -440,6 +440,14 @@ int moe_expert_gemm_kn_supported(const moe_handle* h, int32_t N, int32_t K, int3
 int moe_expert_gemm_kn(moe_handle* h, const void* a_rows, const void* w, const void* u_rows, const void* g_rows,
                        const int32_t* expert_count, const int32_t* expert_offset, int32_t N, int32_t K, void* out_rows,
                        void* out1_rows, void* stream);
+/* Two products of one shape, each as the calls above give it (the same bits), in one launch where there is a kernel for that: a SwiGLU
+ * layer's up and gate projections of the same rows (w0, w1 [E, N, K], no bias, no activation), and their data gradients (w0, w1
+ * [E, K, N], 16-byte aligned pointers, where moe_expert_gemm_kn_supported says 1 or 2).  The results must not overlap any operand. */
+int moe_expert_gemm_pair(moe_handle* h, const void* a_rows, const void* w0, const void* w1, const int32_t* expert_count,
+                         const int32_t* expert_offset, int32_t N, int32_t K, void* out0_rows, void* out1_rows, void* scratch, size_t scratch_bytes,
+                         void* stream);
+int moe_expert_gemm_kn_pair(moe_handle* h, const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* expert_count,
+                            const int32_t* expert_offset, int32_t N, int32_t K, void* out0_rows, void* out1_rows, void* stream);
 /* The router's share of a training step, without the logits' gradients of all experts ever being multiplied:
  * moe_combine_router_backward: moe_combine_backward whose gate-weight gradients go on through the gate -- softmax normalised over the
  *   chosen experts, or sigmoid, normalised or not (logits [S, E] from moe_gate: the normalised sigmoid only) -- into router_grad

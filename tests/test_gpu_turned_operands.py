@@ -65,3 +65,27 @@ def test_weight_gradients_on_rows_as_stored(moe, dtype, shape):
     for x, y in ((a, b), (b, a)):
         got, want = layer.expert_wgrad(x, y, dcount, doff), copies.expert_wgrad(x, y, dcount, doff)
         assert torch.equal(got, want) and not got[0].any() and got[-1].any()
+
+
+@pytest.mark.parametrize("dtype", [ob.BF16, ob.F16])
+@pytest.mark.parametrize("shape", [(1, 64, 64, 2, 1), (520, 576, 320, 2, 1), (1100, 2112, 448, 2, 2), (1900, 2112, 1088, 8, 2), (400, 320, 1088, 70, 2)])
+def test_two_products_in_one_launch(moe, dtype, shape):
+    """A SwiGLU layer's two projections of the same rows, and their data gradients: the bits of a launch each; also where an option asks
+    for the 128 x 128 tile, which takes two."""
+    import torch
+    import cuplayground_amd.api as api
+    S, H, I, E, k = shape
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=S, drop=0, skew=0.3)
+    cfg = dataclasses.replace(cfg, act=ob.ACT_SWIGLU)
+    R = int(count.sum())
+    layer, plain = moe.MoELayer(product_config(cfg)), moe.MoELayer(product_config(cfg), options={"grouped_tile": 0})
+    dev = lambda *s: to_device(ob.from_f32((rng.standard_normal(s) * 0.3).astype(np.float32), dtype), KIND[dtype])
+    dcount, doff = to_device(count, "i32"), to_device(offset, "i32")
+    x, du, dg, w_up, w_gate = dev(S * k, H), dev(S * k, I), dev(S * k, I), dev(E, I, H), dev(E, I, H)
+    for t in (x, du, dg):
+        t[R:] = float("nan")
+    for l in (layer, plain):
+        for got, w in zip(l.expert_gemm_pair(x, w_up, w_gate, dcount, doff), (w_up, w_gate)):
+            assert torch.equal(got[:R], l.expert_gemm(x, w, None, dcount, doff, api.ACT_NONE)[:R])
+    for got, d, w in zip(layer.expert_gemm_kn_pair(du, dg, w_up, w_gate, dcount, doff), (du, dg), (w_up, w_gate)):
+        assert torch.equal(got[:R], layer.expert_gemm_kn(d, w, dcount, doff)[:R])

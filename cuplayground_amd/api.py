@@ -29,7 +29,7 @@ EXPORTS = (
     "moe_set_ffn_mode", "moe_get_ffn_mode", "moe_forward", "moe_forward_static", "moe_set_spin_limit", "moe_clear_stall", "moe_gate", "moe_router_stats", "moe_route", "moe_gemm_bias_act", "moe_combine",
     "moe_set_stage_timing", "moe_get_stage_ms", "moe_get_stage_samples", "moe_get_task_counts", "moe_get_queue_balance", "moe_task_trace_bytes", "moe_set_task_trace", "moe_get_task_trace", "moe_measure_mfma_tflops",
     "moe_measure_hbm_read_gbs", "moe_quant_block128", "moe_dequant_block128", "moe_backward_scratch_bytes", "moe_transpose", "moe_expert_gemm",
-    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_gemm_pair", "moe_expert_gemm_kn_pair", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_gate_wgrad_rows", "moe_last_hip_error", "moe_status_string",
+    "moe_expert_gemm_act_backward", "moe_expert_gemm_act_backward_supported", "moe_expert_gemm_kn", "moe_expert_gemm_kn_supported", "moe_expert_gemm_pair", "moe_expert_gemm_kn_pair", "moe_expert_wgrads", "moe_expert_wgrad", "moe_act_backward", "moe_bias_grad", "moe_combine_backward", "moe_dispatch_rows", "moe_act_forward", "moe_dispatch_backward", "moe_router_grad_bytes", "moe_combine_router_backward", "moe_dispatch_router_backward", "moe_gate_wgrad", "moe_gate_wgrad_rows", "moe_last_hip_error", "moe_status_string",
     "moe_version",
 )
 
@@ -162,6 +162,7 @@ def load_library():
     L.moe_expert_gemm_kn.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp]
     L.moe_expert_gemm_pair.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp, C.c_size_t, vp]
     L.moe_expert_gemm_kn_pair.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp, vp]
+    L.moe_expert_wgrads.argtypes = [vp, i32, C.POINTER(vp), C.POINTER(vp), C.POINTER(vp), C.POINTER(i32), C.POINTER(i32), vp, vp, vp, C.c_size_t, vp]
     L.moe_expert_gemm_kn_supported.argtypes = [vp, i32, i32, C.POINTER(C.c_int32)]
     L.moe_act_backward.argtypes = [vp, vp, vp, vp, i64, vp, vp, vp]
     L.moe_bias_grad.argtypes = [vp, vp, vp, vp, i32, vp, vp]
@@ -632,6 +633,28 @@ class MoELayer:
         sc = self.backward_scratch()
         _check(self.L.moe_expert_wgrad(self._h, _ptr(dy_rows), _ptr(a_rows), _ptr(expert_count), _ptr(expert_offset),
                                        N, K, _ptr(out), _ptr(sc), sc.numel(), _stream()), "moe_expert_wgrad")
+        return out
+
+    def expert_wgrads(self, pairs, expert_count, expert_offset):
+        """The weight gradients of up to three (dy_rows, a_rows), as expert_wgrad gives each."""
+        import torch
+        for dy, a in pairs:
+            for name, t in (("dy_rows", dy), ("a_rows", a)):
+                _operand(name, t, self.act_dtype, self.S * self.k * t.shape[1])
+        for name, t in (("expert_count", expert_count), ("expert_offset", expert_offset)):
+            _operand(name, t, torch.int32, self.E)
+        out = [torch.empty(self.E, dy.shape[1], a.shape[1], dtype=a.dtype, device=a.device) for dy, a in pairs]
+        n, sc = len(pairs), self.backward_scratch()
+
+        def addresses(ts):
+            return (C.c_void_p * n)(*(t.data_ptr() for t in ts))
+
+        def sizes(ts):
+            return (C.c_int32 * n)(*(t.shape[1] for t in ts))
+
+        dys, rows = [dy for dy, _ in pairs], [a for _, a in pairs]
+        _check(self.L.moe_expert_wgrads(self._h, n, addresses(dys), addresses(rows), addresses(out), sizes(dys), sizes(rows), _ptr(expert_count),
+                                        _ptr(expert_offset), _ptr(sc), sc.numel(), _stream()), "moe_expert_wgrads")
         return out
 
     def act_backward(self, dh_rows, u_rows, g_rows=None, du=None, dg=None):

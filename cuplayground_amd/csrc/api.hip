@@ -1270,6 +1270,20 @@ int moe_expert_wgrad(moe_handle* h, const void* dy_rows, const void* a_rows, con
     return e == hipSuccess ? MOE_OK : hip_fail(h, e);
 }
 
+int moe_expert_wgrads(moe_handle* h, int32_t n, const void* const* dy_rows, const void* const* a_rows, void* const* dw, const int32_t* N,
+                      const int32_t* K, const int32_t* expert_count, const int32_t* expert_offset, void* scratch, size_t scratch_bytes, void* stream) {
+    if (!h || n < 1 || n > 3 || !dy_rows || !a_rows || !dw || !N || !K || !expert_count || !expert_offset) return MOE_ERR_BAD_ARGUMENT;
+    WgradOperands ops[3];
+    for (int i = 0; i < n; ++i) {
+        if (!dy_rows[i] || !a_rows[i] || !dw[i]) return MOE_ERR_BAD_ARGUMENT;
+        const int rc = check_backward_call(h, N[i], K[i], scratch, scratch_bytes);
+        if (rc) return rc;
+        ops[i] = WgradOperands{dy_rows[i], a_rows[i], dw[i], N[i], K[i]};
+    }
+    const hipError_t e = launch_expert_wgrads(ops, n, expert_count, expert_offset, h->d.A, h->d.E, h->d.act_dtype, h->opt, scratch, (hipStream_t)stream);
+    return e == hipSuccess ? MOE_OK : hip_fail(h, e);
+}
+
 namespace {
 bool backward_dtype(const moe_handle* h) {
     return h->cfg.torch_dtype != MOE_DTYPE_FP8_E4M3_B128;

@@ -32,8 +32,7 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
 hipError_t launch_grouped_gemm_kn_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* out, void* out1,
                                      const int32_t* count, const int32_t* offset, bool large, int64_t A, int E, int N, int K, int hidden_act, bool f16,
                                      hipStream_t st);
-hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K,
-                                bool f16, hipStream_t st);
+hipError_t launch_wgrad_rows_16(const WgradOperands* ops, int n, const int32_t* count, const int32_t* offset, bool large, int E, bool f16, hipStream_t st);
 hipError_t launch_grouped_gemm_deriv_16(const void* a_rows, const void* w, const void* u, const void* g_rows, void* du, void* dg,
                                         const int32_t* count, const int32_t* offset, int tile, int64_t A, int E, int N, int K,
                                         int hidden_act, bool f16, hipStream_t st);
@@ -798,14 +797,17 @@ hipError_t launch_expert_gemm_kn_pair(const void* a0_rows, const void* a1_rows, 
                                           dtype == MOE_DTYPE_FP16, st);
 }
 
+static bool wgrad_from_rows(const WgradOperands& w, int64_t A, int dtype, const moe_options& opt) {
+    const bool aligned = ((uintptr_t)w.dy | (uintptr_t)w.a | (uintptr_t)w.dw) % 16 == 0;
+    return dtype != MOE_DTYPE_F32 && aligned && opt.grouped_tile == MOE_OPT_AUTO && stored_operands_ok(A, w.N, w.K);
+}
 // dw[e] [N,K] = dy_e^T . a_e, from the rows as they are (product_choice.hpp; not where option grouped_tile asks for a tile) or from
 // transposed copies: scratch holds the window offsets and those.
 hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const int32_t* count, const int32_t* offset,
                                int64_t A, int E, int N, int K, int dtype, const moe_options& opt, void* dw, void* scratch,
                                hipStream_t st) {
-    const bool aligned = ((uintptr_t)dy_rows | (uintptr_t)a_rows | (uintptr_t)dw) % 16 == 0;
-    if (dtype != MOE_DTYPE_F32 && aligned && opt.grouped_tile == MOE_OPT_AUTO && stored_operands_ok(A, N, K))
-        return launch_wgrad_rows_16(dy_rows, a_rows, dw, count, offset, wgrad_large(A, E, N, K), E, N, K, dtype == MOE_DTYPE_FP16, st);
+    const WgradOperands op{dy_rows, a_rows, dw, N, K};
+    if (wgrad_from_rows(op, A, dtype, opt)) return launch_wgrad_rows_16(&op, 1, count, offset, wgrad_large(A, E, N, K), E, dtype == MOE_DTYPE_FP16, st);
     const ScratchTables t = scratch_tables(scratch, A, E);
     const int64_t ld = wgrad_ld(A, E);
     const size_t eb = dtype == MOE_DTYPE_F32 ? 4 : 2;
@@ -827,6 +829,19 @@ hipError_t launch_expert_wgrad(const void* dy_rows, const void* a_rows, const in
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return launch_wgrad_16(dyT, aT, dw, t.poff, E, N, K, ld, dtype == MOE_DTYPE_FP16, st);
+}
+
+// n weight gradients (1 to 3; of N x K or K x N each) in one launch where all come from the rows as they are, else one after the other.
+hipError_t launch_expert_wgrads(const WgradOperands* ops, int n, const int32_t* count, const int32_t* offset, int64_t A, int E, int dtype,
+                                const moe_options& opt, void* scratch, hipStream_t st) {
+    bool together = true;
+    for (int i = 0; i < n; ++i) together = together && wgrad_from_rows(ops[i], A, dtype, opt);
+    if (together) return launch_wgrad_rows_16(ops, n, count, offset, wgrad_large(A, E, ops[0].N, ops[0].K, n), E, dtype == MOE_DTYPE_FP16, st);
+    for (int i = 0; i < n; ++i) {
+        const hipError_t e = launch_expert_wgrad(ops[i].dy, ops[i].a, count, offset, A, E, ops[i].N, ops[i].K, dtype, opt, ops[i].dw, scratch, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <class T16, class RAW>

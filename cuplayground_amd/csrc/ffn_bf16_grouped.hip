@@ -329,16 +329,38 @@ __device__ __forceinline__ TaskPtrs prod_epilogue(uint16_t* c, int N, int n0, in
 // Weight gradient of one projection from the packed rows as they are: dw[e] [N, K] = sum over expert e's rows of
 // dy[r, :]^T a[r, :].  Tiles expert by expert.  The workgroups of an XCD (launched eight apart) take neighbouring tiles, four
 // columns wide, whose operands meet in its L2: 16 experts of 2048 x 1408, 750 rows each, 104 us against 124 with columns fastest.
-template <class T>
-struct WgradTiles {
+// Up to three of them share a launch, a projection's tiles behind another's (a step's tiles need not fill whole rounds projection by
+// projection, and the workgroups that stay fill and drain once).  Three launches / one, us: 4 experts of 2048 x 2560, 4096 rows each
+// 532 / 406; 8 of 1536 x 1920, 512 rows 129 / 106; 8 of 1280 x 1664, 256 rows 79 / 58; 16 of 1152 x 1920, 175 rows 110 / 90; 16 of 2048 x
+// 2048, 512 rows 277 / 256; of 2048 x 1408, 750 rows (whole rounds either way) 250 / 243.
+struct WgradJob {
     const uint16_t* dy;
     const uint16_t* a;
     uint16_t* dw;
+    int N, K;
+};
+template <class T>
+struct WgradTiles {
+    WgradJob p0, p1, p2;         // (selected by comparisons: an index that is not a constant would put them into scratch memory)
     const int32_t* count;
     const int32_t* offset;
-    int E, N, K;
-    __device__ __forceinline__ bool place(int id, int& e, int& n0, int& k0) const {
-        const int cols = (K + T::BN - 1) / T::BN, rows = (N + T::BM - 1) / T::BM, share = (cols * rows + 7) / 8;
+    int E;
+    // ids of one projection; a multiple of 8, so that an id's XCD does not depend on the projection
+    static __host__ __device__ __forceinline__ int64_t ids(const WgradJob& p, int E) {
+        return (int64_t)(((p.K + T::BN - 1) / T::BN * ((p.N + T::BM - 1) / T::BM) + 7) / 8 * 8) * E;
+    }
+    // Tile `id`: which projection, of which expert, from which row and column of its gradient on; false: no such tile.
+    __device__ __forceinline__ bool place(int id, WgradJob& p, int& e, int& n0, int& k0) const {
+        const int ids0 = (int)ids(p0, E), ids1 = ids0 + (int)ids(p1, E);
+        const int which = id < ids0 ? 0 : id < ids1 ? 1 : 2;
+        id -= which == 0 ? 0 : which == 1 ? ids0 : ids1;
+        p.dy = which == 0 ? p0.dy : which == 1 ? p1.dy : p2.dy;
+        p.a = which == 0 ? p0.a : which == 1 ? p1.a : p2.a;
+        p.dw = which == 0 ? p0.dw : which == 1 ? p1.dw : p2.dw;
+        p.N = which == 0 ? p0.N : which == 1 ? p1.N : p2.N;
+        p.K = which == 0 ? p0.K : which == 1 ? p1.K : p2.K;
+        const int cols = (p.K + T::BN - 1) / T::BN, rows = (p.N + T::BM - 1) / T::BM, share = (cols * rows + 7) / 8;
+        if (cols * rows == 0) return false;
         e = id / (8 * share);
         const int r = id - e * 8 * share, t = (r & 7) * share + (r >> 3);
         const int band = t / (4 * rows), in = t - band * 4 * rows, width = min(4, cols - 4 * band);
@@ -347,20 +369,30 @@ struct WgradTiles {
         k0 = (4 * band + in % width) * T::BN;
         return e < E;
     }
-    __device__ __forceinline__ bool job(int id, ProdJob& j) const {
-        int e, n0, k0;
-        if (!place(id, e, n0, k0)) return false;
+    __device__ __forceinline__ ProdJob operands(const WgradJob& p, int e, int n0, int k0) const {
         const int n = max(count[e], 0);
         const int64_t off = offset[e];
-        j.a = ProdOperand{dy + off * N + n0, N, n > 0 ? (uint32_t)(((int64_t)n * N - n0) * 2) : 0u};
-        j.b = ProdOperand{a + off * K + k0, K, n > 0 ? (uint32_t)(((int64_t)n * K - k0) * 2) : 0u};
+        ProdJob j;
+        j.a = ProdOperand{p.dy + off * p.N + n0, p.N, n > 0 ? (uint32_t)(((int64_t)n * p.N - n0) * 2) : 0u};
+        j.b = ProdOperand{p.a + off * p.K + k0, p.K, n > 0 ? (uint32_t)(((int64_t)n * p.K - k0) * 2) : 0u};
         j.slabs = max((n + kBK - 1) / kBK, 1);
+        return j;
+    }
+    __device__ __forceinline__ TaskPtrs result(const WgradJob& p, int e, int n0, int k0) const {
+        return prod_epilogue(p.dw + ((int64_t)e * p.N + n0) * p.K, p.K, k0, min(T::BM, p.N - n0));
+    }
+    __device__ __forceinline__ bool job(int id, ProdJob& j) const {
+        WgradJob p;
+        int e, n0, k0;
+        if (!place(id, p, e, n0, k0)) return false;
+        j = operands(p, e, n0, k0);
         return true;
     }
     __device__ __forceinline__ void finish(int id, f32x4 (&acc)[T::TM][T::TN], unsigned char* smem) const {
+        WgradJob p;
         int e, n0, k0;
-        place(id, e, n0, k0);
-        grouped_epilogue<T, kSums>(prod_epilogue(dw + ((int64_t)e * N + n0) * K, K, k0, min(T::BM, N - n0)), smem, acc);
+        place(id, p, e, n0, k0);
+        grouped_epilogue<T, kSums>(result(p, e, n0, k0), smem, acc);
     }
 };
 template <class T>
@@ -377,12 +409,12 @@ template <class T>
 __global__ __launch_bounds__(T::THREADS) void wgrad_ring_kernel(WgradTiles<T> w, int ids) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto find = [&](int id, TaskPtrs& p) {     // the first tile from `id` on, in steps of the grid
+        WgradJob of;
         int e, n0, k0;
-        while (id < ids && !w.place(id, e, n0, k0)) id += gridDim.x;
+        while (id < ids && !w.place(id, of, e, n0, k0)) id += gridDim.x;
         if (id >= ids) return id;
-        ProdJob j;
-        w.job(id, j);
-        p = prod_epilogue(w.dw + ((int64_t)e * w.N + n0) * w.K, w.K, k0, min(T::BM, w.N - n0));
+        const ProdJob j = w.operands(of, e, n0, k0);
+        p = w.result(of, e, n0, k0);
         p.a_base = j.a.base;
         p.a_ld = j.a.ld;
         p.a_extent = j.a.extent;
@@ -594,7 +626,7 @@ hipError_t launch_wgrad_16(const void* dyT, const void* aT, void* dw, const int3
 
 template <class T>
 static hipError_t launch_wgrad_rows(const WgradTiles<T>& w, hipStream_t st) {
-    const int64_t tiles = ((int64_t)((w.K + T::BN - 1) / T::BN) * ((w.N + T::BM - 1) / T::BM) + 7) / 8 * 8 * w.E;
+    const int64_t tiles = WgradTiles<T>::ids(w.p0, w.E) + WgradTiles<T>::ids(w.p1, w.E) + WgradTiles<T>::ids(w.p2, w.E);
     if (tiles > INT32_MAX) return hipErrorInvalidValue;
     if constexpr (T::TRA) {
         hipError_t e = allow_lds(&wgrad_ring_kernel<T>, T::LDS_BYTES);
@@ -608,15 +640,17 @@ static hipError_t launch_wgrad_rows(const WgradTiles<T>& w, hipStream_t st) {
     return hipGetLastError();
 }
 template <bool F16>
-static hipError_t launch_wgrad_rows(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K, hipStream_t st) {
+static hipError_t launch_wgrad_rows(const WgradOperands* ops, int n, const int32_t* count, const int32_t* offset, bool large, int E, hipStream_t st) {
     using Large = Tile<256, 256, 2, 2, 2, F16, true, true>;
-    if (large) return launch_wgrad_rows(WgradTiles<Large>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K}, st);
-    return launch_wgrad_rows(WgradTiles<ProdTile<F16>>{(const uint16_t*)dy, (const uint16_t*)a, (uint16_t*)dw, count, offset, E, N, K}, st);
+    auto job = [&](int i) {
+        return i < n ? WgradJob{(const uint16_t*)ops[i].dy, (const uint16_t*)ops[i].a, (uint16_t*)ops[i].dw, ops[i].N, ops[i].K} : WgradJob{};
+    };
+    if (large) return launch_wgrad_rows(WgradTiles<Large>{job(0), job(1), job(2), count, offset, E}, st);
+    return launch_wgrad_rows(WgradTiles<ProdTile<F16>>{job(0), job(1), job(2), count, offset, E}, st);
 }
-// large: on the 256 x 256 tile.
-hipError_t launch_wgrad_rows_16(const void* dy, const void* a, void* dw, const int32_t* count, const int32_t* offset, bool large, int E, int N, int K,
-                                bool f16, hipStream_t st) {
-    return f16 ? launch_wgrad_rows<true>(dy, a, dw, count, offset, large, E, N, K, st) : launch_wgrad_rows<false>(dy, a, dw, count, offset, large, E, N, K, st);
+// n weight gradients (1 to 3) in one launch; large: on the 256 x 256 tile.
+hipError_t launch_wgrad_rows_16(const WgradOperands* ops, int n, const int32_t* count, const int32_t* offset, bool large, int E, bool f16, hipStream_t st) {
+    return f16 ? launch_wgrad_rows<true>(ops, n, count, offset, large, E, st) : launch_wgrad_rows<false>(ops, n, count, offset, large, E, st);
 }
 
 template <bool F16, int EPI>

@@ -236,6 +236,14 @@ int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const mo
 hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
                                  const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows,
                                  void* out1_rows, hipStream_t st);
+struct WgradOperands {      // a weight gradient dw[e] [N, K] = dy_e^T . a_e
+    const void* dy;
+    const void* a;
+    void* dw;
+    int N, K;
+};
+hipError_t launch_expert_wgrads(const WgradOperands* ops, int n, const int32_t* count, const int32_t* offset, int64_t A, int E, int dtype,
+                                const moe_options& opt, void* scratch, hipStream_t st);
 hipError_t launch_expert_gemm_pair(const void* a_rows, const void* w0, const void* w1, const int32_t* count, const int32_t* offset, int64_t A,
                                    int E, int N, int K, int dtype, const moe_options& opt, void* out0, void* out1, void* scratch, hipStream_t st);
 hipError_t launch_expert_gemm_kn_pair(const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* count,

@@ -51,11 +51,11 @@ inline bool wgrad_as_stored(int64_t A, int E, int N, int K) {
 // round of 512.  This / 128 x 128 tiles: 16 experts of 2048 x 2048, 512 rows each 81 / 101; of 2048 x 1408, 750 rows 82 / 96; 4 of 2048 x
 // 2560, 4096 rows 174 / 192; 4 of 1024 x 2560, 750 rows 27 / 31; 8 of 1920 x 1536, 500 rows 41 / 43; 8 of 1024 x 2560, 750 rows 50 / 50; 8 of
 // 1280 x 1664, 250 rows 29 / 27; 16 of 1152 x 1920, 175 rows 44 / 36; 16 of 1024 x 2560, 19 rows 32 / 23.
-inline bool wgrad_large(int64_t A, int E, int N, int K) {
+inline bool wgrad_large(int64_t A, int E, int N, int K, int products = 1) {      // (`products` of them, N x K or K x N, in one launch)
     if (!wgrad_as_stored(A, E, N, K)) return true;
-    const double slabs = (double)A / std::max(E, 1) / 64;
-    const double large = std::ceil((double)E * columns256(N) * columns256(K) / 256) * (1.3 * (slabs + 1.0) + 8.5);
-    const double small = std::ceil((double)E * ((N + 127) / 128) * ((K + 127) / 128) / 512) * (1.1 * (slabs + 0.5) + 3.6);
+    const double slabs = (double)A / std::max(E, 1) / 64, experts = (double)products * E;
+    const double large = std::ceil(experts * columns256(N) * columns256(K) / 256) * (1.3 * (slabs + 1.0) + 8.5);
+    const double small = std::ceil(experts * ((N + 127) / 128) * ((K + 127) / 128) / 512) * (1.1 * (slabs + 0.5) + 3.6);
     return large < small;
 }
 // Data gradient [A, N] from rows of K and the weight [E, K, N]: as stored wherever the offsets allow it -- the transposing fragment reads

@@ -150,9 +150,7 @@ def _expert_gradients(layer, needs, dy, kept, count, offset):
         out = torch.empty(a.shape[0], w_t.shape[1], dtype=a.dtype, device=a.device)
         return layer.expert_gemm(a, w_t, None, count, offset, api.ACT_NONE, out=out)
 
-    da = db = dup = dgate = ddown = None
-    if need_down:
-        ddown = layer.expert_wgrad(dy, h, count, offset)
+    da = db = dup = dgate = ddown = du = dg = None
     if need_x or need_up or need_gate:
         if _as_stored(layer, w_down):
             du, dg = layer.expert_gemm_kn(dy, w_down, count, offset, u, g)                         # dH = dY . W_down, times act'
@@ -170,10 +168,14 @@ def _expert_gradients(layer, needs, dy, kept, count, offset):
             else:
                 da = data_gradient(du, w_up)
                 db = None if g is None else data_gradient(dg, w_gate)
-        if need_up:
-            dup = layer.expert_wgrad(du, rows, count, offset)                                      # dW[e] = dU_e^T . A_e
-        if need_gate:
-            dgate = layer.expert_wgrad(dg, rows, count, offset)
+    asked = [p for need, p in ((need_down, (dy, h)), (need_up, (du, rows)), (need_gate, (dg, rows))) if need]      # dW[e] = dU_e^T . A_e
+    if not asked:
+        grads = iter(())
+    elif isinstance(layer, api.MoELayer):
+        grads = iter(layer.expert_wgrads(asked, count, offset))
+    else:
+        grads = iter([layer.expert_wgrad(d, a, count, offset) for d, a in asked])
+    ddown, dup, dgate = (next(grads) if need else None for need in (need_down, need_up, need_gate))
     return da, db, dup, dgate, ddown
 
 

@@ -448,6 +448,10 @@ int moe_expert_gemm_pair(moe_handle* h, const void* a_rows, const void* w0, cons
                          void* stream);
 int moe_expert_gemm_kn_pair(moe_handle* h, const void* a0_rows, const void* a1_rows, const void* w0, const void* w1, const int32_t* expert_count,
                             const int32_t* expert_offset, int32_t N, int32_t K, void* out0_rows, void* out1_rows, void* stream);
+/* n weight gradients (1 to 3) of the layer, each as moe_expert_wgrad gives it (the same bits), in one launch where there is a kernel for
+ * that.  The arrays are on the host and are read before the call returns. */
+int moe_expert_wgrads(moe_handle* h, int32_t n, const void* const* dy_rows, const void* const* a_rows, void* const* dw, const int32_t* N,
+                      const int32_t* K, const int32_t* expert_count, const int32_t* expert_offset, void* scratch, size_t scratch_bytes, void* stream);
 /* The router's share of a training step, without the logits' gradients of all experts ever being multiplied:
  * moe_combine_router_backward: moe_combine_backward whose gate-weight gradients go on through the gate -- softmax normalised over the
  *   chosen experts, or sigmoid, normalised or not (logits [S, E] from moe_gate: the normalised sigmoid only) -- into router_grad

@@ -89,3 +89,24 @@ def test_two_products_in_one_launch(moe, dtype, shape):
             assert torch.equal(got[:R], l.expert_gemm(x, w, None, dcount, doff, api.ACT_NONE)[:R])
     for got, d, w in zip(layer.expert_gemm_kn_pair(du, dg, w_up, w_gate, dcount, doff), (du, dg), (w_up, w_gate)):
         assert torch.equal(got[:R], layer.expert_gemm_kn(d, w, dcount, doff)[:R])
+
+
+@pytest.mark.parametrize("dtype", [ob.F32, ob.BF16, ob.F16])
+@pytest.mark.parametrize("shape", [(1, 64, 64, 2, 1), (750, 2560, 1088, 5, 2), (2304, 2048, 1024, 24, 2), (700, 1152, 1920, 16, 4)])
+def test_weight_gradients_in_one_launch(moe, dtype, shape):
+    """One, two and three weight gradients a call: the bits of a call each, on the rows as they lie and (an option, fp32) from copies."""
+    import torch
+    S, H, I, E, k = shape
+    cfg, rng, count, offset = routed_case(S, H, I, E, k, dtype, seed=S, drop=0, skew=0.2)
+    R = int(count.sum())
+    dev = lambda *s: to_device(ob.from_f32(rng.standard_normal(s).astype(np.float32), dtype), KIND[dtype])
+    dcount, doff = to_device(count, "i32"), to_device(offset, "i32")
+    x, dy, h, du = dev(S * k, H), dev(S * k, H), dev(S * k, I), dev(S * k, I)
+    for t in (x, dy, h, du):
+        t[R:] = float("nan")
+    for options in ({}, {"grouped_tile": 1}):
+        layer = moe.MoELayer(product_config(cfg), options=options)
+        pairs = [(dy, h), (du, x), (h, x)]
+        want = [layer.expert_wgrad(*p, dcount, doff) for p in pairs]
+        for n in (1, 2, 3):
+            assert all(torch.equal(g, w) for g, w in zip(layer.expert_wgrads(pairs[:n], dcount, doff), want))

@@ -597,58 +597,75 @@ __global__ __launch_bounds__(256) void dispatch_rows_kernel(const uint4* __restr
 }
 
 // dx[t, :] = sum over ranks r, ascending, of a[pair_row[t,r], :] + b[pair_row[t,r], :] (b may be null), and, with dl, behind
-// them of dl[t,r] gate_w[topk_idx[t,r], :], in fp32 and rounded once: the adjoint of the dispatch for one or two row gradients.  One wavefront per token and 64 16-byte pieces of its row,
-// the rows of four ranks in flight.  (torch's index_add backward of the same gather, 8192 rows x 2048 columns in bf16:
-// 55 us, behind two zero fills and, for two projections, two more sums over the rows.)  The router's share, a serial loop over the
-// ranks behind each 512 columns, costs 8 us of 19 for 4096 tokens x 2, 10 of 38 for 3000 x 4 with two row gradients.
+// them of dl[t,r] gate_w[topk_idx[t,r], :], in fp32 and rounded once: the adjoint of the dispatch for one or two row gradients.
+// Bound by latency more than by its bytes: what a piece reads hangs on its token's ranks, two trips to memory behind each other.  So a
+// wavefront takes one piece (64 x 16 bytes) of a token, not a token, and asks for the rows of four ranks and the router's weight
+// rows of the same ranks before it adds anything.  A wavefront per token, piece after piece, the router's ranks one after the other / this:
+// us, bf16, with the router's share: 3000 tokens x 4, rows of 2048, two gradients 24.1 / 21.8; 16384 x 6 225 / 183; 8192 x 2, rows of 4096
+// 112 / 70 (a copy of the same bytes 18, 139, 53); 4096 x 2, one gradient 13.4 / 13.7.  (The combine's adjoint with a token's pieces over
+// four wavefronts: 198 / 169 and 91 / 70 for the two large ones, but 20.3 / 21.1 and 16.3 / 18.4 for the others: not done.)
 template <class T16, class RAW = typename RawOf<T16>::type>
 __global__ __launch_bounds__(256) void dispatch_backward_kernel(const RAW* __restrict__ a, const RAW* __restrict__ b,
-                                                                const int32_t* __restrict__ pair_row, int S, int k, int H,
+                                                                const int32_t* __restrict__ pair_row, int S, int k, int H, int pieces,
                                                                 RAW* __restrict__ dx, const int32_t* __restrict__ topk_idx,
                                                                 const float* __restrict__ dl, const RAW* __restrict__ gate_w) {
     constexpr int VEC = 16 / (int)sizeof(RAW);
     union Pack { uint4 q; RAW e[VEC]; };
-    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= S) return;
-    for (int c = lane * VEC; c < H; c += 64 * VEC) {
-        float acc[VEC];
+    const int64_t id = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = (int)(id / pieces), c = ((int)(id - (int64_t)t * pieces) * 64 + (threadIdx.x & 63)) * VEC;
+    if (t >= S || c >= H) return;
+    const int32_t* rows = pair_row + (size_t)t * k;
+    const int32_t* experts = topk_idx + (size_t)t * k;
+    const float* d = dl + (size_t)t * k;
+    Pack w[4];
+    float scale[4];
+    auto router_rows = [&](int r0) {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
-        for (int r0 = 0; r0 < k; r0 += 4) {
-            int row[4];
-            Pack va[4], vb[4];
+        for (int j = 0; j < 4; ++j) {
+            if (r0 + j >= k) continue;
+            scale[j] = d[r0 + j];
+            w[j].q = *reinterpret_cast<const uint4*>(gate_w + (size_t)__builtin_amdgcn_readfirstlane(experts[r0 + j]) * H + c);
+        }
+    };
+    if (dl) router_rows(0);
+    float acc[VEC];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                row[j] = r0 + j < k ? __builtin_amdgcn_readfirstlane(pair_row[(size_t)t * k + r0 + j]) : -1;
-                if (row[j] < 0) continue;
-                va[j].q = *reinterpret_cast<const uint4*>(a + (size_t)row[j] * H + c);
-                if (b) vb[j].q = *reinterpret_cast<const uint4*>(b + (size_t)row[j] * H + c);
-            }
+    for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
+    for (int r0 = 0; r0 < k; r0 += 4) {
+        int row[4];
+        Pack va[4], vb[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (row[j] < 0) continue;
+        for (int j = 0; j < 4; ++j) {
+            row[j] = r0 + j < k ? __builtin_amdgcn_readfirstlane(rows[r0 + j]) : -1;
+            if (row[j] < 0) continue;
+            va[j].q = *reinterpret_cast<const uint4*>(a + (size_t)row[j] * H + c);
+            if (b) vb[j].q = *reinterpret_cast<const uint4*>(b + (size_t)row[j] * H + c);
+        }
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    acc[i] = acc[i] + ld16<T16>(va[j].e, i);
-                    if (b) acc[i] = acc[i] + ld16<T16>(vb[j].e, i);
-                }
+        for (int j = 0; j < 4; ++j) {
+            if (row[j] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                acc[i] = acc[i] + ld16<T16>(va[j].e, i);
+                if (b) acc[i] = acc[i] + ld16<T16>(vb[j].e, i);
             }
         }
-        if (dl) {                          // the router's share: its weight rows of the chosen experts times their logits' gradients
-            for (int j = 0; j < k; ++j) {
-                const int e = __builtin_amdgcn_readfirstlane(topk_idx[(size_t)t * k + j]);
-                const float d = dl[(size_t)t * k + j];
-                Pack w;
-                w.q = *reinterpret_cast<const uint4*>(gate_w + (size_t)e * H + c);
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) acc[i] = fmaf(d, ld16<T16>(w.e, i), acc[i]);
-            }
-        }
-        Pack o;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) o.e[i] = st16<T16>(acc[i]);
-        *reinterpret_cast<uint4*>(dx + (size_t)t * H + c) = o.q;
     }
+    if (dl) {
+        for (int r0 = 0; r0 < k; r0 += 4) {
+            if (r0) router_rows(r0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (r0 + j >= k) continue;
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) acc[i] = fmaf(scale[j], ld16<T16>(w[j].e, i), acc[i]);
+            }
+        }
+    }
+    Pack o;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) o.e[i] = st16<T16>(acc[i]);
+    *reinterpret_cast<uint4*>(dx + (size_t)t * H + c) = o.q;
 }
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -959,11 +976,14 @@ hipError_t launch_dispatch_rows(const void* x, const int32_t* token_indices, int
 hipError_t launch_dispatch_backward(const void* a, const void* b, const int32_t* pair_row, int S, int k, int H, int dtype,
                                     void* dx, const int32_t* topk_idx, const void* grad, const void* gate_w, hipStream_t st) {
     if (S <= 0) return hipSuccess;
-    const int grid = (S + 3) / 4;
+    const int piece = 64 * 16 / (dtype == MOE_DTYPE_F32 ? 4 : 2), pieces = (H + piece - 1) / piece;
+    const int64_t blocks = ((int64_t)S * pieces + 3) / 4;
+    if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    const unsigned grid = (unsigned)blocks;
     const float* dl = static_cast<const float*>(grad);
-    if (dtype == MOE_DTYPE_F32) dispatch_backward_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)a, (const float*)b, pair_row, S, k, H, (float*)dx, topk_idx, dl, (const float*)gate_w);
-    else if (dtype == MOE_DTYPE_FP16) dispatch_backward_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
-    else dispatch_backward_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
+    if (dtype == MOE_DTYPE_F32) dispatch_backward_kernel<f32_s><<<grid, 256, 0, st>>>((const float*)a, (const float*)b, pair_row, S, k, H, pieces, (float*)dx, topk_idx, dl, (const float*)gate_w);
+    else if (dtype == MOE_DTYPE_FP16) dispatch_backward_kernel<f16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, pieces, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
+    else dispatch_backward_kernel<bf16_s><<<grid, 256, 0, st>>>((const uint16_t*)a, (const uint16_t*)b, pair_row, S, k, H, pieces, (uint16_t*)dx, topk_idx, dl, (const uint16_t*)gate_w);
     return hipGetLastError();
 }
 

@@ -10,13 +10,11 @@
 // weight rows of a wavefront's fragments lie in one scale block and the scale of a k block is one scalar (two for a
 // SwiGLU up projection).
 //   * four wavefronts of 64 x 64 outputs, v_mfma_f32_16x16x32_bf16, weights as the "A" operand;
-//   * K slabs of 64: token rows go from global memory straight into LDS (global_load ... lds) as 128-byte rows with
-//     xor-swizzled 16-byte chunks; weight bytes are fetched into registers two slabs ahead, widened to bf16 once per
-//     workgroup (cvt_pk_f32_fp8 + byte permute, exact) and written to LDS in the same layout, so the fragment reads and
-//     MFMAs are those of a bf16 tile;
+//   * K slabs of 64: token rows and weight bytes go from global memory straight into LDS (global_load ... lds), two slabs ahead, as
+//     128- and 64-byte rows with xor-swizzled 16-byte chunks; weight bytes are widened to bf16 (exact) behind their fragment reads;
 //   * a second accumulator set takes the 128-deep partial sums (its first MFMA of a k block starts from zero); after
 //     every second slab acc = fma(scale, partial, acc) in fp32;
-//   * two 32 KiB LDS stages per workgroup, two workgroups per compute unit.
+//   * three 24 KiB LDS stages per workgroup, two workgroups per compute unit.
 #include <type_traits>
 
 #include "ffn_common.hpp"
@@ -26,7 +24,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
@@ -38,12 +35,14 @@ constexpr int PN1 = 128;          // output columns per down-projection task
 constexpr int PBK = 64;           // k per slab
 constexpr int PROW = 128;         // bytes per LDS row (64 bf16)
 constexpr int PSTAGE = (PBM + PBN) * PROW;
-constexpr int PLDS = 2 * PSTAGE;
-constexpr int PLDS_M8 = PLDS + 2 * PBM * 4;       // e4m3 x e4m3 loop: behind the two stages, the token rows' scales of either slab
+constexpr int PLDS_M8 = 2 * PSTAGE + 2 * PBM * 4; // e4m3 x e4m3 loop: behind the two stages, the token rows' scales of either slab
+constexpr int PWROW = 64;         // bytes per LDS row of the weights (64 e4m3)
+constexpr int PWSTAGE = PBM * PROW + PBN * PWROW;
+constexpr int PLDS = 3 * PWSTAGE;
 constexpr int PTHREADS = 256;
 constexpr int PTM = 4, PTN = 4;   // 16 x 16 fragments per wavefront: tokens, weight rows
 constexpr int PRA = PBM * 8 / PTHREADS;        // 16-byte token loads per thread per slab
-constexpr int PRB = PBN * 4 / PTHREADS;        // 16-byte weight loads (16 e4m3 values) per thread per slab
+constexpr int PRW = PBN * 4 / PTHREADS;        // 16-byte weight loads (16 e4m3 values) per thread per slab
 
 struct TileTask {
     const uint16_t* a_base;     // x or h
@@ -62,30 +61,34 @@ struct TileTask {
     const float* sa;            // [*, K / 128]
 };
 
-// 16 e4m3 bytes -> 2 x 8 bf16.  Every e4m3 value is a bf16 value, so the upper half of its fp32 form is exact.
-__device__ __forceinline__ void widen16(const u32x4& q, u32x4& lo, u32x4& hi) {
-    const uint32_t w[4] = {q[0], q[1], q[2], q[3]};
-    uint32_t o[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], false);
-        const f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], true);
-        o[2 * i] = __builtin_amdgcn_perm(__float_as_uint(a[1]), __float_as_uint(a[0]), 0x07060302u);
-        o[2 * i + 1] = __builtin_amdgcn_perm(__float_as_uint(b[1]), __float_as_uint(b[0]), 0x07060302u);
-    }
-    lo = u32x4{o[0], o[1], o[2], o[3]};
-    hi = u32x4{o[4], o[5], o[6], o[7]};
+// 8 e4m3 bytes -> 8 bf16 (exact), two an instruction.
+__device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+    const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+    const u32x4 v = {__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)};
+    return __builtin_bit_cast(bf16x8, v);
 }
 
+// The slab loop.  What bounds it: the latency of its loads; a slab's MFMAs are 0.2 us on a SIMD, a load from beyond the L2 takes 1 us and
+// more.  So both operands go from memory to LDS as they are stored, two slabs ahead, in a ring of three stages (two workgroups
+// per compute unit), and the weight bytes are widened behind their fragment reads: twice per workgroup then (two wavefronts
+// share weight rows), at two values an instruction, but without registers, LDS writes and waits for bytes on their way.
+// Weight bytes through registers, widened once per workgroup and written to LDS, the token rows one slab ahead / this, whole layers, us: 8
+// experts of 4096 x 14336, SwiGLU, 16 rows each 502 / 432, 50 530 / 483, 250 1055 / 974, 500 1867 / 1723, 1024 3517 / 3214; 64 of 7168 x
+// 2048, 37 rows 860 / 782, 500 3757 / 3477; 16 of 2048 x 2048, 500 rows 362 / 330; 256 of 7168 x 2048, 46 rows 3420 / 3149.
 // PARTIAL: the row block holds fewer than 128 rows; fragments that lie entirely in the padding are skipped.
 template <bool PARTIAL>
 __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* smem, f32x4 (&acc)[PTM][PTN]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
 
-    // token rows: 8 threads per row, LDS slot (row, c) holds global chunk c ^ ((row >> 1) & 7)
+    // token rows: 8 threads per 128-byte row.  LDS slot (row, c) holds what a lane of a fragment takes as "chunk c ^ ((row >> 1) & 7)":
+    // a lane's 16 weight bytes are 16 values of k in a row, eight for either half of the slab, so chunk 4 s + f of the tokens is
+    // the one of k = 16 f + 8 s.
     const int prow = tid >> 3;
-    const int chunk = (tid & 7) ^ ((prow >> 1) & 7);
+    const int slot = (tid & 7) ^ ((prow >> 1) & 7);
+    const int chunk = 2 * (slot & 3) + (slot >> 2);
     const uint16_t* a_src[PRA];
 #pragma unroll
     for (int i = 0; i < PRA; ++i) {
@@ -94,21 +97,14 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
         const int64_t src_row = p.gather ? (int64_t)p.gather[r] : p.a_row0 + r;
         a_src[i] = p.a_base + src_row * p.K + chunk * 8;
     }
-    // weight rows: 4 threads per row, 16 e4m3 bytes each = two bf16 chunks of the LDS row.  Which lanes take which rows
-    // decides the bank conflicts of the 16-byte LDS writes: the LDS serves such a write eight consecutive lanes at a time,
-    // 128 bytes a cycle, so the eight must differ in their 16-byte position modulo 128 bytes -- the row does not matter,
-    // rows are 128 bytes apart.  Four lanes of a row write chunks {0, 2, 4, 6} ^ swizzle (then {1, 3, 5, 7} ^ swizzle);
-    // the other four lanes of the pass must therefore sit in a row whose swizzle differs in its lowest bit: rows r and
-    // r + 2.  (With lanes 4..7 in row r + 1, which has the swizzle of row r, every such write took twice its cycles:
-    // a conflict in every fourth LDS cycle of the kernel, measured with two-lane and whole-wavefront probes under
-    // SQ_LDS_BANK_CONFLICT.)
-    const int t = tid >> 2;
-    const int brow = (t & ~3) | ((t & 1) << 1) | ((t >> 1) & 1), bc = tid & 3;
-    const uint8_t* b_src[PRB];
-    int b_dst[PRB][2];
+    // weight rows: 4 threads per 64-byte row; slot c of row j holds chunk c ^ weight_swizzle(j).  The LDS serves a 16-byte read to lanes 0-3,
+    // 12-15 and 20-27 in one cycle, to 4-11, 16-19 and 28-31 in the next (and so on): of rows four apart, which meet the same banks,
+    // two take chunk f and two f ^ 1, and all four must differ.
+    auto weight_swizzle = [](int row) { return (4 - (row >> 2)) & 3; };
+    const uint8_t* b_src[PRW];
 #pragma unroll
-    for (int i = 0; i < PRB; ++i) {
-        const int j = brow + i * 64;                              // row of the weight tile
+    for (int i = 0; i < PRW; ++i) {
+        const int j = (tid >> 2) + i * 64;                        // row of the weight tile
         const uint8_t* base = p.w[0];
         int col;
         if (p.paired) {       // wavefront column w owns tile rows [64 w, 64 w + 64): 32 gate rows, then 32 up rows
@@ -118,47 +114,25 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
         } else {
             col = p.c0 + j;
         }
-        b_src[i] = base + (int64_t)col * p.K + bc * 16;
-        const int sw = (j >> 1) & 7;
-        b_dst[i][0] = PBM * PROW + j * PROW + (((2 * bc) ^ sw) << 4);
-        b_dst[i][1] = PBM * PROW + j * PROW + (((2 * bc + 1) ^ sw) << 4);
+        b_src[i] = base + (int64_t)col * p.K + (((tid & 3) ^ weight_swizzle(j)) << 4);
     }
 
-    const int wrow = __builtin_amdgcn_readfirstlane(prow & ~7);
-    auto issue_a = [&](int kt) {
-        unsigned char* sa = smem + (kt & 1) * PSTAGE;
+    const int awave = __builtin_amdgcn_readfirstlane(prow & ~7) * PROW, bwave = __builtin_amdgcn_readfirstlane((tid >> 2) & ~15) * PWROW;
+    auto issue = [&](int kt, int stage) {
+        unsigned char* st = smem + stage;
 #pragma unroll
         for (int i = 0; i < PRA; ++i)
-            __builtin_amdgcn_global_load_lds((gbl_void*)(a_src[i] + kt * PBK),
-                                             (lds_void*)(sa + (wrow + i * 32) * PROW), 16, 0, 0);
-    };
-    // The weight bytes travel through registers for more than a slab.  Their loads are written in assembly so that the
-    // wait for them can say "all but the PRA token-row loads issued since" -- the compiler, which sees direct-to-LDS
-    // loads and register loads in one counter, would wait for everything.
-    u32x4 breg[PRB];
-    auto fetch_b = [&](int kt) {
+            __builtin_amdgcn_global_load_lds((gbl_void*)(a_src[i] + kt * PBK), (lds_void*)(st + awave + i * 32 * PROW), 16, 0, 0);
 #pragma unroll
-        for (int i = 0; i < PRB; ++i)
-            asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(breg[i]) : "v"(b_src[i] + kt * PBK) : "memory");
-    };
-    auto store_b = [&](int kt) {
-        unsigned char* st = smem + (kt & 1) * PSTAGE;
-        static_assert(PRB == 2, "the wait below names both registers");
-        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(breg[0]), "+v"(breg[1]) : "n"(PRA) : "memory");
-#pragma unroll
-        for (int i = 0; i < PRB; ++i) {
-            u32x4 lo, hi;
-            widen16(breg[i], lo, hi);
-            *reinterpret_cast<u32x4*>(st + b_dst[i][0]) = lo;
-            *reinterpret_cast<u32x4*>(st + b_dst[i][1]) = hi;
-        }
+        for (int i = 0; i < PRW; ++i)
+            __builtin_amdgcn_global_load_lds((gbl_void*)(b_src[i] + kt * PBK), (lds_void*)(st + PBM * PROW + bwave + i * 64 * PWROW), 16, 0, 0);
     };
 
     const int frow = lane & 15, fk = lane >> 4;
     const int sw = (frow >> 1) & 7;
     const int ta = PARTIAL ? min(PTM, max(0, (p.rows - wm * 16 * PTM + 15) >> 4)) : PTM;
     const int a_off = (wm * 16 * PTM + frow) * PROW;
-    const int b_off = PBM * PROW + (wn * 16 * PTN + frow) * PROW;
+    const int b_off = PBM * PROW + (wn * 16 * PTN + frow) * PWROW + ((fk ^ weight_swizzle(frow)) << 4);      // (of rows 16 apart the swizzle is the same)
 
     f32x4 part[PTM][PTN];
 #pragma unroll
@@ -175,56 +149,38 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
     cfloat* sc0 = (cfloat*)(uintptr_t)p.s[0];
     cfloat* sc1 = (cfloat*)(uintptr_t)p.s[1];
 
-    // one k half (32) of a slab: fragments from LDS, PTM x PTN MFMAs into the partial sums.  (Holding both halves'
-    // fragments at once does not fit beside the two accumulator sets in the 256 registers of a wavefront.)
-    auto half_slab = [&](const unsigned char* st, int s, bool from_zero) {
-        const int c = ((s * 4 + fk) ^ sw) << 4;
-        bf16x8 af[PTM], bf[PTN];
+    // One slab: fragments from LDS, two halves of PTM x PTN MFMAs into the partial sums (FIRST: the first of a k block starts from zero).
+    auto slab = [&](int stage, auto first_c) {
+        constexpr bool FIRST = decltype(first_c)::value;
+        const unsigned char* st = smem + stage;
+        u32x4 raw[PTN];
 #pragma unroll
-        for (int j = 0; j < PTN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(st + b_off + j * 16 * PROW + c);
+        for (int j = 0; j < PTN; ++j) raw[j] = *reinterpret_cast<const u32x4*>(st + b_off + j * 16 * PWROW);
 #pragma unroll
-        for (int i = 0; i < PTM; ++i)
-            if (!PARTIAL || i < ta) af[i] = *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * PROW + c);
+        for (int s = 0; s < 2; ++s) {
+            const int c = ((s * 4 + fk) ^ sw) << 4;
+            bf16x8 af[PTM], bf[PTN];
 #pragma unroll
-        for (int i = 0; i < PTM; ++i) {
-            if (PARTIAL && i >= ta) continue;
+            for (int i = 0; i < PTM; ++i)
+                if (!PARTIAL || i < ta) af[i] = *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * PROW + c);
 #pragma unroll
-            for (int j = 0; j < PTN; ++j)
-                part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i],
-                                                                     from_zero ? f32x4{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+            for (int j = 0; j < PTN; ++j) bf[j] = widen8(raw[j][2 * s], raw[j][2 * s + 1]);
+#pragma unroll
+            for (int i = 0; i < PTM; ++i) {
+                if (PARTIAL && i >= ta) continue;
+#pragma unroll
+                for (int j = 0; j < PTN; ++j)
+                    part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], FIRST && s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+            }
         }
     };
-    // The workgroup barrier without the fences of __syncthreads(): a workgroup-scope release would make the compiler
-    // wait for every outstanding vector memory operation, the weight bytes in flight for a later slab included.  The
-    // waits that matter are spelled out in front of it.
-    auto barrier = [&]() {
+    // The next slab has landed (loads return in issue order; LATER: those of the slab behind it may still be on their way), and this
+    // wavefront's reads of LDS are done; then a barrier without the fences of __syncthreads(), which would wait for every load.
+    auto end_slab = [&](auto later_c) {
+        if (decltype(later_c)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PRA + PRW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-    };
-    // Slab kt sits in stage kt & 1 and the other stage is free (every wavefront is past the barrier that ended slab
-    // kt - 1).  The token rows of slab kt + 1 are requested first; with the MFMAs of the first k half the weight bytes
-    // of slab kt + 1 (fetched during slab kt - 1) are widened and written beside them, and the bytes of slab kt + 2 take
-    // their place in the registers.
-    // parity_c: kt & 1; next_c / next2_c: slabs kt + 1 and kt + 2 exist -- constants, so that the steady-state slab is one
-    // basic block (the last k block is peeled off).
-    auto slab = [&](int kt, auto parity_c, auto next_c, auto next2_c) {
-        constexpr int PAR = decltype(parity_c)::value;
-        constexpr bool NEXT = decltype(next_c)::value, NEXT2 = decltype(next2_c)::value;
-        const unsigned char* st = smem + PAR * PSTAGE;
-        if (NEXT) issue_a(kt + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        half_slab(st, 0, PAR == 0);            // a k block starts at an even slab: its first MFMAs start from zero
-        if (NEXT) store_b(kt + 1);
-        if (NEXT2) fetch_b(kt + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        half_slab(st, 1, false);
-    };
-    auto end_slab = [&](auto next2_c) {
-        // token rows of slab kt + 1 landed (loads return in issue order; only the weight bytes of slab kt + 2, requested
-        // behind them, may still be in flight), this wavefront's LDS writes and reads done
-        if (decltype(next2_c)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PRB) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        barrier();
     };
     auto fold = [&](float s0, float s1) {
 #pragma unroll
@@ -236,30 +192,38 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
                 for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(sc, part[i][j][r], acc[i][j][r]);
             }
     };
-    typedef std::integral_constant<int, 0> Even;
-    typedef std::integral_constant<int, 1> Odd;
+    // A slab whose successors exist: the stage that the slab in front of it left takes the slab two behind it.
+    int here = 0, next = PWSTAGE, free_stage = 2 * PWSTAGE;      // stages of slabs kt, kt + 1, kt + 2
+    auto turn = [&]() {
+        const int done = here;
+        here = next;
+        next = free_stage;
+        free_stage = done;
+    };
 
     __syncthreads();                        // the previous task may still be reading the stages
-    fetch_b(0);
-    issue_a(0);
-    store_b(0);
-    fetch_b(1);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PRB) : "memory");
-    barrier();
+    issue(0, here);
+    issue(1, next);
+    end_slab(std::true_type{});
     const int KB = p.K >> 7;
     int kb = 0;
     for (; kb < KB - 1; ++kb) {
         const float s0 = sc0[kb], s1 = sc1[kb];
-        slab(2 * kb, Even{}, std::true_type{}, std::true_type{});
+        issue(2 * kb + 2, free_stage);
+        slab(here, std::true_type{});
         end_slab(std::true_type{});
-        slab(2 * kb + 1, Odd{}, std::true_type{}, std::true_type{});
+        turn();
+        issue(2 * kb + 3, free_stage);
+        slab(here, std::false_type{});
         fold(s0, s1);
         end_slab(std::true_type{});
+        turn();
     }
     const float s0 = sc0[kb], s1 = sc1[kb];
-    slab(2 * kb, Even{}, std::true_type{}, std::false_type{});
+    slab(here, std::true_type{});
     end_slab(std::false_type{});
-    slab(2 * kb + 1, Odd{}, std::false_type{}, std::false_type{});
+    turn();
+    slab(here, std::false_type{});
     fold(s0, s1);
     end_slab(std::false_type{});
 }

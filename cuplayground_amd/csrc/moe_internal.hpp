@@ -28,14 +28,16 @@ struct MTile {
 
 // Words at the start of the queue-state block of the workspace (carved out of the workspace in api.hip).
 constexpr int kMaxQueueGroups = 8;   // XCDs of a gfx950
-// e4m3 layers: average rows per expert from which the tile GEMM replaces the weight streamer.  Measured on two shapes
-// (H 4096, I 14336, 8 experts and H 7168, I 2048, 64 experts): at 16 rows per expert the streamer is 18 % faster, at 32
-// the tile GEMM 13-17 %, at 128 it is 2.5 times and from 1024 on 3.3 times as fast.
-constexpr int kFp8TileRowsPerExpert = 32;
-// ... and from which widening the weights to bf16 in the workspace (one pass over them per call, 4.9 TB/s) and running
-// the bf16 tile GEMM replaces the e4m3 tile GEMM.  Measured, e4m3 tile time / this: H 4096, I 14336, 8 experts 1.01 at
-// 512 rows per expert, 1.08 at 768, 1.18 at 1024, 1.34 at 2048; H 7168, I 2048, 64 experts 0.95 at 512, 1.17 at 1024,
-// 1.30 at 2048; H = I = 2048, 16 experts 1.23 at 1024, 1.36 at 2048.
+// e4m3 layers: average rows per expert from which the tile GEMM replaces the weight streamer, whose row blocks of 16 take each weight byte
+// again for every 16 rows.  Whole layers, streamer / tile, us: 8 experts of 4096 x 14336, 16 rows each 341 / 423, 20 478 / 426, 32 618 /
+// 442; 64 of 7168 x 2048, 16 rows 719 / 717, 20 849 / 723, 32 1061 / 757; 256 of them, 12 rows 2217 / 2670, 16 2648 / 2722, 22 3396 / 2798;
+// 16 of 2048 x 2048, 16 rows 97 / 78, 32 139 / 85.
+constexpr int kFp8TileRowsPerExpert = 18;
+// ... and from which widening the weights to bf16 in the workspace (one pass over them per call, 6.1 TB/s) and running
+// the bf16 tile GEMM replaces the e4m3 tile GEMM.  Whole layers, e4m3 tile / this: 8 experts of 4096 x 14336, 640 rows each 0.88, 768
+// 0.96, 850 0.97, 950 1.04, 1200 1.12, 1500 1.18; 64 of 7168 x 2048, 512 rows 0.85, 768 0.96, 1024 1.03; 16 of 2048 x 2048, 768 rows 0.96,
+// 1024 1.00, 1250 1.06.  (Without the pass, on weights that the caller has prepared, it is the faster one from 768 rows on, and a
+// handle either takes prepared weights or does not, so the line stays where those are accepted.)
 constexpr int kFp8WidenRowsPerExpert = 768;
 // fp32 layers: average rows per expert and number of 128 x 128 tiles from which the matrix-core tile replaces the 64 x 64
 // vector-ALU one.  Measured FFN stage, vector / matrix: the reference's knob file (8192 rows, one expert, H 1024, I 4096)

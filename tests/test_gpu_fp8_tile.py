@@ -25,6 +25,8 @@ SHAPES = {
                         capacity_factor=1.25),
     "relu": ob.Cfg(S=640, H=384, I=128, E=3, k=1, act=ob.ACT_RELU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, norm_topk=0,
                    drop=0),
+    # odd numbers of k blocks, more than the ring of stages holds
+    "long_k": ob.Cfg(S=260, H=1408, I=640, E=3, k=1, act=ob.ACT_SWIGLU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, norm_topk=0, drop=0),
     # fewer rows than one block everywhere (the tile forced onto a decode-sized layer)
     "tiny_rows": ob.Cfg(S=40, H=256, I=128, E=8, k=2, act=ob.ACT_SWIGLU, dtype=ob.FP8, gate_fn=ob.GATE_SIGMOID, drop=0),
 }
@@ -120,4 +122,17 @@ def test_prefill_sized_layer_on_a_stratified_sample():
     layer.set_ffn_mode(FFN_TILED)
     out2 = layer.forward(dev["x"], dev)
     assert torch.equal(out, out2)
+    layer.close()
+
+
+@pytest.mark.parametrize("rows,block_rows", [(17, 16), (18, 128)])
+def test_the_tile_replaces_the_streamer_at_its_threshold(rows, block_rows):
+    import cuplayground_amd as moe
+    cfg = ob.Cfg(S=16 * rows, H=256, I=384, E=16, k=1, act=ob.ACT_SWIGLU, dtype=ob.FP8, norm_topk=0, drop=0)
+    layer = moe.MoELayer(product_config(cfg))
+    assert layer.plan["block_rows"] == block_rows
+    inp = ob.make_inputs(cfg, seed=rows)
+    dev = upload_inputs(cfg, inp)
+    got = ob.to_f32(from_device(layer.forward(dev["x"], dev)), cfg.act_dtype)
+    assert max_rel_err(got, ob.to_f32(ob.forward(cfg, inp)["out"], cfg.act_dtype)) <= OUT_TOL[ob.FP8]
     layer.close()

@@ -37,11 +37,10 @@ constexpr int PROW = 128;         // bytes per LDS row (64 bf16)
 constexpr int PSTAGE = (PBM + PBN) * PROW;
 constexpr int PLDS_M8 = 2 * PSTAGE + 2 * PBM * 4; // e4m3 x e4m3 loop: behind the two stages, the token rows' scales of either slab
 constexpr int PWROW = 64;         // bytes per LDS row of the weights (64 e4m3)
-constexpr int PWSTAGE = PBM * PROW + PBN * PWROW;
-constexpr int PLDS = 3 * PWSTAGE;
+constexpr int PLDS = 3 * (PBM * PROW + PBN * PWROW);
+static_assert(PLDS >= 4 * (PBM / 2 * PROW + PBN * PWROW), "the ring of row blocks of at most 64 rows");
 constexpr int PTHREADS = 256;
 constexpr int PTM = 4, PTN = 4;   // 16 x 16 fragments per wavefront: tokens, weight rows
-constexpr int PRA = PBM * 8 / PTHREADS;        // 16-byte token loads per thread per slab
 constexpr int PRW = PBN * 4 / PTHREADS;        // 16-byte weight loads (16 e4m3 values) per thread per slab
 
 struct TileTask {
@@ -74,12 +73,20 @@ __device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
 // more.  So both operands go from memory to LDS as they are stored, two slabs ahead, in a ring of three stages (two workgroups
 // per compute unit), and the weight bytes are widened behind their fragment reads: twice per workgroup then (two wavefronts
 // share weight rows), at two values an instruction, but without registers, LDS writes and waits for bytes on their way.
-// Weight bytes through registers, widened once per workgroup and written to LDS, the token rows one slab ahead / this, whole layers, us: 8
-// experts of 4096 x 14336, SwiGLU, 16 rows each 502 / 432, 50 530 / 483, 250 1055 / 974, 500 1867 / 1723, 1024 3517 / 3214; 64 of 7168 x
-// 2048, 37 rows 860 / 782, 500 3757 / 3477; 16 of 2048 x 2048, 500 rows 362 / 330; 256 of 7168 x 2048, 46 rows 3420 / 3149.
-// PARTIAL: the row block holds fewer than 128 rows; fragments that lie entirely in the padding are skipped.
-template <bool PARTIAL>
-__device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* smem, f32x4 (&acc)[PTM][PTN]) {
+// Weight bytes through registers, widened once per workgroup and written to LDS, the token rows one slab ahead / this (with blocks of 64,
+// below), whole layers, us: 8 experts of 4096 x 14336, SwiGLU, 50 rows each 530 / 425, 250 1055 / 962, 500 1867 / 1677, 1024 3517 / 3103; 64 of
+// 7168 x 2048, 37 rows 860 / 701, 500 3757 / 3410; 16 of 2048 x 2048, 500 rows 362 / 329; 256 of 7168 x 2048, 46 rows 3420 / 2866.
+// PARTIAL: the row block holds fewer than ROWS rows; fragments that lie entirely in the padding are skipped.  ROWS = 64: a stage is two
+// thirds as large, so that the ring has four and the loads run three slabs ahead (such a block is bound by the weight bytes in
+// flight), and its rows are shared by all four wavefronts.  Blocks of 128 for all /
+// this, us: 8 experts of 4096 x 14336, 32 rows each 458 / 406, 50 478 / 425, 175 (128 + 47) 772 / 737; 64 of 7168 x 2048, 37 rows 775 / 701; 256 of
+// them, 46 rows 3110 / 2866; without such blocks as before.
+template <bool PARTIAL, int ROWS>
+__device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* smem, f32x4 (&acc)[ROWS / 32][PTN]) {
+    constexpr int TM = ROWS / 32;                  // 16 x 16 fragments of token rows per wavefront
+    constexpr int AHEAD = ROWS == 64 ? 3 : 2;
+    constexpr int LOADS_A = ROWS * 8 / PTHREADS;   // 16-byte token loads per thread per slab
+    constexpr int STAGE = ROWS * PROW + PBN * PWROW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
 
@@ -89,9 +96,9 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
     const int prow = tid >> 3;
     const int slot = (tid & 7) ^ ((prow >> 1) & 7);
     const int chunk = 2 * (slot & 3) + (slot >> 2);
-    const uint16_t* a_src[PRA];
+    const uint16_t* a_src[LOADS_A];
 #pragma unroll
-    for (int i = 0; i < PRA; ++i) {
+    for (int i = 0; i < LOADS_A; ++i) {
         int r = prow + i * 32;
         if (r >= p.rows) r = 0;                                   // padding rows re-read row 0; never stored
         const int64_t src_row = p.gather ? (int64_t)p.gather[r] : p.a_row0 + r;
@@ -101,42 +108,34 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
     // 12-15 and 20-27 in one cycle, to 4-11, 16-19 and 28-31 in the next (and so on): of rows four apart, which meet the same banks,
     // two take chunk f and two f ^ 1, and all four must differ.
     auto weight_swizzle = [](int row) { return (4 - (row >> 2)) & 3; };
+    // (a wavefront's 16 rows are rows of one matrix: a scalar address, and one 32-bit offset for both loads)
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave), brow = tid >> 2;
     const uint8_t* b_src[PRW];
 #pragma unroll
-    for (int i = 0; i < PRW; ++i) {
-        const int j = (tid >> 2) + i * 64;                        // row of the weight tile
-        const uint8_t* base = p.w[0];
-        int col;
-        if (p.paired) {       // wavefront column w owns tile rows [64 w, 64 w + 64): 32 gate rows, then 32 up rows
-            const int w = j >> 6, jj = j & 63;
-            col = p.c0 + w * 32 + (jj & 31);
-            base = (jj >> 5) ? p.w[1] : p.w[0];
-        } else {
-            col = p.c0 + j;
-        }
-        b_src[i] = base + (int64_t)col * p.K + (((tid & 3) ^ weight_swizzle(j)) << 4);
-    }
+    for (int i = 0; i < PRW; ++i)         // paired: wavefront column i owns tile rows [64 i, 64 i + 64): 32 gate rows, then 32 up rows
+        b_src[i] = (p.paired && (wave_u >> 1) ? p.w[1] : p.w[0]) + (int64_t)(p.c0 + i * (p.paired ? 32 : 64)) * p.K;
+    const uint32_t b_lane = (uint32_t)(p.paired ? brow & 31 : brow) * (uint32_t)p.K + ((tid & 3) ^ weight_swizzle(brow)) * 16;
 
     const int awave = __builtin_amdgcn_readfirstlane(prow & ~7) * PROW, bwave = __builtin_amdgcn_readfirstlane((tid >> 2) & ~15) * PWROW;
     auto issue = [&](int kt, int stage) {
         unsigned char* st = smem + stage;
 #pragma unroll
-        for (int i = 0; i < PRA; ++i)
+        for (int i = 0; i < LOADS_A; ++i)
             __builtin_amdgcn_global_load_lds((gbl_void*)(a_src[i] + kt * PBK), (lds_void*)(st + awave + i * 32 * PROW), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < PRW; ++i)
-            __builtin_amdgcn_global_load_lds((gbl_void*)(b_src[i] + kt * PBK), (lds_void*)(st + PBM * PROW + bwave + i * 64 * PWROW), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_void*)(b_src[i] + kt * PBK + b_lane), (lds_void*)(st + ROWS * PROW + bwave + i * 64 * PWROW), 16, 0, 0);
     };
 
     const int frow = lane & 15, fk = lane >> 4;
     const int sw = (frow >> 1) & 7;
-    const int ta = PARTIAL ? min(PTM, max(0, (p.rows - wm * 16 * PTM + 15) >> 4)) : PTM;
-    const int a_off = (wm * 16 * PTM + frow) * PROW;
-    const int b_off = PBM * PROW + (wn * 16 * PTN + frow) * PWROW + ((fk ^ weight_swizzle(frow)) << 4);      // (of rows 16 apart the swizzle is the same)
+    const int ta = PARTIAL ? min(TM, max(0, (p.rows - wm * 16 * TM + 15) >> 4)) : TM;
+    const int a_off = (wm * 16 * TM + frow) * PROW;
+    const int b_off = ROWS * PROW + (wn * 16 * PTN + frow) * PWROW + ((fk ^ weight_swizzle(frow)) << 4);      // (of rows 16 apart the swizzle is the same)
 
-    f32x4 part[PTM][PTN];
+    f32x4 part[TM][PTN];
 #pragma unroll
-    for (int i = 0; i < PTM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < PTN; ++j) {
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -149,7 +148,7 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
     cfloat* sc0 = (cfloat*)(uintptr_t)p.s[0];
     cfloat* sc1 = (cfloat*)(uintptr_t)p.s[1];
 
-    // One slab: fragments from LDS, two halves of PTM x PTN MFMAs into the partial sums (FIRST: the first of a k block starts from zero).
+    // One slab: fragments from LDS, two halves of TM x PTN MFMAs into the partial sums (FIRST: the first of a k block starts from zero).
     auto slab = [&](int stage, auto first_c) {
         constexpr bool FIRST = decltype(first_c)::value;
         const unsigned char* st = smem + stage;
@@ -159,14 +158,14 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int c = ((s * 4 + fk) ^ sw) << 4;
-            bf16x8 af[PTM], bf[PTN];
+            bf16x8 af[TM], bf[PTN];
 #pragma unroll
-            for (int i = 0; i < PTM; ++i)
+            for (int i = 0; i < TM; ++i)
                 if (!PARTIAL || i < ta) af[i] = *reinterpret_cast<const bf16x8*>(st + a_off + i * 16 * PROW + c);
 #pragma unroll
             for (int j = 0; j < PTN; ++j) bf[j] = widen8(raw[j][2 * s], raw[j][2 * s + 1]);
 #pragma unroll
-            for (int i = 0; i < PTM; ++i) {
+            for (int i = 0; i < TM; ++i) {
                 if (PARTIAL && i >= ta) continue;
 #pragma unroll
                 for (int j = 0; j < PTN; ++j)
@@ -174,17 +173,18 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
             }
         }
     };
-    // The next slab has landed (loads return in issue order; LATER: those of the slab behind it may still be on their way), and this
+    // The next slab has landed (loads return in issue order; later: how many slabs behind it may still be on their way), and this
     // wavefront's reads of LDS are done; then a barrier without the fences of __syncthreads(), which would wait for every load.
-    auto end_slab = [&](auto later_c) {
-        if (decltype(later_c)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PRA + PRW) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    auto end_slab = [&](auto later) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(later)::value * (LOADS_A + PRW)) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    typedef std::integral_constant<int, 0> None;
+    typedef std::integral_constant<int, AHEAD - 1> Behind;
     auto fold = [&](float s0, float s1) {
 #pragma unroll
-        for (int i = 0; i < PTM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < PTN; ++j) {
                 const float sc = j < PTN / 2 ? s0 : s1;
@@ -192,40 +192,40 @@ __device__ __forceinline__ void tile_mainloop(const TileTask& p, unsigned char* 
                 for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(sc, part[i][j][r], acc[i][j][r]);
             }
     };
-    // A slab whose successors exist: the stage that the slab in front of it left takes the slab two behind it.
-    int here = 0, next = PWSTAGE, free_stage = 2 * PWSTAGE;      // stages of slabs kt, kt + 1, kt + 2
-    auto turn = [&]() {
-        const int done = here;
-        here = next;
-        next = free_stage;
-        free_stage = done;
-    };
-
+    // Stages are taken in turn: here slab kt's, ahead that of slab kt + AHEAD, which slab kt - 1 has left.
+    auto next = [](int stage) { return stage == AHEAD * STAGE ? 0 : stage + STAGE; };
+    int here = 0, ahead = AHEAD * STAGE;
+    const int KT = p.K >> 6;                // even
     __syncthreads();                        // the previous task may still be reading the stages
-    issue(0, here);
-    issue(1, next);
-    end_slab(std::true_type{});
-    const int KB = p.K >> 7;
-    int kb = 0;
-    for (; kb < KB - 1; ++kb) {
-        const float s0 = sc0[kb], s1 = sc1[kb];
-        issue(2 * kb + 2, free_stage);
-        slab(here, std::true_type{});
-        end_slab(std::true_type{});
-        turn();
-        issue(2 * kb + 3, free_stage);
-        slab(here, std::false_type{});
-        fold(s0, s1);
-        end_slab(std::true_type{});
-        turn();
+#pragma unroll
+    for (int kt = 0; kt < AHEAD; ++kt)
+        if (kt < 2 || kt < KT) issue(kt, kt * STAGE);
+    if (KT >= AHEAD) end_slab(Behind{});
+    else end_slab(None{});
+    int kt = 0;
+    auto k_block = [&](auto more0_c, auto more1_c) {     // slabs kt + AHEAD and kt + 1 + AHEAD exist
+        const float s0 = sc0[kt >> 1], s1 = sc1[kt >> 1];
+        auto one = [&](auto half_c, auto more_c) {
+            constexpr int half = decltype(half_c)::value;
+            constexpr bool more = decltype(more_c)::value;
+            if constexpr (more) issue(kt + half + AHEAD, ahead);
+            slab(here, std::integral_constant<bool, half == 0>{});
+            if constexpr (half == 1) fold(s0, s1);
+            end_slab(std::integral_constant<int, more ? AHEAD - 1 : 0>{});
+            here = next(here);
+            ahead = next(ahead);
+        };
+        one(std::integral_constant<int, 0>{}, more0_c);
+        one(std::integral_constant<int, 1>{}, more1_c);
+        kt += 2;
+    };
+    typedef std::true_type Yes;
+    typedef std::false_type No;
+    while (kt + 1 + AHEAD < KT) k_block(Yes{}, Yes{});
+    if constexpr (AHEAD == 3) {
+        if (kt + AHEAD < KT) k_block(Yes{}, No{});
     }
-    const float s0 = sc0[kb], s1 = sc1[kb];
-    slab(here, std::true_type{});
-    end_slab(std::false_type{});
-    turn();
-    slab(here, std::false_type{});
-    fold(s0, s1);
-    end_slab(std::false_type{});
+    k_block(No{}, No{});
 }
 
 // ---- the same tile with both operands e4m3: v_mfma_f32_16x16x128_f8f6f4 ----
@@ -353,14 +353,15 @@ __device__ __forceinline__ void tile_mainloop_mfma8(const TileTask& p, unsigned 
     }
 }
 
-// acc[i][j][r]: token row = 64 wm + 16 i + (lane & 15); weight row inside fragment j = 4 (lane >> 4) + r.
-__device__ __forceinline__ void tile_epilogue(const TileTask& p, f32x4 (&acc)[PTM][PTN]) {
+// acc[i][j][r]: token row = 16 (TM wm + i) + (lane & 15); weight row inside fragment j = 4 (lane >> 4) + r.
+template <int TM>
+__device__ __forceinline__ void tile_epilogue(const TileTask& p, f32x4 (&acc)[TM][PTN]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int frow = lane & 15, fk = lane >> 4;
 #pragma unroll
-    for (int i = 0; i < PTM; ++i) {
-        const int m = wm * 16 * PTM + i * 16 + frow;
+    for (int i = 0; i < TM; ++i) {
+        const int m = wm * 16 * TM + i * 16 + frow;
         if (m >= p.rows) continue;
         uint16_t* crow = p.c_base + (int64_t)m * p.N;
         if (p.paired) {
@@ -399,9 +400,15 @@ __device__ __forceinline__ void tile_epilogue(const TileTask& p, f32x4 (&acc)[PT
 }
 
 __device__ __forceinline__ void fp8_gemm_tile(const TileTask& p, unsigned char* smem) {
+    if (p.rows <= PBM / 2) {
+        f32x4 acc[PTM / 2][PTN];
+        tile_mainloop<true, PBM / 2>(p, smem, acc);
+        tile_epilogue(p, acc);
+        return;
+    }
     f32x4 acc[PTM][PTN];
-    if (p.rows < PBM) tile_mainloop<true>(p, smem, acc);
-    else tile_mainloop<false>(p, smem, acc);
+    if (p.rows < PBM) tile_mainloop<true, PBM>(p, smem, acc);
+    else tile_mainloop<false, PBM>(p, smem, acc);
     tile_epilogue(p, acc);
 }
 __device__ __forceinline__ void fp8_gemm_tile_mfma8(const TileTask& p, unsigned char* smem) {

@@ -29,14 +29,14 @@ struct MTile {
 // Words at the start of the queue-state block of the workspace (carved out of the workspace in api.hip).
 constexpr int kMaxQueueGroups = 8;   // XCDs of a gfx950
 // e4m3 layers: average rows per expert from which the tile GEMM replaces the weight streamer, whose row blocks of 16 take each weight byte
-// again for every 16 rows.  Whole layers, streamer / tile, us: 8 experts of 4096 x 14336, 16 rows each 341 / 423, 20 478 / 426, 32 618 /
-// 442; 64 of 7168 x 2048, 16 rows 719 / 717, 20 849 / 723, 32 1061 / 757; 256 of them, 12 rows 2217 / 2670, 16 2648 / 2722, 22 3396 / 2798;
-// 16 of 2048 x 2048, 16 rows 97 / 78, 32 139 / 85.
+// again for every 16 rows.  Whole layers, streamer / tile, us: 8 experts of 4096 x 14336, 16 rows each 341 / 400, 20 478 / 397, 32 618 /
+// 409; 64 of 7168 x 2048, 16 rows 722 / 658, 20 848 / 665, 32 1061 / 690; 256 of them, 12 rows 2214 / 2438, 16 2643 / 2503, 22 3392 / 2593;
+// 16 of 2048 x 2048, 16 rows 97 / 72, 32 141 / 72.
 constexpr int kFp8TileRowsPerExpert = 18;
 // ... and from which widening the weights to bf16 in the workspace (one pass over them per call, 6.1 TB/s) and running
 // the bf16 tile GEMM replaces the e4m3 tile GEMM.  Whole layers, e4m3 tile / this: 8 experts of 4096 x 14336, 640 rows each 0.88, 768
-// 0.96, 850 0.97, 950 1.04, 1200 1.12, 1500 1.18; 64 of 7168 x 2048, 512 rows 0.85, 768 0.96, 1024 1.03; 16 of 2048 x 2048, 768 rows 0.96,
-// 1024 1.00, 1250 1.06.  (Without the pass, on weights that the caller has prepared, it is the faster one from 768 rows on, and a
+// 0.93, 850 0.94, 950 1.02, 1200 1.10, 1500 1.18; 64 of 7168 x 2048, 512 rows 0.84, 768 0.94, 1024 1.01; 16 of 2048 x 2048, 768 rows 1.01,
+// 1024 1.01, 1250 1.08.  (Without the pass, on weights that the caller has prepared, it is the faster one from 768 rows on, and a
 // handle either takes prepared weights or does not, so the line stays where those are accepted.)
 constexpr int kFp8WidenRowsPerExpert = 768;
 // fp32 layers: average rows per expert and number of 128 x 128 tiles from which the matrix-core tile replaces the 64 x 64

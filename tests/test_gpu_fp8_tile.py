@@ -136,3 +136,14 @@ def test_the_tile_replaces_the_streamer_at_its_threshold(rows, block_rows):
     got = ob.to_f32(from_device(layer.forward(dev["x"], dev)), cfg.act_dtype)
     assert max_rel_err(got, ob.to_f32(ob.forward(cfg, inp)["out"], cfg.act_dtype)) <= OUT_TOL[ob.FP8]
     layer.close()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64, 65, 127, 128, 129, 192, 193])
+@pytest.mark.parametrize("H,I", [(128, 256), (256, 384), (384, 128)])
+def test_row_blocks_of_every_kind(rows, H, I):
+    """One expert of `rows` rows: blocks of at most 64 rows (a ring of four stages) and of up to 128 (three), contractions of one to three
+    blocks of 128, which end before, at and behind what the rings ask for ahead."""
+    cfg = ob.Cfg(S=rows, H=H, I=I, E=1, k=1, act=ob.ACT_SWIGLU, dtype=ob.FP8, norm_topk=0, drop=0)
+    inp = ob.make_inputs(cfg, seed=rows + H)
+    got = _run(cfg, inp, FFN_TILED, 1, calls=2)
+    assert max_rel_err(got["out"], ob.to_f32(ob.forward(cfg, inp)["out"], cfg.act_dtype)) <= OUT_TOL[ob.FP8]

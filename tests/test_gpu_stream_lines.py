@@ -36,6 +36,7 @@ def test_cold_and_kept_weights_give_the_same_bits(S, H, I, k, act, dtype):
             else:
                 d[n] = torch.zeros(E, *t.shape[1:], dtype=adt, device="cuda")
                 d[n][:small] = t.to(adt)
-        outs.append(moe.MoELayer(cfg).forward(x, d))
+        # (26 rows an expert: e4m3 layers of so many take the tile by themselves)
+        outs.append(moe.MoELayer(cfg, options={"fp8_tile": 0} if dtype == 4 else None).forward(x, d))
     assert outs[0].isfinite().all() and outs[0].any()
     assert torch.equal(outs[0], outs[1])

@@ -121,9 +121,10 @@ def test_phase0_results_are_complete_before_they_are_signalled(source):
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_fp8_tile_barriers_sit_behind_their_waits():
     """The e4m3 tile GEMM (ffn_fp8_tile.hip) meets at a bare s_barrier and spells its waits out in front of it: between
-    the wait that covers the direct-to-LDS loads and this wavefront's LDS traffic (s_waitcnt vmcnt(<=2) lgkmcnt(0)) and
-    the barrier the compiler may not have placed an LDS access or a load of either kind; its slab loops hold no spill;
-    and the weight bytes are awaited with the count that leaves only the token-row loads issued since (vmcnt(4))."""
+    the wait that covers the direct-to-LDS loads and this wavefront's LDS traffic (s_waitcnt vmcnt(n) lgkmcnt(0)) and
+    the barrier the compiler may not have placed an LDS access or a load of either kind, and its slab loops hold no spill.  n
+    leaves the slabs behind the next one: one of 4 + 2 loads where a row block has up to 128 rows, two of 2 + 2 where it has up to 64,
+    none at the end."""
     text = _assembly("ffn_fp8_tile.hip")
     kernels = re.findall(r"\n(_ZN6moe355\w*fp8_tile_kernel\w*):[^\n]*\n(.*?)\n\s*s_endpgm", text, re.S)
     assert len(kernels) == 2
@@ -131,7 +132,7 @@ def test_fp8_tile_barriers_sit_behind_their_waits():
         lines = [x.strip() for x in body.split("\n") if x.strip() and not x.strip().startswith(";")]
         mfma = [i for i, x in enumerate(lines) if x.startswith("v_mfma")]
         assert len(mfma) >= 6 * 32, name
-        checked = 0
+        checked, seen = 0, set()
         for i, x in enumerate(lines):
             if not x.startswith("s_barrier") or not any(abs(i - m) < 60 for m in mfma):
                 continue
@@ -139,7 +140,8 @@ def test_fp8_tile_barriers_sit_behind_their_waits():
             for back in range(i - 1, max(i - 40, 0), -1):
                 w = re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)", lines[back])
                 if w:
-                    assert int(w.group(1)) <= 2, (name, lines[back])
+                    assert int(w.group(1)) in (0, 6, 8), (name, lines[back])
+                    seen.add(int(w.group(1)))
                     break
                 between.append(lines[back])
             else:
@@ -147,7 +149,7 @@ def test_fp8_tile_barriers_sit_behind_their_waits():
             assert not [b for b in between if b.startswith(("ds_", "global_load", "buffer_load", "scratch_"))], (name, between)
             checked += 1
         assert checked >= 6, (name, checked)      # prologue + two per steady-state block + two of the peeled block, twice
-        assert any(x == "s_waitcnt vmcnt(4)" for x in lines), name
+        assert seen == {0, 6, 8}, (name, seen)
         # no spill traffic between the first and the last MFMA of a slab loop: loops are the label .. back-branch ranges
         labels = {x.split(":")[0]: i for i, x in enumerate(lines) if re.match(r"\.LBB\d+_\d+:", x)}
         slab_loops = 0
@@ -207,9 +209,9 @@ def _vregs(text):
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_fp8_tile_weight_bytes_are_not_touched_in_flight():
-    """The e4m3 tile GEMM fetches its weight bytes with a load written in assembly, so the compiler does not know that
-    the destination registers are pending until the wait that names them (s_waitcnt vmcnt(4)).  Inside the slab loops
-    nothing between such a load and that wait may read, copy or spill those registers."""
+    """The e4m3 tile GEMM asks for its operands slabs ahead of their use.  Nothing of them may travel through registers on the way (a load
+    written in assembly leaves its destination registers pending without the compiler's knowing): in the slab loops every
+    vector load goes straight to LDS, six a slab (four of token rows, two of weight rows) where a row block has up to 128 rows."""
     text = _assembly("ffn_fp8_tile.hip")
     kernels = re.findall(r"\n(_ZN6moe355\w*fp8_tile_kernel\w*):[^\n]*\n(.*?)\n\s*s_endpgm", text, re.S)
     assert len(kernels) == 2
@@ -224,21 +226,10 @@ def test_fp8_tile_weight_bytes_are_not_touched_in_flight():
             loop = [y for y in lines[labels[j.group(1)]:i] if not re.match(r"\.LBB\d+_\d+:", y)]
             if sum(y.startswith("v_mfma") for y in loop) < 32 or sum(y.startswith("s_barrier") for y in loop) != 2:
                 continue
-            n = len(loop)
-            for k, y in enumerate(loop):
-                m = re.match(r"global_load_dwordx4 v\[(\d+):(\d+)\], v\[\d+:\d+\], off", y)
-                if not m:
-                    continue
-                pending = set(range(int(m.group(1)), int(m.group(2)) + 1))
-                for step in range(1, n + 1):           # the wait may sit behind the loop's back edge
-                    z = loop[(k + step) % n]
-                    if z == "s_waitcnt vmcnt(4)":
-                        break
-                    assert not (_vregs(z) & pending), (name, y, z)
-                else:
-                    raise AssertionError("no wait for " + y)
-                checked += 1
-        assert checked >= 4, (name, checked)       # two loads per slab, two slabs per loop iteration
+            loads = [y for y in loop if y.startswith(("global_load", "buffer_load", "flat_load", "scratch_load"))]
+            assert loads and all(y.startswith("global_load_lds_dwordx4") for y in loads), (name, loads)
+            checked += len(loads) == 12
+        assert checked >= 1, name
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")

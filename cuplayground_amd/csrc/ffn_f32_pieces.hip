@@ -16,7 +16,9 @@
 // for the pieces of tokens and weights at 6.2 TB/s.
 // Values that three pieces do not hold -- infinities and NaN, whose products with a zero piece would be NaN, and magnitudes of 2^100
 // and more or below 2^-100 -- set QueueState::inexact, in the pass that makes the pieces or where the up projection's results become
-// some; then these launches do nothing and the fp32 tiles behind them (ffn_f32_tile.hip), which otherwise do nothing, run instead.
+// some.  So does a sum of either projection that is not finite: the pieces of two values that they hold can overflow where the product
+// of the values is infinite (one of them with the other sign: NaN) or just below the largest number.  The fp32 tiles at the end
+// (ffn_f32_tile.hip), which do nothing otherwise, then take both projections again.
 #include <algorithm>
 
 #include "ffn_bf16_tile.hpp"
@@ -45,6 +47,7 @@ __device__ __forceinline__ bool inexact_as_pieces(float v) {
     const uint32_t a = __float_as_uint(v) & 0x7FFFFFFFu;
     return a != 0u && (a >> 23) - 27u >= 200u;
 }
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
 // Two values as pieces: p[i] their i-th pieces side by side.
 __device__ __forceinline__ void pieces2(float v0, float v1, uint32_t (&p)[3]) {
 #pragma unroll
@@ -149,6 +152,7 @@ __device__ __forceinline__ void piece_epilogue(const PieceEpilogue& e, unsigned 
 #pragma unroll 1
         for (int s = 0; s < 64 / ROWS; ++s) {
             const int row = row0 + s * ROWS;
+            bool over = false;
             const f32x4* g = reinterpret_cast<const f32x4*>(get + s * ROWS * PITCH);
             const f32x4* u = SWIGLU ? g + COLS / 4 : g;
             float v[8];
@@ -158,11 +162,13 @@ __device__ __forceinline__ void piece_epilogue(const PieceEpilogue& e, unsigned 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float x = uu[r] + b0[4 * q + r];
+                    over = over || !finite(x);           // (here: ReLU makes a zero of -inf.  An infinite gate makes a NaN or stays infinite)
                     if constexpr (SWIGLU) v[4 * q + r] = silu(gg[r] + b1[4 * q + r]) * x;
                     else v[4 * q + r] = act_apply(x, EPI == MOE_ACT_GELU ? MOE_ACT_GELU : e.act);
                 }
             }
             if (row >= e.rows || !mine) continue;
+            bad = bad || over;
             if constexpr (UP) {
                 u32x4 out[3];
 #pragma unroll
@@ -183,7 +189,7 @@ __device__ __forceinline__ void piece_epilogue(const PieceEpilogue& e, unsigned 
             }
         }
     }
-    if (UP && bad) e.inexact[1] = 1;
+    if (bad) e.inexact[UP ? 1 : 2] = 1;
 }
 
 struct PieceArgs {
@@ -207,7 +213,7 @@ __global__ __launch_bounds__(P::THREADS) void ffn_tiled_f32_pieces_kernel(PieceA
     constexpr bool SWIGLU = EPI == MOE_ACT_SWIGLU;
     constexpr int COLS = SWIGLU ? P::BN / 2 : P::BN;
     extern __shared__ __align__(16) unsigned char smem[];
-    if (a.inexact[0] || (!UP && a.inexact[1])) return;      // (the up projection sets the second word itself)
+    if (a.inexact[0] || (!UP && a.inexact[1])) return;      // (never a word that this launch sets: all wavefronts go the same way)
     GroupedTask t;
     if (!grouped_task<P::BIG>(a.count, a.offset, a.E, (a.N + COLS - 1) / COLS, blockIdx.x, t)) return;
     const int ld = 3 * a.K;
@@ -266,8 +272,8 @@ hipError_t launch_pieces(const PieceArgs& a, int64_t rows, hipStream_t st) {
 
 }  // namespace
 
-// A whole FFN stage.  x_pieces [S, 3, H], w_pieces the matrices [up | down | gate] as pieces, h_pieces [A, 3, I] (may lie on a.h: the
-// fp32 tiles write that only when the pieces are not used).
+// A whole FFN stage.  x_pieces [S, 3, H], w_pieces the matrices [up | down | gate] as pieces, h_pieces [A, 3, I] (may lie on a.h),
+// inexact: three words that are zero (QueueState::inexact).
 hipError_t launch_ffn_f32_pieces(const FfnArgs& a, const ExpertRows& rows, void* x_pieces, void* w_pieces, void* h_pieces, int32_t* inexact,
                                  int max_mtiles, int nnt0, int nnt1, hipStream_t st) {
     const bool sw = a.act == MOE_ACT_SWIGLU;
@@ -291,11 +297,11 @@ hipError_t launch_ffn_f32_pieces(const FfnArgs& a, const ExpertRows& rows, void*
                 rows.count, rows.offset, inexact, a.E, a.I, a.H, a.act, (uint32_t)((int64_t)a.S * 3 * a.H * 2)};
     e = sw ? launch_pieces<MOE_ACT_SWIGLU, true>(p, A, st) : a.act == MOE_ACT_GELU ? launch_pieces<MOE_ACT_GELU, true>(p, A, st) : launch_pieces<MOE_ACT_NONE, true>(p, A, st);
     if (e != hipSuccess) return e;
-    e = launch_ffn_f32_tile_if(a, 0, inexact, max_mtiles, nnt0, st);
-    if (e != hipSuccess) return e;
     p = PieceArgs{(const uint16_t*)h_pieces, w[1], nullptr, (const float*)a.b_down, nullptr, (float*)a.y, nullptr, nullptr,
                   rows.count, rows.offset, inexact, a.E, a.H, a.I, MOE_ACT_NONE, (uint32_t)(A * 3 * a.I * 2)};
     e = launch_pieces<MOE_ACT_NONE, false>(p, A, st);
+    if (e != hipSuccess) return e;
+    e = launch_ffn_f32_tile_if(a, 0, inexact, max_mtiles, nnt0, st);      // (behind the last reader of h_pieces, on which it may write)
     if (e != hipSuccess) return e;
     return launch_ffn_f32_tile_if(a, 1, inexact, max_mtiles, nnt1, st);
 }

@@ -245,11 +245,11 @@ __device__ __forceinline__ TileTaskF resolve_tile_f32(const FfnArgs& a, const Ta
     return p;
 }
 
-// only_if: null, or two device words; where both are zero there is nothing to do (ffn_f32_pieces.hip).
+// only_if: null, or three device words; where all are zero there is nothing to do (ffn_f32_pieces.hip).
 __global__ __launch_bounds__(GTHREADS) void ffn_tiled_f32_tile_kernel(FfnArgs a, int phase, const int32_t* only_if) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_list[1 + GBM];
-    if (only_if && (only_if[0] | only_if[1]) == 0) return;
+    if (only_if && (only_if[0] | only_if[1] | only_if[2]) == 0) return;
     if (phase == 0) zero_unrouted_rows(a, 4);
     Task t;
     if (!tiled_task(a, phase, blockIdx.x, t)) return;
@@ -396,7 +396,7 @@ hipError_t launch_wgrad_f32_tile(const void* dyT, const void* aT, void* dw, cons
     return hipGetLastError();
 }
 
-// One projection of the two launches, if one of the two words is set.
+// One projection of the two launches, if one of the three words is set.
 hipError_t launch_ffn_f32_tile_if(const FfnArgs& a, int phase, const int32_t* only_if, int max_mtiles, int nnt, hipStream_t st) {
     hipError_t e = allow_lds(&ffn_tiled_f32_tile_kernel);
     if (e != hipSuccess) return e;

@@ -68,8 +68,8 @@ struct QueueState {
     int32_t ids_phase1;
     int32_t split_mt0;     // first row block whose down-projection tiles run as partial sums (num_mtiles: none)
     int32_t nseg_phase1;   // segments of the phase-1 table (the experts, plus one when a run was cut at split_mt0)
-    int32_t inexact[2];    // fp32 layers as bf16 pieces: three pieces do not hold one of the operands / of the up projection's results
-    int32_t pad[1];
+    int32_t inexact[3];    // fp32 layers as bf16 pieces: three pieces do not hold one of the operands / of the up projection's results, or
+                           // a sum of that / of the down projection is not finite
 };
 // State of the combine tasks of the queue kernels, in a cache line of its own: the workgroups that have run out of GEMM
 // tasks poll it, and must not stand in the way of the queue heads that the busy ones pop.

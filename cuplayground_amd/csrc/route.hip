@@ -246,7 +246,7 @@ __device__ __forceinline__ void route_scan_body(const RouteArgs& a, ScanShared& 
         a.q->num_mtiles = total_mt;
         a.q->kept_rows = total_rows;
         a.q->stall = 0;
-        a.q->inexact[0] = a.q->inexact[1] = 0;
+        a.q->inexact[0] = a.q->inexact[1] = a.q->inexact[2] = 0;
         a.q->nseg = nseg_final;
         a.expert_offset[a.E] = total_rows;
     }

@@ -96,6 +96,35 @@ def test_values_that_pieces_do_not_hold(moe, name, what):
     pieces.close(), tile.close()
 
 
+def _same(got, want):
+    import torch
+    return torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(1.0, 2.0, 3.0), want.nan_to_num(1.0, 2.0, 3.0))
+
+
+@pytest.mark.parametrize("what", ["down_infinite", "down_near_largest", "up_negative_infinite"])
+def test_sums_that_overflow_on_pieces_only(moe, what):
+    """Every operand is held by three pieces, but the pieces' products or their sums leave the range before those of the values do."""
+    import torch
+    cfg, pieces, tile, x, w = _layers(moe, "relu_one_expert")
+    S, H = x.shape
+    t, below = torch.arange(S, device="cuda"), 2.0 ** 64 * (1 - 2.0 ** -13)     # below: its first piece is 2^64
+    x.zero_(), w["w_up"].zero_()
+    j = torch.arange(H, device="cuda")
+    if what == "up_negative_infinite":     # -2^128 (1 - 2^-12) and three times nearly 2^127: on pieces -inf, which ReLU turns into a zero
+        for k in (1, 130, 260, 390):
+            x[:, k], w["w_up"][0, :, k] = (-below, below) if k == 1 else (2.0 ** 63 * (1 - 2.0 ** -10), 2.0 ** 64)
+        w["w_down"].fill_(2.0 ** -90)
+    else:                                  # hidden column j is token column j
+        w["w_up"][0, j, j] = 1.0
+        x[t, t % H] = below if what == "down_near_largest" else 2.0 ** 70 * (1 + 2.0 ** -8 + 2.0 ** -12)
+        w["w_down"][:] = below if what == "down_near_largest" else 2.0 ** 70 * 1.9989
+        w["w_down"][:, ::2] *= -1
+    got, want = pieces.forward(x, w), tile.forward(x, w)
+    assert want.isinf().all() if what == "down_infinite" else want.isfinite().all() and want.any()
+    assert _same(got, want)
+    pieces.close(), tile.close()
+
+
 def test_smallest_and_largest_magnitudes_that_pieces_hold(moe):
     """2^-100 and just below 2^100 as operands: all three pieces count."""
     import torch

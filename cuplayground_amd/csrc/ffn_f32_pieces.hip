@@ -14,11 +14,15 @@
 // fp32 product runs at 200 TFLOP/s.  The reference's knob file (8192 rows, one expert of 1024 x 4096, ReLU): up and down projection 577 and
 // 556 us on the fp32 instructions; 339 and 357 here, on 256- and on 128-row blocks (128 tiles of 256 rows, half the chip: 494), behind 27 us
 // for the pieces of tokens and weights at 6.2 TB/s.
-// Values that three pieces do not hold -- infinities and NaN, whose products with a zero piece would be NaN, and magnitudes of 2^100
-// and more or below 2^-100 -- set QueueState::inexact, in the pass that makes the pieces or where the up projection's results become
-// some.  So does a sum of either projection that is not finite: the pieces of two values that they hold can overflow where the product
-// of the values is infinite (one of them with the other sign: NaN) or just below the largest number.  The fp32 tiles at the end
-// (ffn_f32_tile.hip), which do nothing otherwise, then take both projections again.
+// Values are multiplied by 2^24 before they are taken apart, so that the lowest bit of any fp32 number, denormal ones included, is a
+// normal bf16 number, and neither the pieces nor the products that matter of small values (2^-62 times 2^-62, say) fall below the
+// range; the sums are multiplied by 2^-48.  Values that three pieces do not hold even so -- infinities and NaN, whose products with a
+// zero piece would be NaN, and magnitudes of 2^76 and more -- set QueueState::inexact, in the pass that makes the pieces or where the up
+// projection's results become some.  So does a sum of either projection that is not finite: the pieces of two values can overflow where
+// the product of the values does not (or with the other sign: NaN).  The fp32 tiles at the end (ffn_f32_tile.hip), which do nothing
+// otherwise, then take both projections again.  What such a call costs, us, on pieces / on the fp32 tiles without asking / an infinite token /
+// sums of 2^76 in the up projection: the knob file 711 / 1067 / 1098 / 1449; 8 experts of 1024 x 2048, SwiGLU, 2048 rows each 1248 / 1825 /
+// 1885 / 2571.
 #include <algorithm>
 
 #include "ffn_bf16_tile.hpp"
@@ -42,14 +46,15 @@ struct PieceSplit {
     static constexpr int LDS_BYTES = TB::LDS_BYTES;
 };
 
-// Not held by three pieces (zero is).
-__device__ __forceinline__ bool inexact_as_pieces(float v) {
-    const uint32_t a = __float_as_uint(v) & 0x7FFFFFFFu;
-    return a != 0u && (a >> 23) - 27u >= 200u;
-}
+constexpr float kPieceScale = 16777216.0f, kSumScale = 1.0f / kPieceScale / kPieceScale;
+// Not held by three pieces of kPieceScale times it.
+__device__ __forceinline__ bool inexact_as_pieces(float v) { return (__float_as_uint(v) & 0x7FFFFFFFu) >= 0x65800000u; }
+static_assert((0x65800000u >> 23) == 127 + 76, "from 2^76 on");
 __device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
-// Two values as pieces: p[i] their i-th pieces side by side.
+// kPieceScale times two values as pieces: p[i] their i-th pieces side by side.
 __device__ __forceinline__ void pieces2(float v0, float v1, uint32_t (&p)[3]) {
+    v0 *= kPieceScale;
+    v1 *= kPieceScale;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         p[i] = pack2_bf16(v0, v1);
@@ -161,9 +166,9 @@ __device__ __forceinline__ void piece_epilogue(const PieceEpilogue& e, unsigned 
                 const f32x4 uu = u[q], gg = g[q];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float x = uu[r] + b0[4 * q + r];
+                    const float x = uu[r] * kSumScale + b0[4 * q + r];
                     over = over || !finite(x);           // (here: ReLU makes a zero of -inf.  An infinite gate makes a NaN or stays infinite)
-                    if constexpr (SWIGLU) v[4 * q + r] = silu(gg[r] + b1[4 * q + r]) * x;
+                    if constexpr (SWIGLU) v[4 * q + r] = silu(gg[r] * kSumScale + b1[4 * q + r]) * x;
                     else v[4 * q + r] = act_apply(x, EPI == MOE_ACT_GELU ? MOE_ACT_GELU : e.act);
                 }
             }

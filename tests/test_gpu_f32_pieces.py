@@ -70,7 +70,7 @@ def test_no_further_from_float64_than_the_fp32_tile(moe, name):
     pieces.close(), tile.close()
 
 
-@pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_huge", "w_tiny", "x_denormal", "h_huge", "h_tiny"])
+@pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_huge", "h_huge"])
 @pytest.mark.parametrize("name", ["gelu_bias_drop", "swiglu_bias"])
 def test_values_that_pieces_do_not_hold(moe, name, what):
     """The whole call by the fp32 instructions, bit for bit (NaN in the same places)."""
@@ -82,17 +82,39 @@ def test_values_that_pieces_do_not_hold(moe, name, what):
         x[cfg.tokens - 1, 0] = float("nan")
     elif what == "w_huge":
         w["w_down"][1, 3, 64] = 3e38
-    elif what == "w_tiny":
-        w["w_up"][0, 7, 9] = 2.0 ** -101
-    elif what == "x_denormal":
-        x[100, 11] = 1e-41
     else:      # operands that pieces hold, results of the up projection that they do not
-        x *= 1.0 if what == "h_huge" else 1e-15
-        for n in ("w_up", "w_gate", "b_up", "b_gate"):
-            if n in w:
-                w[n] *= 0.0 if n[0] == "b" else 1e30 if what == "h_huge" else 1e-20
+        x *= 1e3
+        w["w_up"] *= 1e21
     got, want = pieces.forward(x, w), tile.forward(x, w)
     assert torch.equal(got.view(torch.int32), want.view(torch.int32)) or (torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()))
+    pieces.close(), tile.close()
+
+
+@pytest.mark.parametrize("name,what", [(n, w) for n in ("gelu_bias_drop", "swiglu_bias") for w in ("w_tiny", "x_denormal", "h_tiny")] + [("swiglu_bias", "silu_tail")])
+def test_small_values_are_held(moe, name, what):
+    """However small a value is, it is held exactly: the call stays on pieces (the fp32 tile's bits are others), and is no further from
+    float64.  A gate of -66 and less makes intermediate values below 2^-100 of ordinary tokens."""
+    import torch
+    cfg, pieces, tile, x, w = _layers(moe, name)
+    if what == "w_tiny":
+        w["w_up"][0, 7, 9] = 2.0 ** -101
+        w["w_down"][:, 5] *= 2.0 ** -120
+    elif what == "x_denormal":
+        x[100, 11] = 1e-41
+        x[:, 12] *= 2.0 ** -125
+    elif what == "h_tiny":
+        x *= 1e-15
+        for n in ("w_up", "w_gate", "b_up", "b_gate", "b_down"):
+            if n in w:
+                w[n] *= 0.0 if n[0] == "b" else 1e15 if n == "w_gate" else 1e-20
+        w["w_down"] *= 1e10
+    else:
+        w["b_gate"][:, ::3] = -torch.linspace(60.0, 90.0, w["b_gate"][:, ::3].shape[1], device="cuda")
+    routing = pieces.new_routing()
+    got, other = pieces.forward(x, w, routing=routing), tile.forward(x, w)
+    ref = _float64(cfg, x, w, routing)
+    far = lambda o: ((o.double() - ref).norm() / ref.norm()).item()
+    assert ref.any() and far(got) <= far(other) and far(got) < 1e-6 and not torch.equal(got, other), (far(got), far(other))
     pieces.close(), tile.close()
 
 
@@ -126,12 +148,15 @@ def test_sums_that_overflow_on_pieces_only(moe, what):
 
 
 def test_smallest_and_largest_magnitudes_that_pieces_hold(moe):
-    """2^-100 and just below 2^100 as operands: all three pieces count."""
+    """Tokens down to the denormal numbers against weights up to just below 2^76: all three pieces count."""
     import torch
     cfg, pieces, tile, x, w = _layers(moe, "relu_one_expert")
-    x *= 2.0 ** -90
-    x[x.abs() < 2.0 ** -100] = 2.0 ** -100
-    w["w_up"] *= 2.0 ** 60
+    x *= 2.0 ** -115
+    x[:, ::5] *= 2.0 ** -15
+    x[0, 0] = 2.0 ** -149
+    w["w_up"] *= 2.0 ** 77
+    w["w_up"].clamp_(-(2.0 ** 76 - 2.0 ** 52), 2.0 ** 76 - 2.0 ** 52)
+    w["w_up"][0, 0, 0] = 2.0 ** 76 - 2.0 ** 52
     routing = pieces.new_routing()
     got, other = pieces.forward(x, w, routing=routing), tile.forward(x, w)
     ref = _float64(cfg, x, w, routing)

@@ -68,7 +68,7 @@ struct Derived {
     int64_t capacity;
     FfnPlan plan;
     int nblk;          // workgroups of the slot-assignment kernels
-    bool f32_pieces;   // fp32 layer that runs on bf16 pieces unless its mode or options ask for a schedule of the fp32 tile
+    bool f32_pieces;   // fp32 layer that runs on bf16 pieces unless the task queue is asked for
     int wide_mats;     // weight matrices per expert (3 with SwiGLU, else 2)
     int max_mtiles;
 };
@@ -324,6 +324,7 @@ template <typename T>
 T* at(void* ws, size_t off) { return reinterpret_cast<T*>(static_cast<char*>(ws) + off); }
 
 int resolved_ffn_mode(const moe_handle* h);
+int combine_run(const moe_handle* h);
 
 RouteArgs route_args(const moe_handle* h, void* ws) {
     const Derived& d = h->d;
@@ -346,8 +347,8 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
     // arrival counters [S, nnt1] of the combine inside the FFN kernels, or the flags [S * slices] of the combine tasks of
     // the queue (a slice is at least 1024 columns, a column tile at most 256: the flags fit the same array); the latter
     // exist in task-queue mode only
-    const bool queue_combine = h->combine_mode == 2 && resolved_ffn_mode(h) == MOE_FFN_PERSISTENT;
-    a.arrive = (h->combine_mode == 1 || queue_combine) ? at<int32_t>(ws, w.arrive) : nullptr;
+    const bool queue_combine = combine_run(h) == 2 && resolved_ffn_mode(h) == MOE_FFN_PERSISTENT;
+    a.arrive = (combine_run(h) == 1 || queue_combine) ? at<int32_t>(ws, w.arrive) : nullptr;
     a.arrive_n = d.S * d.plan.nnt1;
     a.done1 = queue_combine ? at<int32_t>(ws, w.done1) : nullptr;
     a.pair_mt = queue_combine ? at<int32_t>(ws, w.pair_mt) : nullptr;
@@ -375,10 +376,11 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
-// Whether this call's FFN stage runs on bf16 pieces: as two launches, whatever a queue would take.
-bool pieces_run(const moe_handle* h) {
-    return h->d.f32_pieces && h->ffn_mode == MOE_FFN_AUTO && h->combine_mode == 0 && !h->queue_options && !h->task_trace;
-}
+// Whether this call's FFN stage runs on bf16 pieces: as two launches.  Their bits are not those of the fp32 tile, so this is the plan's
+// choice alone -- no option of the queue, way to combine or trace has a say -- but for the mode that only the fp32 tile has.
+bool pieces_run(const moe_handle* h) { return h->d.f32_pieces && h->ffn_mode != MOE_FFN_PERSISTENT; }
+// ... and leave the combine to its own launch.
+int combine_run(const moe_handle* h) { return pieces_run(h) ? 0 : h->combine_mode; }
 int resolved_ffn_mode(const moe_handle* h) {
     if (pieces_run(h)) return MOE_FFN_TILED;
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
@@ -636,7 +638,7 @@ int moe_get_options(const moe_handle* h, moe_options* opt) {
     *opt = h->opt;
     const int kdt = h->d.plan.kernel_dtype;
     // (nor have fp32 layers on bf16 pieces)
-    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && (h->d.plan.tile == kF32StreamTile || h->d.f32_pieces)) opt->f32_tile = MOE_OPT_AUTO;
+    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && (h->d.plan.tile == kF32StreamTile || pieces_run(h))) opt->f32_tile = MOE_OPT_AUTO;
     return MOE_OK;
 }
 

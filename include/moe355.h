@@ -118,7 +118,11 @@ typedef struct moe_options {
     int32_t block_rows;      /* bf16 / fp16 layers: 128 or 256 rows per row block (a coarser way to say tile16 = 0 / 1; 256 needs
                                 H % 256 == 0 and I % 256 == 0, with SwiGLU I % 128 == 0; elsewhere 256 gives the 128x128 tile) */
     int32_t f32_tile;        /* fp32 / tf32 layers: 0 = 64x64 vector-ALU tile, 1 = 128x128 matrix-core tile (AUTO: also the weight
-                                streamer, other bits).  The backward entry points of an fp32 handle use the matrix-core tile,
+                                streamer, and for many rows per expert the bf16 matrix instructions on three bf16 pieces of every
+                                value, in a workspace that is larger by 6 bytes a weight, a token's and 2 an intermediate value; other
+                                bits either of them, no further from the exact result; moe_get_options reports AUTO for both).  Layers
+                                on pieces take two launches and leave the combine to one of its own, whatever the options of the queue,
+                                combine and a task trace say; MOE_FFN_PERSISTENT alone moves them to the 128x128 tile.  The backward entry points of an fp32 handle use the matrix-core tile,
                                 where their shape allows, on a handle whose layer runs on it, and the 64x64 tile on any other
                                 one, the streamer's included (which moe_get_options reports as AUTO) */
     int32_t fp8_tile;        /* e4m3 layers: 0 = weight streamer (decode), 1 = 128x128 tile GEMM */
@@ -133,7 +137,8 @@ typedef struct moe_options {
     int32_t combine;         /* 0 = a launch of its own behind the FFN stage; 1 = inside the FFN kernels, by the workgroup
                                 whose tile completes a token (arrival counters); 2 = as tasks of the FFN queue, taken by
                                 workgroups that find no GEMM task left (task-queue mode only; the rest of the tokens is
-                                combined by a short launch behind it).  All three give the same bits. */
+                                combined by a short launch behind it).  All three give the same bits.  Plans whose kernels leave it to
+                                a launch (fp8_mfma, fp32 on bf16 pieces: f32_tile) do so with every value. */
     int32_t gate_kernel;     /* logits kernel: 0 = register-tiled, 1 = token rows in registers */
     int32_t gate_mfma;       /* 1 = the logits on the matrix cores where the shape allows (16-bit layers, H % 512 == 0), 0 = never */
     int32_t gate_tile;       /* register-tiled logits kernel: 0 = 4x8 pairs per wavefront, 1 = 4x4, 2 = 2x8 */
@@ -228,7 +233,8 @@ typedef struct moe_routing_out {
 int moe_prepared_bytes(const moe_handle* h, size_t* bytes);
 int moe_prepare_weights(moe_handle* h, const moe_weights* w, void* prepared, size_t prepared_bytes, void* stream);
 
-/* Variants of the FFN stage; MOE_FFN_AUTO lets the library choose. */
+/* Variants of the FFN stage; MOE_FFN_AUTO lets the library choose.  They give the same bits, but for fp32 / tf32 layers that run on
+ * bf16 pieces (option f32_tile): those have no task queue, and MOE_FFN_PERSISTENT runs them on the 128x128 fp32 tile as f32_tile = 1 does. */
 enum { MOE_FFN_AUTO = 0, MOE_FFN_TILED = 1 /* one launch per GEMM */, MOE_FFN_PERSISTENT = 2 /* task queue */ };
 int moe_set_ffn_mode(moe_handle* h, int mode);
 /* The variant a forward call on this handle runs (MOE_FFN_TILED or MOE_FFN_PERSISTENT), with AUTO resolved. */
@@ -308,7 +314,8 @@ int moe_get_stage_ms(moe_handle* h, int stage, float* ms, int32_t* calls);
 int moe_get_stage_samples(moe_handle* h, int stage, float* ms, int32_t capacity, int32_t* count);
 
 /* How evenly the task queue of the last moe_forward kept its workgroups busy (task-queue FFN only; MOE_ERR_UNSUPPORTED
- * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers, for single experts and,
+ * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers, for fp32 layers on bf16
+ * pieces (whatever trace and options say; MOE_FFN_PERSISTENT asks for the fp32 tile's queue), for single experts and,
  * in 16-bit layers, for up to about 192 rows per expert (more than 48 where tokens are dropped) and for many rounds of short tasks
  * (where none are dropped): moe_get_ffn_mode tells, moe_set_ffn_mode asks for the queue, and a task trace or an option of the queue
  * -- queue_groups, queue_lag, queue_early, row_chunk, blocks_per_cu, tail_round, combine, tail_split -- with another value than AUTO
@@ -324,7 +331,7 @@ int moe_get_queue_balance(moe_handle* h, const void* workspace, void* stream, in
  * behind the tile (the dependency wait of a down-projection task lies in front of start_us).  The buffer is device
  * memory of the caller (moe_task_trace_bytes(max_tasks) bytes, 8-byte aligned; tasks beyond its capacity are counted
  * but not recorded); it holds the records of the most recent call.  moe_set_task_trace(h, NULL, 0) switches the trace
- * off.  Setting it copies 16 bytes to the device (synchronous; not for the serving loop); moe_get_task_trace copies
+ * off.  A call that runs no queue kernel leaves no records.  Setting it copies 16 bytes to the device (synchronous; not for the serving loop); moe_get_task_trace copies
  * the records back, so it synchronises `stream`; times are microseconds since the earliest recorded start; *count
  * receives the number of records the call left (it may exceed `capacity`).  Cost with the trace on: two clock reads
  * and one atomic per task.  Counterpart in the reference: the clock stamps its kernels print (mma.cuh:51-57,162-169;

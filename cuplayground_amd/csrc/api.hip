@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "moe_internal.hpp"
+#include "f32_pieces_choice.hpp"
 #include "two_launches.hpp"
 
 namespace moe355 {
@@ -97,16 +98,14 @@ int check_supported(const moe_config& c) {
 
 WsLayout layout(const Derived& d);
 
-// Rows per expert from which an fp32 layer on the 128 x 128 matrix-core tile runs on bf16 pieces instead (ffn_f32_pieces.hip): below,
-// making the weights' pieces costs what the products save.  Whole layers, us, fp32 tile / pieces, and their distance (2-norm) from
-// float64: the reference's knob file (8192 rows, one expert of 1024 x 4096) 1053 / 712, 1.0e-6 / 3.7e-7; 2048 rows of it 429 / 385; 8
-// experts of 1024 x 2048, GELU, 512 rows each 561 / 432, 1.1e-6 / 3.6e-7; 16 of 2048 x 2048, 512 rows 1334 / 1256, 1.2e-6 / 4.4e-7; of
-// 2048 x 1408, SwiGLU, 2048 rows 4489 / 2979, 1.4e-6 / 5.0e-7; 8 of 512 x 1024, 2048 rows 440 / 342; 4 of 256 x 512, 4096 rows 184 / 155.
+// An fp32 layer on the 128 x 128 matrix-core tile runs on bf16 pieces instead (ffn_f32_pieces.hip) from this many rows per expert on,
+// where f32_pieces_choice.hpp expects that to be faster and its workspace may grow so far.
 constexpr int64_t kPiecesRowsPerExpert = 512, kPiecesExtraBytes = (int64_t)4 << 30;
-bool f32_pieces_ok(const Derived& d, const moe_options& o) {
+bool f32_pieces_ok(const Derived& d, const moe_options& o, bool drops) {
     if (d.act_dtype != MOE_DTYPE_F32 || d.plan.tile != 1 || o.f32_tile != MOE_OPT_AUTO || d.A < d.E * kPiecesRowsPerExpert) return false;
     const int64_t lim = (int64_t)1 << 32, HI = (int64_t)std::max(d.H, d.I);
     if (HI > 65536 || (int64_t)d.S * d.H * 6 >= lim || (int64_t)d.A * d.I * 6 >= lim || (HI + 256) * 6 * std::min(d.H, d.I) >= lim || (std::min(d.H, d.I) + 256) * 6 * HI >= lim) return false;
+    if (!pieces_pay(PieceShape{d.S, d.A, d.E, d.H, d.I, d.wide_mats == 3, drops ? d.capacity : d.A})) return false;
     // what moe_forward_static took before it takes still, and nobody's workspace grows by more than kPiecesExtraBytes
     Derived with = d;
     with.f32_pieces = true;
@@ -135,7 +134,7 @@ int derive(const moe_config& c, const moe_options& o, Derived* d) {
     d->nblk = ceil_div(d->A, kRouteBlock);
     d->max_mtiles = ceil_div(d->A, d->plan.block_m) + d->E;
     d->f32_pieces = false;
-    d->f32_pieces = f32_pieces_ok(*d, o);
+    d->f32_pieces = f32_pieces_ok(*d, o, c.drop_tokens != 0);
     return MOE_OK;
 }
 

@@ -9,7 +9,9 @@
 // Precision.  Pieces are rounded to nearest, so the second is at most 2^-8 of the first, the third 2^-8 of the second, and either has
 // either sign: the three left-out products are below 2^-22 of a term at the very most, about 2^-27 of it on average, and cancel.  The sums run from the smallest pairs to the largest, so that the pieces'
 // products are added up before the first pieces' raise the rounding error of an addition, and those are added 32 at a time.  Distance
-// from float64 against that of the fp32 instructions: see the rule in api.hip (f32_pieces_ok).
+// from float64 (2-norm), fp32 tile / pieces: the reference's knob file 1.0e-6 / 3.7e-7; 8 experts of 1024 x 2048, GELU, 512 rows each
+// 1.1e-6 / 3.6e-7; 16 of 2048 x 1408, SwiGLU, 2048 rows 1.4e-6 / 5.0e-7; one of 1024 x 2048, ReLU, operands of one sign 7.0e-7 / 2.5e-7, all
+// equal 6.5e-6 / 1.6e-8, of magnitudes spread over 2^40 5.0e-7 / 3.3e-7, tokens with one value that is not zero 5.7e-7 / 2.1e-7.
 // What bounds it: the energy of the bf16 MFMAs on operands whose bits are all random (1.2 PFLOP/s of them, as in a 16-bit layer), so a
 // fp32 product runs at 200 TFLOP/s.  The reference's knob file (8192 rows, one expert of 1024 x 4096, ReLU): up and down projection 577 and
 // 556 us on the fp32 instructions; 339 and 357 here, on 256- and on 128-row blocks (128 tiles of 256 rows, half the chip: 494), behind 27 us
@@ -25,6 +27,7 @@
 // 1885 / 2571.
 #include <algorithm>
 
+#include "f32_pieces_choice.hpp"
 #include "ffn_bf16_tile.hpp"
 #include "grouped_task.hpp"
 
@@ -267,11 +270,7 @@ hipError_t launch_pieces(const PieceArgs& a, int64_t rows, hipStream_t st) {
 }
 template <int EPI, bool UP>
 hipError_t launch_pieces(const PieceArgs& a, int64_t rows, hipStream_t st) {
-    // the row blocks that the estimate of a layer's launches finds faster (two_launches.hpp), the contraction six times as long
-    SplitBlocks n(rows, a.E);
-    if (a.E == 1) n.full = (rows + 127) / 256, n.left = rows > 256 * n.full, n.small = (rows + 127) / 128;      // no two ways about it
-    const double cols = (a.N * (EPI == MOE_ACT_SWIGLU ? 2 : 1) + 255) / 256;
-    const bool large = split_us(n.full * cols, n.left * cols, 6 * a.K) <= split_us(0, n.small * cols, 6 * a.K);
+    const bool large = pieces_large(rows, a.E, (a.N * (EPI == MOE_ACT_SWIGLU ? 2 : 1) + 255) / 256, a.K);
     return large ? launch_pieces<PieceSplit<256>, EPI, UP>(a, rows, st) : launch_pieces<PieceSplit<128>, EPI, UP>(a, rows, st);
 }
 

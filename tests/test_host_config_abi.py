@@ -193,3 +193,16 @@ def test_torch_operator_has_no_cpu_path():
         torch.ops.moe355.forward(x, w, e, None, e, cfg)
     m = torch.ops.moe355.forward(x.to("meta"), w.to("meta"), e.to("meta"), None, e.to("meta"), cfg)
     assert m.shape == x.shape
+
+
+@pytest.mark.parametrize("factor,drop,pieces", [(1.0, 0, True), (1.25, 1, True), (0.5, 1, False), (0.5, 0, True)])
+def test_workspace_of_fp32_layers_that_drop_rows(factor, drop, pieces):
+    """Room for the bf16 pieces of weights and tokens only where the rows that are kept repay making them."""
+    c = moe.MoEConfig(**dict(REFERENCE_JSON, num_experts=8, intermediate_size=2048, hidden_act=1, capacity_factor=factor, drop_tokens=drop)).to_c()
+    size = {}
+    for tile in (-1, 1):
+        n, o = C.c_size_t(0), api.make_options({"f32_tile": tile})
+        assert moe.load_library().moe_workspace_bytes_with_options(C.byref(c), C.byref(o), C.byref(n)) == 0
+        size[tile] = n.value
+    extra = 6 * (8192 * 1024 + 2 * 8 * 2048 * 1024) + 2 * 8192 * 2048
+    assert size[-1] - size[1] == (extra if pieces else 0)

@@ -786,7 +786,7 @@ static bool overlap(const void* a, const void* b, int64_t bytes) {
 // (launch_expert_gemm_dact): no transposed copy of the weight.  16-bit layers.
 int expert_gemm_kn_supported(int64_t A, int E, int N, int K, int dtype, const moe_options& opt) {
     if (dtype == MOE_DTYPE_F32 || !stored_operands_ok(A, N, K)) return 0;
-    return opt.grouped_tile == MOE_OPT_AUTO && grouped_kn_as_stored(A, E, N, K) ? 2 : 1;
+    return opt.grouped_tile == MOE_OPT_AUTO && stored_operands_ok(A, N, K) ? 2 : 1;
 }
 hipError_t launch_expert_gemm_kn(const void* a_rows, const void* w, const void* u_rows, const void* g_rows, const int32_t* count,
                                  const int32_t* offset, int64_t A, int E, int N, int K, int hidden_act, int dtype, void* out_rows, void* out1_rows,

@@ -52,8 +52,8 @@ def test_queue_order_keeps_every_dependency_under_asan_and_ubsan(tmp_path):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("rules", ["two_launches", "product_choice", "f32_pieces_choice"])
 def test_dispatch_rules_under_asan_and_ubsan(tmp_path, rules):
-    """csrc/two_launches.hpp decides which 16-bit layers run as two launches and on which row blocks, csrc/product_choice.hpp whether
-    a training product takes operands as stored; every choice gives the same bits.  csrc/f32_pieces_choice.hpp decides which fp32 layers
+    """csrc/two_launches.hpp decides which 16-bit layers run as two launches and on which row blocks, csrc/product_choice.hpp which
+    tiles a training product takes; every choice gives the same bits.  csrc/f32_pieces_choice.hpp decides which fp32 layers
     run on bf16 pieces.  Their answers on both sides of each line, at
     shapes that were measured both ways, and at the ends of the range."""
     exe = str(tmp_path / rules)

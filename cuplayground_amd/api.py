@@ -263,11 +263,12 @@ def _operand(name, t, dtype, elements=0):
 
 def _stream():
     """The current device's current stream, as torch.cuda.current_stream() gives it, without its Python objects: a training step asks
-    a dozen and a half times (2.7 us each against 0.4)."""
+    a dozen and a half times (2.7 us each against 0.4).  A torch without the two functions is asked for the objects."""
     import torch
     if not torch.cuda.is_initialized():
         torch.cuda.init()
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    return C.c_void_p(raw(device()) if raw and device else torch.cuda.current_stream().cuda_stream)
 
 
 def _torch_act_dtype(torch_dtype: int):

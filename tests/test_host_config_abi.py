@@ -206,3 +206,18 @@ def test_workspace_of_fp32_layers_that_drop_rows(factor, drop, pieces):
         size[tile] = n.value
     extra = 6 * (8192 * 1024 + 2 * 8 * 2048 * 1024) + 2 * 8192 * 2048
     assert size[-1] - size[1] == (extra if pieces else 0)
+
+
+def test_streams_without_the_private_functions_of_torch(monkeypatch):
+    """The current stream's address comes from two functions of torch that are no part of its interface; a torch without them, or with
+    one of them, is asked the documented way."""
+    import torch
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": 0x1230})())
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        with monkeypatch.context() as m:
+            m.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0x4560, raising=False)
+            m.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+            assert api._stream().value == 0x4560
+            m.delattr(torch._C, name)
+            assert api._stream().value == 0x1230

@@ -601,13 +601,21 @@ class MoELayer:
                                          _ptr(expert_offset), N, K, _ptr(out), _ptr(out1), _stream()), "moe_expert_gemm_kn")
         return out if u_rows is None else (out, out1)
 
+    def _rows(self, name, t, columns):
+        """Packed rows of every pair (a product's result is made with as many)."""
+        _operand(name, t, self.act_dtype, self.S * self.k * columns)
+        if t.shape[1] != columns:
+            raise ValueError("%s has rows of %d: expected %d" % (name, t.shape[1], columns))
+
     def expert_gemm_pair(self, a_rows, w0, w1, expert_count, expert_offset):
         """(a_rows[r] . w0[e(r)]^T, a_rows[r] . w1[e(r)]^T), w0 and w1 [E,N,K].  Rows of no expert are not written."""
         import torch
         N, K = w0.shape[1], w0.shape[2]
-        _operand("a_rows", a_rows, self.act_dtype, self.S * self.k * K)
+        self._rows("a_rows", a_rows, K)
         for name, t in (("w0", w0), ("w1", w1)):
             _operand(name, t, self.act_dtype, self.E * N * K)
+        for name, t in (("expert_count", expert_count), ("expert_offset", expert_offset)):
+            _operand(name, t, torch.int32, self.E)
         out = [torch.empty(a_rows.shape[0], N, dtype=a_rows.dtype, device=a_rows.device) for _ in range(2)]
         sc = self.backward_scratch()
         _check(self.L.moe_expert_gemm_pair(self._h, _ptr(a_rows), _ptr(w0), _ptr(w1), _ptr(expert_count), _ptr(expert_offset), N, K, _ptr(out[0]),
@@ -619,7 +627,7 @@ class MoELayer:
         import torch
         K, N = w0.shape[1], w0.shape[2]
         for name, t in (("a0_rows", a0_rows), ("a1_rows", a1_rows)):
-            _operand(name, t, self.act_dtype, self.S * self.k * K)
+            self._rows(name, t, K)
         for name, t in (("w0", w0), ("w1", w1)):
             _operand(name, t, self.act_dtype, self.E * K * N)
         for name, t in (("expert_count", expert_count), ("expert_offset", expert_offset)):

@@ -106,6 +106,43 @@ def test_router_passes_and_stored_weight_products_refuse_operands_they_would_rea
             call()
 
 
+def test_products_that_share_a_launch_refuse_operands_they_would_read_or_write_past(monkeypatch):
+    """Tables, rows and weights of another type, of too few elements or of other columns: refused before the first launch."""
+    layer = api.MoELayer.__new__(api.MoELayer)
+    layer.cfg, layer.S, layer.k, layer.H, layer.E, layer.act_dtype, layer._h = _cfg(), 8, 2, 64, 4, torch.bfloat16, None
+
+    def launched(*a):
+        raise AssertionError("reached the launch")
+    layer.L = type("L", (), dict.fromkeys(("moe_expert_gemm_pair", "moe_expert_gemm_kn_pair", "moe_expert_wgrads"), staticmethod(launched)))
+    monkeypatch.setattr(api.MoELayer, "backward_scratch", lambda self: torch.zeros(16, dtype=torch.uint8))
+    monkeypatch.setattr(api, "_stream", lambda: None)
+    rows, w, count = torch.zeros(16, 64, dtype=torch.bfloat16), torch.zeros(4, 64, 64, dtype=torch.bfloat16), torch.zeros(4, dtype=torch.int32)
+
+    def pair(a=rows, w0=w, w1=w, count=count, offset=count):
+        return lambda: layer.expert_gemm_pair(a, w0, w1, count, offset)
+
+    def kn_pair(a=rows, b=rows, w0=w, w1=w, count=count, offset=count):
+        return lambda: layer.expert_gemm_kn_pair(a, b, w0, w1, count, offset)
+
+    def wgrads(dy=rows, a=rows, count=count, offset=count):
+        return lambda: layer.expert_wgrads([(rows, rows), (dy, a)], count, offset)
+
+    for call in (pair(), kn_pair(), wgrads()):
+        with pytest.raises(AssertionError):
+            call()
+    for f in (pair, kn_pair, wgrads):
+        for call in (f(a=rows.half()), f(count=count.long()), f(offset=count.float())):
+            with pytest.raises(TypeError):
+                call()
+        for call in (f(a=rows[:15]), f(count=count[:3]), f(offset=count[:3])):
+            with pytest.raises(ValueError):
+                call()
+    for f in (pair, kn_pair):
+        for call in (f(w1=w[:3]), f(a=rows.reshape(8, 128))):      # (as many elements, but results of 8 rows where 16 are written)
+            with pytest.raises(ValueError):
+                call()
+
+
 class _RowsLayer:
     """The passes of the expert node as plain torch expressions (one expert, one rank): enough to run the node on the CPU."""
     fused_act_backward = False

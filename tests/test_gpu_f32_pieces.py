@@ -70,6 +70,39 @@ def test_no_further_from_float64_than_the_fp32_tile(moe, name):
     pieces.close(), tile.close()
 
 
+@pytest.mark.parametrize("kind", ["one_sign", "constant", "one_hot", "spread"])
+@pytest.mark.parametrize("act", [0, 2])
+def test_other_distributions_are_no_further_from_float64(moe, act, kind):
+    """Sums of one sign, which an adder that truncates would show; equal terms; single terms, one rounding either way; magnitudes over 2^24."""
+    import torch
+    S, H, I = 4500, 1024, 2048
+    cfg = moe.MoEConfig(capacity_factor=1.0, drop_tokens=0, expert_top_k=1, is_training=0, hidden_act=act, hidden_size=H, intermediate_size=I,
+                        micro_batch=1, num_experts=1, sequence_len=S, torch_dtype=0, gate_fn=0, norm_topk_prob=0)
+    pieces, tile = moe.MoELayer(cfg, options={}), moe.MoELayer(cfg, options={"f32_tile": 1}, ffn_mode=moe.api.FFN_TILED)
+    assert pieces.workspace_bytes > tile.workspace_bytes + 6 * S * H
+    g = torch.Generator(device="cuda").manual_seed(S + act)
+
+    def values(*s, std=1.0):
+        r = torch.randn(*s, generator=g, device="cuda") * std
+        if kind == "spread":
+            r *= torch.exp2(torch.randint(-12, 12, s, generator=g, device="cuda").float())
+        return torch.full_like(r, 1.2345678 * std) if kind == "constant" else r.abs() if kind == "one_sign" else r
+    x = values(S, H)
+    if kind == "one_hot":
+        t = torch.arange(S, device="cuda")
+        x = torch.zeros_like(x).index_put_((t, t % H), x[t, t % H])
+    w = {"gate_w": torch.zeros(1, H, device="cuda"), "w_up": values(1, I, H, std=0.05), "w_down": values(1, H, I, std=0.05)}
+    if act == 2:
+        w["w_gate"] = values(1, I, H, std=0.05)
+    routing = pieces.new_routing()
+    got, other = pieces.forward(x, w, routing=routing), tile.forward(x, w)
+    ref = _float64(cfg, x, w, routing)
+    far = lambda o: ((o.double() - ref).norm() / ref.norm()).item()
+    assert far(got) <= far(other) and not torch.equal(got, other), (far(got), far(other))
+    assert ((got.double() - ref).abs().max() <= (other.double() - ref).abs().max() * 1.5)
+    pieces.close(), tile.close()
+
+
 @pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_huge", "h_huge"])
 @pytest.mark.parametrize("name", ["gelu_bias_drop", "swiglu_bias"])
 def test_values_that_pieces_do_not_hold(moe, name, what):

@@ -34,32 +34,33 @@ PEAK_HBM_GBS = 8000.0         # MI355X HBM3E
 # script (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch), each scaled by what the same counter showed for a 1 GiB
 # device copy in the same run (--calibrate-copy).  Each entry names the summary under profiles/ it comes from and the
 # digest of the kernel sources it was collected with: when the sources have changed since, the figure is withheld.
-BF16_SOURCES = ("ffn_bf16.hip", "ffn_bf16_tile.hpp", "ffn_bf16_slab_steady.inc", "ffn_common.hpp", "route.hip")
-FP8_SOURCES = ("ffn_fp8.hip", "ffn_common.hpp", "route.hip")
+BF16_SOURCES = ("ffn_bf16.hip", "ffn_bf16_tile.hpp", "ffn_bf16_slab.inc", "ffn_bf16_slab_steady.inc", "ffn_common.hpp", "route.hip")
+FP8_SOURCES = ("ffn_fp8.hip", "stream_lines.hpp", "ffn_common.hpp", "route.hip")
 FP8_TILE_SOURCES = ("ffn_fp8_tile.hip", "ffn_common.hpp", "route.hip")
 WIDEN_SOURCES = BF16_SOURCES + ("quant.hip",)
-F32_TILE_SOURCES = ("ffn_f32_tile.hip", "ffn_common.hpp", "route.hip")
+F32_PIECES_SOURCES = ("ffn_f32_pieces.hip", "ffn_bf16_tile.hpp", "ffn_bf16_slab.inc", "ffn_bf16_slab_steady.inc", "ffn_bf16_slab_half.inc", "grouped_task.hpp",
+                      "f32_pieces_choice.hpp", "two_launches.hpp", "ffn_common.hpp", "route.hip")
 FP8_MFMA_SOURCES = FP8_TILE_SOURCES + ("quant.hip",)
 MEASURED_TRAFFIC = {
-    "mixtral": {"bytes": 18.52e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
+    "mixtral": {"bytes": 18.66e9, "sources": BF16_SOURCES, "kernel_digest": "b503db3d00b9",
                 "profile": "profiles/ffn_persistent_kernel_bf16_mixtral_c3_hbm_traffic.txt"},
-    "mid": {"bytes": 0.8063e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
+    "mid": {"bytes": 0.8071e9, "sources": BF16_SOURCES, "kernel_digest": "b503db3d00b9",
             "profile": "profiles/ffn_persistent_kernel_bf16_mid_c2_hbm_traffic.txt"},
-    "finegrained": {"bytes": 3.355e9, "sources": BF16_SOURCES, "kernel_digest": "d7bf5c709d8b",
+    "finegrained": {"bytes": 3.352e9, "sources": BF16_SOURCES, "kernel_digest": "b503db3d00b9",
                     "profile": "profiles/ffn_persistent_kernel_bf16_finegrained_c4_hbm_traffic.txt"},
-    "decode_fp8": {"bytes": 9.907e9, "sources": FP8_SOURCES, "kernel_digest": "db57f455db60",
+    "decode_fp8": {"bytes": 9.685e9, "sources": FP8_SOURCES, "kernel_digest": "9a289dff5a96",
                    "profile": "profiles/ffn_persistent_fp8_kernel_decode_c5_hbm_traffic.txt"},
-    # a single-expert fp32 layer runs as two launches (one per projection); the figure is their sum
-    "reference_default": {"bytes": 0.9174e9, "sources": F32_TILE_SOURCES, "kernel_digest": "18f0fced7a60", "ffn_mode": 1,
-                          "profile": "profiles/ffn_tiled_f32_tile_kernel_reference_default_hbm_traffic.txt"},
+    # fp32 on bf16 pieces: the pass that makes the pieces and a launch per projection; the figure is their sum
+    "reference_default/pieces": {"bytes": 1.81e9, "sources": F32_PIECES_SOURCES, "kernel_digest": "96a8f230a12d", "ffn_mode": 1,
+                                 "profile": "profiles/ffn_tiled_f32_pieces_kernel_reference_default_hbm_traffic.txt"},
     # the widening pass and the bf16 queue kernel together (what the layer's FFN stage launches by default) ...
-    "prefill_fp8": {"bytes": 23.35e9, "sources": WIDEN_SOURCES, "kernel_digest": "1a74032c0fe0",
+    "prefill_fp8": {"bytes": 23.29e9, "sources": WIDEN_SOURCES, "kernel_digest": "930df71c86d1",
                     "profile": "profiles/widen_plus_ffn_persistent_kernel_prefill_fp8_hbm_traffic.txt"},
     # ... the e4m3 tile GEMM on the same layer (option fp8_widen = 0) ...
-    "prefill_fp8/e4m3_tile": {"bytes": 26.44e9, "sources": FP8_TILE_SOURCES, "kernel_digest": "21f3a64c924d",
+    "prefill_fp8/e4m3_tile": {"bytes": 29.91e9, "sources": FP8_TILE_SOURCES, "kernel_digest": "dbe5d179a1db",
                               "profile": "profiles/ffn_persistent_fp8_tile_kernel_prefill_fp8_hbm_traffic.txt"},
     # ... and the e4m3 x e4m3 plan (option fp8_mfma = 1): two quantising passes and two GEMM launches
-    "prefill_fp8/e4m3_mfma": {"bytes": 14.59e9, "sources": FP8_MFMA_SOURCES, "kernel_digest": "3a045167b72d", "ffn_mode": 1,
+    "prefill_fp8/e4m3_mfma": {"bytes": 15e9, "sources": FP8_MFMA_SOURCES, "kernel_digest": "4053f35af63c", "ffn_mode": 1,
                               "profile": "profiles/ffn_tiled_fp8_mfma_kernel_prefill_fp8_hbm_traffic.txt"},
 }
 

@@ -1,5 +1,6 @@
 // Expert FFN in fp32 on the bf16 matrix instructions: every fp32 value as three bf16 pieces that add up to it exactly, the product of
-// two values as the six largest of the nine products of their pieces, each exact in fp32.
+// two values as the six largest of the nine products of their pieces, each exact in fp32 (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype for Higher-Precision Computations", ARITH 2019).
 //
 // v_mfma_f32_32x32x2_f32 multiplies at 157 TFLOP/s, v_mfma_f32_16x16x32_bf16 at 2.5 PFLOP/s: six of the latter for one of the former
 // is 2.6 times the rate.  An operand's row holds its pieces one behind the other, [first | second | third] of K each, and a product
@@ -7,9 +8,9 @@
 // only where a slab's loads begin is different.
 //
 // Precision.  Pieces are rounded to nearest, so the second is at most 2^-8 of the first, the third 2^-8 of the second, and either has
-// either sign: the three left-out products are below 2^-22 of a term at the very most, about 2^-27 of it on average, and cancel.  The sums run from the smallest pairs to the largest, so that the pieces'
-// products are added up before the first pieces' raise the rounding error of an addition, and those are added 32 at a time.  Distance
-// from float64 (2-norm), fp32 tile / pieces: the reference's knob file 1.0e-6 / 3.7e-7; 8 experts of 1024 x 2048, GELU, 512 rows each
+// either sign: the three left-out products are below 2^-22 of a term at the very most, about 2^-27 of it on average, and cancel.
+// The sums run from the smallest pairs to the largest, so that the pieces' products are added up before the first pieces' raise the
+// rounding error of an addition, and those are added 32 at a time.  Distance from float64 (2-norm), fp32 tile / pieces: the reference's knob file 1.0e-6 / 3.7e-7; 8 experts of 1024 x 2048, GELU, 512 rows each
 // 1.1e-6 / 3.6e-7; 16 of 2048 x 1408, SwiGLU, 2048 rows 1.4e-6 / 5.0e-7; one of 1024 x 2048, ReLU, operands of one sign 7.0e-7 / 2.5e-7, all
 // equal 6.5e-6 / 1.6e-8, of magnitudes spread over 2^40 5.0e-7 / 3.3e-7, tokens with one value that is not zero 5.7e-7 / 2.1e-7.
 // What bounds it: the energy of the bf16 MFMAs on operands whose bits are all random (1.2 PFLOP/s of them, as in a 16-bit layer), so a

@@ -385,8 +385,10 @@ hipError_t launch_gate_tiled(const void* x, const void* gate_w, const float* gat
 // A workgroup holds 2 x 2 tiles (32 tokens x 32 experts).  A step's 64 rows of 1 KiB go from memory straight into one of two stages,
 // requested two steps ahead and across the end of a tile too: the workgroups stay, `tiles` of them in steps of the grid.  What bounds
 // it: a SIMD's two wavefronts share the pipe, and the two widening operations an MFMA needs do not run beside fp32 MFMAs (measured on
-// registers: 36 cycles an MFMA without, 48 with them; 64 here).  16384 tokens x 64 experts of 2048, selection included, 83.5 -> 74.5 us
-// against rows fetched into registers, 64 bytes of each of 16 a request, one tile's column of 32 experts a workgroup; 4000 tokens 32.4 -> 23.5.
+// registers: 36 cycles an MFMA without, 48 with them; 64 here).  16384 tokens x 64 experts of 2048 75.6 -> 72.0 us in a trace,
+// against rows fetched into registers, 64 bytes of each of 16 a request, one tile's column of 32 experts a workgroup; with the selection
+// (topk16_kernel) behind it 81 -> 69 us a call, 8192 tokens 42 -> 36, 4000 30.5 -> 22.2; 1024 tokens x 256 of 7168 74 -> 55.  Few tiles, which AUTO
+// leaves to the kernels above, were faster as they were: 1000 tokens x 64 experts 15.4 -> 20.4 with option gate_mfma = 1.
 typedef float gate_f32x16 __attribute__((ext_vector_type(16)));
 
 template <typename T>
@@ -532,9 +534,9 @@ __global__ __launch_bounds__(GateStage<T>::THREADS) __attribute__((amdgpu_waves_
 }
 // The matrix-core kernel takes 16-bit layers whose rows split into full steps of 512 elements, from 150 workgroups' tiles on that the
 // experts fill to three quarters, or where they are many and the experts fill most of 16 columns.  This / the best other kernel, us,
-// selection included, rows of 2048: 64 experts, 2500 tokens (158) 22.4 / 24.3, 2000 (126) 21.0 / 19.8; 32 experts, 8192 tokens (256) 24.7 /
-// 33.7, 4096 (128) 21.2 / 19.5; 24 experts, 16384 (512) 44.8 / 54.3; 128, 4096 (512) 40.9 / 45.7; 256 experts of 7168, 1024 tokens (256)
-// 55.2 / 76.9, 512 (128) 54.2 / 44.7; 16 experts, 8192 tokens (256, half filled) 23.2 / 22.6, 32768 73.4 / 74.0, 12 of 1024 49.8 / 53.4.
+// selection included, rows of 2048: 64 experts, 2500 tokens (158) 21.0 / 22.7, 2000 (126) 20.5 / 19.2; 32 experts, 8192 tokens (256) 20.8 /
+// 28.2, 4096 (128) 18.4 / 16.5; 24 experts, 16384 (512) 36.3 / 46.7; 128, 4096 (512) 34.8 / 49.3; 256 experts of 7168, 1024 tokens (256)
+// 55.2 / 75.1, 512 (128) 54.0 / 44.8; 16 experts, 8192 tokens (256, half filled) 20.0 / 20.1, 32768 64.5 / 68.5.
 // (The selection in the same launch, where a workgroup holds every expert: 27.5 against 24.7 us with 32 experts and 8192 tokens.)
 template <typename T>
 bool launch_gate_mfma(const void* x, const void* gate_w, const float* gate_bias, float* logits, int S, int H, int E, int opt_mfma, hipStream_t st, hipError_t* err) {
@@ -566,8 +568,8 @@ __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ log
 // The same for up to 64 experts, sixteen lanes to a token: lane l of a row of sixteen keeps the logits of experts l, l + 16, l + 32 and
 // l + 48, so that a candidate travels through four DPP moves instead of four and three lane reads, and a wavefront selects for four tokens
 // at a time.  The softmax's sum pairs the experts as the wavefront's butterfly does (e with e + 32, then + 16 in the lane, 8, 4, 2, 1
-// between them): the same bits.  64 experts, k 6, logits included, a token a wavefront / this: 16384 tokens 79 / 69 us, 8192 43 / 39, 4000
-// 24.0 / 22.5, up to 1000 no difference.
+// between them): the same bits.  16384 tokens x 64 experts, k 6, a token a wavefront / this 17.2 / 8.4 us in a trace
+// (profiles/layer_bf16_finegrained_kernel_trace.txt).
 struct Cand16 {
     float key, v;
     int i;

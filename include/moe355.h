@@ -142,8 +142,9 @@ typedef struct moe_options {
     int32_t gate_kernel;     /* logits kernel: 0 = register-tiled, 1 = token rows in registers */
     int32_t gate_mfma;       /* 1 = the logits on the matrix cores where the shape allows (16-bit layers, H % 512 == 0), 0 = never */
     int32_t gate_tile;       /* register-tiled logits kernel: 0 = 4x8 pairs per wavefront, 1 = 4x4, 2 = 2x8 */
-    int32_t gate_fused_topk; /* 1 = top-k inside the logits kernel where one exists for the shape (no logits round trip
-                                through memory unless the caller asks for them), 0 = always a launch of its own */
+    int32_t gate_fused_topk; /* 1 = top-k inside the logits kernel where the one that runs holds a token's logits (the register-tiled
+                                one; no logits round trip through memory unless the caller asks for them), 0 = always a launch of its
+                                own.  The matrix-core kernel (gate_mfma) leaves it to a launch with either. */
     int32_t grouped_tile;    /* moe_expert_gemm on a 16-bit handle: 0 = 128x128, 1 = 256x256, 2 = 128x256; with any of them
                                 moe_expert_wgrad works on transposed copies of the rows, never on the rows as stored */
     int32_t tail_round;      /* task-queue mode: 1 (and AUTO) = the last up-projection segment of the queue is placed so that the

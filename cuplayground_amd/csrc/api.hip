@@ -69,7 +69,7 @@ struct Derived {
     int64_t capacity;
     FfnPlan plan;
     int nblk;          // workgroups of the slot-assignment kernels
-    bool f32_pieces;   // fp32 layer that runs on bf16 pieces unless the task queue is asked for
+    bool f32_pieces;   // fp32 layer that runs on bf16 pieces
     int wide_mats;     // weight matrices per expert (3 with SwiGLU, else 2)
     int max_mtiles;
 };
@@ -323,7 +323,6 @@ template <typename T>
 T* at(void* ws, size_t off) { return reinterpret_cast<T*>(static_cast<char*>(ws) + off); }
 
 int resolved_ffn_mode(const moe_handle* h);
-int combine_run(const moe_handle* h);
 
 RouteArgs route_args(const moe_handle* h, void* ws) {
     const Derived& d = h->d;
@@ -346,8 +345,8 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
     // arrival counters [S, nnt1] of the combine inside the FFN kernels, or the flags [S * slices] of the combine tasks of
     // the queue (a slice is at least 1024 columns, a column tile at most 256: the flags fit the same array); the latter
     // exist in task-queue mode only
-    const bool queue_combine = combine_run(h) == 2 && resolved_ffn_mode(h) == MOE_FFN_PERSISTENT;
-    a.arrive = (combine_run(h) == 1 || queue_combine) ? at<int32_t>(ws, w.arrive) : nullptr;
+    const bool queue_combine = h->combine_mode == 2 && resolved_ffn_mode(h) == MOE_FFN_PERSISTENT;
+    a.arrive = (h->combine_mode == 1 || queue_combine) ? at<int32_t>(ws, w.arrive) : nullptr;
     a.arrive_n = d.S * d.plan.nnt1;
     a.done1 = queue_combine ? at<int32_t>(ws, w.done1) : nullptr;
     a.pair_mt = queue_combine ? at<int32_t>(ws, w.pair_mt) : nullptr;
@@ -375,13 +374,10 @@ RouteArgs route_args(const moe_handle* h, void* ws) {
 // The mode a forward call runs in.  The queue pays off once there are more tasks than resident workgroups; tiny
 // layers launch once per projection.  Row blocks are estimated on the host as the larger of kept rows / block rows
 // and the experts that can be hit at all (every hit expert owns at least one row block).
-// Whether this call's FFN stage runs on bf16 pieces: as two launches.  Their bits are not those of the fp32 tile, so this is the plan's
-// choice alone -- no option of the queue, way to combine or trace has a say -- but for the mode that only the fp32 tile has.
-bool pieces_run(const moe_handle* h) { return h->d.f32_pieces && h->ffn_mode != MOE_FFN_PERSISTENT; }
-// ... and leave the combine to its own launch.
-int combine_run(const moe_handle* h) { return pieces_run(h) ? 0 : h->combine_mode; }
 int resolved_ffn_mode(const moe_handle* h) {
-    if (pieces_run(h)) return MOE_FFN_TILED;
+    // fp32 on bf16 pieces: two launches, whatever mode, option of the queue or trace is set -- its bits are not those of the fp32 tile, which
+    // has the queue, so that no schedule may choose between them
+    if (h->d.f32_pieces) return MOE_FFN_TILED;
     // the e4m3 x e4m3 plan quantises the intermediate rows between the projections: always one launch per projection
     if (h->d.plan.mfma8) return MOE_FFN_TILED;
     if (h->ffn_mode != MOE_FFN_AUTO) return h->ffn_mode;
@@ -596,7 +592,7 @@ int moe_create_with_options(const moe_config* cfg, const moe_options* opt, moe_h
     // +18 %, decode +0.9 %): the workgroup that completes a token holds a whole compute unit while it gathers k rows
     // at memory latency, where the separate launch does the same gather with the whole chip's occupancy in 8-38 us.
     h->combine_mode = opt->combine == MOE_OPT_AUTO ? 0 : opt->combine;
-    if (d.plan.mfma8) h->combine_mode = 0;                // that plan's kernels leave the combine to its own launch
+    if (d.plan.mfma8 || d.f32_pieces) h->combine_mode = 0;      // those plans' kernels leave the combine to its own launch
     h->spin_limit = kDefaultSpinLimit;
     h->task_trace = nullptr;
     h->task_trace_cap = 0;
@@ -637,7 +633,7 @@ int moe_get_options(const moe_handle* h, moe_options* opt) {
     *opt = h->opt;
     const int kdt = h->d.plan.kernel_dtype;
     // (nor have fp32 layers on bf16 pieces)
-    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && (h->d.plan.tile == kF32StreamTile || pieces_run(h))) opt->f32_tile = MOE_OPT_AUTO;
+    if ((kdt == MOE_DTYPE_F32 || kdt == MOE_DTYPE_TF32) && (h->d.plan.tile == kF32StreamTile || h->d.f32_pieces)) opt->f32_tile = MOE_OPT_AUTO;
     return MOE_OK;
 }
 
@@ -911,7 +907,7 @@ int forward_on(moe_handle* h, const void* x, const moe_weights* w, void* out, co
         for (int i = 0; i < d.wide_mats; ++i) *dst[i] = wide + (size_t)i * d.E * d.I * d.H * 2;
         fa.s_up = fa.s_gate = fa.s_down = nullptr;
     }
-    if (pieces_run(h)) {
+    if (d.f32_pieces) {
         e = launch_ffn_f32_pieces(fa, ExpertRows{ra.expert_count, ra.expert_offset}, at<char>(workspace, L.x_pieces), at<char>(workspace, L.w_pieces), fa.h,
                                   ra.q->inexact, d.max_mtiles, d.plan.nnt0, d.plan.nnt1, st);
     } else if (d.plan.mfma8) {

@@ -121,8 +121,8 @@ typedef struct moe_options {
                                 streamer, and for many rows per expert the bf16 matrix instructions on three bf16 pieces of every
                                 value, in a workspace that is larger by 6 bytes a weight, a token's and 2 an intermediate value; other
                                 bits either of them, no further from the exact result; moe_get_options reports AUTO for both).  Layers
-                                on pieces take two launches and leave the combine to one of its own, whatever the options of the queue,
-                                combine and a task trace say; MOE_FFN_PERSISTENT alone moves them to the 128x128 tile.  The backward entry points of an fp32 handle use the matrix-core tile,
+                                on pieces take two launches and leave the combine to one of its own, whatever moe_set_ffn_mode, combine,
+                                the options of the queue and a task trace ask for: the queue is the 128x128 tile's.  The backward entry points of an fp32 handle use the matrix-core tile,
                                 where their shape allows, on a handle whose layer runs on it, and the 64x64 tile on any other
                                 one, the streamer's included (which moe_get_options reports as AUTO) */
     int32_t fp8_tile;        /* e4m3 layers: 0 = weight streamer (decode), 1 = 128x128 tile GEMM */
@@ -234,8 +234,8 @@ typedef struct moe_routing_out {
 int moe_prepared_bytes(const moe_handle* h, size_t* bytes);
 int moe_prepare_weights(moe_handle* h, const moe_weights* w, void* prepared, size_t prepared_bytes, void* stream);
 
-/* Variants of the FFN stage; MOE_FFN_AUTO lets the library choose.  They give the same bits, but for fp32 / tf32 layers that run on
- * bf16 pieces (option f32_tile): those have no task queue, and MOE_FFN_PERSISTENT runs them on the 128x128 fp32 tile as f32_tile = 1 does. */
+/* Variants of the FFN stage; MOE_FFN_AUTO lets the library choose.  They give the same bits.  Plans without a task queue (fp8_mfma, fp32 on
+ * bf16 pieces: f32_tile) take a launch per GEMM in every mode. */
 enum { MOE_FFN_AUTO = 0, MOE_FFN_TILED = 1 /* one launch per GEMM */, MOE_FFN_PERSISTENT = 2 /* task queue */ };
 int moe_set_ffn_mode(moe_handle* h, int mode);
 /* The variant a forward call on this handle runs (MOE_FFN_TILED or MOE_FFN_PERSISTENT), with AUTO resolved. */
@@ -316,7 +316,7 @@ int moe_get_stage_samples(moe_handle* h, int stage, float* ms, int32_t capacity,
 
 /* How evenly the task queue of the last moe_forward kept its workgroups busy (task-queue FFN only; MOE_ERR_UNSUPPORTED
  * in the two-launch mode, which MOE_FFN_AUTO also means for the weight streamers of 16- and 32-bit layers, for fp32 layers on bf16
- * pieces (whatever trace and options say; MOE_FFN_PERSISTENT asks for the fp32 tile's queue), for single experts and,
+ * pieces (in every mode: f32_tile = 1 has the queue), for single experts and,
  * in 16-bit layers, for up to about 192 rows per expert (more than 48 where tokens are dropped) and for many rounds of short tasks
  * (where none are dropped): moe_get_ffn_mode tells, moe_set_ffn_mode asks for the queue, and a task trace or an option of the queue
  * -- queue_groups, queue_lag, queue_early, row_chunk, blocks_per_cu, tail_round, combine, tail_split -- with another value than AUTO

@@ -199,27 +199,27 @@ def test_smallest_and_largest_magnitudes_that_pieces_hold(moe):
 
 
 def test_schedules_options_and_traces_change_no_bits(moe):
-    """The arithmetic is the plan's: two launches asked for by name, every way to combine, options of the queue and a trace leave a layer
-    on pieces.  Asking for the task queue gives the fp32 tile, in the options that are reported as in the bits."""
+    """The arithmetic is the plan's: every mode and way to combine, options of the queue and a trace leave a layer on pieces, and its two
+    launches; the options that a handle reports make another like it."""
     import torch
     api = moe.api
     cfg, pieces, tile, x, w = _layers(moe, "gelu_bias_drop")
-    want, fp32 = pieces.forward(x, w), tile.forward(x, w)
-    assert not torch.equal(want, fp32) and pieces.options["f32_tile"] == -1 and pieces.ffn_mode == api.FFN_TILED
+    want = pieces.forward(x, w)
+    assert not torch.equal(want, tile.forward(x, w)) and tile.options["f32_tile"] == 1
     for options in ({}, {"combine": 0}, {"combine": 1}, {"combine": 2}, {"tail_round": 0}, {"row_chunk": 3}, {"queue_groups": 8}, {"queue_lag": 1}, {"blocks_per_cu": 1}):
-        for mode in (api.FFN_AUTO, api.FFN_TILED):
+        for mode in (api.FFN_AUTO, api.FFN_TILED, api.FFN_PERSISTENT):
             layer = moe.MoELayer(cfg, options=options, ffn_mode=mode)
             assert torch.equal(layer.forward(x, w), want) and layer.options["f32_tile"] == -1 and layer.ffn_mode == api.FFN_TILED, (options, mode)
-            layer.close()
+            same = moe.MoELayer(cfg, options=layer.options, ffn_mode=layer.ffn_mode)
+            assert torch.equal(same.forward(x, w), want)
+            layer.close(), same.close()
     traced = moe.MoELayer(cfg, options={})
     traced.enable_task_trace(1 << 14)
     assert torch.equal(traced.forward(x, w), want) and len(traced.task_trace()) == 0
-    traced.set_ffn_mode(api.FFN_PERSISTENT)
-    assert traced.ffn_mode == api.FFN_PERSISTENT and traced.options["f32_tile"] == 1
-    assert torch.equal(traced.forward(x, w), fp32) and len(traced.task_trace()) > 0 and traced.queue_balance()["span_us"] > 0
-    same = moe.MoELayer(cfg, options=traced.options, ffn_mode=traced.ffn_mode)
-    assert torch.equal(same.forward(x, w), fp32)
-    for l in (pieces, tile, traced, same):
+    queue = moe.MoELayer(cfg, options={"f32_tile": 1}, ffn_mode=api.FFN_PERSISTENT)      # where the queue, its reports and traces are
+    queue.enable_task_trace(1 << 14)
+    assert torch.equal(queue.forward(x, w), tile.forward(x, w)) and len(queue.task_trace()) > 0 and queue.queue_balance()["span_us"] > 0
+    for l in (pieces, tile, traced, queue):
         l.close()
 
 

@@ -51,7 +51,7 @@ MEASURED_TRAFFIC = {
     "decode_fp8": {"bytes": 9.685e9, "sources": FP8_SOURCES, "kernel_digest": "9a289dff5a96",
                    "profile": "profiles/ffn_persistent_fp8_kernel_decode_c5_hbm_traffic.txt"},
     # fp32 on bf16 pieces: the pass that makes the pieces and a launch per projection; the figure is their sum
-    "reference_default/pieces": {"bytes": 1.81e9, "sources": F32_PIECES_SOURCES, "kernel_digest": "96a8f230a12d", "ffn_mode": 1,
+    "reference_default/pieces": {"bytes": 1.81e9, "sources": F32_PIECES_SOURCES, "kernel_digest": "0e48e285d658", "ffn_mode": 1,
                                  "profile": "profiles/ffn_tiled_f32_pieces_kernel_reference_default_hbm_traffic.txt"},
     # the widening pass and the bf16 queue kernel together (what the layer's FFN stage launches by default) ...
     "prefill_fp8": {"bytes": 23.29e9, "sources": WIDEN_SOURCES, "kernel_digest": "930df71c86d1",

@@ -13,9 +13,9 @@
 // rounding error of an addition, and those are added 32 at a time.  Distance from float64 (2-norm), fp32 tile / pieces: the reference's knob file 1.0e-6 / 3.7e-7; 8 experts of 1024 x 2048, GELU, 512 rows each
 // 1.1e-6 / 3.6e-7; 16 of 2048 x 1408, SwiGLU, 2048 rows 1.4e-6 / 5.0e-7; one of 1024 x 2048, ReLU, operands of one sign 7.0e-7 / 2.5e-7, all
 // equal 6.5e-6 / 1.6e-8, of magnitudes spread over 2^40 5.0e-7 / 3.3e-7, tokens with one value that is not zero 5.7e-7 / 2.1e-7.
-// What bounds it: the energy of the bf16 MFMAs on operands whose bits are all random (1.2 PFLOP/s of them, as in a 16-bit layer), so a
-// fp32 product runs at 200 TFLOP/s.  The reference's knob file (8192 rows, one expert of 1024 x 4096, ReLU): up and down projection 577 and
-// 556 us on the fp32 instructions; 339 and 357 here, on 256- and on 128-row blocks (128 tiles of 256 rows, half the chip: 494), behind 27 us
+// What bounds it: the energy of the bf16 MFMAs on operands whose bits are all random (1.25 PFLOP/s of them, as in a 16-bit layer), so a
+// fp32 product runs at 208 TFLOP/s.  The reference's knob file (8192 rows, one expert of 1024 x 4096, ReLU): up and down projection 577 and
+// 556 us on the fp32 instructions; 331 and 329 here, on 256- and on 128-row blocks (128 tiles of 256 rows, half the chip: 494), behind 27 us
 // for the pieces of tokens and weights at 6.2 TB/s.
 // Values are multiplied by 2^24 before they are taken apart, so that the lowest bit of any fp32 number, denormal ones included, is a
 // normal bf16 number, and neither the pieces nor the products that matter of small values (2^-62 times 2^-62, say) fall below the
